@@ -126,8 +126,9 @@ def build_oracle() -> str:
 
 
 def build_reference(ref_root: str = "/root/reference"):
-    """Compile the reference Fortran (checker only) when its sources exist."""
-    if not os.path.isdir(ref_root):
+    """Compile the reference Fortran (checker only) when its sources exist
+    (an empty mount point holds none)."""
+    if not os.path.isfile(os.path.join(ref_root, "lib", "step3.f")):
         return None
     _run(["make", "-s", "-C", os.path.join(ROOT, "oracle", "ref"), f"REF={ref_root}"])
     # the timing build of the same sources (the CPU baseline's reference kind)
