@@ -67,13 +67,14 @@ __device__ __forceinline__ float sqrtT<float>(float x) { return __builtin_amdgcn
 template <bool RF>
 __device__ __forceinline__ double rcp1(double x)
 {
-    if constexpr (RF) {
-        const double r = __builtin_amdgcn_rcp(x);
-        return fma(r, fma(-x, r, 1.0), r);
-    } else {
-        return 1.0 / x;
-    }
+    double r = __builtin_amdgcn_rcp(x);
+    r = fma(r, fma(-x, r, 1.0), r);
+    if constexpr (!RF) r = fma(r, fma(-x, r, 1.0), r);
+    return r;
 }
+// 1/x of the limiters' clamped Courant numbers and 1 + r (normal range)
+__device__ __forceinline__ double rcpL(double x) { return rcp1<false>(x); }
+__device__ __forceinline__ float rcpL(float x) { return __builtin_amdgcn_rcpf(x); }
 template <bool RF>
 __device__ __forceinline__ double sqrt1(double x)
 {
@@ -90,11 +91,39 @@ __device__ __forceinline__ double sqrt1(double x)
     }
 }
 
+// Square root s and its reciprocal i of x > 0 together, from one hardware
+// reciprocal square root and Newton-Goldschmidt steps (one for the FP32
+// form; in FP64 two, and a last residual step for the root).
+template <bool RF>
+__device__ __forceinline__ void root_rcp(double x, double &s, double &i)
+{
+    const double y = __builtin_amdgcn_rsq(x);
+    double g = x * y, h = 0.5 * y;
+    double r = fma(-g, h, 0.5);
+    g = fma(g, r, g);
+    h = fma(h, r, h);
+    if constexpr (!RF) {
+        r = fma(-g, h, 0.5);
+        g = fma(g, r, g);
+        h = fma(h, r, h);
+        g = fma(fma(-g, g, x), h, g);
+    }
+    s = g;
+    i = h + h;
+}
+
 // flang's MIN/MAX: a < b ? a : b, a > b ? a : b
 template <typename T>
 __device__ __forceinline__ T fminF(T a, T b) { return a < b ? a : b; }
 template <typename T>
 __device__ __forceinline__ T fmaxF(T a, T b) { return a > b ? a : b; }
+
+// MIN/MAX in one instruction, where neither operand is NaN in a state that
+// goes on (the limiters' and splits' own)
+__device__ __forceinline__ double fminT(double a, double b) { return __builtin_fmin(a, b); }
+__device__ __forceinline__ double fmaxT(double a, double b) { return __builtin_fmax(a, b); }
+__device__ __forceinline__ float fminT(float a, float b) { return __builtin_fminf(a, b); }
+__device__ __forceinline__ float fmaxT(float a, float b) { return __builtin_fmaxf(a, b); }
 
 // x**y for 0 <= x < 1, y > 0 (suppow's rfrac**pp): the library pow in FP64;
 // in the FP32 form 2**(y log2 x) from the hardware's exp2 and log2
@@ -104,6 +133,66 @@ __device__ __forceinline__ float powT(float x, float y)
 {
     return __builtin_amdgcn_exp2f(y * __builtin_amdgcn_logf(x));
 }
+
+// 1 - x**p for 0 <= x <= 1, p > 0 (suppow's 1 - rfrac**pp).  FP64: ln x from
+// the odd series of ln((1+s)/(1-s)) with x = m 2**k, sqrt(1/2) <= m <
+// sqrt(2), s = (m-1)/(m+1), and -expm1(p ln x) from the Taylor series of the
+// exponential on [-ln 2 / 2, ln 2 / 2]; both series run until the next term is
+// below 2**-54 of the sum, and ln x and p ln x keep their rounding errors.
+// Largest error over 2e7 arguments: 0.74 units of 2**-53, as
+// 1 - pow(x, p) has (0.75).  The limiter needs none of the
+// library function's special cases.
+__device__ __forceinline__ double one_minus_pow(double x, double p)
+{
+    int k;
+    double m = __builtin_frexp(fmaxT(x, 1e-300), &k);   // [1/2, 1); x = 0: the power is 0 either way
+    const bool low = m < 0.70710678118654752;
+    m = low ? m + m : m;
+    const double kd = (double)(low ? k - 1 : k);
+    const double f = m - 1.0, g = m + 1.0;
+    double i = __builtin_amdgcn_rcp(g);
+    i = fma(i, fma(-g, i, 1.0), i);
+    i = fma(i, fma(-g, i, 1.0), i);
+    // (m-1)/(m+1) = s + sl (m - (g - 1): what rounding m + 1 left out)
+    const double s = f * i, sl = fma(-s, m - (g - 1.0), fma(-s, g, f)) * i;
+    const double z = s * s;
+    double h = 1.0 / 21.0;
+    h = fma(h, z, 1.0 / 19.0);
+    h = fma(h, z, 1.0 / 17.0);
+    h = fma(h, z, 1.0 / 15.0);
+    h = fma(h, z, 1.0 / 13.0);
+    h = fma(h, z, 1.0 / 11.0);
+    h = fma(h, z, 1.0 / 9.0);
+    h = fma(h, z, 1.0 / 7.0);
+    h = fma(h, z, 1.0 / 5.0);
+    h = fma(h, z, 1.0 / 3.0);
+    // ln x = hi + lo; ln 2 in two parts, the first with 33 significant bits,
+    // so that kd times it is exact
+    const double s2 = s + s;
+    const double ln2h = 0x1.62e42fefp-1, ln2l = 0x1.473de6af278edp-34;
+    const double A = kd * ln2h, hi = A + s2;
+    const double lo = fma(s2 * z, h, fma(kd, ln2l, (s2 - (hi - A)) + (sl + sl)));
+    const double pc = fminT(p, 4000.0);
+    const double L = fmaxT(pc * hi, -60.0), Ll = fma(pc, hi, -(pc * hi)) + pc * lo;   // the power is below 2**-53 beyond -60
+    const double n = rint((L + Ll) * 1.4426950408889634);
+    const double r = fma(-n, ln2h, L) + fma(-n, ln2l, Ll);
+    double e = 1.0 / 6227020800.0;
+    e = fma(e, r, 1.0 / 479001600.0);
+    e = fma(e, r, 1.0 / 39916800.0);
+    e = fma(e, r, 1.0 / 3628800.0);
+    e = fma(e, r, 1.0 / 362880.0);
+    e = fma(e, r, 1.0 / 40320.0);
+    e = fma(e, r, 1.0 / 5040.0);
+    e = fma(e, r, 1.0 / 720.0);
+    e = fma(e, r, 1.0 / 120.0);
+    e = fma(e, r, 1.0 / 24.0);
+    e = fma(e, r, 1.0 / 6.0);
+    e = fma(e, r, 0.5);
+    const double em1 = fma(e, r * r, r);
+    const double sc = __builtin_ldexp(1.0, (int)n);
+    return fma(-sc, em1, 1.0 - sc);
+}
+__device__ __forceinline__ float one_minus_pow(float x, float p) { return 1.0f - powT(x, p); }
 
 // rpn3euX.f:686-705
 template <typename T>
@@ -144,6 +233,47 @@ __device__ __forceinline__ T suppow(T r, T cfl, T cflup)
     T rfrac = fabs((T(1.0) - rabs) * rcpT(T(1.0) + rabs));
     T signum = fmaxF(T(0.0), copysign(T(1.0), r));
     return signum * (s3 + s2 * r) * (T(1.0) - powT(rfrac, pp));
+}
+
+// The limiters of one interface's waves that move at one speed: with the
+// clamped Courant number e, the reciprocals of e and 1 - e are taken once.
+template <typename T>
+struct LimT {
+    T e, i1mc, icfl;
+    __device__ __forceinline__ explicit LimT(T cfl)
+        : e(fmaxT(T(0.001), fminT(T(0.999), cfl))), i1mc(rcpL(T(1.0) - e)), icfl(rcpL(e)) {}
+    // weight of the upwind interface's Courant number (rpn3euX.f:693)
+    __device__ __forceinline__ T weight(T cflup) const
+    {
+        return (T(1.0) - fmaxT(T(0.001), fminT(T(0.999), cflup))) * i1mc;
+    }
+    // cflsupbee, rpn3euX.f:686-705
+    __device__ __forceinline__ T bee(T theta, T beta, T r, T weight) const
+    {
+        const T s1 = theta * weight * T(2.0) * icfl;
+        const T s2 = (T(1.0) + e) * (T(1.0) / T(3.0));
+        const T ultra = fmaxT(T(0.0), fminT(s1 * r, theta * T(2.0) * i1mc));
+        const T c1 = T(1.0) + (s2 - beta / T(2.0)) * (r - T(1.0));
+        const T c2 = T(1.0) + (s2 + beta / T(2.0)) * (r - T(1.0));
+        return fmaxT(T(0.0), fminT(ultra, fmaxT(c1, c2)));
+    }
+};
+
+// suppow (rpn3euX.f:709-731) with the interface's own Courant number as the
+// upwind one (its weight is then 1), so that each branch of the exponent
+// needs one reciprocal; zero for a ratio that is not positive.
+template <typename T>
+__device__ __forceinline__ T suppow1(T r, T cfl)
+{
+    const T big = sizeof(T) == 4 ? T(1e30) : T(1e300);
+    r = r > big ? big : r;   // a ratio beyond it: (1-r)/(1+r) is 1 to rounding and the limiter 0
+    const T e = fmaxT(T(0.001), fminT(T(0.999), cfl));
+    const T s2 = (T(1.0) + e) * (T(1.0) / T(3.0)), s3 = T(1.0) - s2;
+    const bool lo = r <= T(1.0);
+    const T pp = T(4.0) * (lo ? s3 : s2) * rcpL(lo ? e : T(1.0) - e);
+    const T rfrac = fabs((T(1.0) - r) * rcpL(T(1.0) + r));
+    const T y = (s3 + s2 * r) * one_minus_pow(rfrac, pp);
+    return r <= T(0.0) ? T(0.0) : y;
 }
 
 // Transverse split of a flux difference by the Roe eigensystem of the
@@ -191,26 +321,73 @@ __device__ __forceinline__ void tsplit(const RoeT<T> &R, const T (&in)[NC], T (&
     }
 }
 
-// The split of components M0 .. M0+G-1 alone.  A tracer's split involves
-// only its own component and the contact speed (the v or w of the
-// interface), so a group of tracers (M0 >= 5) is split without the Euler
-// components; M0 = 0 is the split above.
-template <int M0, int G, int ICOOR, bool QUIRK, typename T>
-__device__ __forceinline__ void tsplit_group(const RoeT<T> &R, const T (&in)[G], T (&bm)[G], T (&bp)[G])
-{
-    if constexpr (M0 == 0) {
-        tsplit<G, ICOOR, QUIRK>(R, in, bm, bp);
-    } else {
-        static_assert(M0 >= 5, "a group without the Euler components holds tracers only");
-        const T s = ICOOR == 2 ? R.v : R.w;
-        const T m2 = fminF(s, T(0.0)), p2 = fmaxF(s, T(0.0));
-#pragma unroll
-        for (int m = 0; m < G; m++) {
-            bm[m] = m2 * in[m];
-            bp[m] = p2 * in[m];
-        }
+// A vector of the transverse splits in variables relative to the Roe
+// velocity, scaled so that the splits need the fewest operations: entropy
+// s = rho - p, pressure p (divided by a^2) and the momenta n, a, b along the
+// normal and the two transverse directions, less rho times the Roe velocity.
+// An acoustic wave of strength x along the normal is p = x, n = -+ a x; the
+// contact wave is s; the shear waves are a and b.
+template <typename T>
+struct WaveT {
+    T s, p, n, a, b;
+    __device__ __forceinline__ WaveT() {}
+    __device__ __forceinline__ WaveT(T x1, T x4, T xa, T xb, T x5, T snd)
+        : s(x4), p(x1 + x5), n(snd * (x5 - x1)), a(xa), b(xb) {}
+    __device__ __forceinline__ void add(const WaveT &o) { s += o.s; p += o.p; n += o.n; a += o.a; b += o.b; }
+    // k e - (lo + hi): the middle one of three splits that sum to k e
+    __device__ __forceinline__ static WaveT middle(const WaveT &lo, const WaveT &hi, T k, const WaveT &e)
+    {
+        WaveT o;
+        o.s = k * e.s - (lo.s + hi.s);
+        o.p = k * e.p - (lo.p + hi.p);
+        o.n = k * e.n - (lo.n + hi.n);
+        o.a = k * e.a - (lo.a + hi.a);
+        o.b = k * e.b - (lo.b + hi.b);
+        return o;
     }
-}
+};
+
+// The three speeds of a transverse direction (half of u - c and u + c: a
+// split halves the acoustic parts) and the splits with the weights
+// -min(speed, 0), -|speed| and max(speed, 0) (R = 0, 1, 2).
+template <typename T>
+struct SpeedT {
+    T h1, h2, h3;
+    __device__ __forceinline__ SpeedT(T v, T snd) : h1(T(0.5) * (v - snd)), h2(v), h3(T(0.5) * (v + snd)) {}
+    template <int R>
+    __device__ __forceinline__ static T weight(T x)
+    {
+        return R == 0 ? -fminT(x, T(0.0)) : R == 1 ? -fabs(x) : fmaxT(x, T(0.0));
+    }
+    __device__ __forceinline__ T w2(int r) const { return r == 0 ? weight<0>(h2) : r == 1 ? weight<1>(h2) : weight<2>(h2); }
+    // (normal, other, split) momenta of x -> split along this direction
+    template <int R>
+    __device__ __forceinline__ void split(const WaveT<T> &x, T along, T snd, T isnd, T &p, T &al, T &s) const
+    {
+        const T y1 = weight<R>(h1) * (x.p - along * isnd), y3 = weight<R>(h3) * (x.p + along * isnd);
+        p = y1 + y3;
+        al = snd * (y3 - y1);
+        s = weight<R>(h2) * x.s;
+    }
+    template <int R>
+    __device__ __forceinline__ WaveT<T> split_a(const WaveT<T> &x, T snd, T isnd) const
+    {
+        WaveT<T> o;
+        split<R>(x, x.a, snd, isnd, o.p, o.a, o.s);
+        o.n = weight<R>(h2) * x.n;
+        o.b = weight<R>(h2) * x.b;
+        return o;
+    }
+    template <int R>
+    __device__ __forceinline__ WaveT<T> split_b(const WaveT<T> &x, T snd, T isnd) const
+    {
+        WaveT<T> o;
+        split<R>(x, x.b, snd, isnd, o.p, o.b, o.s);
+        o.n = weight<R>(h2) * x.n;
+        o.a = weight<R>(h2) * x.a;
+        return o;
+    }
+};
 
 // Accumulators D[da+1][db+1][m] of the increments a cell receives, for the
 // target cell offset (da, db) in the (g, h) plane (step3.f:189-226).

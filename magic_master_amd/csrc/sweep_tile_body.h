@@ -68,15 +68,6 @@ constexpr bool tile_flush_atomic() { return sizeof(T) == 8; }
 __device__ __forceinline__ void add_noret(gptr<double> p, double v) { (void)__builtin_amdgcn_global_atomic_fadd_f64(p, v); }
 __device__ __forceinline__ void add_noret(gptr<float> p, float v) { (void)__builtin_amdgcn_global_atomic_fadd_f32(p, v); }
 
-// The Roe state the limiters use: the FP64 form's own; the FP32 form's FP64
-// copy from its solve.
-template <typename T>
-__device__ __forceinline__ const RoeT<double> &limiter_roe(const RoeT<T> &R, const RoeT<double> &RD)
-{
-    if constexpr (sizeof(T) == 8) return R;
-    else return RD;
-}
-
 template <typename AT>
 __device__ __forceinline__ void report_t(const AT &A, int code, int i, int pg, int ph)
 {
@@ -122,15 +113,16 @@ __device__ __forceinline__ void tile_sweep_body(const SweepArgsT<T> &A, int a_is
     const int pg = a_is_g ? a : b, ph = a_is_g ? b : a;   // (g, h) coordinates
     const long long pbase = (long long)(a + A.mbc - 1) * A.sA + (long long)(b + A.mbc - 1) * A.sB;
     const T dtdn = T(A.dtdn);
-    const T cg = T(A.fg), ch = T(A.fh);
     const T d = dtdn;
+    const T ca = T(a_is_g ? A.fg : A.fh), cb2 = T(a_is_g ? A.fh : A.fg);   // dt/da, dt/db
     const gptr<const T> qold = to_global(A.qold);
     const gptr<T> qnew = to_global(A.qnew);
     const gptr<const double> gam = to_global(A.gam), vgrav = to_global(A.vgrav);
     const gptr<const double> crho = to_global(A.crho), cE = to_global(A.cE), cgam = to_global(A.cgam),
                              cvg = to_global(A.cvg), cres = to_global(A.cres);
-    const T k6g = (T(1.0) / T(6.0)) * d * ch;
-    const T k6h = (T(1.0) / T(6.0)) * d * cg;
+    // plane of each tile component: (rho, m_n, m_a, m_b, E, tracers)
+    const int pl2 = a_is_g ? A.comp[2] : A.comp[3], pl3 = a_is_g ? A.comp[3] : A.comp[2];
+    auto plane = [&](int m) { return (long long)(m == 2 ? pl2 : m == 3 ? pl3 : A.comp[m]) * A.P; };
 
     // T index: (m, db, a offset ai, cell ci); the fastest index follows memory
     auto tix = [&](int m, int db, int ai, int ci) {
@@ -176,20 +168,22 @@ __device__ __forceinline__ void tile_sweep_body(const SweepArgsT<T> &A, int a_is
         // chunk's barrier after part 1.
 
         // ---------------- part 1: Roe solve of interface I (rpn3euX.f:138-421)
-        RoeT<T> R = {0, 0, 0, 0, 1, 0, 0, 0, 0};
-        T fw1[NC], fw2[NC], fw3[NC], amdq[NC], apdq[NC];
-        T s1 = 0, s2 = 0, s3 = 0, c1 = 0, c2 = 0, c3 = 0;
+        // The waves stay in their strengths (b1, b5 acoustic, b4 entropy, b2
+        // and b3 shear; W: the same as the solve's FP64 values); the f-wave
+        // vectors of rpn3euX.f:217-271 are never formed.  al1, al5 and lf:
+        // the left-going parts of waves 1, 3 and 2 (rpn3euX.f:311-399).
+        // The solve runs in FP64 in both forms (see rcp1 in magic_solver.h).
+        RoeT<double> R = {0, 0, 0, 0, 1, 0, 0, 0, 0};
+        double b1 = 0, b2 = 0, b3 = 0, b4 = 0, b5 = 0, al1 = 0, al5 = 0;
+        double s1 = 0, s2 = 0, s3 = 0;
+        bool lf = false;
+        T trw[NTR > 0 ? NTR : 1];   // unlimited tracer waves
+        T c1 = 0, c2 = 0, c3 = 0;
         bool f1 = false, f2 = false, f5 = false;
-#pragma unroll
-        for (int m = 0; m < NC; m++) { fw1[m] = fw2[m] = fw3[m] = amdq[m] = apdq[m] = T(0.0); }
-        // The solve runs in FP64 in both forms (T1 = double): the FP64 form
-        // writes its results in place; the FP32 form solves into FP64
-        // arrays and rounds the results (see rcp1 in magic_solver.h).
-        auto riemann = [&](auto &RR, auto &F1, auto &F2, auto &F3, auto &AM, auto &AP, auto &W) {
-            using T1 = double;
+        if (act1) {
             constexpr bool RF = sizeof(T) == 4;
-            T1 qa[NC], qb[NC], vgc = T1(0.0);
-            T1 ga, gb;
+            double qa[NC], qb[NC], vgc = 0.0;
+            double ga, gb;
             if constexpr (PREFETCH) {
 #pragma unroll
                 for (int m = 0; m < NC; m++) {
@@ -216,7 +210,7 @@ __device__ __forceinline__ void tile_sweep_body(const SweepArgsT<T> &A, int a_is
             // perturbation form: q holds q - background; the background is a
             // column at rest (rho_bar(k), E_bar(k), gamma(k)), so the full
             // states differ from q only in rho and E
-            T1 rpa = 0, rpb = 0, ppa = 0, ppb = 0;
+            double rpa = 0, rpb = 0, ppa = 0, ppb = 0;
             int kib = 0;
             if constexpr (PERT) {
                 const int ka = A.sweep == 3 ? I - 1 : b, kb = A.sweep == 3 ? I : b;
@@ -226,492 +220,362 @@ __device__ __forceinline__ void tile_sweep_body(const SweepArgsT<T> &A, int a_is
                 gb = cgam[kib];
                 rpa = qa[0];
                 rpb = qb[0];
-                const T1 epa = qa[4], epb = qb[4];
+                const double epa = qa[4], epb = qb[4];
                 qa[0] = crho[kia] + rpa;
                 qb[0] = crho[kib] + rpb;
                 qa[4] = cE[kia] + epa;
                 qb[4] = cE[kib] + epb;
-                // p - p_bar = (gamma-1) (E' - kinetic energy), p_bar = (gamma-1) E_bar
-                ppa = (ga - T1(1.0)) * (epa - T1(0.5) * (qa[1] * qa[1] + qa[2] * qa[2] + qa[3] * qa[3]) / qa[0]);
-                ppb = (gb - T1(1.0)) * (epb - T1(0.5) * (qb[1] * qb[1] + qb[2] * qb[2] + qb[3] * qb[3]) / qb[0]);
+                ppa = epa;
+                ppb = epb;
             }
-            if (!(qa[0] > T1(0.0)) || !(qb[0] > T1(0.0))) report_t(A, 1, I, pg, ph);
-            const T1 rhsqrtl = sqrt1<RF>(qa[0]), rhsqrtr = sqrt1<RF>(qb[0]);
-            const T1 rhsq2 = rhsqrtl + rhsqrtr;
-            // reciprocals taken once where rpn3euX.f:159-216 divides by the
-            // same value several times (the products differ from the
-            // quotients by at most one rounding)
-            const T1 il = rcp1<RF>(rhsqrtl), ir = rcp1<RF>(rhsqrtr), i2 = rcp1<RF>(rhsq2);
-            const T1 iqa = rcp1<RF>(qa[0]), iqb = rcp1<RF>(qb[0]);
-            const T1 gamma = (rhsqrtr * gb + rhsqrtl * ga) * i2;
-            const T1 gamma1 = gamma - T1(1.0);
-            const T1 pl = pressure_nc(ga, qa[4], qa[1], qa[2], qa[3], iqa);
-            const T1 pr = pressure_nc(gb, qb[4], qb[1], qb[2], qb[3], iqb);
-            RR.u = (qa[1] * il + qb[1] * ir) * i2;
-            RR.v = (qa[2] * il + qb[2] * ir) * i2;
-            RR.w = (qa[3] * il + qb[3] * ir) * i2;
-            RR.enth = ((qa[4] + pl) * il + (qb[4] + pr) * ir) * i2;
-            RR.u2v2w2 = RR.u * RR.u + RR.v * RR.v + RR.w * RR.w;
-            const T1 a2 = gamma1 * (RR.enth - T1(0.5) * RR.u2v2w2);
-            if (!(a2 > T1(0.0))) report_t(A, 2, I, pg, ph);
-            RR.a = sqrt1<RF>(a2);
-            RR.i2a = rcp1<RF>(T1(2.0) * RR.a);
-            RR.g1a2 = gamma1 / a2;
-            RR.euv = RR.enth - RR.u2v2w2;
-            const T1 ur = qb[1] * iqb, ul = qa[1] * iqa;
-            const T1 d1 = qb[1] - qa[1];
-            T1 d2;
+            if (!(qa[0] > 0.0) || !(qb[0] > 0.0)) report_t(A, 1, I, pg, ph);
+            // square root, its reciprocal and the reciprocal of both densities
+            double rhsqrtl, il, iqa, rhsqrtr, ir, iqb;
+            root_rcp<RF>(qa[0], rhsqrtl, il);
+            root_rcp<RF>(qb[0], rhsqrtr, ir);
+            iqa = rcp1<RF>(qa[0]);
+            iqb = rcp1<RF>(qb[0]);
+            const double i2 = rcp1<RF>(rhsqrtl + rhsqrtr);
+            const double gamma = (rhsqrtr * gb + rhsqrtl * ga) * i2;
+            const double gamma1 = gamma - 1.0;
+            if constexpr (PERT) {
+                // p - p_bar = (gamma-1) (E' - kinetic energy), p_bar = (gamma-1) E_bar
+                ppa = (ga - 1.0) * (ppa - 0.5 * (qa[1] * qa[1] + qa[2] * qa[2] + qa[3] * qa[3]) * iqa);
+                ppb = (gb - 1.0) * (ppb - 0.5 * (qb[1] * qb[1] + qb[2] * qb[2] + qb[3] * qb[3]) * iqb);
+            }
+            const double pl = pressure_nc(ga, qa[4], qa[1], qa[2], qa[3], iqa);
+            const double pr = pressure_nc(gb, qb[4], qb[1], qb[2], qb[3], iqb);
+            R.u = (qa[1] * il + qb[1] * ir) * i2;
+            R.v = (qa[2] * il + qb[2] * ir) * i2;
+            R.w = (qa[3] * il + qb[3] * ir) * i2;
+            R.enth = ((qa[4] + pl) * il + (qb[4] + pr) * ir) * i2;
+            R.u2v2w2 = R.u * R.u + R.v * R.v + R.w * R.w;
+            const double a2 = gamma1 * (R.enth - 0.5 * R.u2v2w2);
+            if (!(a2 > 0.0)) report_t(A, 2, I, pg, ph);
+            double ia;
+            root_rcp<RF>(a2, R.a, ia);
+            R.i2a = 0.5 * ia;
+            R.g1a2 = gamma1 * (ia * ia);
+            R.euv = R.enth - R.u2v2w2;
+            const double ur = qb[1] * iqb, ul = qa[1] * iqa;
+            const double d1 = qb[1] - qa[1];
+            double d2;
             if constexpr (PERT) d2 = (qb[1] * ur + ppb) - (qa[1] * ul + ppa);   // background part below
             else d2 = flux_jump_nc(qb[1], ur, pr, qa[1], ul, pl);
-            const T1 d3 = ur * qb[2] - ul * qa[2];
-            const T1 d4 = ur * qb[3] - ul * qa[3];
-            T1 d5 = (qb[4] + pr) * ur - (qa[4] + pl) * ul;
+            const double d3 = ur * qb[2] - ul * qa[2];
+            const double d4 = ur * qb[3] - ul * qa[3];
+            double d5 = (qb[4] + pr) * ur - (qa[4] + pl) * ul;
             if (A.gravity) {
                 if constexpr (PERT) {
                     // the background's own jump p_bar_b - p_bar_a - .5 (rho_bar_a +
                     // rho_bar_b) aux17 is the column residual (zero to FP64 rounding)
-                    const T1 vg = cvg[kib];
-                    d2 = d2 - T1(0.5) * (rpb + rpa) * vg + cres[kib];
-                    d5 = d5 - T1(0.5) * (qb[1] + qa[1]) * vg;
+                    const double vg = cvg[kib];
+                    d2 = d2 - 0.5 * (rpb + rpa) * vg + cres[kib];
+                    d5 = d5 - 0.5 * (qb[1] + qa[1]) * vg;
                 } else {
-                    const T1 vg = vgc;
-                    d2 = gravity_jump_nc(d2, qa[0], qb[0], vg);
-                    d5 = d5 - T1(0.5) * (qb[1] + qa[1]) * vg;
+                    d2 = gravity_jump_nc(d2, qa[0], qb[0], vgc);
+                    d5 = d5 - 0.5 * (qb[1] + qa[1]) * vgc;
                 }
             }
-            const T1 b4 = RR.g1a2 * (RR.euv * d1 + RR.u * d2 + RR.v * d3 + RR.w * d4 - d5);
-            const T1 b2 = d3 - RR.v * d1;
-            const T1 b3 = d4 - RR.w * d1;
-            const T1 b5 = (d2 + (RR.a - RR.u) * d1 - RR.a * b4) * RR.i2a;
-            const T1 b1 = d1 - b4 - b5;
-            F1[0] = b1; F1[1] = b1 * (RR.u - RR.a); F1[2] = b1 * RR.v; F1[3] = b1 * RR.w;
-            F1[4] = b1 * (RR.enth - RR.u * RR.a);
-            s1 = RR.u - RR.a;
-            F2[0] = b4; F2[1] = b4 * RR.u; F2[2] = b2 + b4 * RR.v; F2[3] = b3 + b4 * RR.w;
-            F2[4] = b2 * RR.v + b3 * RR.w + b4 * T1(0.5) * RR.u2v2w2;
-            s2 = RR.u;
-            F3[0] = b5; F3[1] = b5 * (RR.u + RR.a); F3[2] = b5 * RR.v; F3[3] = b5 * RR.w;
-            F3[4] = b5 * (RR.enth + RR.u * RR.a);
-            s3 = RR.u + RR.a;
+            b4 = R.g1a2 * (R.euv * d1 + R.u * d2 + R.v * d3 + R.w * d4 - d5);
+            b2 = d3 - R.v * d1;
+            b3 = d4 - R.w * d1;
+            b5 = (d2 + (R.a - R.u) * d1 - R.a * b4) * R.i2a;
+            b1 = d1 - b4 - b5;
+            s1 = R.u - R.a;
+            s2 = R.u;
+            s3 = R.u + R.a;
 #pragma unroll
-            for (int m = 5; m < NC; m++)
-                F2[m] = (m - 4 <= A.nspecadv) ? s2 * (qb[m] - qa[m]) : ur * qb[m] - ul * qa[m];
-            // entropy fix and amdq: rpn3euX.f:316-398
+            for (int k = 0; k < NTR; k++)
+                trw[k] = (T)((k + 1 <= A.nspecadv) ? s2 * (qb[5 + k] - qa[5 + k]) : ur * qb[5 + k] - ul * qa[5 + k]);
+            // Entropy fix (rpn3euX.f:316-398).  The signs of the speeds it
+            // compares, u -+ c of a state with c**2 = gamma p/rho, are taken
+            // from u**2 against c**2 with the intermediate states scaled by
+            // the wave speed, without their square roots and reciprocals;
+            // those are formed only in a transonic wave.
             {
-                const T1 gmm = ga, gm1 = ga - T1(1.0);
-                const T1 pim1 = gm1 * (qa[4] - T1(0.5) * (qa[1] * qa[1] + qa[2] * qa[2] + qa[3] * qa[3]) * iqa);
-                const T1 cim1 = sqrt1<RF>(gmm * pim1 * iqa);
-                const T1 s0 = qa[1] * iqa - cim1;
-                if (!(s0 >= T1(0.0) && s1 > T1(0.0))) {
-                    const T1 is1 = rcp1<RF>(s1);
-                    const T1 rho1 = qa[0] + F1[0] * is1;
-                    const T1 rhou1 = qa[1] + F1[1] * is1;
-                    const T1 rhov1 = qa[2] + F1[2] * is1;
-                    const T1 rhow1 = qa[3] + F1[3] * is1;
-                    const T1 en1 = qa[4] + F1[4] * is1;
-                    const T1 ir1 = rcp1<RF>(rho1);
-                    const T1 p1 = gm1 * (en1 - T1(0.5) * (rhou1 * rhou1 + rhov1 * rhov1 + rhow1 * rhow1) * ir1);
-                    const T1 cc1 = sqrt1<RF>(gmm * p1 * ir1);
-                    const T1 sa = rhou1 * ir1 - cc1;
-                    T1 sfract;
-                    if (s0 < T1(0.0) && sa > T1(0.0)) sfract = s0 * (sa - s1) / (sa - s0);
-                    else if (s1 < T1(0.0)) sfract = s1;
-                    else sfract = T1(0.0);
-#pragma unroll
-                    for (int m = 0; m < NC; m++) AM[m] = sfract * F1[m] * is1;
-                    if (s2 < T1(0.0)) {
-#pragma unroll
-                        for (int m = 0; m < NC; m++) AM[m] = AM[m] + F2[m];
-                        const T1 gm = gb, g1 = gb - T1(1.0);
-                        const T1 pi_ = g1 * (qb[4] - T1(0.5) * (qb[1] * qb[1] + qb[2] * qb[2] + qb[3] * qb[3]) * iqb);
-                        const T1 ci = sqrt1<RF>(gm * pi_ * iqb);
-                        const T1 s3r = qb[1] * iqb + ci;
-                        const T1 is3 = rcp1<RF>(s3);
-                        const T1 rho2 = qb[0] - F3[0] * is3;
-                        const T1 rhou2 = qb[1] - F3[1] * is3;
-                        const T1 rhov2 = qb[2] - F3[2] * is3;
-                        const T1 rhow2 = qb[3] - F3[3] * is3;
-                        const T1 en2 = qb[4] - F3[4] * is3;
-                        const T1 ir2 = rcp1<RF>(rho2);
-                        const T1 p2 = g1 * (en2 - T1(0.5) * (rhou2 * rhou2 + rhov2 * rhov2 + rhow2 * rhow2) * ir2);
-                        const T1 cc2 = sqrt1<RF>(gm * p2 * ir2);
-                        const T1 sb = rhou2 * ir2 + cc2;
-                        bool add = true;
-                        if (sb < T1(0.0) && s3r > T1(0.0)) sfract = sb * (s3r - s3) / (s3r - sb);
-                        else if (s3 < T1(0.0)) sfract = s3;
-                        else add = false;
-                        if (add) {
-#pragma unroll
-                            for (int m = 0; m < NC; m++) AM[m] = AM[m] + sfract * F3[m] * is3;
-                        }
+                const double cca = ga * pl * qa[0];   // (rho c)**2
+                const bool super = pl >= 0.0 && qa[1] >= 0.0 && qa[1] * qa[1] >= cca && s1 > 0.0;
+                // state behind wave 1, times s1
+                const double r1 = qa[0] * s1 + b1, m1 = qa[1] * s1 + b1 * s1;
+                const double m2 = qa[2] * s1 + b1 * R.v, m3 = qa[3] * s1 + b1 * R.w;
+                const double e1 = qa[4] * s1 + b1 * (R.enth - R.u * R.a);
+                const double cc1 = ga * (ga - 1.0) * (e1 * r1 - 0.5 * (m1 * m1 + m2 * m2 + m3 * m3));
+                al1 = s1 < 0.0 ? b1 : 0.0;
+                if (m1 * s1 > 0.0 && m1 * m1 > cc1 && !(qa[1] >= 0.0 && qa[1] * qa[1] >= cca)) {
+                    const double s0 = ul - sqrt1<RF>(ga * pl * iqa);
+                    const double sa = m1 / r1 - sqrt1<RF>(cc1) / fabs(r1);
+                    if (s0 < 0.0 && sa > 0.0) al1 = s0 * (sa - s1) / (sa - s0) / s1 * b1;
+                }
+                if (super) al1 = 0.0;
+                lf = s2 < 0.0 && !super;
+                if (lf) {
+                    const double ccb = gb * pr * qb[0];
+                    // state ahead of wave 3, times s3
+                    const double r2 = qb[0] * s3 - b5, n1 = qb[1] * s3 - b5 * s3;
+                    const double n2 = qb[2] * s3 - b5 * R.v, n3 = qb[3] * s3 - b5 * R.w;
+                    const double e2 = qb[4] * s3 - b5 * (R.enth + R.u * R.a);
+                    const double cc2 = gb * (gb - 1.0) * (e2 * r2 - 0.5 * (n1 * n1 + n2 * n2 + n3 * n3));
+                    al5 = s3 < 0.0 ? b5 : 0.0;
+                    if (n1 * s3 < 0.0 && n1 * n1 > cc2 && !(qb[1] <= 0.0 && qb[1] * qb[1] >= ccb)) {
+                        const double sr = ur + sqrt1<RF>(gb * pr * iqb);
+                        const double sb = n1 / r2 + sqrt1<RF>(cc2) / fabs(r2);
+                        if (sb < 0.0 && sr > 0.0) al5 = sb * (sr - s3) / (sr - sb) / s3 * b5;
                     }
                 }
             }
-#pragma unroll
-            for (int m = 0; m < NC; m++) AP[m] = ((T1(0.0) + F1[m]) + F2[m]) + F3[m] - AM[m];
-            c1 = fabs(s1 * dtdn); c2 = fabs(s2 * dtdn); c3 = fabs(s3 * dtdn);
-            const T1 b2r = F2[2] - b4 * RR.v;
-            f1 = b1 != T1(0.0); f2 = b2r != T1(0.0); f5 = b5 != T1(0.0);
-            W[0] = b1; W[1] = b2r; W[2] = F2[3] - b4 * RR.w; W[3] = b4; W[4] = b5;
+            c1 = fabs((T)s1 * dtdn); c2 = fabs((T)s2 * dtdn); c3 = fabs((T)s3 * dtdn);
+            f1 = b1 != 0.0; f2 = b2 != 0.0; f5 = b5 != 0.0;
             s_del[0][t] = d1; s_del[1][t] = d2; s_del[2][t] = d3; s_del[3][t] = d4; s_del[4][t] = d5;
-            s_s2[t] = s2;
+            s_s2[t] = (T)s2;
 #pragma unroll
-            for (int k = 0; k < NTR; k++) s_trw[k][t] = F2[5 + k];
+            for (int k = 0; k < NTR; k++) s_trw[k][t] = trw[k];
             s_flag[t] = (act2 && (f1 || f2 || f5)) ? 1 : 0;
             s_cfo[t] = f5 ? c3 : (f2 ? c2 : c1);
-        };
-        // FP32 form: the solve's FP64 Roe state and wave strengths (b1 .. b5),
-        // kept for the limiters' Lax-Liu ratios, whose upwind wave strengths
-        // cancel as the solve's do
-        RoeT<double> RD = {0, 0, 0, 0, 1, 0, 0, 0, 0};
-        double WB[5] = {0.0, 0.0, 0.0, 0.0, 0.0};
-        if (act1) {
-            if constexpr (sizeof(T) == 8) {
-                riemann(R, fw1, fw2, fw3, amdq, apdq, WB);
-            } else {
-                RoeT<double> &RR = RD;
-                // zero as the FP32 arrays above: the solve leaves the tracer
-                // entries of waves 1 and 3 at zero
-                double F1[NC], F2[NC], F3[NC], AM[NC], AP[NC];
-#pragma unroll
-                for (int m = 0; m < NC; m++) F1[m] = F2[m] = F3[m] = AM[m] = AP[m] = 0.0;
-                riemann(RR, F1, F2, F3, AM, AP, WB);
-#pragma unroll
-                for (int m = 0; m < NC; m++) {
-                    fw1[m] = (T)F1[m]; fw2[m] = (T)F2[m]; fw3[m] = (T)F3[m];
-                    amdq[m] = (T)AM[m]; apdq[m] = (T)AP[m];
-                }
-                R = {(T)RR.u, (T)RR.v, (T)RR.w, (T)RR.enth, (T)RR.a, (T)RR.g1a2, (T)RR.euv, (T)RR.u2v2w2, (T)RR.i2a};
-            }
         } else {
             s_flag[t] = 0;
         }
         __syncthreads();
 
-        // ---------------- part 2: limiters and cqxx (rpn3euX.f:434-676, flux3fw.f:270-284)
-        T cqxx[NC];
-#pragma unroll
-        for (int m = 0; m < NC; m++) cqxx[m] = T(0.0);
+        // ---------------- part 2: limiters (rpn3euX.f:434-676) and the strengths
+        // of the second-order correction (flux3fw.f:270-284).  From here on the
+        // transverse directions are the tile axis a and the coloured axis b.
+        T un = 0, ua = 0, ub = 0, snd = 1, isnd = 1, kin = 0, hk = 0;   // Roe state: kin = |u|^2/2, hk = H - kin
+        T x1 = 0, x4 = 0, xa = 0, xb = 0, x5 = 0, l1 = 0, l5 = 0;       // strengths, left-going acoustic parts
+        T q1 = 0, q4 = 0, qsa = 0, qsb = 0, q5 = 0;                     // strengths of cqxx
+        T trq[NTR > 0 ? NTR : 1];
+        T nrm[2][5];   // FP32 form: the cell's own normal update
         if (act2) {
+            const T ts1 = (T)s1, ts2 = (T)s2, ts3 = (T)s3;
+            const T k1 = T(0.5) * copysign(T(1.0), ts1) * (T(1.0) - fabs(ts1) * dtdn);
+            const T k2 = T(0.5) * copysign(T(1.0), ts2) * (T(1.0) - fabs(ts2) * dtdn);
+            const T k3 = T(0.5) * copysign(T(1.0), ts3) * (T(1.0) - fabs(ts3) * dtdn);
+            const int up1 = signbit(s1) ? t + nb : t - nb, up2 = signbit(s2) ? t + nb : t - nb,
+                      up3 = signbit(s3) ? t + nb : t - nb;
+            const LimT<T> lim2(c2);
 #pragma unroll
             for (int k = 0; k < NTR; k++) {
-                const T fc = fw2[5 + k];
+                const T fc = trw[k];
+                T wl = T(0.0);
                 if (fc != T(0.0)) {
-                    const T r = (s2 > T(0.0)) ? s_trw[k][t - nb] / fc : s_trw[k][t + nb] / fc;
-                    T wl;
-                    if (k + 1 <= A.nspecadv) {
-                        const int up = (int)(-copysign(T(1.0), s2));      // Id(2,i) - i
-                        wl = cflsupbee(T(0.5), beta, r, c2, fabs(s_s2[t + up * nb] * dtdn));
-                    } else {
-                        wl = fmaxF(T(0.0), fminF(T(1.0), r));
-                    }
-                    fw2[5 + k] = wl * fc;
+                    const T r = s_trw[k][s2 > 0.0 ? t - nb : t + nb] / fc;
+                    if (k + 1 <= A.nspecadv) wl = lim2.bee(T(0.5), beta, r, lim2.weight(fabs(s_s2[up2] * dtdn)));
+                    else wl = fmaxF(T(0.0), fminF(T(1.0), r));
                 }
+                trq[k] = k2 * (wl * fc);
             }
-            // wave strengths and ratios in FP64 (TL); the limiter functions
-            // in the form's type
-            using TL = double;
-            const RoeT<double> &RL = limiter_roe(R, RD);
-            TL b1, b2, b3, b4, b5;
-            if constexpr (sizeof(T) == 8) {
-                b1 = fw1[0];
-                b4 = fw2[0];
-                b2 = fw2[2] - b4 * R.v;
-                b3 = fw2[3] - b4 * R.w;
-                b5 = fw3[0];
-            } else {
-                b1 = WB[0]; b2 = WB[1]; b3 = WB[2]; b4 = WB[3]; b5 = WB[4];
-            }
+            // the upwind interfaces' strengths in this interface's waves: those
+            // of wave 2 come from one of the two acoustic waves' sides
+            double g1 = 0, g2 = 0, g3 = 0, g4 = 0, g5 = 0;
             T wl1 = T(1.0), wl2 = T(1.0), wl3 = T(1.0), wl4 = T(1.0), wl5 = T(1.0);
-            auto del = [&](int k, int up) { return s_del[k][t + up * nb]; };
-            if (b1 != TL(0.0)) {
-                const int up = (int)(-copysign(T(1.0), s1));
-                const TL b4Id = RL.g1a2 * (RL.euv * del(0, up) + RL.u * del(1, up) + RL.v * del(2, up) +
-                                           RL.w * del(3, up) - del(4, up));
-                const TL b5Id = (del(1, up) + (RL.a - RL.u) * del(0, up) - RL.a * b4Id) * RL.i2a;
-                const TL b1Id = del(0, up) - b4Id - b5Id;
-                wl1 = suppow((T)(b1Id / b1), c1, c1);
-            }
-            if (b2 != TL(0.0)) {
-                const int up = (int)(-copysign(T(1.0), s2));
-                const TL b2Id = del(2, up) - RL.v * del(0, up);
-                wl2 = cflsupbee(T(1.0), beta, (T)(b2Id / b2), c2, c2);
-            }
-            if (b3 != TL(0.0) || b4 != TL(0.0)) {
-                T cflup;
-                if (f2) cflup = c2;
-                else if (f1) cflup = c1;
-                else {
-                    cflup = s_cprev[pa];
-                    for (int j = c - 1; j >= 1; j--)
-                        if (s_flag[t - (c - j) * nb]) { cflup = s_cfo[t - (c - j) * nb]; break; }
+            if (b1 != 0.0 || b2 != 0.0 || b3 != 0.0 || b4 != 0.0 || b5 != 0.0) {
+                auto b4of = [&](int e) {
+                    return R.g1a2 * (R.euv * s_del[0][e] + R.u * s_del[1][e] + R.v * s_del[2][e] + R.w * s_del[3][e] -
+                                     s_del[4][e]);
+                };
+                auto b5of = [&](int e, double b4e) {
+                    return (s_del[1][e] + (R.a - R.u) * s_del[0][e] - R.a * b4e) * R.i2a;
+                };
+                const double b4l = b4of(up1), b4r = b4of(up3);
+                g1 = s_del[0][up1] - b4l - b5of(up1, b4l);
+                g5 = b5of(up3, b4r);
+                g4 = up2 == up1 ? b4l : b4r;
+                g2 = s_del[2][up2] - R.v * s_del[0][up2];
+                g3 = s_del[3][up2] - R.w * s_del[0][up2];
+                if (f1 || f5) {
+                    const T r1 = (T)(g1 / b1), r5 = (T)(g5 / b5);
+                    const T p1 = suppow1(r1, c1), p5 = suppow1(r5, c3);
+                    wl1 = f1 ? p1 : T(1.0);
+                    wl5 = f5 ? p5 : T(1.0);
                 }
-                const int up = (int)(-copysign(T(1.0), s2));
-                if (b3 != TL(0.0)) {
-                    const TL b3Id = del(3, up) - RL.w * del(0, up);
-                    wl3 = cflsupbee(T(1.0), beta, (T)(b3Id / b3), c2, cflup);
-                }
-                if (b4 != TL(0.0)) {
-                    const TL b4Id = RL.g1a2 * (RL.euv * del(0, up) + RL.u * del(1, up) + RL.v * del(2, up) +
-                                               RL.w * del(3, up) - del(4, up));
-                    wl4 = cflsupbee(T(1.0), beta, (T)(b4Id / b4), c2, cflup);
+                if (f2 || b3 != 0.0 || b4 != 0.0) {
+                    T wt = T(1.0);   // the upwind Courant number's weight: 1 where it is c2 itself
+                    if (!f2 && (b3 != 0.0 || b4 != 0.0)) {
+                        T cflup;
+                        if (f1) cflup = c1;
+                        else {
+                            cflup = s_cprev[pa];
+                            for (int j = c - 1; j >= 1; j--)
+                                if (s_flag[t - (c - j) * nb]) { cflup = s_cfo[t - (c - j) * nb]; break; }
+                        }
+                        wt = lim2.weight(cflup);
+                    }
+                    const T r2 = (T)(g2 / b2), r3 = (T)(g3 / b3), r4 = (T)(g4 / b4);
+                    const T p2 = lim2.bee(T(1.0), beta, r2, T(1.0)), p3 = lim2.bee(T(1.0), beta, r3, wt),
+                            p4 = lim2.bee(T(1.0), beta, r4, wt);
+                    wl2 = f2 ? p2 : T(1.0);
+                    wl3 = b3 != 0.0 ? p3 : T(1.0);
+                    wl4 = b4 != 0.0 ? p4 : T(1.0);
                 }
             }
-            if (b5 != TL(0.0)) {
-                const int up = (int)(-copysign(T(1.0), s3));
-                const TL b4Id = RL.g1a2 * (RL.euv * del(0, up) + RL.u * del(1, up) + RL.v * del(2, up) +
-                                           RL.w * del(3, up) - del(4, up));
-                const TL b5Id = (del(1, up) + (RL.a - RL.u) * del(0, up) - RL.a * b4Id) * RL.i2a;
-                wl5 = suppow((T)(b5Id / b5), c3, c3);
-            }
+            // strengths of cqxx, in FP64 up to here
+            const double w1 = (double)(k1 * wl1) * b1, w2 = (double)(k2 * wl2) * b2, w3 = (double)(k2 * wl3) * b3,
+                         w4 = (double)(k2 * wl4) * b4, w5 = (double)(k3 * wl5) * b5;
+            if constexpr (PERT) {
+                // The FP32 form forms the cell's own normal update in FP64 with
+                // the unrounded dt/dn and rounds it once: the second-order
+                // correction nearly cancels the fluctuation in smooth flow, and
+                // rounding the two products apart (with dt/dn in FP32) grew,
+                // over some 300 steps, into an error of T' of 1e-4 of its peak
+                // in the thin upper layers of weak plumes.
 #pragma unroll
-            for (int m = 0; m < 5; m++) {
-                fw1[m] = fw1[m] * wl1;
-                fw3[m] = fw3[m] * wl5;
-            }
-            const TL b2l = wl2 * b2, b3l = wl3 * b3, b4l = wl4 * b4;
-            fw2[0] = (T)b4l;
-            fw2[1] = (T)(b4l * RL.u);
-            fw2[2] = (T)(b2l + b4l * RL.v);
-            fw2[3] = (T)(b3l + b4l * RL.w);
-            fw2[4] = (T)(b2l * RL.v + b3l * RL.w + b4l * TL(0.5) * RL.u2v2w2);
-            const T k1 = T(0.5) * copysign(T(1.0), s1) * (T(1.0) - fabs(s1) * dtdn);
-            const T k2 = T(0.5) * copysign(T(1.0), s2) * (T(1.0) - fabs(s2) * dtdn);
-            const T k3 = T(0.5) * copysign(T(1.0), s3) * (T(1.0) - fabs(s3) * dtdn);
-#pragma unroll
-            for (int m = 0; m < NC; m++) cqxx[m] = k1 * fw1[m] + k2 * fw2[m] + k3 * fw3[m];
-            if constexpr (PERT)
-                cflmax = fmaxF(cflmax, fmaxF(fmaxF(fabs((double)s1), fabs((double)s2)), fabs((double)s3)) * A.dtdn);
-            else
+                for (int ph2 = 0; ph2 < 2; ph2++) {
+                    const double dD = -A.dtdn, sg = ph2 == 0 ? 1.0 : -1.0;
+                    const bool has = (ph2 == 0) == lf;
+                    const double n1 = dD * ((ph2 == 0 ? al1 : b1 - al1) + sg * w1);
+                    const double n5 = dD * ((ph2 == 0 ? al5 : b5 - al5) + sg * w5);
+                    const double n4 = dD * ((has ? b4 : 0.0) + sg * w4);
+                    const double nv = dD * ((has ? b2 : 0.0) + sg * w2), nw = dD * ((has ? b3 : 0.0) + sg * w3);
+                    const double pp = n1 + n5, nn = R.a * (n5 - n1), rho = pp + n4, kk = 0.5 * R.u2v2w2;
+                    const double mv = R.v * rho + nv, mw = R.w * rho + nw;
+                    nrm[ph2][0] = (T)rho;
+                    nrm[ph2][1] = (T)(R.u * rho + nn);
+                    nrm[ph2][2] = (T)(a_is_g ? mv : mw);
+                    nrm[ph2][3] = (T)(a_is_g ? mw : mv);
+                    nrm[ph2][4] = (T)((R.enth - kk) * pp + kk * rho + R.u * nn + R.v * nv + R.w * nw);
+                }
+                cflmax = fmaxF(cflmax, fmaxF(fmaxF(fabs((double)ts1), fabs((double)ts2)), fabs((double)ts3)) * A.dtdn);
+            } else {
                 cflmax = fmaxF(cflmax, fmaxF(fmaxF(c1, c2), c3));
+            }
+            un = (T)R.u;
+            ua = (T)(a_is_g ? R.v : R.w);
+            ub = (T)(a_is_g ? R.w : R.v);
+            snd = (T)R.a;
+            isnd = (T)(2.0 * R.i2a);
+            kin = (T)(0.5 * R.u2v2w2);
+            hk = (T)(R.enth - 0.5 * R.u2v2w2);
+            x1 = (T)b1; x4 = (T)b4; x5 = (T)b5;
+            xa = (T)(a_is_g ? b2 : b3);
+            xb = (T)(a_is_g ? b3 : b2);
+            l1 = (T)al1; l5 = (T)al5;
+            q1 = (T)w1; q4 = (T)w4; q5 = (T)w5;
+            qsa = (T)(a_is_g ? w2 : w3);
+            qsb = (T)(a_is_g ? w3 : w2);
         }
         if (PREFETCH && chunk + 1 < nchunk) fetch(S + (CH - 2) + c);
 
-        // ---------------- part 3: transverse terms, two phases
-        // Each phase recomputes the two cqxx splits it needs, in an order that
-        // keeps at most four split vectors alive next to the accumulator.
-        // Each lane folds its increments into a register accumulator, added
-        // to the tile in three barrier-separated sub-steps (one per a offset,
-        // so no two lanes add to one entry at once): deterministic.  (Adding
-        // each increment to the tile with shared-memory atomics instead, with
-        // or without a two-waves-per-SIMD register budget, measured 3-5 %
-        // slower in FP64 and 7x slower in FP32 on the full-domain workload.)
-        // In FP64 with tracers the components go in groups, the Euler
-        // components and then the tracers, at most three at a time, with one
-        // accumulator alive at a time (at ten components it spilled a
-        // kilobyte per lane, and the full-domain step with five tracers ran
-        // 2.8x slower; with one tracer the groups hold 19 fewer AGPRs, and
-        // the full-domain step runs 4 % faster, bit for bit the same).
-        // Groups add to disjoint tile entries, so a group's first sub-step
-        // needs no barrier after the previous group's last one.  FP32
-        // accumulators fit without groups, and the extra barriers cost 3 %
-        // there.
-        if constexpr (NTR == 0 || sizeof(T) == 4) {
-            for (int phase = 0; phase < 2; phase++) {
-                // phase 0 (L): interface I -> cell I-1; phase 1 (R): -> cell I
-                const bool on = act2 && (phase == 0 ? I >= 2 : I <= n);
-                const int ci = phase == 0 ? c - 1 : c;  // cell index within the chunk's tile
-                auto transverse = [&](auto &acc) {
-                    const T sgn = phase == 0 ? T(1.0) : -T(1.0);   // +3 cqxx mixing for amdq, -3 for apdq
-                    const T cc = phase == 0 ? -d : d;        // sign of the correction-wave term
-                    T asd[NC];
+        // ---------------- part 3: transverse terms (flux3fw.f:297-625), two phases
+        // The transverse splits by the interface's Roe eigensystem
+        // (rpt3euX.f:106-214, rptt3euX.f:108-214) run in variables relative to
+        // the Roe velocity (WaveT: entropy s, pressure p/a^2, momenta n, a, b),
+        // in which a split is a few products and nested splits need no change
+        // of variables.  A split along a with weights w (of the speeds u_a - c,
+        // u_a, u_a + c) is S_a[w].  With w_j = -min(speed, 0), -|speed|,
+        // max(speed, 0) for the target offsets j = -1, 0, +1, the reference's
+        // 9-point increments of one interface (step3.f:189-226) are
+        //   D[r][j] = S_a[w_r] y_j + S_b[w_j] z_r,
+        //   y_j = S_b[w_j] F - (d c_a / 2) E [j = 0],
+        //   z_r = S_a[w_r] F - (d c_b / 2) E [r = 0],
+        // E = asdq +- 2 cqxx, F = -(d c_a c_b / 6)(asdq +- 3 cqxx), plus the
+        // cell's own normal update in the centre.  Each D is carried to the
+        // conserved components once, when it is added to the tile, in three
+        // sub-steps (one per a offset, so no two lanes add to one entry at
+        // once): deterministic.  Against splitting conserved vectors and
+        // summing a 3 x 3 x NC register accumulator this halves the sweep's
+        // arithmetic, and nothing wider than the y and z vectors stays live.
+        const T kf = -(T(1.0) / T(6.0)) * d * ca * cb2, kea = -T(0.5) * d * ca, keb = -T(0.5) * d * cb2;
+        const SpeedT<T> va(ua, snd), vb(ub, snd);
+#pragma unroll 1
+        for (int phase = 0; phase < 2; phase++) {
+            // phase 0 (L): interface I -> cell I-1; phase 1 (R): -> cell I
+            const bool on = act2 && (phase == 0 ? I >= 2 : I <= n);
+            const int ci = phase == 0 ? c - 1 : c;  // cell index within the chunk's tile
+            const T sg = phase == 0 ? T(1.0) : -T(1.0);
+            const bool has = (phase == 0) == lf;    // the contact waves belong to this phase
+            WaveT<T> y[3], z[3], N;
+            T yt[3][NTR > 0 ? NTR : 1], zt[3][NTR > 0 ? NTR : 1], Nt[NTR > 0 ? NTR : 1];
+            if (on) {
+                const T a1 = phase == 0 ? l1 : x1 - l1, a5 = phase == 0 ? l5 : x5 - l5;
+                const T a4 = has ? x4 : T(0.0), aa = has ? xa : T(0.0), ab = has ? xb : T(0.0);
+                const T s3q = T(3.0) * sg, s2q = T(2.0) * sg;
+                const WaveT<T> F(kf * (a1 + s3q * q1), kf * (a4 + s3q * q4), kf * (aa + s3q * qsa), kf * (ab + s3q * qsb),
+                                 kf * (a5 + s3q * q5), snd);
+                const WaveT<T> E(a1 + s2q * q1, a4 + s2q * q4, aa + s2q * qsa, ab + s2q * qsb, a5 + s2q * q5, snd);
+                if constexpr (!PERT)
+                    N = WaveT<T>(-d * (a1 + sg * q1), -d * (a4 + sg * q4), -d * (aa + sg * qsa), -d * (ab + sg * qsb),
+                                 -d * (a5 + sg * q5), snd);
+                y[0] = vb.template split_b<0>(F, snd, isnd);
+                y[2] = vb.template split_b<2>(F, snd, isnd);
+                z[0] = va.template split_a<0>(F, snd, isnd);
+                z[2] = va.template split_a<2>(F, snd, isnd);
+                // rptt3euX.f:169: the split along h takes its first shear
+                // from the h momentum
+                if (a_is_g) {
 #pragma unroll
-                    for (int m = 0; m < NC; m++) asd[m] = phase == 0 ? amdq[m] : apdq[m];
-                    {
-                        // C splits (h direction): 2-D part, correction, then the
-                        // g-direction corner terms of c*asdq +- 3 c*cqxx (flux3fw.f:388-412)
-                        T Cm[NC], Cp[NC], Cmq[NC], Cpq[NC];
-                        tsplit<NC, 3, false>(R, cqxx, Cmq, Cpq);
-                        tsplit<NC, 3, false>(R, asd, Cm, Cp);
-                        acc.h(1, 0, -T(0.5) * d * ch, Cm); acc.h(2, 0, -T(0.5) * d * ch, Cp);
-                        acc.h(1, 0, cc * ch, Cmq);      acc.h(2, 0, cc * ch, Cpq);
-                        axpy3(Cp, Cp, T(3.0) * sgn, Cpq);
-                        axpy3(Cm, Cm, T(3.0) * sgn, Cmq);
-                        tsplit<NC, 2, true>(R, Cp, Cmq, Cpq);      // B-, B+ of c+asdq2
-                        acc.g(2, 0, k6g * cg, Cpq);  acc.g(1, 0, k6g * cg, Cmq);
-                        acc.g(2, 1, -k6g * cg, Cpq); acc.g(1, 1, -k6g * cg, Cmq);
-                        tsplit<NC, 2, true>(R, Cm, Cmq, Cpq);      // B-, B+ of c-asdq2
-                        acc.g(2, 0, -k6g * cg, Cpq); acc.g(1, 0, -k6g * cg, Cmq);
-                        acc.g(2, -1, k6g * cg, Cpq); acc.g(1, -1, k6g * cg, Cmq);
-                    }
-                    {
-                        // B splits (g direction): 2-D part, correction, then the
-                        // h-direction corner terms of b*asdq +- 3 b*cqxx (flux3fw.f:510-538)
-                        T Bm[NC], Bp[NC], Bmq[NC], Bpq[NC];
-                        tsplit<NC, 2, false>(R, cqxx, Bmq, Bpq);
-                        tsplit<NC, 2, false>(R, asd, Bm, Bp);
-                        acc.g(1, 0, -T(0.5) * d * cg, Bm); acc.g(2, 0, -T(0.5) * d * cg, Bp);
-                        acc.g(1, 0, cc * cg, Bmq);      acc.g(2, 0, cc * cg, Bpq);
-                        axpy3(Bp, Bp, T(3.0) * sgn, Bpq);
-                        axpy3(Bm, Bm, T(3.0) * sgn, Bmq);
-                        tsplit<NC, 3, true>(R, Bp, Bmq, Bpq);      // C-, C+ of b+asdq
-                        acc.h(2, 0, k6h * ch, Bpq);  acc.h(1, 0, k6h * ch, Bmq);
-                        acc.h(2, 1, -k6h * ch, Bpq); acc.h(1, 1, -k6h * ch, Bmq);
-                        tsplit<NC, 3, true>(R, Bm, Bmq, Bpq);      // C-, C+ of b-asdq
-                        acc.h(2, 0, -k6h * ch, Bpq); acc.h(1, 0, -k6h * ch, Bmq);
-                        acc.h(2, -1, k6h * ch, Bpq); acc.h(1, -1, k6h * ch, Bmq);
-                    }
-                    if constexpr (sizeof(T) == 4) {
-                        // The FP32 form forms the cell's own normal update in
-                        // FP64 with the unrounded dt/dn and rounds it once: the
-                        // second-order correction nearly cancels the fluctuation
-                        // in smooth flow, and rounding the two products apart
-                        // (with dt/dn in FP32) grew, over some 300 steps, into
-                        // an error of T' of 1e-4 of its peak in the thin upper
-                        // layers of weak plumes.
-                        const double dD = A.dtdn;
-#pragma unroll
-                        for (int m = 0; m < NC; m++)
-                            acc.c11(m, (T)(phase == 0 ? -dD * (double)amdq[m] - dD * (double)cqxx[m]
-                                                      : -dD * (double)apdq[m] + dD * (double)cqxx[m]));
-                    } else {
-#pragma unroll
-                        for (int m = 0; m < NC; m++)
-                            acc.c11(m, phase == 0 ? -d * amdq[m] - d * cqxx[m] : -d * apdq[m] + d * cqxx[m]);
-                    }
-                };
-                Acc<NC, T> acc;
-                acc.zero();
-                if (on) transverse(acc);
-                // one sub-step per offset along a: lanes then add to distinct T entries
-#pragma unroll
-                for (int da = 0; da < 3; da++) {
-                    if (on) {
-                        // the accumulator is indexed [g offset][h offset]; both
-                        // branches keep every index a compile-time constant so
-                        // it stays in registers
-                        if (a_is_g) {
-#pragma unroll
-                            for (int db = 0; db < 3; db++)
-#pragma unroll
-                                for (int m = 0; m < NC; m++) LT[tix(m, db, pa + da, ci)] += acc.D[da][db][m];
-                        } else {
-#pragma unroll
-                            for (int db = 0; db < 3; db++)
-#pragma unroll
-                                for (int m = 0; m < NC; m++) LT[tix(m, db, pa + da, ci)] += acc.D[db][da][m];
-                        }
-                    }
-                    // With tile-axis-major lanes a wave holds every pencil of
-                    // its chunk cells, so the entries one phase's sub-steps add
-                    // to are the wave's own (cells c-1 or c of its lanes): only
-                    // the wave's program order separates its sub-steps (the
-                    // fence keeps the compiler from moving one sub-step's tile
-                    // reads above the previous one's writes; it emits nothing),
-                    // and the workgroup waits once per phase.  Pencil-major
-                    // waves share entries: a barrier after every sub-step.
-                    if (PM || da == 2) __syncthreads();
-                    else __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
-                    if (phase == 0 && da == (PM ? 0 : 2) && t < TA) {
-                        // CFLup carried into the next chunk: the last assignment
-                        // among this chunk's interfaces (every lane is past part
-                        // 2, which reads s_cprev, once this barrier is passed)
-                        for (int j = CH - 2; j >= 1; j--) {
-                            const int tt = PM ? t * CH + j : j * TA + t;
-                            if (s_flag[tt]) { s_cprev[t] = s_cfo[tt]; break; }
-                        }
-                    }
-                }
-            }
-        } else {
-            for (int phase = 0; phase < 2; phase++) {
-                // phase 0 (L): interface I -> cell I-1; phase 1 (R): -> cell I
-                const bool on = act2 && (phase == 0 ? I >= 2 : I <= n);
-                const int ci = phase == 0 ? c - 1 : c;  // cell index within the chunk's tile
-                const T sgn = phase == 0 ? T(1.0) : -T(1.0);   // +3 cqxx mixing for amdq, -3 for apdq
-                const T cc = phase == 0 ? -d : d;        // sign of the correction-wave term
-                // components M0 .. M0+GW-1; `final`: the phase's last group
-                auto group = [&](auto m0c, auto gwc, bool final) {
-                    constexpr int M0 = decltype(m0c)::value, GW = decltype(gwc)::value;
-                    Acc<GW, T> acc;
-                    acc.zero();
-                    if (on) {
-                        T asd[GW];
-#pragma unroll
-                        for (int m = 0; m < GW; m++) asd[m] = phase == 0 ? amdq[M0 + m] : apdq[M0 + m];
-                        const T(&cq)[GW] = *reinterpret_cast<const T(*)[GW]>(cqxx + M0);
-                        {
-                            // C splits (h direction): 2-D part, correction, then the
-                            // g-direction corner terms of c*asdq +- 3 c*cqxx (flux3fw.f:388-412)
-                            T Cm[GW], Cp[GW], Cmq[GW], Cpq[GW];
-                            tsplit_group<M0, GW, 3, false>(R, cq, Cmq, Cpq);
-                            tsplit_group<M0, GW, 3, false>(R, asd, Cm, Cp);
-                            acc.h(1, 0, -T(0.5) * d * ch, Cm); acc.h(2, 0, -T(0.5) * d * ch, Cp);
-                            acc.h(1, 0, cc * ch, Cmq);      acc.h(2, 0, cc * ch, Cpq);
-                            axpy3(Cp, Cp, T(3.0) * sgn, Cpq);
-                            axpy3(Cm, Cm, T(3.0) * sgn, Cmq);
-                            tsplit_group<M0, GW, 2, true>(R, Cp, Cmq, Cpq);      // B-, B+ of c+asdq2
-                            acc.g(2, 0, k6g * cg, Cpq);  acc.g(1, 0, k6g * cg, Cmq);
-                            acc.g(2, 1, -k6g * cg, Cpq); acc.g(1, 1, -k6g * cg, Cmq);
-                            tsplit_group<M0, GW, 2, true>(R, Cm, Cmq, Cpq);      // B-, B+ of c-asdq2
-                            acc.g(2, 0, -k6g * cg, Cpq); acc.g(1, 0, -k6g * cg, Cmq);
-                            acc.g(2, -1, k6g * cg, Cpq); acc.g(1, -1, k6g * cg, Cmq);
-                        }
-                        {
-                            // B splits (g direction): 2-D part, correction, then the
-                            // h-direction corner terms of b*asdq +- 3 b*cqxx (flux3fw.f:510-538)
-                            T Bm[GW], Bp[GW], Bmq[GW], Bpq[GW];
-                            tsplit_group<M0, GW, 2, false>(R, cq, Bmq, Bpq);
-                            tsplit_group<M0, GW, 2, false>(R, asd, Bm, Bp);
-                            acc.g(1, 0, -T(0.5) * d * cg, Bm); acc.g(2, 0, -T(0.5) * d * cg, Bp);
-                            acc.g(1, 0, cc * cg, Bmq);      acc.g(2, 0, cc * cg, Bpq);
-                            axpy3(Bp, Bp, T(3.0) * sgn, Bpq);
-                            axpy3(Bm, Bm, T(3.0) * sgn, Bmq);
-                            tsplit_group<M0, GW, 3, true>(R, Bp, Bmq, Bpq);      // C-, C+ of b+asdq
-                            acc.h(2, 0, k6h * ch, Bpq);  acc.h(1, 0, k6h * ch, Bmq);
-                            acc.h(2, 1, -k6h * ch, Bpq); acc.h(1, 1, -k6h * ch, Bmq);
-                            tsplit_group<M0, GW, 3, true>(R, Bm, Bmq, Bpq);      // C-, C+ of b-asdq
-                            acc.h(2, 0, -k6h * ch, Bpq); acc.h(1, 0, -k6h * ch, Bmq);
-                            acc.h(2, -1, k6h * ch, Bpq); acc.h(1, -1, k6h * ch, Bmq);
-                        }
-#pragma unroll
-                        for (int m = 0; m < GW; m++)
-                            acc.c11(m, phase == 0 ? -d * amdq[M0 + m] - d * cqxx[M0 + m] : -d * apdq[M0 + m] + d * cqxx[M0 + m]);
-                    }
-                    // one sub-step per offset along a: lanes then add to distinct T entries
-#pragma unroll
-                    for (int da = 0; da < 3; da++) {
-                        if (on) {
-                            // the accumulator is indexed [g offset][h offset]; both
-                            // branches keep every index a compile-time constant so
-                            // it stays in registers
-                            if (a_is_g) {
-#pragma unroll
-                                for (int db = 0; db < 3; db++)
-#pragma unroll
-                                    for (int m = 0; m < GW; m++) LT[tix(M0 + m, db, pa + da, ci)] += acc.D[da][db][m];
-                            } else {
-#pragma unroll
-                                for (int db = 0; db < 3; db++)
-#pragma unroll
-                                    for (int m = 0; m < GW; m++) LT[tix(M0 + m, db, pa + da, ci)] += acc.D[db][da][m];
-                            }
-                        }
-                        // as in the branch above: tile-axis-major waves wait
-                        // once per phase (after its final group), pencil-major
-                        // ones after every sub-step but a group's last
-                        if (PM ? (da < 2 || (final && phase == 1)) : (da == 2 && final)) __syncthreads();
-                        else if (!PM) __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
-                        if (phase == 0 && (PM ? (M0 == 0 && da == 0) : (final && da == 2)) && t < TA) {
-                            // CFLup carried into the next chunk: the last assignment
-                            // among this chunk's interfaces (every lane is past part
-                            // 2, which reads s_cprev, once this barrier is passed)
-                            for (int j = CH - 2; j >= 1; j--) {
-                                const int tt = PM ? t * CH + j : j * TA + t;
-                                if (s_flag[tt]) { s_cprev[t] = s_cfo[tt]; break; }
-                            }
-                        }
-                    }
-                };
-                if constexpr (NTR <= 3) {
-                    group(IConst<0>{}, IConst<5>{}, false);
-                    group(IConst<5>{}, IConst<NTR>{}, true);
+                    for (int r = 0; r < 3; r += 2) z[r].n = z[r].b + (ub - un) * (z[r].s + z[r].p);
                 } else {
-                    group(IConst<0>{}, IConst<5>{}, false);
-                    group(IConst<5>{}, IConst<3>{}, false);
-                    group(IConst<8>{}, IConst<NTR - 3>{}, true);
+#pragma unroll
+                    for (int r = 0; r < 3; r += 2) y[r].n = y[r].a + (ua - un) * (y[r].s + y[r].p);
+                }
+                y[1] = WaveT<T>::middle(y[0], y[2], kea, E);
+                z[1] = WaveT<T>::middle(z[0], z[2], keb, E);
+#pragma unroll
+                for (int k = 0; k < NTR; k++) {
+                    const T at = has ? trw[k] : T(0.0);
+                    const T ft = kf * (at + s3q * trq[k]), et = at + s2q * trq[k];
+                    Nt[k] = -d * (at + sg * trq[k]);
+#pragma unroll
+                    for (int r = 0; r < 3; r += 2) {
+                        yt[r][k] = vb.w2(r) * ft;
+                        zt[r][k] = va.w2(r) * ft;
+                    }
+                    yt[1][k] = kea * et - (yt[0][k] + yt[2][k]);
+                    zt[1][k] = keb * et - (zt[0][k] + zt[2][k]);
                 }
             }
+            // one sub-step per offset along a: lanes then add to distinct T entries
+            auto substep = [&](auto rc) {
+                constexpr int r = decltype(rc)::value;
+                if (on) {
+                    auto target = [&](auto jc) {
+                        constexpr int j = decltype(jc)::value;
+                        WaveT<T> D = va.template split_a<r>(y[j], snd, isnd);
+                        D.add(vb.template split_b<j>(z[r], snd, isnd));
+                        if constexpr (!PERT && r == 1 && j == 1) D.add(N);
+                        const T rho = D.s + D.p;
+                        T o[5] = {rho, un * rho + D.n, ua * rho + D.a, ub * rho + D.b,
+                                  hk * D.p + kin * rho + un * D.n + ua * D.a + ub * D.b};
+                        if constexpr (PERT && r == 1 && j == 1) {
+#pragma unroll
+                            for (int m = 0; m < 5; m++) o[m] += phase == 0 ? nrm[0][m] : nrm[1][m];
+                        }
+#pragma unroll
+                        for (int m = 0; m < 5; m++) LT[tix(m, j, pa + r, ci)] += o[m];
+#pragma unroll
+                        for (int k = 0; k < NTR; k++) {
+                            T v = va.w2(r) * yt[j][k] + vb.w2(j) * zt[r][k];
+                            if (r == 1 && j == 1) v += Nt[k];
+                            LT[tix(5 + k, j, pa + r, ci)] += v;
+                        }
+                    };
+                    target(IConst<0>{});
+                    target(IConst<1>{});
+                    target(IConst<2>{});
+                }
+                // With tile-axis-major lanes a wave holds every pencil of
+                // its chunk cells, so the entries one phase's sub-steps add
+                // to are the wave's own (cells c-1 or c of its lanes): only
+                // the wave's program order separates its sub-steps (the
+                // fence keeps the compiler from moving one sub-step's tile
+                // reads above the previous one's writes; it emits nothing),
+                // and the workgroup waits once per phase.  Pencil-major
+                // waves share entries: a barrier after every sub-step.
+                if (PM || r == 2) __syncthreads();
+                else __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
+                if (phase == 0 && r == (PM ? 0 : 2) && t < TA) {
+                    // CFLup carried into the next chunk: the last assignment
+                    // among this chunk's interfaces (every lane is past part
+                    // 2, which reads s_cprev, once this barrier is passed)
+                    for (int j = CH - 2; j >= 1; j--) {
+                        const int tt = PM ? t * CH + j : j * TA + t;
+                        if (s_flag[tt]) { s_cprev[t] = s_cfo[tt]; break; }
+                    }
+                }
+            };
+            substep(IConst<0>{});
+            substep(IConst<1>{});
+            substep(IConst<2>{});
         }
 
         // ---------------- flush the tile to q (one read-modify-write per row)
@@ -742,7 +606,7 @@ __device__ __forceinline__ void tile_sweep_body(const SweepArgsT<T> &A, int a_is
 #pragma unroll
                     for (int db = 0; db < 3; db++) {
                         const gptr<T> base =
-                            qnew + (long long)A.comp[m] * A.P + (long long)(b + db - 1 + A.mbc - 1) * A.sB;
+                            qnew + plane(m) + (long long)(b + db - 1 + A.mbc - 1) * A.sB;
 #pragma unroll
                         for (int k = 0; k < PPT; k++) {
                             const int e = t + k * NT;
@@ -759,7 +623,7 @@ __device__ __forceinline__ void tile_sweep_body(const SweepArgsT<T> &A, int a_is
             for (int m = 0; m < NC; m++)
 #pragma unroll
                 for (int db = 0; db < 3; db++) {
-                    const gptr<T> base = qnew + (long long)A.comp[m] * A.P + (long long)(b + db - 1 + A.mbc - 1) * A.sB;
+                    const gptr<T> base = qnew + plane(m) + (long long)(b + db - 1 + A.mbc - 1) * A.sB;
 #pragma unroll
                     for (int k = 0; k < PPT; k++) val[m][db][k] = *(pok[k] ? base + poff[k] : sink);
                 }
@@ -778,7 +642,7 @@ __device__ __forceinline__ void tile_sweep_body(const SweepArgsT<T> &A, int a_is
             for (int m = 0; m < NC; m++)
 #pragma unroll
                 for (int db = 0; db < 3; db++) {
-                    const gptr<T> base = qnew + (long long)A.comp[m] * A.P + (long long)(b + db - 1 + A.mbc - 1) * A.sB;
+                    const gptr<T> base = qnew + plane(m) + (long long)(b + db - 1 + A.mbc - 1) * A.sB;
 #pragma unroll
                     for (int k = 0; k < PPT; k++) *(pok[k] ? base + poff[k] : sink) = val[m][db][k];
                 }
