@@ -163,13 +163,12 @@ int magic_global_sums_noalloc(magic_ctx *ctx, double *sums);
  * (rpn3euX.f:145-150). */
 int magic_error_location(magic_ctx *ctx, int *sweep, int *i, int *j, int *k);
 
-/* Per-kernel-class timing with HIP events on the library's streams
- * (0 = off): each class's launches are bracketed on the stream they run on
- * (the second stream for the y-sweep and half of the z-sweep while the
- * sweep overlap is on, so those spans include time shared with the other
- * stream).  Classes: 0 sweep x, 1 sweep y, 2 sweep z, 3 bc3, 4 src3,
- * 5 other.  magic_timing_read returns milliseconds and launch counts
- * accumulated since the last reset. */
+/* Per-kernel-class timing with HIP events on the context's stream (0 = off):
+ * each class's launches are bracketed.  Classes: 0 sweep x, 1 sweep y, 2
+ * sweep z, 3 bc3, 4 src3, 5 other.  Directions of one tile shape are swept by
+ * one launch; its time is shared by them in proportion to their blocks, and
+ * it counts as a launch of each.  magic_timing_read returns milliseconds and
+ * launch counts accumulated since the last reset. */
 int magic_timing_enable(magic_ctx *ctx, int on);
 int magic_timing_read(magic_ctx *ctx, double ms[6], long long launches[6]);
 int magic_timing_reset(magic_ctx *ctx);
@@ -187,9 +186,6 @@ int magic_timing_reset(magic_ctx *ctx);
  * set, dt > 0: one untimed and reps timed sweeps each), keeps the fastest
  * per direction and returns them in shapes_out (and, if ms_out is not NULL,
  * the mean ms per sweep in ms_out[3 * MAGIC_TILE_NSHAPE], direction-major).
- * With the sweep overlap on (magic_set_sweep_overlap), it then varies each
- * direction's shape in turn, timing the overlapped sweeps of step3 as a
- * whole, and keeps an assignment that is at least 1 % faster.
  * q is unchanged bit for bit; the backup copy then holds q.
  * MAGIC_EUNSUPPORTED for the FP64 pencil kernel (MAGIC_SWEEP=pencil). */
 #define MAGIC_TILE_NSHAPE 4
@@ -198,16 +194,10 @@ int magic_get_tile_shapes(magic_ctx *ctx, int shapes[3]);
 int magic_tune(magic_ctx *ctx, double dt, int reps, int shapes_out[3], float *ms_out);
 
 /* ---- Order of the sweeps (no counterpart in the reference) -------------
- * on = 1 (default): the y-sweep of step3 and half of the z-sweep's colour
- * launches run on a second stream next to the x-sweep and the other z
- * launches, adding into a scratch copy of the state's shape that is added
- * to q once both streams are done (the compute units the last workgroups of
- * one stream's launches leave idle take the other stream's workgroups).
- * on = 0: the three sweeps add into q in turn on the context's stream, the
- * order of additions of the batched driver, whose scenarios then equal the
- * same grids stepped alone bit for bit.  Either way the result is the same
- * on every run; the two orders differ in the last bits.  The environment
- * variable MAGIC_SWEEP_OVERLAP=0 turns the overlap off for every context. */
+ * The three sweeps of a step run as one launch, and their increments are
+ * added to q in one fixed order (x, y, z) whatever this setting says: both
+ * values give the same state, bit for bit, on one grid and in a batch.
+ * Kept so that programs that set it keep working. */
 int magic_set_sweep_overlap(magic_ctx *ctx, int on);
 
 /* ---- Batched driver: many grids of one form advanced together ----------
@@ -216,10 +206,11 @@ int magic_set_sweep_overlap(magic_ctx *ctx, int on);
  * (claw3_mpi.f:736-927) but lives on the device, and one attempted step of
  * every scenario is one replay of a HIP graph captured at the first
  * magic_batch_run.  Each kernel of the attempt is one launch over all
- * scenarios (the sweeps as persistent launches per direction and tile
- * colour over a work list of tiles, the boundary, copy and source-pass
+ * scenarios (the sweeps over a list of the grids' blocks, in groups of
+ * scenarios whose increments fit 8 GB, the boundary, copy and source-pass
  * kernels over the scenarios' grids laid end to end), so the launches per
- * attempt do not grow with the number of scenarios.  No counterpart in the
+ * attempt do not grow with the number of scenarios but by one group's three
+ * per 8 GB of increments.  No counterpart in the
  * reference. */
 typedef struct magic_batch magic_batch;
 /* dims: (mx, my, mz) per scenario; geom: (xlower, ylower, zlower, dx, dy, dz)
@@ -258,20 +249,15 @@ int magic_batch_state(magic_batch *b, int s, double real_out[5], int int_out[6])
 /* Tile shapes of the batch's x-, y- and z-sweeps (one per direction for all
  * scenarios; default 0, 0, 0); setting them captures the graph again.
  * magic_batch_tune is the autotuner of the batch: every shape of every
- * direction is timed as one persistent launch per tile colour over the
- * tiles of all scenarios (their current states and next dt; one untimed
+ * direction is timed as launches over the blocks of all scenarios (their current states and next dt; one untimed
  * and reps timed sweeps), and the fastest per direction is kept.  The
  * scenarios' states are unchanged bit for bit. */
 int magic_batch_set_tile_shapes(magic_batch *b, const int shapes[3]);
 int magic_batch_get_tile_shapes(magic_batch *b, int shapes[3]);
 int magic_batch_tune(magic_batch *b, int reps, int shapes_out[3], float *ms_out);
-/* The batch's sweeps in the same two orders as magic_set_sweep_overlap.
- * Off by default: the batch's persistent launches leave few compute units
- * idle, and the per-scenario merge costs more than the overlap gains.
- * While on, each scenario holds one more buffer of its state's size.
- * Setting it captures the graph again.  A scenario equals the same grid
- * stepped alone bit for bit when both use the same order and tile shapes.
- * No counterpart in the reference. */
+/* As magic_set_sweep_overlap: accepted, without effect on the result.  A
+ * scenario equals the same grid stepped alone bit for bit when both use the
+ * same tile shapes.  Setting it captures the graph again. */
 int magic_batch_set_sweep_overlap(magic_batch *b, int on);
 
 #ifdef __cplusplus

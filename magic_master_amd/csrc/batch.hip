@@ -5,12 +5,17 @@
 //
 // One attempt:
 //   prepare  (dt clip, per-grid sweep factors, source-pass substep counts)
-//   bc3 (x, y, z faces), b4step3, copyq3 backup
-//   3 directions x 6 tile colours of the sweep  (persistent work-list launches)
-//   decide   (accept / reject from the Courant number)
-//   restore of rejected scenarios, src3 of accepted ones
+//   bc3 (x, y, z faces), b4step3
+//   per group of scenarios (as many as the increment buffer holds):
+//     the sweeps    (one launch over the blocks of the group's grids)
+//     decide        (accept / reject from the Courant number)
+//     src3's conversion of the accepted scenarios, which adds the increments
+//     to q and leaves the state before the step in the backup
+//   the rest of src3 of accepted scenarios
 //   finalize (next dt, step count, end of interval)
-// Every launch covers all scenarios: the sweeps through tile work lists,
+// The sweeps read q itself, which only an accepted step's conversion changes,
+// so nothing is copied before a step or restored after a rejected one.
+// Every launch covers all scenarios: the sweeps through lists of their blocks,
 // the other kernels through block lists that lay the scenarios' own grids
 // end to end (batch_ops.h), each scenario gated by its control block.  The
 // number of launches per attempt does not depend on the number of
@@ -37,38 +42,36 @@ struct magic_batch {
     std::vector<int> mthbc;              // 6 per scenario
     ScenCtl *ctl_d = nullptr;
     ScenCtl *ctl_pin = nullptr;          // pinned read-back buffer
-    void *args_d = nullptr;              // SweepArgsT of the form, 18 per slot: direction x colour
+    void *args_d = nullptr;              // SweepArgsT of the form, 3 per slot: one per direction
     const int **run_d = nullptr;         // per argument block: &ctl_d[s].run
     int4 *items_d = nullptr;
-    int item_off[19] = {0};              // work list of direction d, colour k at [item_off[6d+k], ..)
-    int *counters_d = nullptr;           // 18 pairs of work counters (tile_sweep_list)
+    // Groups of slots [lo, hi) whose increments the part buffer holds at
+    // once; blocks of the group's direction d at items_d[off[d], off[d + 1])
+    struct Group { int lo, hi, off[4]; };
+    std::vector<Group> groups;
+    std::vector<StepParts<double>> sp64; // per slot, by form: the increments of its sweeps
+    std::vector<StepParts<float>> sp32;
+    void *parts = nullptr;
+    size_t parts_bytes = 0;
+    bool parts_one = false;              // room for one direction at a time only
     int shape[3] = {0, 0, 0};            // tile shape of the x-, y- and z-sweeps
-    int grid[3] = {0, 0, 0};             // persistent grid size of each direction's kernel
     int *one_d = nullptr;                // a device 1: the run flag of every tile while tuning
     // boundary, copy and source-pass kernels (batch_ops.h)
     void *ops_d = nullptr;               // BatchOps of the form, one per slot
     int *loff_d = nullptr;               // NLG block lists: cap + 1 offsets each
     int4 *lgdim_d = nullptr;             //                  cap grid shapes each
-    long long ltotal[NLG] = {0};         // blocks of each list
+    std::vector<int> loff;               // loff_d's host copy
     int ndtr_cap = 0, ndtrc_cap = 0;     // substep loops of the captured attempt
     int opgrid[NOP] = {0};               // persistent grid of each kernel class
-    // Sweep overlap, as for a single grid (off by default): the y-sweep and
-    // the last three colour launches of the z-sweep add into each
-    // scenario's dq (ctx dq[0]) on a second stream, the rest into q on the
-    // main stream; each scenario then adds dq into q and clears it.  The
-    // same order of additions as a single grid with the overlap on.  The
-    // batch's persistent launches leave few compute units idle, and on the
-    // 64-scenario ensemble the merge's traffic outweighs the gain (3 %
-    // slower), hence the default.
-    bool overlap = false;
-    hipStream_t side = nullptr;
-    hipEvent_t sw_fork = nullptr, sw_join = nullptr;
+    bool overlap = false;                // accepted for the ABI; the order of the sums does not depend on it
     hipGraph_t graph = nullptr;
     hipGraphExec_t exec = nullptr;
     bool dirty = true;                   // control blocks changed on the host
     bool graph_ok = false;
 };
 
+static StepParts<double> &slot_parts(magic_batch *b, int s, double) { return b->sp64[s]; }
+static StepParts<float> &slot_parts(magic_batch *b, int s, float) { return b->sp32[s]; }
 static bool fp32(const magic_batch *b) { return b->form == MAGIC_FORM_FP32P; }
 static size_t elt(const magic_batch *b) { return fp32(b) ? sizeof(float) : sizeof(double); }
 static void *state_q(const magic_ctx *c) { return c->form == MAGIC_FORM_FP32P ? (void *)c->q32 : (void *)c->q; }
@@ -79,10 +82,9 @@ static void *state_qold(const magic_ctx *c)
 
 // ------------------------------------------------------- control kernels --
 template <typename T>
-__global__ void k_batch_prepare(ScenCtl *ctl, int n, SweepArgsT<T> *args, int *counters)
+__global__ void k_batch_prepare(ScenCtl *ctl, int n, SweepArgsT<T> *args)
 {
     const int s = (int)(blockIdx.x * blockDim.x + threadIdx.x);
-    if (s < 36) counters[s] = 0;   // the sweeps' counter pairs (the kernel also resets them)
     if (s >= n) return;
     ScenCtl &c = ctl[s];
     c.accepted = 0;
@@ -98,12 +100,10 @@ __global__ void k_batch_prepare(ScenCtl *ctl, int n, SweepArgsT<T> *args, int *c
     for (int e = 0; e < 6; e++) c.err[e] = 0;
     const double dt = c.dt;
     const double dtdx = dt / c.dx, dtdy = dt / c.dy, dtdz = dt / c.dz;
-    for (int k = 0; k < 6; k++) {
-        SweepArgsT<T> &ax = args[s * 18 + 0 * 6 + k], &ay = args[s * 18 + 1 * 6 + k], &az = args[s * 18 + 2 * 6 + k];
-        ax.dtdn = dtdx; ax.fg = dtdy; ax.fh = dtdz;
-        ay.dtdn = dtdy; ay.fg = dtdz; ay.fh = dtdx;
-        az.dtdn = dtdz; az.fg = dtdx; az.fh = dtdy;
-    }
+    SweepArgsT<T> &ax = args[s * 3], &ay = args[s * 3 + 1], &az = args[s * 3 + 2];
+    ax.dtdn = dtdx; ax.fg = dtdy; ax.fh = dtdz;
+    ay.dtdn = dtdy; ay.fg = dtdz; ay.fh = dtdx;
+    az.dtdn = dtdz; az.fg = dtdx; az.fh = dtdy;
     // src3.f90:314-322
     const int ndtr = (int)ceil((dt * c.difmax / (c.dxyzmin2)) / 0.45);
     const double dtr = dt / ndtr;
@@ -206,67 +206,27 @@ static void src_caps(const magic_ctx *c, double dtbound, int *ndtr, int *ndtrc)
     if (*ndtrc < 1) *ndtrc = 1;
 }
 
-// tracers 0, 1, 2 and 5 (the sweep kernels' instantiations)
+// the blocks of directions d0 .. d1-1 (of one shape) of a group's grids
 template <typename T, bool PERT>
-static const void *list_fn(const magic_batch *b, int dir)
+static int launch_dirs(magic_batch *b, const magic_batch::Group &g, int d0, int d1)
 {
-    switch (b->meqn - 5) {
-    case 0: return tile_list_fn<T, PERT, 0>(b->shape[dir]);
-    case 1: return tile_list_fn<T, PERT, 1>(b->shape[dir]);
-    case 2: return tile_list_fn<T, PERT, 2>(b->shape[dir]);
-    case 3: return tile_list_fn<T, PERT, 3>(b->shape[dir]);
-    case 4: return tile_list_fn<T, PERT, 4>(b->shape[dir]);
-    case 5: return tile_list_fn<T, PERT, 5>(b->shape[dir]);
-    default: return nullptr;
-    }
-}
-
-// colour launches k0 .. k1-1 of direction dir on stream st
-template <typename T, bool PERT>
-static int launch_dir(magic_batch *b, int dir, hipStream_t st = nullptr, int k0 = 0, int k1 = 6)
-{
-    if (!st) st = b->stream;
-    const void *fn = list_fn<T, PERT>(b, dir);
-    if (!fn || b->grid[dir] < 1) return MAGIC_EARG;
-    for (int k = k0; k < k1; k++) {
-        const int lo = b->item_off[6 * dir + k];
-        int n = b->item_off[6 * dir + k + 1] - lo;
-        if (n <= 0) continue;
-        const SweepArgsT<T> *args = (const SweepArgsT<T> *)b->args_d;
-        const int4 *items = b->items_d + lo;
-        const int *const *run = b->run_d;
-        int *cnt = b->counters_d + 2 * (6 * dir + k);
-        int4 grid = make_int4(0, 0, 0, 0);   // the work list
-        void *kargs[] = {&args, &items, &n, &run, &cnt, &grid};
-        HIPCHECK(hipLaunchKernel(fn, dim3(b->grid[dir]), dim3(256), kargs, 0, st));
-        TRY(launch_check());
-    }
-    return MAGIC_OK;
-}
-
-template <typename T, bool PERT>
-static int launch_sweeps(magic_batch *b)
-{
-    if (b->overlap) {
-        HIPCHECK(hipEventRecord(b->sw_fork, b->stream));
-        HIPCHECK(hipStreamWaitEvent(b->side, b->sw_fork, 0));
-        TRY((launch_dir<T, PERT>(b, 1, b->side)));
-        TRY((launch_dir<T, PERT>(b, 2, b->side, 3, 6)));
-        TRY((launch_dir<T, PERT>(b, 0)));
-        TRY((launch_dir<T, PERT>(b, 2, b->stream, 0, 3)));
-        HIPCHECK(hipEventRecord(b->sw_join, b->side));
-        HIPCHECK(hipStreamWaitEvent(b->stream, b->sw_join, 0));
-        return MAGIC_OK;
-    }
-    for (int dir = 0; dir < 3; dir++) TRY((launch_dir<T, PERT>(b, dir)));
-    return MAGIC_OK;
+    const void *fn = tile_fn<T, PERT>(b->meqn - 5, b->shape[d0]);
+    const int nblk = g.off[d1] - g.off[d0];
+    if (!fn) return MAGIC_EARG;
+    if (nblk <= 0) return MAGIC_OK;
+    const SweepArgsT<T> *args = (const SweepArgsT<T> *)b->args_d;
+    const int4 *items = b->items_d + g.off[d0];
+    const int *const *run = b->run_d;
+    void *kargs[] = {&args, &items, &run};
+    HIPCHECK(hipLaunchKernel(fn, dim3((unsigned)nblk), dim3(256), kargs, 0, b->stream));
+    return launch_check();
 }
 
 // Workgroup shape of the kernels that use block list lg
 static dim3 list_block(int lg)
 {
     switch (lg) {
-    case LG_ALL: case LG_CPY: case LG_CP1: case LG_MRG: return dim3(256);
+    case LG_ALL: case LG_CPY: case LG_CP1: return dim3(256);
     case LG_PAD: case LG_DIF: case LG_INT: return cell_block();
     default: return dim3(64);
     }
@@ -276,24 +236,26 @@ static dim3 list_block(int lg)
 static int op_list(int op)
 {
     static const int lg[NOP] = {LG_FX,  LG_FY,  LG_BCZ, LG_ALL, LG_CPY, LG_CPY, LG_PAD, LG_FZ, LG_DIF,
-                                LG_DIF, LG_CP1, LG_INT, LG_FZ,  LG_SPL, LG_INT, LG_INT, LG_MRG};
+                                LG_DIF, LG_CP1, LG_INT, LG_FZ,  LG_SPL, LG_INT, LG_INT, LG_PAD};
     return lg[op];
 }
 
-// One launch of kernel class op over its block list: a persistent grid of
-// at most as many workgroups as fit on the chip at once
+// One launch of kernel class op over its block list (slots lo .. hi-1; all
+// by default): a persistent grid of at most as many workgroups as fit on the
+// chip at once
 template <typename T>
-static int launch_op(magic_batch *b, int op, GateSpec gs, int arg = 0)
+static int launch_op(magic_batch *b, int op, GateSpec gs, int arg = 0, int lo = 0, int hi = -1)
 {
     const int lg = op_list(op);
-    const int total = (int)b->ltotal[lg];
+    if (hi < 0) hi = b->n;
+    const int total = (int)(b->loff[(size_t)lg * (b->cap + 1) + hi] - b->loff[(size_t)lg * (b->cap + 1) + lo]);
     if (total <= 0) return MAGIC_OK;
     const void *fn = batch_op_fn<T>(op);
     if (!fn || b->opgrid[op] < 1) return MAGIC_EARG;
-    const BatchOps<T> *ops = (const BatchOps<T> *)b->ops_d;
-    const int *off = b->loff_d + (size_t)lg * (b->cap + 1);
-    const int4 *gd = b->lgdim_d + (size_t)lg * b->cap;
-    int n = b->n;
+    const BatchOps<T> *ops = (const BatchOps<T> *)b->ops_d + lo;
+    const int *off = b->loff_d + (size_t)lg * (b->cap + 1) + lo;
+    const int4 *gd = b->lgdim_d + (size_t)lg * b->cap + lo;
+    int n = hi - lo;
     void *kargs[] = {&ops, &off, &gd, &n, &gs, &arg};
     HIPCHECK(hipLaunchKernel(fn, dim3(std::min(total, b->opgrid[op])), list_block(lg), kargs, 0, b->stream));
     return launch_check();
@@ -301,13 +263,13 @@ static int launch_op(magic_batch *b, int op, GateSpec gs, int arg = 0)
 
 static GateSpec gs(int mode, int nn = 0, int kk = 0, int fslot = -1) { return GateSpec{mode, nn, kk, fslot}; }
 
-// src3 of the accepted scenarios: src3_passes32 / src3_passes64's sequence
+// src3 of the accepted scenarios after its conversion (launch_group):
+// src3_passes32 / src3_passes64's sequence
 // with the substep loops run to the captured caps, each scenario gated by
 // its own counts (src3.f90:203-634, diffuse.f:37-210, conduct.f:245-332)
 template <typename T>
 static int launch_src(magic_batch *b)
 {
-    TRY(launch_op<T>(b, OP_CONVERT, gs(GATE_ACCEPTED)));
     for (int nn = 1; nn <= b->ndtr_cap; nn++) {
         const GateSpec gd = gs(GATE_DIFF, nn);
         // bc3 with the z faces skipped (src3.f90:333-336)
@@ -334,24 +296,42 @@ static int launch_src(magic_batch *b)
     return launch_op<T>(b, OP_FINISH, gs(GATE_ACCEPTED));
 }
 
+// Sweeps, decision and conversion of one group.  With room for one
+// direction's increments only, each direction's are added to q before the
+// next runs, from the copied backup, as one grid does (capi.hip).
+template <typename T, bool PERT>
+static int launch_group(magic_batch *b, const magic_batch::Group &g)
+{
+    if (b->parts_one) {
+        TRY(launch_op<T>(b, OP_BACKUP, gs(GATE_RUN), 0, g.lo, g.hi));
+        for (int d = 0; d < 3; d++) {
+            TRY((launch_dirs<T, PERT>(b, g, d, d + 1)));
+            TRY(launch_op<T>(b, OP_ADD_PARTS, gs(GATE_SWEPT), d, g.lo, g.hi));
+        }
+    } else {
+        for (int d0 = 0, d1; d0 < 3; d0 = d1) {
+            for (d1 = d0 + 1; d1 < 3 && b->shape[d1] == b->shape[d0];) d1++;
+            TRY((launch_dirs<T, PERT>(b, g, d0, d1)));
+        }
+    }
+    k_batch_decide<<<blocks(g.hi - g.lo, 256), 256, 0, b->stream>>>(b->ctl_d + g.lo, g.hi - g.lo);
+    TRY(launch_check());
+    if (b->parts_one) TRY(launch_op<T>(b, OP_RESTORE, gs(GATE_REJECTED), 0, g.lo, g.hi));
+    return launch_op<T>(b, OP_CONVERT, gs(GATE_ACCEPTED), 0, g.lo, g.hi);
+}
+
 // one attempt of every scenario, as launched into the capture
 template <typename T, bool PERT>
 static int record_attempt(magic_batch *b)
 {
-    const unsigned nb = blocks(b->n > 18 ? b->n : 18, 256);
-    k_batch_prepare<T><<<nb, 256, 0, b->stream>>>(b->ctl_d, b->n, (SweepArgsT<T> *)b->args_d, b->counters_d);
+    k_batch_prepare<T><<<blocks(b->n, 256), 256, 0, b->stream>>>(b->ctl_d, b->n, (SweepArgsT<T> *)b->args_d);
     TRY(launch_check());
     const GateSpec run = gs(GATE_RUN);
     TRY(launch_op<T>(b, OP_BCX, run));
     TRY(launch_op<T>(b, OP_BCY, run));
     TRY(launch_op<T>(b, OP_BCZ, run));
     if (b->meqn > 5) TRY(launch_op<T>(b, OP_CLAMP, run));
-    TRY(launch_op<T>(b, OP_BACKUP, run));
-    TRY((launch_sweeps<T, PERT>(b)));
-    k_batch_decide<<<blocks(b->n, 256), 256, 0, b->stream>>>(b->ctl_d, b->n);
-    TRY(launch_check());
-    if (b->overlap) TRY(launch_op<T>(b, OP_MERGE, gs(GATE_SWEPT)));
-    TRY(launch_op<T>(b, OP_RESTORE, gs(GATE_REJECTED)));
+    for (const auto &g : b->groups) TRY((launch_group<T, PERT>(b, g)));
     TRY(launch_src<T>(b));
     k_batch_finalize<<<blocks(b->n, 256), 256, 0, b->stream>>>(b->ctl_d, b->n);
     return launch_check();
@@ -361,105 +341,124 @@ static int record_attempt(magic_batch *b)
 static void sweep_form_args(const magic_ctx *c, SweepArgsT<float> &a)
 {
     const int NZ = c->d.NZ;
-    a.qold = c->qold32;
-    a.qnew = c->q32;
+    a.qold = c->q32;
     a.crho = c->bg64 + B64_RHO * NZ;
     a.cE = c->bg64 + B64_E * NZ;
     a.cgam = c->bg64 + B64_GAM * NZ;
     a.cvg = c->bg64 + B64_VG * NZ;
     a.cres = c->bg64 + B64_RES * NZ;
-    a.sink = (float *)c->sink;
 }
 
 static void sweep_form_args(const magic_ctx *c, SweepArgsT<double> &a)
 {
-    a.qold = c->qold;
-    a.qnew = c->q;
+    a.qold = c->q;
     a.gam = c->aux + AX_GAM * c->P;
     a.vgrav = c->aux + AX_VG * c->P;
-    a.sink = (double *)c->sink;
 }
 
-// Sweep argument blocks and tile work lists (geometry only; the step's dt
-// factors are written by k_batch_prepare).  For the autotuner (tuning) every
-// tile runs and the dt factors come from each scenario's next dt.
+// Room for the increments of a batch's grids.  A batch of more grids than
+// this holds runs its sweeps in groups; 8 GB (40 million FP64 cells of six
+// components, twice that in FP32) fill the chip many times over, so that the
+// groups cost nothing, and the bound keeps the batch's memory near what its
+// scenarios' own states take.
+constexpr size_t PARTS_BYTES = size_t(8) << 30;
+
+// The part buffer and the groups for the batch's shapes
+template <typename T>
+static int build_groups(magic_batch *b)
+{
+    std::vector<size_t> all(b->n, 0), most(b->n, 0);
+    size_t sum = 0, big = 0, big1 = 0;
+    for (int s = 0; s < b->n; s++) {
+        if (!b->sc[s]) continue;
+        for (int dir = 0; dir < 3; dir++) {
+            SweepArgsT<T> a;
+            SweepParts<T> p;
+            sweep_geometry(b->sc[s], dir, b->shape[dir], a, p);
+            const size_t bytes = (size_t)parts_size(p, b->meqn, b->shape[dir]) * sizeof(T);
+            all[s] += bytes;
+            most[s] = std::max(most[s], bytes);
+        }
+        sum += all[s];
+        big = std::max(big, all[s]);
+        big1 = std::max(big1, most[s]);
+    }
+    const size_t want = std::max(big, std::min(sum, PARTS_BYTES));
+    if (b->parts_bytes < want) {
+        hipFree(b->parts);
+        b->parts = nullptr;
+        b->parts_bytes = 0;
+        b->parts_one = false;
+        size_t got = want;
+        // less room: smaller groups, down to the largest grid; then one
+        // direction of it
+        while (hipMalloc(&b->parts, got) != hipSuccess) {
+            (void)hipGetLastError();
+            b->parts = nullptr;
+            if (got > big) got = std::max(big, got / 2);
+            else if (!b->parts_one) { b->parts_one = true; got = big1; }
+            else return MAGIC_ENOMEM;
+        }
+        b->parts_bytes = got;
+    }
+    b->groups.clear();
+    const std::vector<size_t> &need = b->parts_one ? most : all;
+    size_t used = 0;
+    for (int s = 0; s < b->n; s++) {
+        if (b->groups.empty() || used + need[s] > b->parts_bytes) {
+            b->groups.push_back({s, s, {0, 0, 0, 0}});
+            used = 0;
+        }
+        used += need[s];
+        b->groups.back().hi = s + 1;
+    }
+    return MAGIC_OK;
+}
+
+// Sweep argument blocks, the groups and their blocks' lists (geometry only;
+// the step's dt factors are written by k_batch_prepare).  For the autotuner
+// (tuning) every block runs and the dt factors come from each scenario's
+// next dt.
 template <typename T>
 static int build_lists(magic_batch *b, bool tuning = false)
 {
-    std::vector<SweepArgsT<T>> args((size_t)b->n * 18);
-    std::vector<const int *> run((size_t)b->n * 18);
-    std::vector<std::vector<int4>> lists(18);
-    // tiles of longer pencils first (they take longest)
-    std::vector<int> order;
-    for (int s = 0; s < b->n; s++)
-        if (b->sc[s]) order.push_back(s);
-    for (int dir = 0; dir < 3; dir++) {
-        auto len = [&](int s) { return dir == 0 ? b->sc[s]->mx : dir == 1 ? b->sc[s]->my : b->sc[s]->mz; };
-        std::stable_sort(order.begin(), order.end(), [&](int x, int y) { return len(x) > len(y); });
-        for (int s : order) {
-            magic_ctx *c = b->sc[s];
-            const Dims &d = c->d;
-            const long long NXY = (long long)d.NX * d.NY;
-            SweepArgsT<T> a;
-            memset(&a, 0, sizeof(a));
-            sweep_form_args(c, a);
-            a.P = c->P;
-            a.mbc = c->mbc;
-            a.nspecadv = c->have_params ? c->prm.nspecadv : 0;
-            a.cfl_bits = &b->ctl_d[s].cfl_bits;
-            a.status = &b->ctl_d[s].err[0];
-            for (int m = 5; m < c->meqn; m++) a.comp[m] = m;
-            int a_is_g;
-            const double dt = b->ctl[s].dt > 0.0 ? b->ctl[s].dt : 1.0;
-            if (dir == 0) {          // step3.f:121-280 (g = y, h = z), tile axis y = g
-                a.comp[0] = 0; a.comp[1] = 1; a.comp[2] = 2; a.comp[3] = 3; a.comp[4] = 4;
-                a.n = c->mx; a.nA = c->my; a.nB = c->mz;
-                a.sN = 1; a.sA = d.NX; a.sB = NXY;
-                a.gravity = 0; a.sweep = 1;
-                a_is_g = 1;
-                if (tuning) { a.dtdn = dt / c->dx; a.fg = dt / c->dy; a.fh = dt / c->dz; }
-            } else if (dir == 1) {   // step3.f:289-450 (g = z, h = x), tile axis x = h
-                a.comp[0] = 0; a.comp[1] = 2; a.comp[2] = 3; a.comp[3] = 1; a.comp[4] = 4;
-                a.n = c->my; a.nA = c->mx; a.nB = c->mz;
-                a.sN = d.NX; a.sA = 1; a.sB = NXY;
-                a.gravity = 0; a.sweep = 2;
-                a_is_g = 0;
-                if (tuning) { a.dtdn = dt / c->dy; a.fg = dt / c->dz; a.fh = dt / c->dx; }
-            } else {                 // step3.f:459-621 (g = x, h = y), tile axis x = g
-                a.comp[0] = 0; a.comp[1] = 3; a.comp[2] = 1; a.comp[3] = 2; a.comp[4] = 4;
-                a.n = c->mz; a.nA = c->mx; a.nB = c->my;
-                a.sN = NXY; a.sA = 1; a.sB = d.NX;
-                a.gravity = 1; a.sweep = 3;
-                a_is_g = 1;
-                if (tuning) { a.dtdn = dt / c->dz; a.fg = dt / c->dx; a.fh = dt / c->dy; }
-            }
-            const int TA = tile_ta(b->shape[dir]);
-            const int ntiles = (a.nA + 2 + TA - 1) / TA;
-            for (int ca = 0; ca < 2; ca++)
-                for (int cb = 0; cb < 3; cb++) {
-                    const int k = ca * 3 + cb, ai = s * 18 + dir * 6 + k;
-                    SweepArgsT<T> t = a;
-                    t.cA = ca;
-                    t.cB = cb;
-                    if (!tuning && b->overlap && (dir == 1 || (dir == 2 && k >= 3))) t.qnew = (T *)c->dq[0];
-                    args[ai] = t;
-                    run[ai] = tuning ? b->one_d : &b->ctl_d[s].run;
-                    const int gx = (ntiles - ca + 1) / 2, gy = (a.nB + 1 - cb) / 3 + 1;
-                    for (int by = 0; by < gy; by++)
-                        for (int bx = 0; bx < gx; bx++) lists[dir * 6 + k].push_back(make_int4(ai, a_is_g, bx, by));
-                }
-        }
-    }
-    size_t total = 0;
-    for (int k = 0; k < 18; k++) {
-        b->item_off[k] = (int)total;
-        total += lists[k].size();
-    }
-    if (total > 0x7fffffff) return MAGIC_EUNSUPPORTED;
-    b->item_off[18] = (int)total;
+    TRY(build_groups<T>(b));
+    std::vector<SweepArgsT<T>> args((size_t)b->n * 3);
+    std::vector<const int *> run((size_t)b->n * 3);
     std::vector<int4> items;
-    items.reserve(total);
-    for (auto &l : lists) items.insert(items.end(), l.begin(), l.end());
+    b->sp64.assign(b->n, StepParts<double>{});
+    b->sp32.assign(b->n, StepParts<float>{});
+    for (auto &g : b->groups) {
+        T *next = (T *)b->parts;
+        for (int dir = 0; dir < 3; dir++) {
+            if (b->parts_one) next = (T *)b->parts;
+            g.off[dir] = (int)items.size();
+            for (int s = g.lo; s < g.hi; s++) {
+                magic_ctx *c = b->sc[s];
+                if (!c) continue;
+                SweepArgsT<T> &a = args[3 * s + dir];
+                StepParts<T> &sp = slot_parts(b, s, T());
+                memset(&a, 0, sizeof(a));
+                sweep_form_args(c, a);
+                sweep_geometry(c, dir, b->shape[dir], a, sp.d[dir]);
+                sp.nc = c->meqn;
+                a.nspecadv = c->have_params ? c->prm.nspecadv : 0;
+                a.cfl_bits = &b->ctl_d[s].cfl_bits;
+                a.status = &b->ctl_d[s].err[0];
+                if (b->parts_one) a.qold = (const T *)state_qold(c);
+                const double dt = b->ctl[s].dt > 0.0 ? b->ctl[s].dt : 1.0;
+                if (tuning) sweep_factors(c, dir, dt, a);
+                a.parts = next;
+                sp.d[dir].base = next;
+                next += parts_size(sp.d[dir], c->meqn, b->shape[dir]);
+                run[3 * s + dir] = tuning ? b->one_d : &b->ctl_d[s].run;
+                push_items(items, sp.d[dir], 3 * s + dir);
+                if (items.size() > 0x7fffffff) return MAGIC_EUNSUPPORTED;
+            }
+        }
+        g.off[3] = (int)items.size();
+    }
+    const size_t total = items.size();
     hipFree(b->items_d);
     b->items_d = nullptr;
     HIPCHECK(hipMalloc(&b->items_d, (total ? total : 1) * sizeof(int4)));
@@ -523,10 +522,6 @@ static int4 list_grid(const magic_batch *b, const magic_ctx *c, const int *bc, i
     case LG_DIF: return make_int4(blocks(d.mx, 64), blocks(d.my, 4), blocks(d.mz, batch_kb(d)), 0);
     case LG_INT: { const dim3 g = interior_grid(d); return make_int4(g.x, g.y, g.z, 0); }
     case LG_SPL: return g1(c->mz > c->mx ? blocks(c->mz - c->mx, 64) : 0);
-    case LG_MRG: {
-        const long long nv = P * b->meqn / (long long)(16 / elt(b)) + 1;
-        return g1(std::min<long long>(8192, blocks(nv, 256)));
-    }
     default: return g1(0);
     }
 }
@@ -553,7 +548,6 @@ static int build_ops(magic_batch *b)
             if (total > 0x7fffffff) return MAGIC_EUNSUPPORTED;
         }
         off[(size_t)lg * (b->cap + 1) + b->n] = (int)total;
-        b->ltotal[lg] = total;
     }
     for (int s = 0; s < b->n; s++) {
         magic_ctx *c = b->sc[s];
@@ -563,7 +557,8 @@ static int build_ops(magic_batch *b)
         if (!c) continue;
         o.d = c->d;
         form_ops(c, o);
-        o.dq = (T *)c->dq[0];
+        o.sp = slot_parts(b, s, T());
+        o.one = b->parts_one;
         o.nc = c->meqn;
         o.kb = batch_kb(c->d);
         o.spill = c->mz > c->mx ? c->mz - c->mx : 0;
@@ -581,6 +576,7 @@ static int build_ops(magic_batch *b)
         b->ndtr_cap = std::max(b->ndtr_cap, b->ctl[s].ndtr_cap);
         b->ndtrc_cap = std::max(b->ndtrc_cap, b->ctl[s].ndtrc_cap);
     }
+    b->loff = off;
     HIPCHECK(hipMemcpyAsync(b->ops_d, ops.data(), ops.size() * sizeof(ops[0]), hipMemcpyHostToDevice, b->stream));
     HIPCHECK(hipMemcpyAsync(b->loff_d, off.data(), off.size() * sizeof(int), hipMemcpyHostToDevice, b->stream));
     HIPCHECK(hipMemcpyAsync(b->lgdim_d, gdim.data(), gdim.size() * sizeof(int4), hipMemcpyHostToDevice, b->stream));
@@ -588,21 +584,14 @@ static int build_ops(magic_batch *b)
     return MAGIC_OK;
 }
 
-// persistent grid of each sweep direction and of each kernel class of the
-// work-list launches: as many workgroups as fit on the chip at once
-template <typename T, bool PERT>
+// persistent grid of each kernel class of the work-list launches: as many
+// workgroups as fit on the chip at once
+template <typename T>
 static int list_grids(magic_batch *b)
 {
     int dev = 0, ncu = 0;
     HIPCHECK(hipGetDevice(&dev));
     HIPCHECK(hipDeviceGetAttribute(&ncu, hipDeviceAttributeMultiprocessorCount, dev));
-    for (int dir = 0; dir < 3; dir++) {
-        const void *fn = list_fn<T, PERT>(b, dir);
-        if (!fn) return MAGIC_EUNSUPPORTED;
-        int occ = 0;
-        HIPCHECK(hipOccupancyMaxActiveBlocksPerMultiprocessor(&occ, fn, 256, 0));
-        b->grid[dir] = ncu * (occ > 0 ? occ : 1);
-    }
     for (int op = 0; op < NOP; op++) {
         const void *fn = batch_op_fn<T>(op);
         if (!fn) return MAGIC_EUNSUPPORTED;
@@ -614,8 +603,7 @@ static int list_grids(magic_batch *b)
     return MAGIC_OK;
 }
 
-// Retire the captured attempt: wait until no replay runs (the main stream
-// and the sweep overlap's stream), then destroy the executable graph and
+// Retire the captured attempt: wait until no replay runs, then destroy the executable graph and
 // the graph itself.  Called before any device buffer its kernels address
 // (control blocks, argument blocks, work and block lists, a scenario's
 // state) is freed or reallocated, so that no instantiated graph ever holds
@@ -624,7 +612,6 @@ static int drop_graph(magic_batch *b)
 {
     int st = MAGIC_OK;
     if (b->stream && hipStreamSynchronize(b->stream) != hipSuccess) st = MAGIC_EHIP;
-    if (b->side && hipStreamSynchronize(b->side) != hipSuccess) st = MAGIC_EHIP;
     if (b->exec) hipGraphExecDestroy(b->exec);
     if (b->graph) hipGraphDestroy(b->graph);
     b->exec = nullptr;
@@ -637,17 +624,7 @@ template <typename T, bool PERT>
 static int build_graph_t(magic_batch *b)
 {
     TRY(drop_graph(b));
-    TRY((list_grids<T, PERT>(b)));
-    if (b->overlap)
-        for (magic_ctx *c : b->sc) {
-            if (!c || c->dq[0]) continue;
-            const size_t bytes = (size_t)c->P * c->meqn * sizeof(T);
-            if (hipMalloc(&c->dq[0], bytes) != hipSuccess) {
-                c->dq[0] = nullptr;
-                return MAGIC_ENOMEM;
-            }
-            HIPCHECK(hipMemsetAsync(c->dq[0], 0, bytes, b->stream));   // before the capture
-        }
+    TRY(list_grids<T>(b));
     TRY(build_lists<T>(b));
     TRY(build_ops<T>(b));
     HIPCHECK(hipStreamBeginCapture(b->stream, hipStreamCaptureModeThreadLocal));
@@ -689,8 +666,8 @@ static int reserve(magic_batch *b, int want)
     const size_t ops_bytes = fp32(b) ? sizeof(BatchOps<float>) : sizeof(BatchOps<double>);
     if (hipMalloc(&b->ctl_d, cap * sizeof(ScenCtl)) != hipSuccess ||
         hipHostMalloc(&b->ctl_pin, cap * sizeof(ScenCtl), hipHostMallocDefault) != hipSuccess ||
-        hipMalloc(&b->args_d, (size_t)cap * 18 * args_bytes) != hipSuccess ||
-        hipMalloc(&b->run_d, (size_t)cap * 18 * sizeof(int *)) != hipSuccess ||
+        hipMalloc(&b->args_d, (size_t)cap * 3 * args_bytes) != hipSuccess ||
+        hipMalloc(&b->run_d, (size_t)cap * 3 * sizeof(int *)) != hipSuccess ||
         hipMalloc(&b->ops_d, (size_t)cap * ops_bytes) != hipSuccess ||
         hipMalloc(&b->loff_d, (size_t)NLG * (cap + 1) * sizeof(int)) != hipSuccess ||
         hipMalloc(&b->lgdim_d, (size_t)NLG * cap * sizeof(int4)) != hipSuccess)
@@ -762,14 +739,8 @@ extern "C" int magic_batch_create(int nscen, const int *dims, int meqn, int mbc,
     b->maux = maux;
     b->form = form;
     int st = MAGIC_OK;
-    if (hipStreamCreateWithFlags(&b->stream, hipStreamNonBlocking) != hipSuccess ||
-        hipStreamCreateWithFlags(&b->side, hipStreamNonBlocking) != hipSuccess)
-        st = MAGIC_EHIP;
-    if (st == MAGIC_OK && (hipEventCreateWithFlags(&b->sw_fork, hipEventDisableTiming) != hipSuccess ||
-                           hipEventCreateWithFlags(&b->sw_join, hipEventDisableTiming) != hipSuccess))
-        st = MAGIC_EHIP;
+    if (hipStreamCreateWithFlags(&b->stream, hipStreamNonBlocking) != hipSuccess) st = MAGIC_EHIP;
     if (st == MAGIC_OK) st = reserve(b, nscen > 0 ? nscen : 1);
-    if (st == MAGIC_OK) st = hipMalloc(&b->counters_d, 36 * sizeof(int)) == hipSuccess ? MAGIC_OK : MAGIC_ENOMEM;
     if (st == MAGIC_OK) st = hipMalloc(&b->one_d, sizeof(int)) == hipSuccess ? MAGIC_OK : MAGIC_ENOMEM;
     if (st == MAGIC_OK) {
         const int one = 1;
@@ -793,12 +764,9 @@ extern "C" int magic_batch_destroy(magic_batch *b)
     drop_graph(b);
     for (auto c : b->sc)
         if (c) magic_destroy(c);
-    hipFree(b->ctl_d); hipFree(b->args_d); hipFree(b->run_d); hipFree(b->items_d); hipFree(b->counters_d);
+    hipFree(b->ctl_d); hipFree(b->args_d); hipFree(b->run_d); hipFree(b->items_d); hipFree(b->parts);
     hipFree(b->one_d); hipFree(b->ops_d); hipFree(b->loff_d); hipFree(b->lgdim_d);
     if (b->ctl_pin) hipHostFree(b->ctl_pin);
-    if (b->sw_fork) hipEventDestroy(b->sw_fork);
-    if (b->sw_join) hipEventDestroy(b->sw_join);
-    if (b->side) hipStreamDestroy(b->side);
     if (b->stream) hipStreamDestroy(b->stream);
     delete b;
     return MAGIC_OK;
@@ -945,22 +913,20 @@ extern "C" int magic_batch_get_tile_shapes(magic_batch *b, int shapes[3])
     return MAGIC_OK;
 }
 
-// Every candidate reads the backup planes and adds into q (one list build
-// per shape and round, all directions); q is restored from the backup
-// afterwards.  The candidates' Courant numbers and reports land in the
-// control blocks' reduction fields, which the next attempt's prepare clears.
+// Every candidate reads q and writes its own increment blocks (one list
+// build per shape and round, all directions), so the states do not change.
+// The candidates' Courant numbers and reports land in the control blocks'
+// reduction fields, which the next attempt's prepare clears.
 template <typename T, bool PERT>
 static int tune_rounds(magic_batch *b, int reps, TuneClock &clk)
 {
     for (int r = 0; r <= reps; r++) {   // repetition 0 warms up and is not timed
         for (int sh = 0; sh < TILE_NSHAPE; sh++) {
             for (int k = 0; k < 3; k++) b->shape[k] = sh;
-            TRY((list_grids<T, PERT>(b)));
             TRY(build_lists<T>(b, true));
             for (int dir = 0; dir < 3; dir++) {
                 TRY(clk.mark(dir, sh, 0, b->stream));
-                HIPCHECK(hipMemsetAsync(b->counters_d, 0, 36 * sizeof(int), b->stream));
-                TRY((launch_dir<T, PERT>(b, dir)));
+                for (const auto &g : b->groups) TRY((launch_dirs<T, PERT>(b, g, dir, dir + 1)));
                 TRY(clk.mark(dir, sh, 1, b->stream));
             }
         }
@@ -986,12 +952,6 @@ extern "C" int magic_batch_tune(magic_batch *b, int reps, int shapes_out[3], flo
                                     hipMemcpyDeviceToDevice, b->stream));
     }
     int st = fp32(b) ? tune_rounds<float, true>(b, reps, clk) : tune_rounds<double, false>(b, reps, clk);
-    for (int s = 0; s < b->n; s++) {   // also after a failed round
-        magic_ctx *c = b->sc[s];
-        if (c && hipMemcpyAsync(state_q(c), state_qold(c), (size_t)c->P * c->meqn * elt(b), hipMemcpyDeviceToDevice,
-                                b->stream) != hipSuccess)
-            st = MAGIC_EHIP;
-    }
     if (st == MAGIC_OK && hipStreamSynchronize(b->stream) != hipSuccess) st = MAGIC_EHIP;
     if (st != MAGIC_OK) {
         for (int k = 0; k < 3; k++) b->shape[k] = saved[k];

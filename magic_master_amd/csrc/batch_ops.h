@@ -16,6 +16,7 @@
 #pragma once
 #include "batch.h"
 #include "bc_src.h"
+#include "parts.h"
 
 namespace magic {
 
@@ -23,7 +24,9 @@ namespace magic {
 template <typename T>
 struct BatchOps {
     Dims d;
-    T *q, *qold, *u, *qt, *ut, *dq;
+    T *q, *qold, *u, *qt, *ut;
+    StepParts<T> sp;  // the sweeps' increments, added in the conversion, or with one set by OP_ADD_PARTS
+    int one;          // the increments have room for one direction at a time
     int nc;          // meqn
     int kb;          // layers per block of the diffusion kernels (diff_kb)
     int spill;       // conduct.f:86-91 out-of-row writes (mz - mx when mz > mx, else 0)
@@ -42,7 +45,7 @@ struct BatchOps {
 // Kernel classes of the batched attempt
 enum {
     OP_BCX = 0, OP_BCY, OP_BCZ, OP_CLAMP, OP_BACKUP, OP_RESTORE, OP_CONVERT, OP_ZGHOST_UVW, OP_DIFF_CROSS,
-    OP_DIFF_XYZ, OP_COPY_Q5, OP_PASS, OP_CONDUCT_ZGHOST, OP_ZSPILL, OP_COPY_INTERIOR, OP_FINISH, OP_MERGE, NOP
+    OP_DIFF_XYZ, OP_COPY_Q5, OP_PASS, OP_CONDUCT_ZGHOST, OP_ZSPILL, OP_COPY_INTERIOR, OP_FINISH, OP_ADD_PARTS, NOP
 };
 // Block lists, one per launch geometry (a scenario whose faces of a bc3
 // kernel are all left to the caller has no blocks in that kernel's list):
@@ -53,8 +56,7 @@ enum {
 //   DIF diffusion passes     (mx/64, my/4, mz/kb)
 //   INT interior cells       (mx/64, my/4, mz)
 //   SPL conduct.f's out-of-row writes ((mz-mx)/64)
-//   MRG grid-stride q += dq of meqn planes
-enum { LG_FX = 0, LG_FY, LG_BCZ, LG_FZ, LG_ALL, LG_CPY, LG_CP1, LG_PAD, LG_DIF, LG_INT, LG_SPL, LG_MRG, NLG };
+enum { LG_FX = 0, LG_FY, LG_BCZ, LG_FZ, LG_ALL, LG_CPY, LG_CP1, LG_PAD, LG_DIF, LG_INT, LG_SPL, NLG };
 // OP_PASS variants: (out, interior source) = (qt, ut), (ut, qt), (q(5), ut)
 enum { PASS_QT_UT = 0, PASS_UT_QT, PASS_Q5_UT };
 
@@ -81,38 +83,14 @@ __device__ __forceinline__ int active_find(const int *pre, int n, int a)
 
 __device__ __forceinline__ int lohi(int m) { return m < 0 ? 0 : m; }
 
-// q += dq, dq = 0 over n elements for a scenario whose sweeps ran (the
-// sweep overlap of the batch): float4 or double2 vectors, grid-stride over
-// nblk blocks of 256 lanes
-template <typename T, class G>
-__device__ __forceinline__ void b_merge(const uint3 BI, unsigned nblk, T *__restrict__ q, T *__restrict__ dq,
-                                        long long n, const G &gate)
-{
-    if (!gate.on()) return;
-    constexpr int N = 16 / sizeof(T);
-    const long long nv = n / N;
-    const long long stride = (long long)nblk * blockDim.x;
-    const long long t0 = (long long)BI.x * blockDim.x + threadIdx.x;
-    for (long long i = t0; i < nv; i += stride)
-#pragma unroll
-        for (int e = 0; e < N; e++) {
-            q[i * N + e] = q[i * N + e] + dq[i * N + e];
-            dq[i * N + e] = T(0.0);
-        }
-    const long long r = nv * N + t0;   // the last n mod N elements
-    if (r < n) {
-        q[r] = q[r] + dq[r];
-        dq[r] = T(0.0);
-    }
-}
-
 // One launch of kernel class OP over the blocks of the scenarios' list
 // (off, gdim) whose gates are on.  Each workgroup of the persistent grid
 // first evaluates every slot's gate and lays the active slots' blocks end to
 // end in LDS (pre: active blocks before each slot), then takes active
 // blocks blockIdx.x, blockIdx.x + gridDim.x, ...; a launch whose gates are
 // all off ends after that scan.  arg: the velocity component of
-// OP_DIFF_XYZ (1-3), PASS_* * 4 + axis of OP_PASS.  The form's own bodies
+// OP_DIFF_XYZ (1-3), PASS_* * 4 + axis of OP_PASS, the direction of
+// OP_ADD_PARTS.  The form's own bodies
 // are reached through the FORM functor (FP32: bc_src32.hip, FP64:
 // bc_src.hip).  n <= BATCH_MAX_SLOTS (the host checks).
 template <typename T, int OP, class FORM>
@@ -222,8 +200,12 @@ __global__ __launch_bounds__(256) void k_batch_op(const BatchOps<T> *__restrict_
             b_copy_interior(bi, o.d, o.ut, o.qt, 1, g);
         } else if constexpr (OP == OP_FINISH) {
             FORM::finish(bi, o, g);
-        } else if constexpr (OP == OP_MERGE) {
-            b_merge(bi, (unsigned)gx, o.q, o.dq, P * o.nc, g);
+        } else if constexpr (OP == OP_ADD_PARTS) {
+            StepParts<T> one = o.sp;   // direction arg alone
+#pragma unroll
+            for (int k = 0; k < 3; k++)
+                if (k != arg) one.d[k].base = nullptr;
+            b_add_parts(bi, o.d, o.q, one, g);
         }
     }
 }

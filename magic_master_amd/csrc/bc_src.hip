@@ -69,26 +69,40 @@ __global__ void k_bc_z(Dims d, double *q, int nc, int lo, int hi, const double *
 // ---------------------------------------------------------------- src3 ---
 // conserved -> (rho, u', v', w', T') on every cell: src3.f90:242-304.
 // COL: the background comes as columns (index kk), else as planes.
-// dq (one grid's sweeps on two streams): the second stream's increments,
-// added to every component of the cell first, as a separate q += dq pass
-// would add them (nc components; tracers are only added).
+// sp: the sweeps' increments still to be added (sp.d[0].base null: none), to
+// every component of the cell first; tracers are only added.  The state is
+// read from qin and written to q: one grid hands over its two state buffers,
+// so that the state before the step stays behind as copyq3's backup without
+// a copy; a batch works in place (qin = q) and writes that state to keep.
+// Against adding a finished increment buffer this pass reads up to 1.36
+// times the increments, but they were written once and never added to.
 template <bool COL, class G>
-__device__ __forceinline__ void b_src_convert(const uint3 BI, Dims d, double *q, const Aux a, const G &gate,
-                                              const double *dq = nullptr, int nc = 0)
+__device__ __forceinline__ void b_src_convert(const uint3 BI, Dims d, const double *qin, double *q, double *keep, const Aux a,
+                                              const G &gate, const StepParts<double> &sp)
 {
     if (!gate.on()) return;
     PADDED_IJK
     const long long P = d.P;
-    if (dq) {
-        q[c] = q[c] + dq[c];
-        for (int m = 1; m < nc; m++) q[m * P + c] = q[m * P + c] + dq[m * P + c];
+    const bool has = sp.d[0].base != nullptr;
+    double v[10];
+#pragma unroll
+    for (int m = 0; m < 10; m++) v[m] = m < 5 || (has && m < sp.nc) ? qin[m * P + c] : 0.0;
+    if (has) {
+        double acc[10];
+        step_parts(sp, ip, jp, kk, d.mbc, acc);
+#pragma unroll
+        for (int m = 0; m < 10; m++) {
+            if (m >= 5 && m >= sp.nc) continue;
+            if (keep) keep[m * P + c] = v[m];
+            v[m] = v[m] + acc[m];
+            if (m == 0 || m >= 5) q[m * P + c] = v[m];
+        }
     }
     const long long x = COL ? (long long)kk : c;
     const double gamma1 = a.gam[x] - 1.0;
-    const double q1 = q[c], q2 = q[P + c], q3 = q[2 * P + c], q4 = q[3 * P + c];
+    const double q1 = v[0], q2 = v[1], q3 = v[2], q4 = v[3];
     const double a1 = a.rho[x], a2 = a.mx[x], a3 = a.my[x], a4 = a.mz[x];
-    const double qtemp = gamma1 * (q[4 * P + c] - 0.5 * (1.0 / q1) * (q2 * q2 + q3 * q3 + q4 * q4)) /
-                         (q1 * a.R[x]);
+    const double qtemp = gamma1 * (v[4] - 0.5 * (1.0 / q1) * (q2 * q2 + q3 * q3 + q4 * q4)) / (q1 * a.R[x]);
     const double auxtemp = gamma1 * (a.E[x] - 0.5 * (1.0 / a1) * (a2 * a2 + a3 * a3 + a4 * a4)) /
                            (a1 * a.R[x]);
     q[4 * P + c] = qtemp - auxtemp;
@@ -97,9 +111,9 @@ __device__ __forceinline__ void b_src_convert(const uint3 BI, Dims d, double *q,
     q[3 * P + c] = q4 / q1 - a4 / a1;
 }
 template <bool COL, class G>
-__global__ void k_src_convert(Dims d, double *q, const Aux a, G gate, const double *dq, int nc)
+__global__ void k_src_convert(Dims d, const double *qin, double *q, const Aux a, G gate, StepParts<double> sp)
 {
-    b_src_convert<COL>(uint3{blockIdx.x, blockIdx.y, blockIdx.z}, d, q, a, gate, dq, nc);
+    b_src_convert<COL>(uint3{blockIdx.x, blockIdx.y, blockIdx.z}, d, qin, q, (double *)nullptr, a, gate, sp);
 }
 
 // src3.f90:380-418 (reassembly), 430-445 / 514-607 (forcing), 616-626
@@ -182,7 +196,9 @@ struct Form64 {
     }
     __device__ static void convert(uint3 bi, const BatchOps<double> &o, const StepGate &g)
     {
-        b_src_convert<true>(bi, o.d, o.q, o.ax, g);
+        StepParts<double> sp = o.sp;
+        if (o.one) sp.d[0].base = nullptr;   // already in q
+        b_src_convert<true>(bi, o.d, o.q, o.q, o.qold, o.ax, g, sp);
     }
     __device__ static void finish(uint3 bi, const BatchOps<double> &o, const StepGate &g)
     {
@@ -200,7 +216,7 @@ const void *batch_op_fn<double>(int op)
     MAGIC_OP(OP_BCX) MAGIC_OP(OP_BCY) MAGIC_OP(OP_BCZ) MAGIC_OP(OP_CLAMP) MAGIC_OP(OP_BACKUP) MAGIC_OP(OP_RESTORE)
     MAGIC_OP(OP_CONVERT) MAGIC_OP(OP_ZGHOST_UVW) MAGIC_OP(OP_DIFF_CROSS) MAGIC_OP(OP_DIFF_XYZ) MAGIC_OP(OP_COPY_Q5)
     MAGIC_OP(OP_PASS) MAGIC_OP(OP_CONDUCT_ZGHOST) MAGIC_OP(OP_ZSPILL) MAGIC_OP(OP_COPY_INTERIOR) MAGIC_OP(OP_FINISH)
-    MAGIC_OP(OP_MERGE)
+    MAGIC_OP(OP_ADD_PARTS)
 #undef MAGIC_OP
     default: return nullptr;
     }
@@ -213,8 +229,9 @@ template __global__ void k_clamp<double, NoGate>(double *, long long, int, NoGat
 template __global__ void k_zghost_uvw<double, NoGate>(Dims, double *, NoGate);
 template __global__ void k_bc_z<NoGate>(Dims, double *, int, int, int, const double *, const double *, const double *,
                                         const double *, const double *, NoGate);
-template __global__ void k_src_convert<false, NoGate>(Dims, double *, const Aux, NoGate, const double *, int);
-template __global__ void k_src_convert<true, NoGate>(Dims, double *, const Aux, NoGate, const double *, int);
+template __global__ void k_src_convert<false, NoGate>(Dims, const double *, double *, const Aux, NoGate, StepParts<double>);
+template __global__ void k_src_convert<true, NoGate>(Dims, const double *, double *, const Aux, NoGate, StepParts<double>);
+template __global__ void k_add_parts<double, NoGate>(Dims, double *, StepParts<double>, NoGate);
 template __global__ void k_src_finish<false, NoGate>(Dims, double *, int, const Aux, Forcing, NoGate);
 template __global__ void k_src_finish<true, NoGate>(Dims, double *, int, const Aux, Forcing, NoGate);
 template __global__ void k_diff_xyz<double, true, NoGate>(Dims, double *, const double *, const double *, double, double,

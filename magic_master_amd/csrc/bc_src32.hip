@@ -90,22 +90,33 @@ __global__ void k32_bc_z(Dims d, float *q, int nc, int lo, int hi, Zr32 zr, G ga
 // stored values are FP32): T' is a small difference of the pressure and
 // density perturbations' background-weighted parts, and E' a sum of such
 // parts, whose FP32 rounding the flow carries into the thin upper layers.
-// dq: as the FP64 form's conversion (bc_src.hip), the second sweep
-// stream's increments added first, each rounded to FP32 as q += dq rounds
+// qin, q, keep and the step's increments: as the FP64 form's conversion
+// (bc_src.hip)
 template <class G>
-__device__ __forceinline__ void b32_src_convert(const uint3 BI, Dims d, float *q, Col32 col, const G &gate,
-                                                const float *dq = nullptr, int nc = 0)
+__device__ __forceinline__ void b32_src_convert(const uint3 BI, Dims d, const float *qin, float *q, float *keep, Col32 col,
+                                                const G &gate, const StepParts<float> &sp)
 {
     if (!gate.on()) return;
     PADDED_IJK
     const long long P = d.P;
-    if (dq) {
-        q[c] = q[c] + dq[c];
-        for (int m = 1; m < nc; m++) q[m * P + c] = q[m * P + c] + dq[m * P + c];
+    const bool has = sp.d[0].base != nullptr;
+    float v[10];
+#pragma unroll
+    for (int m = 0; m < 10; m++) v[m] = m < 5 || (has && m < sp.nc) ? qin[m * P + c] : 0.0f;
+    if (has) {
+        float acc[10];
+        step_parts(sp, ip, jp, kk, d.mbc, acc);
+#pragma unroll
+        for (int m = 0; m < 10; m++) {
+            if (m >= 5 && m >= sp.nc) continue;
+            if (keep) keep[m * P + c] = v[m];
+            v[m] = v[m] + acc[m];
+            if (m == 0 || m >= 5) q[m * P + c] = v[m];
+        }
     }
     const double rb = col.rho[kk], Eb = col.E[kk], g1 = col.gam[kk] - 1.0, R = col.R[kk];
-    const double rp = q[c], rho = rb + rp;
-    const double m2 = q[P + c], m3 = q[2 * P + c], m4 = q[3 * P + c], ep = q[4 * P + c];
+    const double rp = v[0], rho = rb + rp;
+    const double m2 = v[1], m3 = v[2], m4 = v[3], ep = v[4];
     const double irho = 1.0 / rho;
     const double pp = g1 * (ep - 0.5 * (m2 * m2 + m3 * m3 + m4 * m4) * irho);
     q[4 * P + c] = (float)((pp - rp * (g1 * Eb / rb)) * irho / R);
@@ -114,9 +125,9 @@ __device__ __forceinline__ void b32_src_convert(const uint3 BI, Dims d, float *q
     q[3 * P + c] = (float)(m4 * irho);
 }
 template <class G>
-__global__ void k32_src_convert(Dims d, float *q, Col32 col, G gate, const float *dq, int nc)
+__global__ void k32_src_convert(Dims d, const float *qin, float *q, Col32 col, G gate, StepParts<float> sp)
 {
-    b32_src_convert(uint3{blockIdx.x, blockIdx.y, blockIdx.z}, d, q, col, gate, dq, nc);
+    b32_src_convert(uint3{blockIdx.x, blockIdx.y, blockIdx.z}, d, qin, q, (float *)nullptr, col, gate, sp);
 }
 
 // Reassembly, plume forcing and tracer clamp on the interior
@@ -178,7 +189,9 @@ struct Form32 {
     }
     __device__ static void convert(uint3 bi, const BatchOps<float> &o, const StepGate &g)
     {
-        b32_src_convert(bi, o.d, o.q, o.col, g);
+        StepParts<float> sp = o.sp;
+        if (o.one) sp.d[0].base = nullptr;   // already in q
+        b32_src_convert(bi, o.d, o.q, o.q, o.qold, o.col, g, sp);
     }
     __device__ static void finish(uint3 bi, const BatchOps<float> &o, const StepGate &g)
     {
@@ -196,7 +209,7 @@ const void *batch_op_fn<float>(int op)
     MAGIC_OP(OP_BCX) MAGIC_OP(OP_BCY) MAGIC_OP(OP_BCZ) MAGIC_OP(OP_CLAMP) MAGIC_OP(OP_BACKUP) MAGIC_OP(OP_RESTORE)
     MAGIC_OP(OP_CONVERT) MAGIC_OP(OP_ZGHOST_UVW) MAGIC_OP(OP_DIFF_CROSS) MAGIC_OP(OP_DIFF_XYZ) MAGIC_OP(OP_COPY_Q5)
     MAGIC_OP(OP_PASS) MAGIC_OP(OP_CONDUCT_ZGHOST) MAGIC_OP(OP_ZSPILL) MAGIC_OP(OP_COPY_INTERIOR) MAGIC_OP(OP_FINISH)
-    MAGIC_OP(OP_MERGE)
+    MAGIC_OP(OP_ADD_PARTS)
 #undef MAGIC_OP
     default: return nullptr;
     }
@@ -205,7 +218,8 @@ const void *batch_op_fn<float>(int op)
 // instantiations of the single-grid kernels (the batched driver's are
 // k_batch_op, above)
 template __global__ void k32_bc_z<NoGate>(Dims, float *, int, int, int, Zr32, NoGate);
-template __global__ void k32_src_convert<NoGate>(Dims, float *, Col32, NoGate, const float *, int);
+template __global__ void k32_src_convert<NoGate>(Dims, const float *, float *, Col32, NoGate, StepParts<float>);
+template __global__ void k_add_parts<float, NoGate>(Dims, float *, StepParts<float>, NoGate);
 template __global__ void k32_src_finish<NoGate>(Dims, float *, int, Col32, Forcing, NoGate);
 
 // reference AoS q(meqn, i, j, k) (FP64, full state) <-> perturbation planes:

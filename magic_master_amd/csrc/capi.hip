@@ -148,7 +148,6 @@ extern "C" int magic_create_form(int mx, int my, int mz, int meqn, int mbc, int 
     bool ok = hipStreamCreateWithFlags(&c->stream, hipStreamNonBlocking) == hipSuccess;
     ok = ok && hipMalloc(&c->stage, P * meqn * sizeof(double)) == hipSuccess;
     ok = ok && hipMalloc(&c->dscal, 8 * sizeof(unsigned long long)) == hipSuccess;
-    ok = ok && hipMalloc(&c->sink, 4096) == hipSuccess;
     ok = ok && hipHostMalloc(&c->hscal, HSCAL_WORDS * sizeof(unsigned long long), hipHostMallocDefault) == hipSuccess;
     if (ok && form == MAGIC_FORM_FP32P) {
         const size_t NZ = (size_t)c->d.NZ;
@@ -210,18 +209,10 @@ extern "C" int magic_destroy(magic_ctx *c)
     drain_timing(c);
     for (auto e : c->pool) hipEventDestroy(e);
     hipFree(c->q); hipFree(c->qold); hipFree(c->aux); hipFree(c->zratio); hipFree(c->stage);
-    hipFree(c->u); hipFree(c->qt); hipFree(c->ut); hipFree(c->dscal); hipFree(c->sink);
+    hipFree(c->u); hipFree(c->qt); hipFree(c->ut); hipFree(c->dscal);
     hipFree(c->q32); hipFree(c->qold32); hipFree(c->u32); hipFree(c->qt32); hipFree(c->ut32);
     hipFree(c->col32); hipFree(c->bg64); hipFree(c->col64); hipFree(c->sums_d);
-    hipFree(c->largs); hipFree(c->lrun); hipFree(c->lone); hipFree(c->lcnt);
-    for (auto &d : c->litems)
-        for (int4 *p : d) hipFree(p);
-    if (c->side) hipStreamSynchronize(c->side);
-    hipFree(c->dq[0]);
-    hipFree(c->dq[1]);
-    if (c->ev_fork) hipEventDestroy(c->ev_fork);
-    if (c->ev_join) hipEventDestroy(c->ev_join);
-    if (c->side) hipStreamDestroy(c->side);
+    hipFree(c->largs); hipFree(c->lrun); hipFree(c->lone); hipFree(c->items); hipFree(c->parts);
     if (c->hscal) hipHostFree(c->hscal);
     if (c->snap_conv) hipEventDestroy(c->snap_conv);
     if (c->snap_done) hipEventDestroy(c->snap_done);
@@ -636,129 +627,6 @@ static int launch_sweep(magic_ctx *c, SweepArgs a, int *nl)
     return MAGIC_OK;
 }
 
-// Argument blocks of colours k0 .. k1-1 of direction dir (slot 6 dir + k),
-// written on the stream of their launches, so that a later call may change
-// them while these launches are still queued
-template <typename T>
-__global__ void k_put_args(SweepArgsT<T> *slots, SweepArgsT<T> a, int dir, int k0, int k1)
-{
-    const int k = k0 + (int)threadIdx.x;
-    if (k >= k1) return;
-    SweepArgsT<T> s = a;
-    s.cA = k / 3;
-    s.cB = k % 3;
-    slots[dir * 6 + k] = s;
-}
-
-// The work-list buffers of the context (first tiled sweep)
-template <typename T>
-static int list_setup(magic_ctx *c)
-{
-    if (c->largs) return MAGIC_OK;
-    if (hipMalloc(&c->largs, 18 * sizeof(SweepArgsT<T>)) != hipSuccess ||
-        hipMalloc(&c->lrun, 18 * sizeof(int *)) != hipSuccess || hipMalloc(&c->lone, sizeof(int)) != hipSuccess ||
-        hipMalloc(&c->lcnt, 36 * sizeof(int)) != hipSuccess) {
-        hipFree(c->largs); hipFree(c->lrun); hipFree(c->lone); hipFree(c->lcnt);
-        c->largs = nullptr; c->lrun = nullptr; c->lone = nullptr; c->lcnt = nullptr;
-        return MAGIC_ENOMEM;
-    }
-    const int one = 1;
-    const int *run[18];
-    for (auto &r : run) r = c->lone;
-    const int zero[36] = {};
-    HIPCHECK(hipMemcpy(c->lone, &one, sizeof(int), hipMemcpyHostToDevice));
-    HIPCHECK(hipMemcpy(c->lrun, run, sizeof(run), hipMemcpyHostToDevice));
-    HIPCHECK(hipMemcpy(c->lcnt, zero, sizeof(zero), hipMemcpyHostToDevice));
-    return MAGIC_OK;
-}
-
-// The tiles of direction dir in shape sh, colour by colour (built once)
-static int list_items(magic_ctx *c, int dir, int sh, int nA, int nB, int a_is_g)
-{
-    if (c->litems[dir][sh]) return MAGIC_OK;
-    const int TA = tile_ta(sh);
-    const int ntiles = (nA + 2 + TA - 1) / TA;
-    std::vector<int4> items;
-    int *off = c->litem_off[dir][sh];
-    for (int ca = 0; ca < 2; ca++)
-        for (int cb = 0; cb < 3; cb++) {
-            const int k = 3 * ca + cb;
-            off[k] = (int)items.size();
-            const int gx = (ntiles - ca + 1) / 2, gy = (nB + 1 - cb) / 3 + 1;
-            for (int by = 0; by < gy; by++)
-                for (int bx = 0; bx < gx; bx++) items.push_back(make_int4(dir * 6 + k, a_is_g, bx, by));
-        }
-    off[6] = (int)items.size();
-    int4 *d = nullptr;
-    HIPCHECK(hipMalloc(&d, (items.size() ? items.size() : 1) * sizeof(int4)));
-    if (hipMemcpy(d, items.data(), items.size() * sizeof(int4), hipMemcpyHostToDevice) != hipSuccess) {
-        hipFree(d);
-        return MAGIC_EHIP;
-    }
-    c->litems[dir][sh] = d;
-    return MAGIC_OK;
-}
-
-// Colour launches k0 .. k1-1 (k = 3 ca + cb) of one direction: the sweep
-// kernel over this grid's tiles of each colour.  The FP64 form runs it as a
-// persistent grid over the work list (925 Mcell-updates/s on the full-domain
-// workload, against 918 for one tile per workgroup), the FP32 form one tile
-// per workgroup (1785 against 1728), which lets the two streams of the sweep
-// overlap share the compute units tile by tile.
-template <typename T, bool PERT, int NTR>
-static int launch_tile(magic_ctx *c, SweepArgsT<T> a, int sh, int a_is_g, int *nl, hipStream_t s, int k0, int k1,
-                       bool put)
-{
-    const void *fn = tile_list_fn<T, PERT, NTR>(sh);
-    if (!fn) return MAGIC_EARG;
-    const int dir = a.sweep - 1;
-    TRY(list_setup<T>(c));
-    TRY(list_items(c, dir, sh, a.nA, a.nB, a_is_g));
-    if (put) {   // else the caller wrote every slot of this step (k_put_step_args)
-        k_put_args<T><<<1, 64, 0, s>>>((SweepArgsT<T> *)c->largs, a, dir, k0, k1);
-        TRY(launch_check());
-    }
-    constexpr bool PER_TILE = sizeof(T) == 4;
-    if (!PER_TILE && !c->lgrid[sh]) {
-        int dev = 0, ncu = 0, occ = 0;
-        HIPCHECK(hipGetDevice(&dev));
-        HIPCHECK(hipDeviceGetAttribute(&ncu, hipDeviceAttributeMultiprocessorCount, dev));
-        HIPCHECK(hipOccupancyMaxActiveBlocksPerMultiprocessor(&occ, fn, 256, 0));
-        c->lgrid[sh] = ncu * (occ > 0 ? occ : 1);
-    }
-    const int *off = c->litem_off[dir][sh];
-    for (int k = k0; k < k1; k++) {
-        int n = off[k + 1] - off[k];
-        if (n <= 0) continue;
-        const SweepArgsT<T> *args = (const SweepArgsT<T> *)c->largs;
-        const int4 *items = c->litems[dir][sh] + off[k];
-        const int *const *run = c->lrun;
-        int *cnt = c->lcnt + 2 * (dir * 6 + k);
-        // one tile per workgroup: tiles (bx, by) of colour k as the list holds them
-        const int TA = tile_ta(sh), ntiles = (a.nA + 2 + TA - 1) / TA, ca = k / 3;
-        int4 grid = PER_TILE ? make_int4((ntiles - ca + 1) / 2, dir * 6 + k, a_is_g, 0) : make_int4(0, 0, 0, 0);
-        void *kargs[] = {&args, &items, &n, &run, &cnt, &grid};
-        HIPCHECK(hipLaunchKernel(fn, dim3(PER_TILE ? n : std::min(c->lgrid[sh], n)), dim3(256), kargs, 0, s));
-        ++*nl;
-    }
-    return MAGIC_OK;
-}
-
-template <typename T, bool PERT>
-static int tile_dispatch(magic_ctx *c, const SweepArgsT<T> &a, int sh, int a_is_g, int *nl, hipStream_t s, int k0,
-                         int k1, bool put)
-{
-    switch (ntracer(c)) {
-    case 0: return launch_tile<T, PERT, 0>(c, a, sh, a_is_g, nl, s, k0, k1, put);
-    case 1: return launch_tile<T, PERT, 1>(c, a, sh, a_is_g, nl, s, k0, k1, put);
-    case 2: return launch_tile<T, PERT, 2>(c, a, sh, a_is_g, nl, s, k0, k1, put);
-    case 3: return launch_tile<T, PERT, 3>(c, a, sh, a_is_g, nl, s, k0, k1, put);
-    case 4: return launch_tile<T, PERT, 4>(c, a, sh, a_is_g, nl, s, k0, k1, put);
-    case 5: return launch_tile<T, PERT, 5>(c, a, sh, a_is_g, nl, s, k0, k1, put);
-    default: return MAGIC_EUNSUPPORTED;
-    }
-}
-
 static bool use_tile()
 {
     const char *e = getenv("MAGIC_SWEEP");
@@ -808,225 +676,172 @@ static void dir_args(const magic_ctx *c, SweepArgsT<T> &a, int dir, double dt)
     }
 }
 
-// One directional sweep with the tiled kernel of shape sh (or the pencil
-// kernel of the FP64 form).  The tile axis is g for the x- and z-sweeps and
-// x = h for the y-sweep, so that the y- and z-sweeps tile along rows of x.
+// Buffers of the tiled sweeps for the context's shapes: argument blocks and
+// run flags, the workgroups' blocks, and the increment buffer.  Where the
+// device has no room for the three directions' increments, one direction's
+// are kept and added to q before the next direction runs.
 template <typename T>
-static int tile_dir_args(const magic_ctx *c, SweepArgsT<T> &a, int dir, double dt)
+static int sweep_setup(magic_ctx *c)
 {
-    dir_args(c, a, dir, dt);
-    if (dir == 1) {
-        a.nA = c->mx; a.nB = c->mz;
-        a.sA = 1; a.sB = (long long)c->d.NX * c->d.NY;
-        return 0;
-    }
-    return 1;
-}
-
-// Argument blocks of all 18 launches of one step3 (slot 6 dir + k), from
-// each direction's block; dq: the sweep overlap's buffer, which the y-sweep
-// and the last three z colours add into (nullptr: no overlap).  Launched on
-// the context's stream before any of the step's sweeps, while nothing else
-// runs, so it never waits for a compute unit behind a sweep.
-template <typename T>
-__global__ void k_put_step_args(SweepArgsT<T> *slots, SweepArgsT<T> ax, SweepArgsT<T> ay, SweepArgsT<T> az, T *dq)
-{
-    const int k = (int)threadIdx.x;
-    if (k >= 18) return;
-    const int dir = k / 6, kk = k % 6;
-    SweepArgsT<T> s = dir == 0 ? ax : dir == 1 ? ay : az;
-    s.cA = kk / 3;
-    s.cB = kk % 3;
-    if (dq && (dir == 1 || (dir == 2 && kk >= 3))) s.qnew = dq;
-    slots[k] = s;
-}
-
-template <typename T>
-static int put_step_args(magic_ctx *c, const SweepArgsT<T> &a, double dt, T *dq)
-{
-    TRY(list_setup<T>(c));
-    SweepArgsT<T> ax = a, ay = a, az = a;
-    tile_dir_args(c, ax, 0, dt);
-    tile_dir_args(c, ay, 1, dt);
-    tile_dir_args(c, az, 2, dt);
-    k_put_step_args<T><<<1, 64, 0, c->stream>>>((SweepArgsT<T> *)c->largs, ax, ay, az, dq);
-    return launch_check();
-}
-
-template <typename T, bool PERT>
-static int sweep_dir(magic_ctx *c, SweepArgsT<T> a, int dir, double dt, int sh, bool tile, int *nl,
-                     hipStream_t s = nullptr, int k0 = 0, int k1 = 6, bool put = true)
-{
-    if (!s) s = c->stream;
-    if (tile) {
-        const int a_is_g = tile_dir_args(c, a, dir, dt);
-        return tile_dispatch<T, PERT>(c, a, sh, a_is_g, nl, s, k0, k1, put);
-    }
-    dir_args(c, a, dir, dt);
-    if (s != c->stream || k0 != 0 || k1 != 6) return MAGIC_EUNSUPPORTED;
-    if constexpr (!PERT) return sweep_dispatch(c, a, nl);
-    return MAGIC_EUNSUPPORTED;
-}
-
-// 16-byte vectors of the state's type
-template <typename T>
-struct Vec16;
-template <>
-struct Vec16<double> { typedef double2 type; static constexpr int N = 2; };
-template <>
-struct Vec16<float> { typedef float4 type; static constexpr int N = 4; };
-
-// q += dq over n elements (both 16-byte aligned): 16-byte loads and stores,
-// four of each pair in flight per lane
-template <typename T>
-__device__ __forceinline__ void vadd(typename Vec16<T>::type &a, const typename Vec16<T>::type &b)
-{
-    a.x = a.x + b.x;
-    a.y = a.y + b.y;
-    if constexpr (Vec16<T>::N == 4) {
-        a.z = a.z + b.z;
-        a.w = a.w + b.w;
-    }
-}
-
-template <typename T>
-__global__ void k_merge(T *__restrict__ q, const T *__restrict__ dq, long long n)
-{
-    using V = typename Vec16<T>::type;
-    constexpr int N = Vec16<T>::N, U = 4;
-    const long long nv = n / N;
-    V *qv = reinterpret_cast<V *>(q);
-    const V *dv = reinterpret_cast<const V *>(dq);
-    const long long stride = (long long)gridDim.x * blockDim.x;
-    const long long t0 = (long long)blockIdx.x * blockDim.x + threadIdx.x;
-    long long i = t0;
-    for (; i + (U - 1) * stride < nv; i += U * stride) {
-        V a[U], b[U];
-#pragma unroll
-        for (int u = 0; u < U; u++) {
-            a[u] = qv[i + u * stride];
-            b[u] = dv[i + u * stride];
-        }
-#pragma unroll
-        for (int u = 0; u < U; u++) {
-            vadd<T>(a[u], b[u]);
-            qv[i + u * stride] = a[u];
-        }
-    }
-    for (; i < nv; i += stride) {
-        V a = qv[i];
-        vadd<T>(a, dv[i]);
-        qv[i] = a;
-    }
-    const long long r = nv * N + t0;   // the last n mod N elements
-    if (r < n) q[r] = q[r] + dq[r];
-}
-
-template <typename T>
-__global__ void k_fill_zero(T *__restrict__ p, long long n)
-{
-    const long long stride = (long long)gridDim.x * blockDim.x;
-    for (long long i = (long long)blockIdx.x * blockDim.x + threadIdx.x; i < n; i += stride) p[i] = T(0.0);
-}
-
-// Whether the y-sweep runs on the second stream (a context that owns its
-// stream and has not turned the overlap off; MAGIC_SWEEP_OVERLAP=0 keeps
-// the three sweeps on one stream for every context).
-static bool overlap_sweeps(const magic_ctx *c)
-{
-    const char *e = getenv("MAGIC_SWEEP_OVERLAP");
-    return c->overlap && c->own_stream && !(e && strcmp(e, "0") == 0);
-}
-
-template <typename T>
-static int side_setup(magic_ctx *c)
-{
-    if (!c->side) {
-        HIPCHECK(hipStreamCreateWithFlags(&c->side, hipStreamNonBlocking));
-        HIPCHECK(hipEventCreateWithFlags(&c->ev_fork, hipEventDisableTiming));
-        HIPCHECK(hipEventCreateWithFlags(&c->ev_join, hipEventDisableTiming));
-    }
-    if (c->dq_clear) return MAGIC_OK;
-    const long long n = (long long)c->meqn * c->P;
-    for (int k = 0; k < 2; k++) {
-        if (!c->dq[k] && hipMalloc(&c->dq[k], (size_t)n * sizeof(T)) != hipSuccess) {
-            c->dq[k] = nullptr;
+    if (!c->largs) {
+        if (hipMalloc(&c->largs, 3 * sizeof(SweepArgsT<T>)) != hipSuccess ||
+            hipMalloc(&c->lrun, 3 * sizeof(int *)) != hipSuccess || hipMalloc(&c->lone, sizeof(int)) != hipSuccess) {
+            hipFree(c->largs); hipFree(c->lrun); hipFree(c->lone);
+            c->largs = nullptr; c->lrun = nullptr; c->lone = nullptr;
+            (void)hipGetLastError();
             return MAGIC_ENOMEM;
         }
-        k_fill_zero<T><<<(unsigned)std::min<long long>(blocks(n, 256), 8192), 256, 0, c->stream>>>((T *)c->dq[k], n);
-        TRY(launch_check());
+        const int one = 1;
+        const int *run[3] = {c->lone, c->lone, c->lone};
+        HIPCHECK(hipMemcpy(c->lone, &one, sizeof(int), hipMemcpyHostToDevice));
+        HIPCHECK(hipMemcpy(c->lrun, run, sizeof(run), hipMemcpyHostToDevice));
     }
-    c->dq_clear = true;
+    if (c->items && memcmp(c->item_shape, c->shape, sizeof(c->shape)) == 0) return MAGIC_OK;
+    std::vector<int4> items;
+    int off[4] = {0, 0, 0, 0};
+    size_t all = 0, most = 0;
+    for (int dir = 0; dir < 3; dir++) {
+        SweepArgsT<T> a;
+        SweepParts<T> p;
+        sweep_geometry(c, dir, c->shape[dir], a, p);
+        push_items(items, p, dir);
+        off[dir + 1] = (int)items.size();
+        const size_t bytes = (size_t)parts_size(p, c->meqn, c->shape[dir]) * sizeof(T);
+        all += bytes;
+        most = std::max(most, bytes);
+    }
+    HIPCHECK(hipStreamSynchronize(c->stream));   // nothing reads the old lists or increments any more
+    hipFree(c->items);
+    c->items = nullptr;
+    if (c->parts_bytes < all) {
+        hipFree(c->parts);
+        c->parts = nullptr;
+        c->parts_bytes = 0;
+        c->parts_one = false;
+        size_t got = all;
+        if (hipMalloc(&c->parts, all) != hipSuccess) {
+            (void)hipGetLastError();
+            got = most;
+            c->parts_one = true;
+            if (hipMalloc(&c->parts, most) != hipSuccess) {
+                (void)hipGetLastError();
+                c->parts = nullptr;
+                return MAGIC_ENOMEM;
+            }
+        }
+        c->parts_bytes = got;
+    } else {
+        c->parts_one = false;
+    }
+    if (hipMalloc(&c->items, items.size() * sizeof(int4)) != hipSuccess) {
+        (void)hipGetLastError();
+        c->items = nullptr;
+        return MAGIC_ENOMEM;
+    }
+    HIPCHECK(hipMemcpy(c->items, items.data(), items.size() * sizeof(int4), hipMemcpyHostToDevice));
+    memcpy(c->item_off, off, sizeof(off));
+    memcpy(c->item_shape, c->shape, sizeof(c->shape));
     return MAGIC_OK;
 }
 
-// The three sweeps of step3 (lib/step3.f:121-621) on argument block a,
-// whose state pointers and form-specific fields are already set.
-//
-// The sweeps only add into q, each from the backup, so they can run on two
-// streams into two buffers: the x-sweep and the first three colour launches
-// of the z-sweep add into q on the context's stream, the y-sweep and the
-// other three z launches into a zeroed buffer dq on the second stream (9
-// launches each), and q += dq once both are done.  Each launch's last wave
-// of workgroups leaves most compute units idle (4-7 rounds of one workgroup
-// per CU per launch); with two streams the other stream's workgroups fill
-// them.  Two buffers alternate: the one the previous call added to q is
-// cleared on the second stream while this call's sweeps run.  The order of
-// the additions into every element is fixed (x and the first z colours,
-// then dq's sum of y and the other z colours), so the result is the same
-// on every run.
-template <typename T, bool PERT>
-static int step3_sweeps(magic_ctx *c, const SweepArgsT<T> &a, double dt, bool defer_merge = false)
+// The argument blocks of one step's sweeps, and the step's reductions back
+// to zero.  Launched before the sweeps on their stream.
+template <typename T>
+struct StepArgs {
+    SweepArgsT<T> d[3];
+};
+template <typename T>
+__global__ void k_put_step_args(SweepArgsT<T> *slots, StepArgs<T> a, unsigned long long *scal)
 {
-    const bool tile = PERT || use_tile();
-    if (tile && overlap_sweeps(c)) {
-        TRY(side_setup<T>(c));
-        // a launch that fails below leaves the buffers unknown: cleared again next time
-        c->dq_clear = false;
-        const long long n = (long long)c->meqn * c->P;
-        T *dq = (T *)c->dq[c->dq_cur], *dq_next = (T *)c->dq[c->dq_cur ^ 1];
-        SweepArgsT<T> ay = a;
-        ay.qnew = dq;
-        TRY(put_step_args<T>(c, a, dt, dq));
-        HIPCHECK(hipEventRecord(c->ev_fork, c->stream));
-        HIPCHECK(hipStreamWaitEvent(c->side, c->ev_fork, 0));
-        // dq_next was added to q by the previous call, before the fork
-        k_fill_zero<T><<<(unsigned)std::min<long long>(blocks(n, 256), 8192), 256, 0, c->side>>>(dq_next, n);
-        TRY(launch_check());
-        {
-            Span sp(c, TC_SWY, 0, c->side);
-            TRY((sweep_dir<T, PERT>(c, ay, 1, dt, c->shape[1], true, &sp.n, c->side, 0, 6, false)));
+    if (threadIdx.x < 3) slots[threadIdx.x] = a.d[threadIdx.x];
+    else if (threadIdx.x >= 8 && threadIdx.x < 16) scal[threadIdx.x - 8] = 0ull;
+}
+
+// Argument blocks for step dt from base (state pointers and form-specific
+// fields set), and the descriptors of the parts they fill
+template <typename T>
+static int put_step_args(magic_ctx *c, const SweepArgsT<T> &base, double dt, StepParts<T> &sp)
+{
+    TRY(sweep_setup<T>(c));
+    StepArgs<T> s;
+    sp.nc = c->meqn;
+    T *next = (T *)c->parts;
+    for (int dir = 0; dir < 3; dir++) {
+        s.d[dir] = base;
+        sweep_geometry(c, dir, c->shape[dir], s.d[dir], sp.d[dir]);
+        sweep_factors(c, dir, dt, s.d[dir]);
+        s.d[dir].parts = next;
+        sp.d[dir].base = next;
+        if (!c->parts_one) next += parts_size(sp.d[dir], c->meqn, c->shape[dir]);
+    }
+    k_put_step_args<T><<<1, 64, 0, c->stream>>>((SweepArgsT<T> *)c->largs, s, c->dscal);
+    return launch_check();
+}
+
+// One launch over the blocks of directions d0 .. d1-1 (of one shape)
+template <typename T, bool PERT>
+static int launch_tile(magic_ctx *c, int d0, int d1)
+{
+    const void *fn = tile_fn<T, PERT>(ntracer(c), c->shape[d0]);
+    if (!fn) return MAGIC_EARG;
+    const SweepArgsT<T> *args = (const SweepArgsT<T> *)c->largs;
+    const int4 *items = c->items + c->item_off[d0];
+    const int *const *run = c->lrun;
+    void *kargs[] = {&args, &items, &run};
+    Span sp(c, NTC, 1);
+    const float blocks_ = (float)(c->item_off[d1] - c->item_off[d0]);
+    for (int d = d0; d < d1; d++) sp.share[d] = (c->item_off[d + 1] - c->item_off[d]) / blocks_;
+    HIPCHECK(hipLaunchKernel(fn, dim3((unsigned)(c->item_off[d1] - c->item_off[d0])), dim3(256), kargs, 0, c->stream));
+    return MAGIC_OK;
+}
+
+// q += the increments of sp (directions with a base), every cell
+template <typename T>
+static int add_parts_launch(magic_ctx *c, T *q, const StepParts<T> &sp)
+{
+    Span s(c, TC_OTHER, 1);
+    k_add_parts<T, NoGate><<<padded_cells(c->d), cell_block(), 0, c->stream>>>(c->d, q, sp, NoGate{});
+    return launch_check();
+}
+
+// The three sweeps of step3 (lib/step3.f:121-621) on argument block a, whose
+// state pointers and form-specific fields are already set.  The sweeps only
+// read a.qold and write their blocks' increments, so they are one launch
+// (one per run of directions that share a tile shape); sp returns the
+// increments, which add_parts or the source pass's conversion adds to q.
+// With one direction's room (parts_one) each direction's increments are
+// added to q at once, and sp is left empty.
+template <typename T, bool PERT>
+static int step3_sweeps(magic_ctx *c, const SweepArgsT<T> &a, T *q, double dt, StepParts<T> &sp)
+{
+    TRY(put_step_args<T>(c, a, dt, sp));
+    if (c->parts_one) {
+        for (int dir = 0; dir < 3; dir++) {
+            TRY((launch_tile<T, PERT>(c, dir, dir + 1)));
+            StepParts<T> one = sp;
+            for (int k = 0; k < 3; k++)
+                if (k != dir) one.d[k].base = nullptr;
+            TRY(add_parts_launch(c, q, one));
         }
-        {
-            Span sp(c, TC_SWZ, 0, c->side);
-            TRY((sweep_dir<T, PERT>(c, ay, 2, dt, c->shape[2], true, &sp.n, c->side, 3, 6, false)));
-        }
-        {
-            Span sp(c, TC_SWX, 0);
-            TRY((sweep_dir<T, PERT>(c, a, 0, dt, c->shape[0], true, &sp.n, c->stream, 0, 6, false)));
-        }
-        {
-            Span sp(c, TC_SWZ, 0);
-            TRY((sweep_dir<T, PERT>(c, a, 2, dt, c->shape[2], true, &sp.n, c->stream, 0, 3, false)));
-        }
-        HIPCHECK(hipEventRecord(c->ev_join, c->side));
-        HIPCHECK(hipStreamWaitEvent(c->stream, c->ev_join, 0));
-        c->dq_cur ^= 1;
-        c->dq_clear = true;
-        if (defer_merge) {
-            c->merge_dq = dq;
-            return MAGIC_OK;
-        }
-        Span sp(c, TC_OTHER, 1);
-        k_merge<T><<<(unsigned)std::min<long long>(blocks(n / Vec16<T>::N + 1, 256), 8192), 256, 0, c->stream>>>(
-            a.qnew, dq, n);
-        TRY(launch_check());
+        for (auto &p : sp.d) p.base = nullptr;
         return MAGIC_OK;
     }
-    if (tile) TRY(put_step_args<T>(c, a, dt, (T *)nullptr));
+    for (int d0 = 0, d1; d0 < 3; d0 = d1) {
+        for (d1 = d0 + 1; d1 < 3 && c->shape[d1] == c->shape[d0];) d1++;
+        TRY((launch_tile<T, PERT>(c, d0, d1)));
+    }
+    return MAGIC_OK;
+}
+
+// The FP64 form's one-workgroup-per-pencil kernel (MAGIC_SWEEP=pencil), which
+// adds into q in nine colour launches per direction
+static int pencil_sweeps(magic_ctx *c, const SweepArgs &a, double dt)
+{
     for (int dir = 0; dir < 3; dir++) {
         Span sp(c, TC_SWX + dir, 0);
-        TRY((sweep_dir<T, PERT>(c, a, dir, dt, c->shape[dir], tile, &sp.n, c->stream, 0, 6, !tile)));
+        SweepArgs d = a;
+        dir_args(c, d, dir, dt);
+        TRY(sweep_dispatch(c, d, &sp.n));
     }
     return MAGIC_OK;
 }
@@ -1050,7 +865,6 @@ static SweepArgsT<float> args32(magic_ctx *c)
     a.cgam = c->bg64 + B64_GAM * NZ;
     a.cvg = c->bg64 + B64_VG * NZ;
     a.cres = c->bg64 + B64_RES * NZ;
-    a.sink = (float *)c->sink;
     return a;
 }
 
@@ -1068,19 +882,51 @@ static SweepArgs args64(magic_ctx *c)
     a.cfl_bits = c->dscal;
     a.status = (int *)(c->dscal + 1);
     for (int m = 5; m < c->meqn; m++) a.comp[m] = m;
-    a.sink = (double *)c->sink;
     return a;
 }
 
-// defer_merge: leave the overlapped sweeps' q += dq to the caller (merge_dq)
-static int step3_launch(magic_ctx *c, double dt, bool defer_merge = false)
+// the pending increments of a step, added to q as a pass of their own
+static int parts_flush(magic_ctx *c)
 {
-    k_zero_scalars<<<1, 64, 0, c->stream>>>(c->dscal);
-    TRY(launch_check());
-    if (c->form == MAGIC_FORM_FP32P) TRY((step3_sweeps<float, true>(c, args32(c), dt, defer_merge)));
-    else TRY((step3_sweeps<double, false>(c, args64(c), dt, defer_merge)));
+    if (!c->pending_parts) return MAGIC_OK;
+    c->pending_parts = false;
+    return c->form == MAGIC_FORM_FP32P ? add_parts_launch(c, c->q32, c->parts32) : add_parts_launch(c, c->q, c->parts64);
+}
+
+// whether the sweeps leave their increments in the part buffer (known once
+// sweep_setup has run) rather than in q
+static bool form_tile(const magic_ctx *c) { return c->form == MAGIC_FORM_FP32P || use_tile(); }
+static int setup_sweeps(magic_ctx *c)
+{
+    if (!form_tile(c)) return MAGIC_OK;
+    return c->form == MAGIC_FORM_FP32P ? sweep_setup<float>(c) : sweep_setup<double>(c);
+}
+static bool sweeps_defer(const magic_ctx *c) { return form_tile(c) && !c->parts_one; }
+
+// The sweeps of one step and the read-back of its reductions.  from_q: they
+// read q itself (with deferred increments q does not change meanwhile);
+// else the backup.  The increments end up in q, or with defer stay pending
+// in the part buffer (c->pending_parts).
+static int step3_launch(magic_ctx *c, double dt, bool from_q = false, bool defer = false)
+{
+    if (!form_tile(c)) {
+        k_zero_scalars<<<1, 64, 0, c->stream>>>(c->dscal);
+        TRY(launch_check());
+        TRY(pencil_sweeps(c, args64(c), dt));
+    } else if (c->form == MAGIC_FORM_FP32P) {
+        SweepArgsT<float> a = args32(c);
+        if (from_q) a.qold = c->q32;
+        TRY((step3_sweeps<float, true>(c, a, c->q32, dt, c->parts32)));
+        c->pending_parts = c->parts32.d[0].base != nullptr;
+    } else {
+        SweepArgs a = args64(c);
+        if (from_q) a.qold = c->q;
+        TRY((step3_sweeps<double, false>(c, a, c->q, dt, c->parts64)));
+        c->pending_parts = c->parts64.d[0].base != nullptr;
+    }
     HIPCHECK(hipMemcpyAsync(c->hscal, c->dscal, 8 * sizeof(unsigned long long), hipMemcpyDeviceToHost,
                             c->stream));
+    if (!defer) TRY(parts_flush(c));
     return MAGIC_OK;
 }
 
@@ -1096,24 +942,6 @@ static int step3_finish(magic_ctx *c, double *cfl)
         return st[0] == 1 ? MAGIC_ERHO : MAGIC_EA2;
     }
     return MAGIC_OK;
-}
-
-// the pending q += dq of a deferred merge, as its own pass
-template <typename T>
-static int merge_launch(magic_ctx *c, T *q)
-{
-    const long long n = (long long)c->meqn * c->P;
-    Span sp(c, TC_OTHER, 1);
-    k_merge<T><<<(unsigned)std::min<long long>(blocks(n / Vec16<T>::N + 1, 256), 8192), 256, 0, c->stream>>>(
-        q, (const T *)c->merge_dq, n);
-    return launch_check();
-}
-static int merge_flush(magic_ctx *c)
-{
-    if (!c->merge_dq) return MAGIC_OK;
-    const int st = c->form == MAGIC_FORM_FP32P ? merge_launch<float>(c, c->q32) : merge_launch<double>(c, c->q);
-    c->merge_dq = nullptr;
-    return st;
 }
 
 extern "C" int magic_step3(magic_ctx *c, double dt, double *cfl)
@@ -1148,98 +976,43 @@ extern "C" int magic_set_sweep_overlap(magic_ctx *c, int on)
 }
 
 // Autotuner: every tile shape of every sweep direction is timed on this
-// grid's current state (one untimed sweep, then reps timed ones, HIP
-// events on the grid's stream) and the fastest shape of each direction is
-// kept.  The candidates read the backup copy and add into q; q is restored
-// from the backup afterwards, so the state is unchanged bit for bit (the
-// backup then holds the current state).
-static int tune_rounds(magic_ctx *c, double dt, int reps, TuneClock &clk)
+// grid's current state (one untimed sweep, then reps timed ones, HIP events
+// on the grid's stream) and the fastest shape of each direction is kept.
+// The candidates read the backup copy and write only their increment
+// blocks, so q does not change (the backup then holds it).
+template <typename T, bool PERT>
+static int tune_rounds(magic_ctx *c, const SweepArgsT<T> &a, double dt, int reps, TuneClock &clk)
 {
     for (int r = 0; r <= reps; r++) {   // repetition 0 warms up and is not timed
-        for (int dir = 0; dir < 3; dir++)
-            for (int sh = 0; sh < TILE_NSHAPE; sh++) {
-                int nl = 0;
+        for (int sh = 0; sh < TILE_NSHAPE; sh++) {
+            for (int k = 0; k < 3; k++) c->shape[k] = sh;
+            StepParts<T> sp;
+            TRY(put_step_args<T>(c, a, dt, sp));
+            for (int dir = 0; dir < 3; dir++) {
                 TRY(clk.mark(dir, sh, 0, c->stream));
-                TRY((c->form == MAGIC_FORM_FP32P ? sweep_dir<float, true>(c, args32(c), dir, dt, sh, true, &nl)
-                                                 : sweep_dir<double, false>(c, args64(c), dir, dt, sh, true, &nl)));
+                TRY((launch_tile<T, PERT>(c, dir, dir + 1)));
                 TRY(clk.mark(dir, sh, 1, c->stream));
             }
+        }
         if (r > 0) TRY(clk.add_round());
     }
     return MAGIC_OK;
 }
 
-// With the sweeps overlapped on two streams the directions share the
-// device, and the fastest assignment need not be each direction's fastest
-// shape alone.  Starting from those, each direction's shape is varied in
-// turn (at most two passes) and the whole set of step3 sweeps is timed on
-// the context's stream (one untimed and reps timed runs); a candidate
-// replaces the best one when it is at least 1 % faster.
-static int tune_joint(magic_ctx *c, double dt, int reps, int best[3])
-{
-    hipEvent_t e0 = nullptr, e1 = nullptr;
-    HIPCHECK(hipEventCreate(&e0));
-    if (hipEventCreate(&e1) != hipSuccess) {
-        hipEventDestroy(e0);
-        return MAGIC_EHIP;
-    }
-    auto time_assignment = [&](const int sh[3], float &ms) -> int {
-        for (int k = 0; k < 3; k++) c->shape[k] = sh[k];
-        ms = 0.f;
-        for (int r = 0; r <= reps; r++) {
-            if (hipEventRecord(e0, c->stream) != hipSuccess) return MAGIC_EHIP;
-            TRY((c->form == MAGIC_FORM_FP32P ? step3_sweeps<float, true>(c, args32(c), dt)
-                                             : step3_sweeps<double, false>(c, args64(c), dt)));
-            float t = 0.f;
-            if (hipEventRecord(e1, c->stream) != hipSuccess || hipEventSynchronize(e1) != hipSuccess ||
-                hipEventElapsedTime(&t, e0, e1) != hipSuccess)
-                return MAGIC_EHIP;
-            if (r > 0) ms += t / reps;
-        }
-        return MAGIC_OK;
-    };
-    float bms = 0.f;
-    int st = time_assignment(best, bms);
-    for (int pass = 0; pass < 2 && st == MAGIC_OK; pass++) {
-        bool changed = false;
-        for (int d = 0; d < 3 && st == MAGIC_OK; d++)
-            for (int sh = 0; sh < TILE_NSHAPE && st == MAGIC_OK; sh++) {
-                if (sh == best[d]) continue;
-                int cand[3] = {best[0], best[1], best[2]};
-                cand[d] = sh;
-                float ms = 0.f;
-                st = time_assignment(cand, ms);
-                if (st == MAGIC_OK && ms < 0.99f * bms) {
-                    bms = ms;
-                    best[d] = sh;
-                    changed = true;
-                }
-            }
-        if (!changed) break;
-    }
-    hipEventDestroy(e0);
-    hipEventDestroy(e1);
-    return st;
-}
-
 extern "C" int magic_tune(magic_ctx *c, double dt, int reps, int shapes_out[3], float *ms_out)
 {
     if (!c || !c->have_aux || !(dt > 0.0) || reps < 1) return MAGIC_EARG;
-    if (!(c->form == MAGIC_FORM_FP32P || use_tile()) || !sweep_supported(ntracer(c))) return MAGIC_EUNSUPPORTED;
+    if (!form_tile(c) || !sweep_supported(ntracer(c))) return MAGIC_EUNSUPPORTED;
     TuneClock clk;
     if (!clk.ok) return MAGIC_EHIP;
     const int keep[3] = {c->shape[0], c->shape[1], c->shape[2]};
     TRY(copy_state(c, true));
-    int st = tune_rounds(c, dt, reps, clk);
-    int best[3];
-    if (st == MAGIC_OK) {
-        clk.result(reps, best, ms_out);
-        if (overlap_sweeps(c)) st = tune_joint(c, dt, reps, best);
-    }
-    if (st != MAGIC_OK)
-        for (int k = 0; k < 3; k++) c->shape[k] = keep[k];
-    TRY(copy_state(c, false));   // also after a failed round
+    const int st = c->form == MAGIC_FORM_FP32P ? tune_rounds<float, true>(c, args32(c), dt, reps, clk)
+                                               : tune_rounds<double, false>(c, args64(c), dt, reps, clk);
+    for (int k = 0; k < 3; k++) c->shape[k] = keep[k];
     TRY(st);
+    int best[3];
+    clk.result(reps, best, ms_out);
     k_zero_scalars<<<1, 64, 0, c->stream>>>(c->dscal);   // the candidates' Courant numbers and reports
     TRY(launch_check());
     HIPCHECK(hipStreamSynchronize(c->stream));
@@ -1264,11 +1037,14 @@ static int src3_passes32(magic_ctx *c, const int *mthbc, int ndtr, double dtr, i
     const Col32 col = col32_of(c);
     {
         Span sp(c, TC_SRC, 1);
-        // the pending q += dq of the overlapped sweeps, if any, goes with the conversion
-        k32_src_convert<<<padded_cells(c->d), cell_block(), 0, c->stream>>>(d, c->q32, col, NoGate{},
-                                                                             (const float *)c->merge_dq, c->meqn);
-        c->merge_dq = nullptr;
+        if (!c->pending_parts) c->parts32.d[0].base = nullptr;
+        // with pending increments the new state goes to the other buffer and
+        // the old one stays behind as the backup
+        float *to = c->pending_parts ? c->qold32 : c->q32;
+        k32_src_convert<<<padded_cells(c->d), cell_block(), 0, c->stream>>>(d, c->q32, to, col, NoGate{}, c->parts32);
         TRY(launch_check());
+        if (c->pending_parts) std::swap(c->q32, c->qold32);
+        c->pending_parts = false;
     }
     for (int nn = 1; nn <= ndtr; nn++) {
         TRY(bc3_launch(c, mthbc));
@@ -1346,11 +1122,14 @@ static int src3_passes64(magic_ctx *c, const int *mthbc, int ndtr, double dtr, i
     const dim3 gface(blocks(d.NX, 64), d.NY);
     {
         Span sp(c, TC_SRC, 1);
-        // the pending q += dq of the overlapped sweeps, if any, goes with the conversion
-        k_src_convert<COL><<<padded_cells(d), cell_block(), 0, c->stream>>>(d, c->q, ax, NoGate{},
-                                                                            (const double *)c->merge_dq, c->meqn);
-        c->merge_dq = nullptr;
+        if (!c->pending_parts) c->parts64.d[0].base = nullptr;
+        // with pending increments the new state goes to the other buffer and
+        // the old one stays behind as the backup
+        double *to = c->pending_parts ? c->qold : c->q;
+        k_src_convert<COL><<<padded_cells(d), cell_block(), 0, c->stream>>>(d, c->q, to, ax, NoGate{}, c->parts64);
         TRY(launch_check());
+        if (c->pending_parts) std::swap(c->q, c->qold);
+        c->pending_parts = false;
     }
     for (int nn = 1; nn <= ndtr; nn++) {
         TRY(bc3_launch(c, mthbc));
@@ -1477,14 +1256,21 @@ extern "C" int magic_claw3(magic_ctx *c, double tstart, double *tend, double dtv
     const int maxn = nv[0];
     int st = MAGIC_OK, nl = 0;
     nv[1] = 0;
+    // With deferred increments the sweeps read q itself, which changes only in
+    // an accepted step's source pass (into the other state buffer): the state
+    // before the step needs no copy and a rejected step no restoring.  A
+    // batch's grid keeps its buffers' places (its captured kernels hold them)
+    // and takes the copying way.
+    if (maxn > 0 && (st = setup_sweeps(c))) return st;
+    const bool defer = sweeps_defer(c) && c->own_stream;
     for (int n = 1; n <= maxn; n++) {
         const double told = t;
         if (told + dt > *tend && tstart < *tend) dt = *tend - told;   // claw3_mpi.f:741
         for (;;) {
             if ((st = bc3_launch(c, mthbc))) goto out;
             if ((st = b4step3_launch(c))) goto out;
-            if ((st = copy_state(c, true))) goto out;
-            if ((st = step3_launch(c, dt, true))) goto out;
+            if (!defer && (st = copy_state(c, true))) goto out;
+            if ((st = step3_launch(c, dt, defer, defer))) goto out;
             if ((st = step3_finish(c, &cfl))) goto out;
             t = told + dt;
             if (log_dt && nl < maxlog) {
@@ -1498,8 +1284,8 @@ extern "C" int magic_claw3(magic_ctx *c, double tstart, double *tend, double dtv
                 break;
             }
             t = told;
-            c->merge_dq = nullptr;   // the rejected step's increments are dropped with it
-            if ((st = copy_state(c, false))) goto out;
+            c->pending_parts = false;   // the rejected step's increments are dropped with it
+            if (!defer && (st = copy_state(c, false))) goto out;
             dt = dtv[1] < dt * cflv[1] / cfl ? dtv[1] : dt * cflv[1] / cfl;
         }
         {
@@ -1515,8 +1301,10 @@ extern "C" int magic_claw3(magic_ctx *c, double tstart, double *tend, double dtv
     }
 out:
     {
-        // a step that stopped before its source pass still ends with q += dq
-        const int sm = merge_flush(c);
+        // a step that stopped before its source pass still leaves its
+        // increments in q and the state before it in the backup
+        int sm = MAGIC_OK;
+        if (c->pending_parts && (sm = copy_state(c, true)) == MAGIC_OK) sm = parts_flush(c);
         if (st == MAGIC_OK) st = sm;
     }
     hipStreamSynchronize(c->stream);

@@ -13,6 +13,7 @@
 #include "../../include/magic_hip.h"
 #include "bc_src.h"
 #include "magic_dev.h"
+#include "parts.h"
 
 using namespace magic;
 
@@ -39,9 +40,10 @@ enum { AX_RHO = 0, AX_MX, AX_MY, AX_MZ, AX_E, AX_NU, AX_KAP, AX_VG, AX_R, AX_GAM
 enum { TC_SWX = 0, TC_SWY, TC_SWZ, TC_BC, TC_SRC, TC_OTHER, NTC };
 
 struct TimedSpan {
-    int cls;
+    int cls;               // NTC: a launch of several sweep directions, shared by them
     hipEvent_t a, b;
     int nlaunch;
+    float share[3];        // of each direction (cls = NTC)
 };
 
 struct magic_ctx {
@@ -65,20 +67,18 @@ struct magic_ctx {
     double *col64 = nullptr;
     bool aux_layered = false;
     bool own_stream = true;   // false when a batch lends its stream
-    // The y-sweep of a single grid runs on a second stream next to the x-
-    // and z-sweeps and adds into dq[dq_cur] (meqn planes of the form's
-    // type), added to q after both; the other buffer is cleared meanwhile
-    // for the next step3.  Allocated on first use.
-    bool overlap = true;
-    hipStream_t side = nullptr;
-    hipEvent_t ev_fork = nullptr, ev_join = nullptr;
-    void *dq[2] = {nullptr, nullptr};
-    int dq_cur = 0;
-    bool dq_clear = false;   // dq[dq_cur] holds zeros (false until set up, and after a failed overlapped step)
-    // Inside magic_claw3 the q += dq pass after an overlapped step3 is left
-    // to the source pass's conversion (one pass over q instead of two);
-    // merge_dq is the buffer still to be added (null: nothing pending).
-    void *merge_dq = nullptr;
+    // The sweeps' increment blocks (SweepParts) of one step, for all three
+    // directions at once or, where the device has no room for that, for one
+    // direction at a time (parts_one).  Allocated on first use.
+    void *parts = nullptr;
+    size_t parts_bytes = 0;
+    bool parts_one = false;
+    // Inside magic_claw3 the increments of a step are left to the source
+    // pass's conversion (pending), which adds them on its way
+    bool pending_parts = false;
+    StepParts<double> parts64;   // the last sweeps' increments, by form
+    StepParts<float> parts32;
+    bool overlap = true;   // accepted for the ABI; the sweeps of a step are one launch
     // Asynchronous snapshots (magic_snapshot_begin): the conversion into
     // stage runs on the context's stream, the copy out of stage on cstream
     // (created on first use), so that later work on the stream need not
@@ -88,21 +88,18 @@ struct magic_ctx {
     hipEvent_t snap_conv = nullptr, snap_done = nullptr;
     bool snap_pending = false;
     unsigned long long *dscal = nullptr;   // [0] cfl bits, [1..] status ints
-    void *sink = nullptr;                  // 4 KiB the sweep's tile flush may write (never read back)
     int shape[3] = {0, 0, 0};              // tile shape of the x-, y- and z-sweeps
-    // The sweep kernel's operands (set up on the first tiled sweep): 18
-    // argument blocks (direction x colour, written by a kernel at the start
-    // of each step3 or of each tuner launch), run flags all pointing at a
-    // device 1, 18 pairs of work counters, and per direction and shape the
-    // tiles of each colour (items of colour k at [litem_off[dir][sh][k],
-    // ..[k + 1])
+    // The sweep kernel's operands (set up on the first tiled sweep): an
+    // argument block per direction (written by a kernel at the start of each
+    // step3 or of each tuner round), run flags all pointing at a device 1, and
+    // the workgroups' blocks, direction by direction (those of direction d at
+    // [item_off[d], item_off[d + 1]))
     void *largs = nullptr;
     const int **lrun = nullptr;
     int *lone = nullptr;
-    int *lcnt = nullptr;
-    int4 *litems[3][TILE_NSHAPE] = {};
-    int litem_off[3][TILE_NSHAPE][7] = {};
-    int lgrid[TILE_NSHAPE] = {};           // persistent grid of each shape's kernel (0: not yet known)
+    int4 *items = nullptr;
+    int item_off[4] = {0, 0, 0, 0};
+    int item_shape[3] = {-1, -1, -1};      // the shapes the items were laid out for
     unsigned long long *hscal = nullptr;   // pinned host words: [0, 8) mirror dscal, [HSCAL_SUMS, +10) global sums
     void *sums_d = nullptr;                // global sums: partials and results (first magic_global_sums)
     magic_params prm;
@@ -134,6 +131,7 @@ struct Span {
     int cls, n;
     hipStream_t s;
     hipEvent_t a = nullptr;
+    float share[3] = {0.f, 0.f, 0.f};
     Span(magic_ctx *c_, int cls_, int n_, hipStream_t s_ = nullptr) : c(c_), cls(cls_), n(n_), s(s_ ? s_ : c_->stream)
     {
         if (c->timing && (a = ev_get(c))) hipEventRecord(a, s);
@@ -146,7 +144,7 @@ struct Span {
         hipEvent_t b = ev_get(c);
         if (a && b) {
             hipEventRecord(b, s);
-            c->pending.push_back({cls, a, b, n});
+            c->pending.push_back({cls, a, b, n, {share[0], share[1], share[2]}});
         }
     }
 };
@@ -156,8 +154,16 @@ static inline void drain_timing(magic_ctx *c)
     for (auto &s : c->pending) {
         float ms = 0.f;
         if (hipEventSynchronize(s.b) == hipSuccess && hipEventElapsedTime(&ms, s.a, s.b) == hipSuccess) {
-            c->ms[s.cls] += ms;
-            c->launches[s.cls] += s.nlaunch;
+            if (s.cls < NTC) {
+                c->ms[s.cls] += ms;
+                c->launches[s.cls] += s.nlaunch;
+            } else {
+                for (int d = 0; d < 3; d++)
+                    if (s.share[d] > 0.f) {
+                        c->ms[TC_SWX + d] += ms * s.share[d];
+                        c->launches[TC_SWX + d] += s.nlaunch;
+                    }
+            }
         }
         c->pool.push_back(s.a);
         c->pool.push_back(s.b);
@@ -201,20 +207,118 @@ static inline dim3 diff_grid(const Dims &d) { return dim3(blocks(d.mx, 64), bloc
 static inline bool sweep_supported(int ntr) { return ntr >= 0 && ntr <= 5; }
 
 // ------------------------------------------------------- tile shapes ----
-// The tiled sweep kernel of shape sh (0 .. TILE_NSHAPE-1): the persistent
-// work-list kernel that one grid and a batch of grids both launch.
+// The tiled sweep kernel of shape sh (0 .. TILE_NSHAPE-1), launched for one
+// grid and for a batch of grids alike.
 template <typename T, bool PERT, int NTR>
-static inline const void *tile_list_fn(int sh)
+static inline const void *tile_fn_n(int sh)
 {
     switch (sh) {
-    case 0: return reinterpret_cast<const void *>(&tile_sweep_list<T, PERT, NTR, 0>);
-    case 1: return reinterpret_cast<const void *>(&tile_sweep_list<T, PERT, NTR, 1>);
-    case 2: return reinterpret_cast<const void *>(&tile_sweep_list<T, PERT, NTR, 2>);
-    case 3: return reinterpret_cast<const void *>(&tile_sweep_list<T, PERT, NTR, 3>);
+    case 0: return reinterpret_cast<const void *>(&tile_sweep<T, PERT, NTR, 0>);
+    case 1: return reinterpret_cast<const void *>(&tile_sweep<T, PERT, NTR, 1>);
+    case 2: return reinterpret_cast<const void *>(&tile_sweep<T, PERT, NTR, 2>);
+    case 3: return reinterpret_cast<const void *>(&tile_sweep<T, PERT, NTR, 3>);
     default: return nullptr;
     }
 }
-static_assert(TILE_NSHAPE == 4, "tile_list_fn lists every shape");
+static_assert(TILE_NSHAPE == 4, "tile_fn_n lists every shape");
+template <typename T, bool PERT>
+static inline const void *tile_fn(int ntr, int sh)
+{
+    switch (ntr) {
+    case 0: return tile_fn_n<T, PERT, 0>(sh);
+    case 1: return tile_fn_n<T, PERT, 1>(sh);
+    case 2: return tile_fn_n<T, PERT, 2>(sh);
+    case 3: return tile_fn_n<T, PERT, 3>(sh);
+    case 4: return tile_fn_n<T, PERT, 4>(sh);
+    case 5: return tile_fn_n<T, PERT, 5>(sh);
+    default: return nullptr;
+    }
+}
+
+// log2 of the planes per segment of a grid's sweeps.  Longer segments write
+// and read fewer edge planes (L + 2 for L) and start less often; shorter ones
+// give more workgroups.  The estimate, in planes of work: a segment costs L
+// and one more for its start and its two extra planes, 512 workgroups run at
+// once, and the last ones leave half a segment of the chip idle.  It depends
+// on the grid alone (not on the device or on a batch's other grids), since
+// the sums' grouping, and so the last bits, depend on it.  Full domain
+// (250 x 200 x 300): 16; 64 x 64 x 48: 8; a dozen cells: 1.
+static inline int segment_lg(const Dims &d)
+{
+    auto cols = [](int n, int a) { return (long long)((a + 2 + 15) / 16) * ((n + 1 + 13) / 14); };
+    const long long cx = cols(d.mx, d.my), cy = cols(d.my, d.mx), cz = cols(d.mz, d.mx);
+    int best = 0;
+    double fbest = 0.0;
+    for (int lg = 0; lg <= 5; lg++) {
+        auto segs = [&](int nB) { return (long long)((nB + 2 + (1 << lg) - 1) >> lg); };
+        const double rounds = (double)(cx * segs(d.mz) + cy * segs(d.mz) + cz * segs(d.my)) / 512.0;
+        const double w = (1 << lg) + 1.0, f = rounds <= 1.0 ? w : (rounds + 0.5) * w;
+        if (lg == 0 || f < fbest) {
+            best = lg;
+            fbest = f;
+        }
+    }
+    return best;
+}
+
+// The part of direction dir's argument block that the grid fixes: planes of
+// the components, strides and the layout of its blocks.  The tile axis is g
+// for the x- and z-sweeps (lib/step3.f:121-280 g = y, h = z; 459-621 g = x,
+// h = y) and x = h for the y-sweep (289-450 g = z, h = x), so that the y- and
+// z-sweeps tile along rows of x.
+template <typename T>
+static inline void sweep_geometry(const magic_ctx *c, int dir, int sh, SweepArgsT<T> &a, SweepParts<T> &p)
+{
+    const Dims &d = c->d;
+    const long long NXY = (long long)d.NX * d.NY;
+    static const int comp[3][5] = {{0, 1, 2, 3, 4}, {0, 2, 3, 1, 4}, {0, 3, 1, 2, 4}};
+    for (int m = 0; m < 5; m++) a.comp[m] = comp[dir][m];
+    for (int m = 5; m < c->meqn; m++) a.comp[m] = m;
+    a.P = c->P;
+    a.mbc = c->mbc;
+    a.n = dir == 0 ? c->mx : dir == 1 ? c->my : c->mz;
+    a.nA = dir == 0 ? c->my : c->mx;
+    a.nB = dir == 2 ? c->my : c->mz;
+    a.sN = dir == 0 ? 1 : dir == 1 ? d.NX : NXY;
+    a.sA = dir == 0 ? d.NX : 1;
+    a.sB = dir == 2 ? d.NX : NXY;
+    a.a_is_g = dir != 1;
+    a.gravity = dir == 2;
+    a.sweep = dir + 1;
+    memset(&p, 0, sizeof(p));
+    p.n = a.n; p.nA = a.nA; p.nB = a.nB;
+    p.lgTA = tile_lgta(sh);
+    p.lgL = segment_lg(d);
+    p.CI = tile_ci(sh);
+    p.iCI = (unsigned)(((1ull << 32) + p.CI - 1) / p.CI);
+    p.nt = (a.nA + 2 + tile_ta(sh) - 1) / tile_ta(sh);
+    p.nk = (a.n + 1 + p.CI - 1) / p.CI;
+    p.ns = (a.nB + 2 + (1 << p.lgL) - 1) >> p.lgL;
+    p.pm = tile_pm(sh);
+    p.mbc = c->mbc;
+    a.lgL = p.lgL; a.nt = p.nt; a.nk = p.nk;
+}
+template <typename T>
+static inline void sweep_factors(const magic_ctx *c, int dir, double dt, SweepArgsT<T> &a)
+{
+    const double x = dt / c->dx, y = dt / c->dy, z = dt / c->dz;
+    a.dtdn = dir == 0 ? x : dir == 1 ? y : z;
+    a.fg = dir == 0 ? y : dir == 1 ? z : x;
+    a.fh = dir == 0 ? z : dir == 1 ? x : y;
+}
+template <typename T>
+static inline long long parts_size(const SweepParts<T> &p, int nc, int sh)   // elements
+{
+    return (long long)p.ns * p.nk * p.nt * ((1 << p.lgL) + 2) * nc * part_npos(sh);
+}
+// the blocks of one direction, as they lie in the part buffer
+template <typename T>
+static inline void push_items(std::vector<int4> &items, const SweepParts<T> &p, int arg)
+{
+    for (int s = 0; s < p.ns; s++)
+        for (int k = 0; k < p.nk; k++)
+            for (int t = 0; t < p.nt; t++) items.push_back(make_int4(arg, t, k, s));
+}
 
 // Event pairs of the autotuners, one per (direction, shape).  The shapes
 // are timed round-robin (every round times each candidate once), so that a

@@ -38,7 +38,11 @@ struct SweepArgsT {
     // (rho_bar, E_bar, gamma, aux17, and the background's own z jump
     // p_bar(k) - p_bar(k-1) - .5 (rho_bar(k) + rho_bar(k-1)) aux17(k))
     const double *crho, *cE, *cgam, *cvg, *cres;
-    T *sink;                           // >= 256 elements of scratch the tile flush may write
+    // tiled sweep: sA/sB/nA/nB then describe the tile axis a and the marching
+    // axis b; a_is_g: the tile axis is the sweep's g direction
+    int a_is_g;
+    T *parts;                          // the direction's increment blocks (SweepParts)
+    int lgL, nt, nk;                   // log2 planes per segment, tiles along a, chunks along n
 };
 using SweepArgs = SweepArgsT<double>;
 
@@ -46,20 +50,38 @@ template <int NTR>
 __global__ void sweep_kernel(SweepArgs a);
 
 // Tiled sweep, one instantiation per tile shape SH (0 .. TILE_NSHAPE-1):
-// TA = tile_ta(SH) pencils along the tile axis a per workgroup, 256/TA
-// interfaces per chunk along the pencil.  a_is_g says whether the tile axis
-// is the sweep's g direction; sA/sB/nA/nB then describe the tile axis a and
-// the coloured axis b.  (T, PERT) = (double, false): FP64 form; (float,
-// true): FP32 perturbation form.  A persistent kernel over a work list of
-// tiles of one or several grids (items: {argument block, a_is_g, bx, by};
-// run[argument block] points at the grid's "runs in this attempt" flag;
-// next: the work counter and the count of finished workgroups, both 0 at
-// launch and set back to 0 by the kernel; grid: {tiles along a, argument
-// block, a_is_g, 0} for one tile per workgroup, x = 0 for the work list).
+// a workgroup sweeps TA = tile_ta(SH) pencils along the tile axis a by 256/TA
+// interfaces along the pencils, over a segment of planes along b, and writes
+// the increments of its block to the block's part.  (T, PERT) = (double,
+// false): FP64 form; (float, true): FP32 perturbation form.  items: {argument
+// block, tile, chunk, segment} of each workgroup; run[argument block] points
+// at the grid's "runs in this attempt" flag.
 constexpr int TILE_NSHAPE = 4;
 __host__ __device__ constexpr int tile_ta(int sh) { return sh == 0 ? 16 : sh == 3 ? 4 : 8; }
+__host__ __device__ constexpr int tile_lgta(int sh) { return sh == 0 ? 4 : sh == 3 ? 2 : 3; }
+__host__ __device__ constexpr bool tile_pm(int sh) { return sh >= 2; }
+// cells along the pencil a chunk completes, and positions of a part's plane
+__host__ __device__ constexpr int tile_ci(int sh) { return 256 / tile_ta(sh) - 2; }
+__host__ __device__ constexpr int part_npos(int sh) { return (tile_ta(sh) + 2) * (tile_ci(sh) + 1); }
 template <typename T, bool PERT, int NTR, int SH>
-__global__ void tile_sweep_list(const SweepArgsT<T> *args, const int4 *items, int nitems, const int *const *run,
-                                int *next, int4 grid);
+__global__ void tile_sweep(const SweepArgsT<T> *args, const int4 *items, const int *const *run);
+
+// The increment blocks of one sweep direction.  Block (segment s, chunk k,
+// tile t) lies at ((s nk + k) nt + t) * (L+2) * nc * npos: planes b = s L - 1
+// .. s L + L, of each plane nc components (tile order: rho, m_n, m_a, m_b, E,
+// tracers) of npos positions (a offsets t TA - 1 .. t TA + TA by cells k CI ..
+// k CI + CI).  A cell's increments are its own block's entry and, next to a
+// block's edge, the neighbouring blocks' entries for it.
+template <typename T>
+struct SweepParts {
+    const T *base;         // nullptr: no increments pending
+    int n, nA, nB;         // interior cells along the pencils, a and b
+    int lgTA, lgL;         // log2 pencils per tile, planes per segment
+    int CI;                // cells a chunk completes
+    unsigned iCI;          // ceil(2**32 / CI)
+    int nt, nk, ns;        // tiles, chunks, segments
+    int pm;                // positions run along the pencils (else along a)
+    int mbc;
+};
 
 }  // namespace magic

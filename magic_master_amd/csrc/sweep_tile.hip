@@ -15,8 +15,8 @@
 namespace magic {
 
 #define MAGIC_TILE64(NTR)                                                                                  \
-    template __global__ void tile_sweep_list<double, false, NTR, MAGIC_TILE_SHAPE>(                     \
-        const SweepArgsT<double> *, const int4 *, int, const int *const *, int *, int4);
+    template __global__ void tile_sweep<double, false, NTR, MAGIC_TILE_SHAPE>(                     \
+        const SweepArgsT<double> *, const int4 *, const int *const *);
 MAGIC_TILE64(0)
 MAGIC_TILE64(1)
 MAGIC_TILE64(2)

@@ -12,8 +12,8 @@
 namespace magic {
 
 #define MAGIC_TILE32(NTR)                                                                                  \
-    template __global__ void tile_sweep_list<float, true, NTR, MAGIC_TILE_SHAPE>(                        \
-        const SweepArgsT<float> *, const int4 *, int, const int *const *, int *, int4);
+    template __global__ void tile_sweep<float, true, NTR, MAGIC_TILE_SHAPE>(                        \
+        const SweepArgsT<float> *, const int4 *, const int *const *);
 MAGIC_TILE32(0)
 MAGIC_TILE32(1)
 MAGIC_TILE32(2)

@@ -10,20 +10,28 @@
 //
 // Same per-interface algebra as sweep.hip (rpn3euX.f, rpt3euX.f, rptt3euX.f,
 // flux3fw.f, step3.f); different data movement:
-//   * a workgroup owns TA pencils that are neighbours along the tile axis "a"
-//     (x-sweep: a = y; y- and z-sweeps: a = x, so that tile-axis-major lanes
-//     read rows of x) and marches along the pencils in chunks of CH
-//     interfaces (overlap 2); TA, CH and the lane order form the tile shape;
+//   * a workgroup takes one block of pencils and interfaces: TA pencils that
+//     are neighbours along the tile axis "a" (x-sweep: a = y; y- and z-sweeps:
+//     a = x, so that tile-axis-major lanes read rows of x) by CH interfaces
+//     along the pencils (chunks overlap by 2: the limiter's upwind
+//     neighbours), and marches over a segment of L planes along the other
+//     transverse axis b; TA, CH and the lane order form the tile shape;
 //   * the 3x3 increments of each interface (its cells i-1 and i into the
-//     pencil and its 8 transverse neighbours, step3.f:189-226) are summed in
-//     an LDS tile LT[b offset][a][cell] in sub-steps (one per phase and a
-//     offset, so no two lanes add to the same entry at once; separated by the
-//     wave's program order or by barriers, see the sub-step loop), and the
-//     tile is flushed to q once per chunk (FP64: one atomic add per entry;
-//     FP32: one coalesced read-modify-write per row);
-//   * tiles are coloured 2 ways along a and 3 ways along the other transverse
-//     axis b, so no two workgroups of a launch flush to the same rows.
-// The result is deterministic.
+//     pencil and its 8 transverse neighbours, step3.f:189-226) are summed in a
+//     ring of three planes in LDS, LT[plane][component][position], in
+//     sub-steps (one per phase and a offset, so no two lanes add to the same
+//     entry at once; separated by the wave's program order or by barriers,
+//     see the sub-step loop).  A plane is complete once the planes on both
+//     sides have been swept; it is then written, contiguous and once, to the
+//     block's own part of the increment buffer (SweepParts);
+//   * the parts of all blocks of the three directions are added to q
+//     afterwards (parts.h), each cell's in a fixed order: no two workgroups
+//     write the same memory, so the blocks need no colouring, no atomics and
+//     no order, and one launch covers the whole step.
+// The result is deterministic.  Against the earlier tile, which marched along
+// the pencils and added each chunk's three planes to q with FP64 atomics in
+// six colour launches per direction, q moves once instead of three times per
+// direction.
 #pragma once
 #include "magic_dev.h"
 #include "magic_solver.h"
@@ -47,7 +55,7 @@ template <>
 struct TileShape<3> { static constexpr int TA = 4; static constexpr bool PM = true; };
 static_assert(TileShape<TILE_NSHAPE - 1>::TA > 0, "one TileShape per shape index");
 
-// Pointer into global memory.  The work-list kernel reads its state pointers
+// Pointer into global memory.  The kernel reads its state pointers
 // from an argument block in memory, where the compiler cannot tell their
 // address space and would use flat loads and stores; flat accesses count on
 // the LDS counter too, so every LDS wait would also wait for them.
@@ -55,18 +63,6 @@ template <typename T>
 using gptr = __attribute__((address_space(1))) T *;
 template <typename T>
 __device__ __forceinline__ gptr<T> to_global(T *p) { return (gptr<T>)p; }
-
-// The FP64 tile flush adds each tile entry to q with one atomic add per
-// element and discards the result, so no wave waits for q to arrive (one
-// wave per SIMD has nothing else to run meanwhile); the colouring keeps
-// every element of q to one adding workgroup per launch, so the sum is the
-// same as a read-modify-write.  Measured on the full-domain workload: FP64
-// step +3 %; in FP32 (two waves per SIMD) the atomics cost 17 % (one grid)
-// and 27 % (ensemble), so FP32 keeps the read-modify-write.
-template <typename T>
-constexpr bool tile_flush_atomic() { return sizeof(T) == 8; }
-__device__ __forceinline__ void add_noret(gptr<double> p, double v) { (void)__builtin_amdgcn_global_atomic_fadd_f64(p, v); }
-__device__ __forceinline__ void add_noret(gptr<float> p, float v) { (void)__builtin_amdgcn_global_atomic_fadd_f32(p, v); }
 
 template <typename AT>
 __device__ __forceinline__ void report_t(const AT &A, int code, int i, int pg, int ph)
@@ -80,18 +76,19 @@ __device__ __forceinline__ void report_t(const AT &A, int code, int i, int pg, i
     }
 }
 
-// One tile (bx along the tile axis, by along the coloured axis) of one
-// colour launch; called by every lane of a 256-lane workgroup.
+// One block (tile bt along the tile axis, chunk bk along the pencils, segment
+// bs along b) of direction A; called by every lane of a 256-lane workgroup.
 template <typename T, bool PERT, int NTR, int SH>
-__device__ __forceinline__ void tile_sweep_body(const SweepArgsT<T> &A, int a_is_g, int bx, int by)
+__device__ __forceinline__ void tile_sweep_body(const SweepArgsT<T> &A, int bt, int bk, int bs)
 {
     constexpr int NC = 5 + NTR;
     constexpr int NT = 256, TA = TileShape<SH>::TA, CH = NT / TA;
     constexpr bool PM = TileShape<SH>::PM;
     constexpr int NCELL = CH - 1;               // cells S .. S+CH-2 of a chunk
     constexpr int TROW = TA + 2;                // a offsets A0-1 .. A0+TA
+    constexpr int NPOS = TROW * NCELL;          // positions of a plane
     constexpr T beta = T(0.666666666666666);
-    static_assert(TA * CH == NT && TA == tile_ta(SH), "tile is 256 lanes");
+    static_assert(TA * CH == NT && TA == tile_ta(SH) && NPOS == part_npos(SH), "tile is 256 lanes");
 
     __shared__ double s_del[5][NT];   // FP64 in both forms: the limiters' upwind wave strengths
     __shared__ T s_s2[NT];
@@ -99,73 +96,98 @@ __device__ __forceinline__ void tile_sweep_body(const SweepArgsT<T> &A, int a_is
     __shared__ T s_cfo[NT];
     __shared__ int s_flag[NT];
     __shared__ T s_cprev[TA];
-    __shared__ T LT[NC * 3 * TROW * NCELL + 1];   // + a slot that only ever holds 0
+    __shared__ int s_found[TA];
+    __shared__ int s_need;
+    __shared__ T LT[3 * NC * NPOS];
 
     const int t = threadIdx.x;
     const int pa = PM ? (t / CH) : (t % TA);    // pencil within the tile
     const int c = PM ? (t % CH) : (t / TA);     // interface offset within the chunk
     const int nb = PM ? 1 : TA;                 // lane distance between neighbouring interfaces
-    const int n = A.n;
-    const int A0 = (2 * bx + A.cA) * TA;
+    const int n = A.n, a_is_g = A.a_is_g;
+    const int A0 = bt * TA, B0 = bs << A.lgL;
+    const int nplane = min(1 << A.lgL, A.nB + 2 - B0);   // planes B0 .. B0 + nplane - 1
     const int a = A0 + pa;                      // tile-axis coordinate of this lane's pencil
-    const int b = A.cB + 3 * by;                // other transverse coordinate
     const bool pen = a <= A.nA + 1;
-    const int pg = a_is_g ? a : b, ph = a_is_g ? b : a;   // (g, h) coordinates
-    const long long pbase = (long long)(a + A.mbc - 1) * A.sA + (long long)(b + A.mbc - 1) * A.sB;
     const T dtdn = T(A.dtdn);
     const T d = dtdn;
     const T ca = T(a_is_g ? A.fg : A.fh), cb2 = T(a_is_g ? A.fh : A.fg);   // dt/da, dt/db
     const gptr<const T> qold = to_global(A.qold);
-    const gptr<T> qnew = to_global(A.qnew);
     const gptr<const double> gam = to_global(A.gam), vgrav = to_global(A.vgrav);
     const gptr<const double> crho = to_global(A.crho), cE = to_global(A.cE), cgam = to_global(A.cgam),
                              cvg = to_global(A.cvg), cres = to_global(A.cres);
-    // plane of each tile component: (rho, m_n, m_a, m_b, E, tracers)
-    const int pl2 = a_is_g ? A.comp[2] : A.comp[3], pl3 = a_is_g ? A.comp[3] : A.comp[2];
-    auto plane = [&](int m) { return (long long)(m == 2 ? pl2 : m == 3 ? pl3 : A.comp[m]) * A.P; };
 
-    // T index: (m, db, a offset ai, cell ci); the fastest index follows memory
-    auto tix = [&](int m, int db, int ai, int ci) {
-        return PM ? ((m * 3 + db) * TROW + ai) * NCELL + ci : ((m * 3 + db) * NCELL + ci) * TROW + ai;
-    };
-    for (int e = t; e <= NC * 3 * TROW * NCELL; e += NT) LT[e] = T(0.0);
+    // position within a plane; the fastest index follows memory
+    auto pix = [&](int ai, int ci) { return PM ? ai * NCELL + ci : ci * TROW + ai; };
+    for (int e = t; e < 3 * NC * NPOS; e += NT) LT[e] = T(0.0);
     if (t < TA) s_cprev[t] = T(0.0);
+    if (t == 0) s_need = 0;
+    __syncthreads();
     double cflmax = 0.0;            // Courant number, reduced in FP64
-    const int nchunk = (n + 1 + (CH - 2) - 1) / (CH - 2);
 
-    // The states of a lane's interface in the next chunk are loaded while
-    // the current chunk's transverse terms are computed (registers), so the
-    // HBM latency of part 1 is hidden behind part 3.  Not in the FP64
-    // pencil-major kernels, where the registers would spill.
-    constexpr bool PREFETCH = !(PM && sizeof(T) == 8) && !(sizeof(T) == 8 && NTR > 2);
+    // cell I-1 of interface I on plane b; the states of a lane's interface
+    const long long cell0 = (long long)(a + A.mbc - 1) * A.sA + (long long)(c - 1 + A.mbc - 1) * A.sN;
     T pqa[NC], pqb[NC], pga = T(0.0), pgb = T(0.0), pvg = T(0.0);
-    auto fetch = [&](int Iq) {
+    auto fetch = [&](int Iq, int b) {
         if (pen && Iq <= n + 2) {
-            const long long ca = pbase + (long long)(Iq - 1 + A.mbc - 1) * A.sN;
-            const long long cb = ca + A.sN;
+            const long long x = cell0 + (long long)(Iq - c) * A.sN + (long long)(b + A.mbc - 1) * A.sB;
+            const long long y = x + A.sN;
 #pragma unroll
             for (int m = 0; m < NC; m++) {
-                pqa[m] = qold[(long long)A.comp[m] * A.P + ca];
-                pqb[m] = qold[(long long)A.comp[m] * A.P + cb];
+                pqa[m] = qold[(long long)A.comp[m] * A.P + x];
+                pqb[m] = qold[(long long)A.comp[m] * A.P + y];
             }
             if constexpr (!PERT) {
-                pga = gam[ca];
-                pgb = gam[cb];
-                if (A.gravity) pvg = vgrav[cb];
+                pga = gam[x];
+                pgb = gam[y];
+                if (A.gravity) pvg = vgrav[y];
             }
         }
     };
-    if constexpr (PREFETCH) fetch(c);
+    // The next plane's states are loaded while the current plane's transverse
+    // terms are computed, so that part 3 hides their latency: in the FP32
+    // form, whose registers hold them next to two waves per SIMD.  In FP64
+    // they would not fit (two waves per SIMD hide the latency instead).
+    constexpr bool PREFETCH = sizeof(T) == 4;
+    const int I0 = bk * (CH - 2) + c;
 
-    for (int chunk = 0; chunk < nchunk; chunk++) {
-        const int S = chunk * (CH - 2);
-        const int I = S + c;                    // Fortran interface index
-        const bool act1 = pen && I <= n + 2;
-        const bool act2 = act1 && c >= 1 && c <= CH - 2 && I >= 1 && I <= n + 1;
-        // No barrier here: the previous chunk's last readers of the s_*
-        // arrays (part 2 and the CFLup carry) are behind its sub-step
-        // barriers, and its flush's reads of the tile are behind this
-        // chunk's barrier after part 1.
+    // one plane of the ring to the block's part, as it lies in LDS: whole
+    // contiguous lines, nothing read back
+    gptr<T> part = to_global(A.parts) + (long long)((bs * A.nk + bk) * A.nt + bt) * (((1 << A.lgL) + 2) * NC * NPOS);
+    auto flush = [&](int p, int slot) {
+        T *src = LT + slot * (NC * NPOS);
+        const gptr<T> dst = part + p * (NC * NPOS);
+#pragma unroll
+        for (int k = 0; k < (NC * NPOS + NT - 1) / NT; k++) {
+            const int e = t + k * NT;
+            if (e < NC * NPOS) {
+                dst[e] = src[e];
+                src[e] = T(0.0);
+            }
+        }
+    };
+    if constexpr (PREFETCH) fetch(I0, B0);
+
+    for (int plane = 0; plane < nplane; plane++) {
+        const int b = B0 + plane;               // other transverse coordinate
+        const int pg = a_is_g ? a : b, ph = a_is_g ? b : a;   // (g, h) coordinates
+        // No barrier here: the previous plane's last readers of the s_*
+        // arrays (part 2) are behind its sub-step barriers, and its flush's
+        // accesses of the ring are behind this plane's barrier after part 1.
+        int kk = bk;                            // chunk being solved (an earlier one while looking for CFLup)
+        int looked = 0;
+        asm volatile("" : "+s"(looked));        // one copy of the solve in the loop below
+        RoeT<double> R;
+        double b1, b2, b3, b4, b5, al1, al5, s1, s2, s3;
+        bool lf, f1, f2, f5, act1, act2;
+        T trw[NTR > 0 ? NTR : 1];   // unlimited tracer waves
+        T c1, c2, c3;
+        int I;
+        for (;;) {
+        I = kk * (CH - 2) + c;                  // Fortran interface index
+        act1 = pen && I <= n + 2;
+        act2 = act1 && c >= 1 && c <= CH - 2 && I >= 1 && I <= n + 1;
+        if (!PREFETCH || looked) fetch(I, b);
 
         // ---------------- part 1: Roe solve of interface I (rpn3euX.f:138-421)
         // The waves stay in their strengths (b1, b5 acoustic, b4 entropy, b2
@@ -173,40 +195,22 @@ __device__ __forceinline__ void tile_sweep_body(const SweepArgsT<T> &A, int a_is
         // vectors of rpn3euX.f:217-271 are never formed.  al1, al5 and lf:
         // the left-going parts of waves 1, 3 and 2 (rpn3euX.f:311-399).
         // The solve runs in FP64 in both forms (see rcp1 in magic_solver.h).
-        RoeT<double> R = {0, 0, 0, 0, 1, 0, 0, 0, 0};
-        double b1 = 0, b2 = 0, b3 = 0, b4 = 0, b5 = 0, al1 = 0, al5 = 0;
-        double s1 = 0, s2 = 0, s3 = 0;
-        bool lf = false;
-        T trw[NTR > 0 ? NTR : 1];   // unlimited tracer waves
-        T c1 = 0, c2 = 0, c3 = 0;
-        bool f1 = false, f2 = false, f5 = false;
+        R = {0, 0, 0, 0, 1, 0, 0, 0, 0};
+        b1 = b2 = b3 = b4 = b5 = al1 = al5 = s1 = s2 = s3 = 0;
+        lf = f1 = f2 = f5 = false;
+        c1 = c2 = c3 = 0;
         if (act1) {
             constexpr bool RF = sizeof(T) == 4;
             double qa[NC], qb[NC], vgc = 0.0;
             double ga, gb;
-            if constexpr (PREFETCH) {
 #pragma unroll
-                for (int m = 0; m < NC; m++) {
-                    qa[m] = pqa[m];
-                    qb[m] = pqb[m];
-                }
-                ga = pga;
-                gb = pgb;
-                vgc = pvg;
-            } else {
-                const long long ca = pbase + (long long)(I - 1 + A.mbc - 1) * A.sN;
-                const long long cb = ca + A.sN;
-#pragma unroll
-                for (int m = 0; m < NC; m++) {
-                    qa[m] = qold[(long long)A.comp[m] * A.P + ca];
-                    qb[m] = qold[(long long)A.comp[m] * A.P + cb];
-                }
-                if constexpr (!PERT) {
-                    ga = gam[ca];
-                    gb = gam[cb];
-                    if (A.gravity) vgc = vgrav[cb];
-                }
+            for (int m = 0; m < NC; m++) {
+                qa[m] = pqa[m];
+                qb[m] = pqb[m];
             }
+            ga = pga;
+            gb = pgb;
+            vgc = pvg;
             // perturbation form: q holds q - background; the background is a
             // column at rest (rho_bar(k), E_bar(k), gamma(k)), so the full
             // states differ from q only in rho and E
@@ -330,16 +334,37 @@ __device__ __forceinline__ void tile_sweep_body(const SweepArgsT<T> &A, int a_is
             s_s2[t] = (T)s2;
 #pragma unroll
             for (int k = 0; k < NTR; k++) s_trw[k][t] = trw[k];
-            s_flag[t] = (act2 && (f1 || f2 || f5)) ? 1 : 0;
+            s_flag[t] = (c <= CH - 2 && I >= 1 && I <= n + 1 && (f1 || f2 || f5)) ? 1 : 0;
             s_cfo[t] = f5 ? c3 : (f2 ? c2 : c1);
+            // the limiters may need the Courant number an earlier chunk left
+            if (bk > 0 && act2 && !f1 && !f2 && (b3 != 0.0 || b4 != 0.0)) s_need = 1;
         } else {
             s_flag[t] = 0;
         }
         __syncthreads();
+        // CFLup (rpn3euX.f:563-619) is the Courant number last assigned along
+        // the pencil.  It is needed from an interface before this chunk only
+        // where waves 1 and 2 vanish exactly and wave 3 or 4 does not (pure
+        // shear or contact): then the earlier chunks are solved again, from
+        // the nearest back, until every pencil of the tile has met an
+        // assignment, and this chunk once more.
+        if (bk == 0 || s_need == 0 || (looked && kk == bk)) break;
+        if (!looked) {
+            looked = 1;
+            if (t < TA) { s_cprev[t] = T(0.0); s_found[t] = 0; }
+        } else if (t < TA && !s_found[t]) {
+            for (int j = CH - 2; j >= 0; j--) {
+                const int tt = PM ? t * CH + j : j * TA + t;
+                if (s_flag[tt]) { s_cprev[t] = s_cfo[tt]; s_found[t] = 1; break; }
+            }
+        }
+        kk = __syncthreads_and(t >= TA || (kk < bk && s_found[t])) ? -1 : kk - 1;
+        if (kk < 0) kk = bk;
+        }
 
         // ---------------- part 2: limiters (rpn3euX.f:434-676) and the strengths
         // of the second-order correction (flux3fw.f:270-284).  From here on the
-        // transverse directions are the tile axis a and the coloured axis b.
+        // transverse directions are the tile axis a and the marching axis b.
         T un = 0, ua = 0, ub = 0, snd = 1, isnd = 1, kin = 0, hk = 0;   // Roe state: kin = |u|^2/2, hk = H - kin
         T x1 = 0, x4 = 0, xa = 0, xb = 0, x5 = 0, l1 = 0, l5 = 0;       // strengths, left-going acoustic parts
         T q1 = 0, q4 = 0, qsa = 0, qsb = 0, q5 = 0;                     // strengths of cqxx
@@ -395,7 +420,7 @@ __device__ __forceinline__ void tile_sweep_body(const SweepArgsT<T> &A, int a_is
                         if (f1) cflup = c1;
                         else {
                             cflup = s_cprev[pa];
-                            for (int j = c - 1; j >= 1; j--)
+                            for (int j = c - 1; j >= 0; j--)
                                 if (s_flag[t - (c - j) * nb]) { cflup = s_cfo[t - (c - j) * nb]; break; }
                         }
                         wt = lim2.weight(cflup);
@@ -453,7 +478,7 @@ __device__ __forceinline__ void tile_sweep_body(const SweepArgsT<T> &A, int a_is
             qsa = (T)(a_is_g ? w2 : w3);
             qsb = (T)(a_is_g ? w3 : w2);
         }
-        if (PREFETCH && chunk + 1 < nchunk) fetch(S + (CH - 2) + c);
+        if (PREFETCH && plane + 1 < nplane) fetch(I0, b + 1);
 
         // ---------------- part 3: transverse terms (flux3fw.f:297-625), two phases
         // The transverse splits by the interface's Roe eigensystem
@@ -474,6 +499,8 @@ __device__ __forceinline__ void tile_sweep_body(const SweepArgsT<T> &A, int a_is
         // once): deterministic.  Against splitting conserved vectors and
         // summing a 3 x 3 x NC register accumulator this halves the sweep's
         // arithmetic, and nothing wider than the y and z vectors stays live.
+        // the ring's planes of b-1, b and b+1
+        const int r0 = plane % 3, r1 = r0 == 2 ? 0 : r0 + 1, r2 = r1 == 2 ? 0 : r1 + 1;
         const T kf = -(T(1.0) / T(6.0)) * d * ca * cb2, kea = -T(0.5) * d * ca, keb = -T(0.5) * d * cb2;
         const SpeedT<T> va(ua, snd), vb(ub, snd);
 #pragma unroll 1
@@ -481,6 +508,7 @@ __device__ __forceinline__ void tile_sweep_body(const SweepArgsT<T> &A, int a_is
             // phase 0 (L): interface I -> cell I-1; phase 1 (R): -> cell I
             const bool on = act2 && (phase == 0 ? I >= 2 : I <= n);
             const int ci = phase == 0 ? c - 1 : c;  // cell index within the chunk's tile
+            if (phase == 1 && t == 0) s_need = 0;   // every lane has read it (phase 0's barrier)
             const T sg = phase == 0 ? T(1.0) : -T(1.0);
             const bool has = (phase == 0) == lf;    // the contact waves belong to this phase
             WaveT<T> y[3], z[3], N;
@@ -530,6 +558,7 @@ __device__ __forceinline__ void tile_sweep_body(const SweepArgsT<T> &A, int a_is
                 if (on) {
                     auto target = [&](auto jc) {
                         constexpr int j = decltype(jc)::value;
+                        T *row = LT + (j == 0 ? r0 : j == 1 ? r1 : r2) * (NC * NPOS) + pix(pa + r, ci);
                         WaveT<T> D = va.template split_a<r>(y[j], snd, isnd);
                         D.add(vb.template split_b<j>(z[r], snd, isnd));
                         if constexpr (!PERT && r == 1 && j == 1) D.add(N);
@@ -541,12 +570,12 @@ __device__ __forceinline__ void tile_sweep_body(const SweepArgsT<T> &A, int a_is
                             for (int m = 0; m < 5; m++) o[m] += phase == 0 ? nrm[0][m] : nrm[1][m];
                         }
 #pragma unroll
-                        for (int m = 0; m < 5; m++) LT[tix(m, j, pa + r, ci)] += o[m];
+                        for (int m = 0; m < 5; m++) row[m * NPOS] += o[m];
 #pragma unroll
                         for (int k = 0; k < NTR; k++) {
                             T v = va.w2(r) * yt[j][k] + vb.w2(j) * zt[r][k];
                             if (r == 1 && j == 1) v += Nt[k];
-                            LT[tix(5 + k, j, pa + r, ci)] += v;
+                            row[(5 + k) * NPOS] += v;
                         }
                     };
                     target(IConst<0>{});
@@ -563,157 +592,48 @@ __device__ __forceinline__ void tile_sweep_body(const SweepArgsT<T> &A, int a_is
                 // waves share entries: a barrier after every sub-step.
                 if (PM || r == 2) __syncthreads();
                 else __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
-                if (phase == 0 && r == (PM ? 0 : 2) && t < TA) {
-                    // CFLup carried into the next chunk: the last assignment
-                    // among this chunk's interfaces (every lane is past part
-                    // 2, which reads s_cprev, once this barrier is passed)
-                    for (int j = CH - 2; j >= 1; j--) {
-                        const int tt = PM ? t * CH + j : j * TA + t;
-                        if (s_flag[tt]) { s_cprev[t] = s_cfo[tt]; break; }
-                    }
-                }
             };
             substep(IConst<0>{});
             substep(IConst<1>{});
             substep(IConst<2>{});
         }
 
-        // ---------------- flush the tile to q (one read-modify-write per row)
-        // Each lane owns PPT (a offset, cell) positions of every (m, db) plane
-        // of the tile; m and db are compile-time so the plane bases come from
-        // scalar registers.  The flush is branch-free so that all loads are
-        // in flight together and no store waits for another: a position
-        // outside the grid reads and writes the lane's slot of A.sink, and
-        // its tile entry is the shared zero slot.
-        {
-            constexpr int NPOS = TROW * NCELL;
-            constexpr int PPT = (NPOS + NT - 1) / NT;
-            constexpr int ZERO = NC * 3 * NPOS;
-            long long poff[PPT];
-            bool pok[PPT];
-#pragma unroll
-            for (int k = 0; k < PPT; k++) {
-                const int e = t + k * NT;
-                const int ai = PM ? e / NCELL : e % TROW, ci = PM ? e % NCELL : e / TROW;
-                const int cell = S + ci;                // Fortran index along the pencil
-                const int aa = A0 - 1 + ai;             // tile-axis coordinate of the target row
-                pok[k] = e < NPOS && cell >= 1 && cell <= n && aa <= A.nA + 2;
-                poff[k] = (long long)(cell + A.mbc - 1) * A.sN + (long long)(aa + A.mbc - 1) * A.sA;
-            }
-            if constexpr (tile_flush_atomic<T>()) {
-#pragma unroll
-                for (int m = 0; m < NC; m++)
-#pragma unroll
-                    for (int db = 0; db < 3; db++) {
-                        const gptr<T> base =
-                            qnew + plane(m) + (long long)(b + db - 1 + A.mbc - 1) * A.sB;
-#pragma unroll
-                        for (int k = 0; k < PPT; k++) {
-                            const int e = t + k * NT;
-                            const int li = e < NPOS ? (m * 3 + db) * NPOS + e : ZERO;
-                            const T v = LT[li];
-                            LT[li] = T(0.0);
-                            if (pok[k]) add_noret(base + poff[k], v);
-                        }
-                    }
-            } else {
-            const gptr<T> sink = to_global(A.sink) + t;
-            T val[NC][3][PPT];
-#pragma unroll
-            for (int m = 0; m < NC; m++)
-#pragma unroll
-                for (int db = 0; db < 3; db++) {
-                    const gptr<T> base = qnew + plane(m) + (long long)(b + db - 1 + A.mbc - 1) * A.sB;
-#pragma unroll
-                    for (int k = 0; k < PPT; k++) val[m][db][k] = *(pok[k] ? base + poff[k] : sink);
-                }
-#pragma unroll
-            for (int m = 0; m < NC; m++)
-#pragma unroll
-                for (int db = 0; db < 3; db++)
-#pragma unroll
-                    for (int k = 0; k < PPT; k++) {
-                        const int e = t + k * NT;
-                        const int li = e < NPOS ? (m * 3 + db) * NPOS + e : ZERO;   // = tix(m, db, ai, ci)
-                        val[m][db][k] = val[m][db][k] + LT[li];
-                        LT[li] = T(0.0);
-                    }
-#pragma unroll
-            for (int m = 0; m < NC; m++)
-#pragma unroll
-                for (int db = 0; db < 3; db++) {
-                    const gptr<T> base = qnew + plane(m) + (long long)(b + db - 1 + A.mbc - 1) * A.sB;
-#pragma unroll
-                    for (int k = 0; k < PPT; k++) *(pok[k] ? base + poff[k] : sink) = val[m][db][k];
-                }
-            }
-        }
+        // ---------------- flush: plane b-1 has all its increments
+        flush(plane, r0);
     }
+    flush(nplane, nplane % 3);
+    flush(nplane + 1, (nplane + 1) % 3);
     for (int o = 32; o > 0; o >>= 1) cflmax = fmaxF(cflmax, __shfl_xor(cflmax, o, 64));
     if ((threadIdx.x & 63) == 0) atomicMax(A.cfl_bits, (unsigned long long)__double_as_longlong(cflmax));
 }
 
 
-// Waves per SIMD the register allocation aims at: two for the FP32 form
-// with tile-axis-major lanes and at most one tracer (left to themselves
-// these kernels miss 256 registers by a few, since the Riemann solve runs in
-// FP64, and halve the occupancy: 50 % slower on the full-domain FP32 step),
-// one otherwise.
+// Waves per SIMD the register allocation aims at: two, except where the LDS
+// of two workgroups does not fit a compute unit (FP64 with four tracers or
+// more) or the registers would spill (pencil-major lanes).
 template <typename T, int NTR, int SH>
 constexpr int tile_waves()
 {
-    if (sizeof(T) != 4 || TileShape<SH>::PM) return 1;
-    return NTR <= 1 ? 2 : 1;
+    if (TileShape<SH>::PM) return 1;
+    return sizeof(T) == 8 ? (NTR <= 3 ? 2 : 1) : (NTR <= 1 ? 2 : 1);
 }
 
 // The sweep kernel, for one grid and for a batch of grids alike (one
-// compiled body with one call site, so both round alike), in two modes:
-//  * work list (grid.x = 0): a persistent grid whose workgroups take tiles
-//    from a work list (item = {argument block, a_is_g, bx, by}) through the
-//    atomic counter next[0] until it runs out; tiles of grids whose control
-//    flag (*run) is 0 in this attempt are skipped.  next[1] counts the
-//    workgroups that are done; the last one sets both back to 0 for the
-//    next launch (every other workgroup has taken its last item by then);
-//  * one tile per workgroup (grid.x > 0 tiles along a): workgroup b takes
-//    tile {argument block grid.y, a_is_g grid.z, b mod grid.x, b / grid.x},
-//    as the hardware dispatches them, so that the launches of two streams
-//    share the compute units tile by tile (one grid's sweep overlap).
+// compiled body with one call site, so both round alike): workgroup g takes
+// block items[g] = {argument block, tile, chunk, segment}; blocks of grids
+// whose control flag (*run) is 0 in this attempt end at once.
 template <typename T, bool PERT, int NTR, int SH>
 __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(tile_waves<T, NTR, SH>())))
-void tile_sweep_list(const SweepArgsT<T> *__restrict__ args, const int4 *items, int nitems,
-                                                        const int *const *run, int *next, int4 grid)
+void tile_sweep(const SweepArgsT<T> *__restrict__ args, const int4 *__restrict__ items,
+                const int *const *__restrict__ run)
 {
-    __shared__ int s_item;
-    bool first = true;
-    for (;;) {
-        int4 w;
-        if (grid.x > 0) {
-            if (!first) break;
-            first = false;
-            w = make_int4(grid.y, grid.z, (int)blockIdx.x % grid.x, (int)blockIdx.x / grid.x);
-        } else {
-            __syncthreads();   // the previous tile's readers of s_item and of the tile arrays are done
-            if (threadIdx.x == 0) s_item = atomicAdd(next, 1);
-            __syncthreads();
-            const int it = s_item;
-            if (it >= nitems) break;
-            w = items[it];
-        }
-        // the item is the same for the whole workgroup: scalar, so that the
-        // argument block is read with scalar loads
-        const int ai = __builtin_amdgcn_readfirstlane(w.x);
-        if (*run[ai] == 0) continue;
-        tile_sweep_body<T, PERT, NTR, SH>(args[ai], __builtin_amdgcn_readfirstlane(w.y),
-                                          __builtin_amdgcn_readfirstlane(w.z), __builtin_amdgcn_readfirstlane(w.w));
-    }
-    if (grid.x == 0 && threadIdx.x == 0) {
-        __threadfence();   // this workgroup's last take precedes its count
-        if (atomicAdd(next + 1, 1) == (int)gridDim.x - 1) {
-            __threadfence();
-            atomicExch(next, 0);
-            atomicExch(next + 1, 0);
-        }
-    }
+    // the item is the same for the whole workgroup: scalar, so that the
+    // argument block is read with scalar loads
+    const int4 w = items[blockIdx.x];
+    const int ai = __builtin_amdgcn_readfirstlane(w.x);
+    if (*run[ai] == 0) return;
+    tile_sweep_body<T, PERT, NTR, SH>(args[ai], __builtin_amdgcn_readfirstlane(w.y),
+                                      __builtin_amdgcn_readfirstlane(w.z), __builtin_amdgcn_readfirstlane(w.w));
 }
 
 }  // namespace magic

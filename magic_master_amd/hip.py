@@ -356,8 +356,8 @@ class MagicHIP:
         return list(sh)
 
     def set_sweep_overlap(self, on: bool):
-        """y-sweep on a second stream (True, the default) or the three sweeps
-        in turn (False: the batched driver's order of additions)."""
+        """Accepted for programs that set it: a step's sweeps are one launch
+        and their sums have one order, whatever it says."""
         self._check(self.L.magic_set_sweep_overlap(self.h, 1 if on else 0), "magic_set_sweep_overlap")
 
     def tune(self, dt: float, reps: int = 3):
@@ -489,7 +489,7 @@ class MagicBatch:
                     "magic_batch_set_tile_shapes")
 
     def set_sweep_overlap(self, on: bool):
-        """The sweeps' order of additions, as MagicHIP.set_sweep_overlap."""
+        """Accepted, without effect, as MagicHIP.set_sweep_overlap."""
         self._check(self.L.magic_batch_set_sweep_overlap(self.h, 1 if on else 0), "magic_batch_set_sweep_overlap")
 
     def tile_shapes(self):
