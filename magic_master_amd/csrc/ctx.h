@@ -294,9 +294,10 @@ static inline void sweep_geometry(const magic_ctx *c, int dir, int sh, SweepArgs
     p.nt = (a.nA + 2 + tile_ta(sh) - 1) / tile_ta(sh);
     p.nk = (a.n + 1 + p.CI - 1) / p.CI;
     p.ns = (a.nB + 2 + (1 << p.lgL) - 1) >> p.lgL;
-    p.pm = tile_pm(sh);
-    p.mbc = c->mbc;
-    a.lgL = p.lgL; a.nt = p.nt; a.nk = p.nk;
+    p.sT = dir == 0 ? p.nk : 1;
+    p.sK = dir == 0 ? 1 : p.nt;
+    p.sS = p.nk * p.nt;
+    a.lgL = p.lgL; a.sT = p.sT; a.sK = p.sK; a.sS = p.sS;
 }
 template <typename T>
 static inline void sweep_factors(const magic_ctx *c, int dir, double dt, SweepArgsT<T> &a)

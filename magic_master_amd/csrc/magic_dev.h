@@ -42,7 +42,7 @@ struct SweepArgsT {
     // axis b; a_is_g: the tile axis is the sweep's g direction
     int a_is_g;
     T *parts;                          // the direction's increment blocks (SweepParts)
-    int lgL, nt, nk;                   // log2 planes per segment, tiles along a, chunks along n
+    int lgL, sT, sK, sS;               // log2 planes per segment; blocks between tiles, chunks, segments
 };
 using SweepArgs = SweepArgsT<double>;
 
@@ -67,11 +67,14 @@ template <typename T, bool PERT, int NTR, int SH>
 __global__ void tile_sweep(const SweepArgsT<T> *args, const int4 *items, const int *const *run);
 
 // The increment blocks of one sweep direction.  Block (segment s, chunk k,
-// tile t) lies at ((s nk + k) nt + t) * (L+2) * nc * npos: planes b = s L - 1
-// .. s L + L, of each plane nc components (tile order: rho, m_n, m_a, m_b, E,
-// tracers) of npos positions (a offsets t TA - 1 .. t TA + TA by cells k CI ..
-// k CI + CI).  A cell's increments are its own block's entry and, next to a
-// block's edge, the neighbouring blocks' entries for it.
+// tile t) is number s sS + k sK + t sT, of (L+2) * nc * npos elements: planes
+// b = s L - 1 .. s L + L, of each plane nc components (tile order: rho, m_n,
+// m_a, m_b, E, tracers) of npos positions (a offsets t TA - 1 .. t TA + TA by
+// cells k CI .. k CI + CI).  A cell's increments are its own block's entry
+// and, next to a block's edge, the neighbouring blocks' entries for it.
+// Whatever the tile's lane order, positions and blocks run fastest along x
+// (the pencils of the x-sweep, the tile axis of the others), as the lanes
+// that add them to q do.
 template <typename T>
 struct SweepParts {
     const T *base;         // nullptr: no increments pending
@@ -80,8 +83,7 @@ struct SweepParts {
     int CI;                // cells a chunk completes
     unsigned iCI;          // ceil(2**32 / CI)
     int nt, nk, ns;        // tiles, chunks, segments
-    int pm;                // positions run along the pencils (else along a)
-    int mbc;
+    int sT, sK, sS;        // blocks between neighbouring tiles, chunks, segments
 };
 
 }  // namespace magic

@@ -117,8 +117,10 @@ __device__ __forceinline__ void tile_sweep_body(const SweepArgsT<T> &A, int bt, 
     const gptr<const double> crho = to_global(A.crho), cE = to_global(A.cE), cgam = to_global(A.cgam),
                              cvg = to_global(A.cvg), cres = to_global(A.cres);
 
-    // position within a plane; the fastest index follows memory
-    auto pix = [&](int ai, int ci) { return PM ? ai * NCELL + ci : ci * TROW + ai; };
+    // position within a plane: fastest along x, as the part's (the x-sweep's
+    // odd row length also keeps lanes on neighbouring pencils in different banks)
+    const int pA = A.sweep == 1 ? NCELL : 1, pN = A.sweep == 1 ? 1 : TROW;
+    auto pix = [&](int ai, int ci) { return ai * pA + ci * pN; };
     for (int e = t; e < 3 * NC * NPOS; e += NT) LT[e] = T(0.0);
     if (t < TA) s_cprev[t] = T(0.0);
     if (t == 0) s_need = 0;
@@ -153,7 +155,7 @@ __device__ __forceinline__ void tile_sweep_body(const SweepArgsT<T> &A, int bt, 
 
     // one plane of the ring to the block's part, as it lies in LDS: whole
     // contiguous lines, nothing read back
-    gptr<T> part = to_global(A.parts) + (long long)((bs * A.nk + bk) * A.nt + bt) * (((1 << A.lgL) + 2) * NC * NPOS);
+    gptr<T> part = to_global(A.parts) + (long long)(bs * A.sS + bk * A.sK + bt * A.sT) * (((1 << A.lgL) + 2) * NC * NPOS);
     auto flush = [&](int p, int slot) {
         T *src = LT + slot * (NC * NPOS);
         const gptr<T> dst = part + p * (NC * NPOS);
