@@ -12,7 +12,7 @@
 
 namespace magic {
 
-enum { GATE_RUN = 0, GATE_ACCEPTED, GATE_REJECTED, GATE_DIFF, GATE_COND, GATE_COND_MORE, GATE_COND_LAST, GATE_SWEPT };
+enum { GATE_RUN = 0, GATE_ACCEPTED, GATE_REJECTED, GATE_DIFF, GATE_COND, GATE_MORE, GATE_SWEPT };
 
 // factor slots of ScenCtl::fac (source pass, src3.f90:314-322 and the
 // passes of diffuse.f / conduct.f)
@@ -71,14 +71,14 @@ struct StepGate {
         case GATE_REJECTED: return c->rejected != 0;
         case GATE_DIFF: return c->accepted != 0 && nn <= c->ndtr;
         case GATE_COND: return c->accepted != 0 && nn <= c->ndtr && kk <= c->ndtrc;
-        case GATE_COND_MORE: return c->accepted != 0 && nn <= c->ndtr && kk < c->ndtrc;
-        case GATE_COND_LAST: return c->accepted != 0 && nn <= c->ndtr && kk == c->ndtrc;
+        case GATE_MORE: return c->accepted != 0 && nn < c->ndtr;
         case GATE_SWEPT: return c->swept != 0;
         default: return false;
         }
     }
     template <typename T>
     __device__ __forceinline__ T f(T x, int i) const { return fslot < 0 ? x : (T)c->fac[fslot + i]; }
+    __device__ __forceinline__ bool conducts(int k) const { return k <= c->ndtrc; }
     // the forcing of src3 is evaluated at the step's start time and dt
     __device__ __forceinline__ void forcing(double &t, double &dt, double &tgauss) const
     {

@@ -226,17 +226,16 @@ static int launch_dirs(magic_batch *b, const magic_batch::Group &g, int d0, int 
 static dim3 list_block(int lg)
 {
     switch (lg) {
-    case LG_ALL: case LG_CPY: case LG_CP1: return dim3(256);
-    case LG_PAD: case LG_DIF: case LG_INT: return cell_block();
-    default: return dim3(64);
+    case LG_BC: case LG_BCUVW: case LG_CPY: return dim3(256);
+    case LG_BCZ: return dim3(64);
+    default: return cell_block();
     }
 }
 
 // The block list each kernel class walks
 static int op_list(int op)
 {
-    static const int lg[NOP] = {LG_FX,  LG_FY,  LG_BCZ, LG_ALL, LG_CPY, LG_CPY, LG_PAD, LG_FZ, LG_DIF,
-                                LG_DIF, LG_CP1, LG_INT, LG_FZ,  LG_SPL, LG_INT, LG_INT, LG_PAD};
+    static const int lg[NOP] = {LG_BC, LG_BCUVW, LG_BCZ, LG_CPY, LG_CPY, LG_PAD, LG_DIF, LG_DF4, LG_DIF, LG_INT, LG_INT, LG_PAD};
     return lg[op];
 }
 
@@ -271,27 +270,12 @@ template <typename T>
 static int launch_src(magic_batch *b)
 {
     for (int nn = 1; nn <= b->ndtr_cap; nn++) {
-        const GateSpec gd = gs(GATE_DIFF, nn);
-        // bc3 with the z faces skipped (src3.f90:333-336)
-        TRY(launch_op<T>(b, OP_BCX, gd));
-        TRY(launch_op<T>(b, OP_BCY, gd));
-        TRY(launch_op<T>(b, OP_ZGHOST_UVW, gd));
+        // bc3 with the z faces skipped (src3.f90:333-336) and diffuse's z ghosts
+        TRY(launch_op<T>(b, OP_BCUVW, gs(GATE_DIFF, nn)));
         TRY(launch_op<T>(b, OP_DIFF_CROSS, gs(GATE_DIFF, nn, 0, FAC_CROSS)));
-        for (int cc = 1; cc <= 3; cc++)
-            TRY(launch_op<T>(b, OP_DIFF_XYZ, gs(GATE_DIFF, nn, 0, FAC_DIFF + 3 * (cc - 1)), cc));
-        TRY(launch_op<T>(b, OP_COPY_Q5, gd));
-        for (int kk = 1; kk <= b->ndtrc_cap; kk++) {
-            const GateSpec gk = gs(GATE_COND, nn, kk);
-            TRY(launch_op<T>(b, OP_PASS, gs(GATE_COND, nn, kk, FAC_COND + 0), PASS_QT_UT * 4 + 0));
-            TRY(launch_op<T>(b, OP_PASS, gs(GATE_COND, nn, kk, FAC_COND + 1), PASS_UT_QT * 4 + 1));
-            TRY(launch_op<T>(b, OP_CONDUCT_ZGHOST, gk));
-            TRY(launch_op<T>(b, OP_ZSPILL, gk));
-            if (kk < b->ndtrc_cap) {   // at kk = ndtrc_cap >= ndtrc these never run
-                TRY(launch_op<T>(b, OP_PASS, gs(GATE_COND_MORE, nn, kk, FAC_COND + 2), PASS_QT_UT * 4 + 2));
-                TRY(launch_op<T>(b, OP_COPY_INTERIOR, gs(GATE_COND_MORE, nn, kk)));
-            }
-            TRY(launch_op<T>(b, OP_PASS, gs(GATE_COND_LAST, nn, kk, FAC_COND + 2), PASS_Q5_UT * 4 + 2));
-        }
+        TRY(launch_op<T>(b, OP_DIFF, gs(GATE_DIFF, nn, 1, FAC_DIFF)));
+        for (int kk = 2; kk <= b->ndtrc_cap; kk++) TRY(launch_op<T>(b, OP_CONDUCT, gs(GATE_COND, nn, kk, FAC_DIFF), kk));
+        if (nn < b->ndtr_cap) TRY(launch_op<T>(b, OP_COPY_T, gs(GATE_MORE, nn)));
     }
     return launch_op<T>(b, OP_FINISH, gs(GATE_ACCEPTED));
 }
@@ -327,10 +311,8 @@ static int record_attempt(magic_batch *b)
     k_batch_prepare<T><<<blocks(b->n, 256), 256, 0, b->stream>>>(b->ctl_d, b->n, (SweepArgsT<T> *)b->args_d);
     TRY(launch_check());
     const GateSpec run = gs(GATE_RUN);
-    TRY(launch_op<T>(b, OP_BCX, run));
-    TRY(launch_op<T>(b, OP_BCY, run));
-    TRY(launch_op<T>(b, OP_BCZ, run));
-    if (b->meqn > 5) TRY(launch_op<T>(b, OP_CLAMP, run));
+    TRY(launch_op<T>(b, OP_BC, run));   // with b4step3
+    TRY(launch_op<T>(b, OP_BCZ, run));            // grids with mz < mbc only
     for (const auto &g : b->groups) TRY((launch_group<T, PERT>(b, g)));
     TRY(launch_src<T>(b));
     k_batch_finalize<<<blocks(b->n, 256), 256, 0, b->stream>>>(b->ctl_d, b->n);
@@ -504,24 +486,28 @@ static void form_ops(const magic_ctx *c, BatchOps<double> &o)
 // the layer count.
 static int batch_kb(const Dims &d) { return std::max(diff_kb(d), std::min(16, d.mz)); }
 
+// whether a scenario's z faces run after the others in their own pass (capi.hip's bc_launch)
+static bool z_apart(const magic_ctx *c, const int *bc) { return c->mz < c->mbc && (bc[4] > 0 || bc[5] > 0); }
+
 // Grid of list lg for one scenario (x, y, z blocks; x = 0: no blocks)
 static int4 list_grid(const magic_batch *b, const magic_ctx *c, const int *bc, int lg)
 {
     const Dims &d = c->d;
     const long long P = c->P;
     auto g1 = [](long long x) { return make_int4((int)x, 1, 1, 0); };
+    const int kb = batch_kb(d), nzb = (int)blocks(d.mz, kb);
     switch (lg) {
-    case LG_FX: return bc[0] >= 0 || bc[1] >= 0 ? make_int4(blocks(d.NY, 64), d.NZ, 1, 0) : g1(0);
-    case LG_FY: return bc[2] >= 0 || bc[3] >= 0 ? make_int4(blocks(d.NX, 64), d.NZ, 1, 0) : g1(0);
-    case LG_BCZ: return bc[4] >= 0 || bc[5] >= 0 ? make_int4(blocks(d.NX, 64), d.NY, 1, 0) : g1(0);
-    case LG_FZ: return make_int4(blocks(d.NX, 64), d.NY, 1, 0);
-    case LG_ALL: return g1(blocks(P, 256));
+    case LG_BC: case LG_BCUVW: {
+        long long n = (long long)bc_lanes(d, 0) + bc_lanes(d, 1) + bc_lanes(d, 2);
+        if (lg == LG_BC && b->meqn > 5) n += bc_lanes(d, 3);
+        return g1(blocks(n, 256));
+    }
+    case LG_BCZ: return z_apart(c, bc) ? make_int4(blocks(d.NX, 64), d.NY, 1, 0) : g1(0);
     case LG_CPY: return g1(std::min<long long>(8192, blocks(P * b->meqn, 256)));
-    case LG_CP1: return g1(std::min<long long>(8192, blocks(P, 256)));
     case LG_PAD: { const dim3 g = padded_cells(d); return make_int4(g.x, g.y, g.z, 0); }
-    case LG_DIF: return make_int4(blocks(d.mx, 64), blocks(d.my, 4), blocks(d.mz, batch_kb(d)), 0);
+    case LG_DIF: return make_int4(blocks(d.mx, 64), blocks(d.my, 4), nzb, 0);
+    case LG_DF4: return make_int4(blocks(d.mx, 64), blocks(d.my, 4), 4 * nzb, 0);
     case LG_INT: { const dim3 g = interior_grid(d); return make_int4(g.x, g.y, g.z, 0); }
-    case LG_SPL: return g1(c->mz > c->mx ? blocks(c->mz - c->mx, 64) : 0);
     default: return g1(0);
     }
 }
@@ -562,7 +548,8 @@ static int build_ops(magic_batch *b)
         o.nc = c->meqn;
         o.kb = batch_kb(c->d);
         o.spill = c->mz > c->mx ? c->mz - c->mx : 0;
-        memcpy(o.bc, &b->mthbc[6 * s], sizeof(o.bc));
+        for (int f = 0; f < 6; f++) o.bc.m[f] = std::max(0, b->mthbc[6 * s + f]);
+        o.bcz = z_apart(c, &b->mthbc[6 * s]);
         const magic_params &p = c->prm;
         Forcing &f = o.f;
         f.forcemth = (int)p.forcemth;

@@ -17,6 +17,7 @@
 #include "batch.h"
 #include "bc_src.h"
 #include "parts.h"
+#include "stencil_body.h"
 
 namespace magic {
 
@@ -30,7 +31,8 @@ struct BatchOps {
     int nc;          // meqn
     int kb;          // layers per block of the diffusion kernels (diff_kb)
     int spill;       // conduct.f:86-91 out-of-row writes (mz - mx when mz > mx, else 0)
-    int bc[6];       // mthbc (bc3 faces; the source pass's substeps skip z)
+    Faces bc;        // bc3's faces (the source pass's substeps skip z)
+    int bcz;         // the z faces run apart, after the others (mz < mbc)
     ScenCtl *ctl;
     // FP32 form: background columns, z-face factors, diffusivity columns
     Col32 col;
@@ -44,21 +46,18 @@ struct BatchOps {
 
 // Kernel classes of the batched attempt
 enum {
-    OP_BCX = 0, OP_BCY, OP_BCZ, OP_CLAMP, OP_BACKUP, OP_RESTORE, OP_CONVERT, OP_ZGHOST_UVW, OP_DIFF_CROSS,
-    OP_DIFF_XYZ, OP_COPY_Q5, OP_PASS, OP_CONDUCT_ZGHOST, OP_ZSPILL, OP_COPY_INTERIOR, OP_FINISH, OP_ADD_PARTS, NOP
+    OP_BC = 0, OP_BCUVW, OP_BCZ, OP_BACKUP, OP_RESTORE, OP_CONVERT, OP_DIFF_CROSS, OP_DIFF, OP_CONDUCT, OP_COPY_T, OP_FINISH,
+    OP_ADD_PARTS, NOP
 };
-// Block lists, one per launch geometry (a scenario whose faces of a bc3
-// kernel are all left to the caller has no blocks in that kernel's list):
-//   FX  bc3 x faces          (NY/64, NZ)      FY  bc3 y faces      (NX/64, NZ)
-//   BCZ bc3 z faces          (NX/64, NY)      FZ  z-ghost fills    (NX/64, NY)
-//   ALL one lane per cell    (P/256)          CPY grid-stride copy of meqn planes
-//   CP1 grid-stride copy of one plane         PAD padded cells     (NX/64, NY/4, NZ)
-//   DIF diffusion passes     (mx/64, my/4, mz/kb)
-//   INT interior cells       (mx/64, my/4, mz)
-//   SPL conduct.f's out-of-row writes ((mz-mx)/64)
-enum { LG_FX = 0, LG_FY, LG_BCZ, LG_FZ, LG_ALL, LG_CPY, LG_CP1, LG_PAD, LG_DIF, LG_INT, LG_SPL, NLG };
-// OP_PASS variants: (out, interior source) = (qt, ut), (ut, qt), (q(5), ut)
-enum { PASS_QT_UT = 0, PASS_UT_QT, PASS_Q5_UT };
+// Block lists, one per launch geometry:
+//   BC  boundary lanes and, with tracers, the interior's (1-D, 256 lanes)
+//   BCUVW boundary lanes (1-D, 256 lanes)
+//   BCZ bc3 z faces of grids with mz < mbc   (NX/64, NY)
+//   CPY grid-stride copy of meqn planes       PAD padded cells     (NX/64, NY/4, NZ)
+//   DIF cross terms, and conduct's substeps kk >= 2  (mx/64, my/4, mz/kb)
+//   DF4 directional passes of four components, conduct's first substep among them (mx/64, my/4, 4 * mz/kb)
+//   INT interior cells   (mx/64, my/4, mz)
+enum { LG_BC = 0, LG_BCUVW, LG_BCZ, LG_CPY, LG_PAD, LG_DIF, LG_DF4, LG_INT, NLG };
 
 struct GateSpec {
     int mode, nn, kk, fslot;
@@ -81,16 +80,22 @@ __device__ __forceinline__ int active_find(const int *pre, int n, int a)
     return lo;
 }
 
-__device__ __forceinline__ int lohi(int m) { return m < 0 ? 0 : m; }
+// T' after the substeps: conduct's last one wrote ut (odd count) or qt; with no
+// substep it is still q's own plane
+template <typename T>
+__device__ __forceinline__ const T *conducted(const BatchOps<T> &o, const StepGate &g)
+{
+    const int n = g.c->ndtr > 0 ? g.c->ndtrc : 0;
+    return n == 0 ? o.q + 4 * o.d.P : (n & 1) ? o.ut : o.qt;
+}
 
 // One launch of kernel class OP over the blocks of the scenarios' list
 // (off, gdim) whose gates are on.  Each workgroup of the persistent grid
 // first evaluates every slot's gate and lays the active slots' blocks end to
 // end in LDS (pre: active blocks before each slot), then takes active
 // blocks blockIdx.x, blockIdx.x + gridDim.x, ...; a launch whose gates are
-// all off ends after that scan.  arg: the velocity component of
-// OP_DIFF_XYZ (1-3), PASS_* * 4 + axis of OP_PASS, the direction of
-// OP_ADD_PARTS.  The form's own bodies
+// all off ends after that scan.  arg: conduct's substep of
+// OP_CONDUCT, the direction of OP_ADD_PARTS.  The form's own bodies
 // are reached through the FORM functor (FP32: bc_src32.hip, FP64:
 // bc_src.hip).  n <= BATCH_MAX_SLOTS (the host checks).
 template <typename T, int OP, class FORM>
@@ -162,42 +167,29 @@ __global__ __launch_bounds__(256) void k_batch_op(const BatchOps<T> *__restrict_
         const int gx = cgdim[4 * s], gy = cgdim[4 * s + 1];
         const uint3 bi = make_uint3((unsigned)(l % gx), (unsigned)((l / gx) % gy), (unsigned)(l / (gx * gy)));
         const long long P = o.d.P;
-        if constexpr (OP == OP_BCX) {
-            b_bc_x(bi, o.d, o.q, o.nc, lohi(o.bc[0]), lohi(o.bc[1]), g);
-        } else if constexpr (OP == OP_BCY) {
-            b_bc_y(bi, o.d, o.q, o.nc, lohi(o.bc[2]), lohi(o.bc[3]), g);
+        if constexpr (OP == OP_BC || OP == OP_BCUVW) {
+            // the boundary pass of a step, or of a diffusion substep, which skips z
+            Faces f = o.bc;
+            if (OP == OP_BCUVW || o.bcz) f.m[4] = f.m[5] = 0;
+            b_bc(bi, o.d, o.q, o.nc, f, OP == OP_BC ? CLAMP_BC : UVW_BC, FORM::zscale(o, CS + s), g);
         } else if constexpr (OP == OP_BCZ) {
             FORM::bc_z(bi, o, CS + s, g);
-        } else if constexpr (OP == OP_CLAMP) {
-            b_clamp(bi, o.q, P, o.nc, g);
         } else if constexpr (OP == OP_BACKUP) {
             b_copy(bi, (unsigned)gx, o.qold, o.q, P * o.nc, g);
         } else if constexpr (OP == OP_RESTORE) {
             b_copy(bi, (unsigned)gx, o.q, o.qold, P * o.nc, g);
         } else if constexpr (OP == OP_CONVERT) {
             FORM::convert(bi, o, g);
-        } else if constexpr (OP == OP_ZGHOST_UVW) {
-            b_zghost_uvw(bi, o.d, o.q, g);
         } else if constexpr (OP == OP_DIFF_CROSS) {
             b_diff_cross<T, true>(bi, o.d, o.u, o.q, FORM::nu(o), T(0.0), T(0.0), T(0.0), o.kb, g);
             __syncthreads();   // the next block's writers of the tile arrays wait for this one's readers
-        } else if constexpr (OP == OP_DIFF_XYZ) {
-            b_diff_xyz<T, true>(bi, o.d, o.q + arg * P, o.u + (arg - 1) * P, FORM::nu(o), T(0.0), T(0.0), T(0.0), o.kb,
-                                g);
+        } else if constexpr (OP == OP_DIFF || OP == OP_CONDUCT) {
+            // arg (OP_CONDUCT): the substep kk >= 2
+            const DiffArgs<T> a = {o.q, o.u, o.ut, o.qt, FORM::nu(o), FORM::kap(o), {}, o.spill, o.kb};
+            b_diff<T, true>(bi, o.d, a, [&](int i) { return g.f(T(0.0), i); }, OP == OP_DIFF ? 1 : arg, g);
             __syncthreads();
-        } else if constexpr (OP == OP_COPY_Q5) {
-            b_copy(bi, (unsigned)gx, o.ut, o.q + 4 * P, P, g);
-        } else if constexpr (OP == OP_PASS) {
-            const int v = arg >> 2, axis = arg & 3;
-            T *out = v == PASS_QT_UT ? o.qt : v == PASS_UT_QT ? o.ut : o.q + 4 * P;
-            const T *src = v == PASS_UT_QT ? o.qt : o.ut;
-            b_pass<T, true>(bi, o.d, out, src, o.ut, FORM::kap(o), T(0.0), axis, g);
-        } else if constexpr (OP == OP_CONDUCT_ZGHOST) {
-            b_conduct_zghost(bi, o.d, o.ut, g);
-        } else if constexpr (OP == OP_ZSPILL) {
-            b_conduct_zspill(bi, o.d, o.ut, o.spill, g);
-        } else if constexpr (OP == OP_COPY_INTERIOR) {
-            b_copy_interior(bi, o.d, o.ut, o.qt, 1, g);
+        } else if constexpr (OP == OP_COPY_T) {
+            b_copy_interior(bi, o.d, o.q + 4 * P, conducted(o, g), 1, g);
         } else if constexpr (OP == OP_FINISH) {
             FORM::finish(bi, o, g);
         } else if constexpr (OP == OP_ADD_PARTS) {

@@ -35,13 +35,43 @@ struct NoGate {
     __device__ __forceinline__ bool on() const { return true; }
     template <typename T>
     __device__ __forceinline__ T f(T x, int) const { return x; }
+    // whether conduct has a substep kk
+    __device__ __forceinline__ bool conducts(int) const { return true; }
     __device__ __forceinline__ void forcing(double &, double &, double &) const {}
 };
 
-template <typename T, class G>
-__global__ void k_bc_x(Dims d, T *q, int nc, int lo, int hi, G gate);
-template <typename T, class G>
-__global__ void k_bc_y(Dims d, T *q, int nc, int lo, int hi, G gate);
+enum { CLAMP_BC = 1, UVW_BC = 2 };   // modes of the boundary kernel (b_bc)
+// Lanes of the boundary kernel: ghost layers, ghost rows of interior layers,
+// ghost columns of interior rows, and with the clamp the interior cells.
+__host__ __device__ __forceinline__ unsigned bc_lanes(const Dims &d, int part)
+{
+    const unsigned g = 2u * d.mbc;
+    return part == 0 ? g * d.NX * d.NY : part == 1 ? g * d.NX * d.mz : part == 2 ? g * d.my * d.mz
+                                                                                 : (unsigned)d.mx * d.my * d.mz;
+}
+
+// bc3's faces (mthbc; 0: skipped)
+struct Faces {
+    int m[6];
+};
+// The z pass's scaling (bc3_mpi.f:544-809) of component m's value v of the
+// column's boundary cell for its ghost layer kbc: FP64 form with the aux
+// planes and the precomputed factors
+struct ZScale64 {
+    const double *aux1, *aux2, *aux3, *aux5, *zratio;
+    int mbc;
+    long long NXY;
+    __device__ __forceinline__ double operator()(int m, int side, int kbc, double v, long long cg, long long cb,
+                                                 long long col) const
+    {
+        if (m >= 5) return v;
+        const double sc = zratio[((long long)side * mbc + (kbc - 1)) * NXY + col];
+        if (m == 3) return v * sc;
+        const double *a = m == 0 ? aux1 : m == 1 ? aux2 : m == 2 ? aux3 : aux5;
+        return a[cg] + (v - a[cb]) * sc;
+    }
+};
+
 // Stephan & Alexander convective heating profile (src3.f90:534-572) for a
 // precipitation rate precipw > 0.1 at height zcell (m): K/s.
 __device__ __forceinline__ double sa_heating(double precipw, double zcell)
@@ -65,6 +95,8 @@ template <class G>
 __global__ void k_bc_z(Dims d, double *q, int nc, int lo, int hi, const double *aux1,
                        const double *aux2, const double *aux3, const double *aux5,
                        const double *zratio, G gate);
+template <typename T, class ZF, class G>
+__global__ void k_bc(Dims d, T *q, int nc, Faces f, int mode, ZF zf, G gate);
 template <typename T, class G>
 __global__ void k_clamp(T *q, long long P, int nc, G gate);
 template <typename T>
@@ -73,22 +105,27 @@ template <bool COL, class G>
 __global__ void k_src_convert(Dims d, const double *qin, double *q, const Aux a, G gate, StepParts<double> sp);
 template <typename T, class G>
 __global__ void k_add_parts(Dims d, T *q, StepParts<T> sp, G gate);
-template <typename T, class G>
-__global__ void k_zghost_uvw(Dims d, T *q, G gate);
 template <typename T, bool COLC, class G>
 __global__ void k_diff_cross(Dims d, T *u, const T *q, const T *coef, T dxy, T dxz, T dyz, int kb, G gate);
+// The operands of the directional passes: diffuse's per velocity component,
+// and a substep of conduct.
+template <typename T>
+struct DiffArgs {
+    T *q;                  // component planes; 1..3: velocities, 4: T'
+    const T *u;            // cross-term result of the velocities
+    T *ut, *qt;            // conduction buffers: substep kk writes ut (odd) or qt (even)
+    const T *nu, *kap;
+    T f[12];               // dt/dx**2, dt/dy**2, dt/dz**2 of each component in turn, with their factors
+    int S;                 // out-of-row z-ghost writes of conduct (mz - mx, or 0)
+    int kb;                // layers per workgroup
+};
+
 template <typename T, bool COLC, class G>
-__global__ void k_diff_xyz(Dims d, T *q, const T *u, const T *coef, T fx, T fy, T fz, int kb, G gate);
+__global__ void k_diff(Dims d, DiffArgs<T> a, int kk, G gate);
 template <typename T, class G>
 __global__ void k_copy_interior(Dims d, T *dst, const T *src, int nplanes, G gate);
-template <typename T, class G>
-__global__ void k_conduct_zghost(Dims d, T *u, G gate);
-template <typename T, class G>
-__global__ void k_conduct_zspill(Dims d, T *u, int S, G gate);
-template <typename T, bool COLC, class G>
-__global__ void k_pass(Dims d, T *out, const T *src, const T *ghost, const T *coef, T f, int axis, G gate);
 template <bool COL, class G>
-__global__ void k_src_finish(Dims d, double *q, int nc, const Aux a, Forcing f, G gate);
+__global__ void k_src_finish(Dims d, double *q, const double *t5, int nc, const Aux a, Forcing f, G gate);
 __global__ void k_aos_to_planes(double *planes, const double *aos, long long P, int nc);
 
 // ---- FP32 perturbation form (bc_src32.hip) ----
@@ -101,12 +138,21 @@ struct Col32 {
 struct Zr32 {
     double s[2][8];
 };
+// FP32 form: with a background at rest every component's perturbation is
+// scaled, in FP64 with one rounding
+struct ZScale32 {
+    Zr32 zr;
+    __device__ __forceinline__ float operator()(int m, int side, int kbc, float v, long long, long long, long long) const
+    {
+        return m >= 5 ? v : (float)((double)v * zr.s[side][kbc - 1]);
+    }
+};
 template <class G>
 __global__ void k32_bc_z(Dims d, float *q, int nc, int lo, int hi, Zr32 zr, G gate);
 template <class G>
 __global__ void k32_src_convert(Dims d, const float *qin, float *q, Col32 col, G gate, StepParts<float> sp);
 template <class G>
-__global__ void k32_src_finish(Dims d, float *q, int nc, Col32 col, Forcing f, G gate);
+__global__ void k32_src_finish(Dims d, float *q, const float *t5, int nc, Col32 col, Forcing f, G gate);
 template <typename T, class G>
 __global__ void k_copy(T *dst, const T *src, long long n, G gate);
 __global__ void k32_aos_to_pert(Dims d, float *q, const double *aos, int nc, const double *bgrho,

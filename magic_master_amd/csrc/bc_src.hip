@@ -116,10 +116,11 @@ __global__ void k_src_convert(Dims d, const double *qin, double *q, const Aux a,
     b_src_convert<COL>(uint3{blockIdx.x, blockIdx.y, blockIdx.z}, d, qin, q, (double *)nullptr, a, gate, sp);
 }
 
+// t5: T' (q's own plane, or the buffer of conduct's last substep).
 // src3.f90:380-418 (reassembly), 430-445 / 514-607 (forcing), 616-626
 // (tracer clamp), on the interior.
 template <bool COL, class G>
-__device__ __forceinline__ void b_src_finish(const uint3 BI, Dims d, double *q, int nc, const Aux a, Forcing f, const G &gate)
+__device__ __forceinline__ void b_src_finish(const uint3 BI, Dims d, double *q, const double *t5, int nc, const Aux a, Forcing f, const G &gate)
 {
     if (!gate.on()) return;
     gate.forcing(f.t, f.dt, f.tgauss);
@@ -133,7 +134,7 @@ __device__ __forceinline__ void b_src_finish(const uint3 BI, Dims d, double *q, 
     const double q3 = q[2 * P + c] * q1 + (a3 / a1) * q1;
     double q4 = q[3 * P + c] * q1 + (a4 / a1) * q1;
     const double auxtemp = gamma1 * (a.E[x] - 0.5 * (1.0 / a1) * (a2 * a2 + a3 * a3 + a4 * a4)) / (a1 * R);
-    double q5 = (auxtemp + q[4 * P + c]) * q1 * R / gamma1 + 0.5 * (1.0 / q1) * (q2 * q2 + q3 * q3 + q4 * q4);
+    double q5 = (auxtemp + t5[c]) * q1 * R / gamma1 + 0.5 * (1.0 / q1) * (q2 * q2 + q3 * q3 + q4 * q4);
     const double xcell = f.xlower + (i - 0.5) * f.dx - f.t * f.vsrcx;
     const double ycell = f.ylower + (j - 0.5) * f.dy;
     const double zcell = f.zlower + (k - 0.5) * f.dz;
@@ -154,9 +155,9 @@ __device__ __forceinline__ void b_src_finish(const uint3 BI, Dims d, double *q, 
         if (precipw > 0.1) {
             const double heat = sa_heating(precipw, zcell);
             const double qtemp = gamma1 * (q5 - 0.5 * (1.0 / q1) * (q2 * q2 + q3 * q3 + q4 * q4)) / (q1 * R);
-            double t5 = qtemp - auxtemp;
-            t5 = t5 + f.dt * heat;
-            q5 = (auxtemp + t5) * q1 * R / gamma1 + 0.5 * (1.0 / q1) * (q2 * q2 + q3 * q3 + q4 * q4);
+            double tp = qtemp - auxtemp;
+            tp = tp + f.dt * heat;
+            q5 = (auxtemp + tp) * q1 * R / gamma1 + 0.5 * (1.0 / q1) * (q2 * q2 + q3 * q3 + q4 * q4);
         }
     }
     q[P + c] = q2;
@@ -166,9 +167,9 @@ __device__ __forceinline__ void b_src_finish(const uint3 BI, Dims d, double *q, 
     for (int m = 5; m < nc; m++) q[m * P + c] = fmaxD(0.0, fminD(q[m * P + c], 1.0));
 }
 template <bool COL, class G>
-__global__ void k_src_finish(Dims d, double *q, int nc, const Aux a, Forcing f, G gate)
+__global__ void k_src_finish(Dims d, double *q, const double *t5, int nc, const Aux a, Forcing f, G gate)
 {
-    b_src_finish<COL>(uint3{blockIdx.x, blockIdx.y, blockIdx.z}, d, q, nc, a, f, gate);
+    b_src_finish<COL>(uint3{blockIdx.x, blockIdx.y, blockIdx.z}, d, q, t5, nc, a, f, gate);
 }
 
 // ---------------------------------------------------------- layout I/O ---
@@ -190,9 +191,13 @@ __global__ void k_planes_to_aos(double *aos, const double *planes, long long P, 
 // The FP64 form's own bodies for the batched work-list kernels
 // (batch_ops.h); its scenarios keep background columns
 struct Form64 {
+    __device__ static ZScale64 zscale(const BatchOps<double> &o, cptr<BatchOps<double>>)
+    {
+        return {o.aux1, o.aux2, o.aux3, o.aux5, o.zratio, o.d.mbc, (long long)o.d.NX * o.d.NY};
+    }
     __device__ static void bc_z(uint3 bi, const BatchOps<double> &o, cptr<BatchOps<double>>, const StepGate &g)
     {
-        b_bc_z(bi, o.d, o.q, o.nc, lohi(o.bc[4]), lohi(o.bc[5]), o.aux1, o.aux2, o.aux3, o.aux5, o.zratio, g);
+        b_bc_z(bi, o.d, o.q, o.nc, o.bcz ? o.bc.m[4] : 0, o.bcz ? o.bc.m[5] : 0, o.aux1, o.aux2, o.aux3, o.aux5, o.zratio, g);
     }
     __device__ static void convert(uint3 bi, const BatchOps<double> &o, const StepGate &g)
     {
@@ -202,7 +207,7 @@ struct Form64 {
     }
     __device__ static void finish(uint3 bi, const BatchOps<double> &o, const StepGate &g)
     {
-        b_src_finish<true>(bi, o.d, o.q, o.nc, o.ax, o.f, g);
+        b_src_finish<true>(bi, o.d, o.q, conducted(o, g), o.nc, o.ax, o.f, g);
     }
     __device__ static const double *nu(const BatchOps<double> &o) { return o.nu64; }
     __device__ static const double *kap(const BatchOps<double> &o) { return o.kap64; }
@@ -213,9 +218,8 @@ const void *batch_op_fn<double>(int op)
 {
     switch (op) {
 #define MAGIC_OP(X) case X: return reinterpret_cast<const void *>(&k_batch_op<double, X, Form64>);
-    MAGIC_OP(OP_BCX) MAGIC_OP(OP_BCY) MAGIC_OP(OP_BCZ) MAGIC_OP(OP_CLAMP) MAGIC_OP(OP_BACKUP) MAGIC_OP(OP_RESTORE)
-    MAGIC_OP(OP_CONVERT) MAGIC_OP(OP_ZGHOST_UVW) MAGIC_OP(OP_DIFF_CROSS) MAGIC_OP(OP_DIFF_XYZ) MAGIC_OP(OP_COPY_Q5)
-    MAGIC_OP(OP_PASS) MAGIC_OP(OP_CONDUCT_ZGHOST) MAGIC_OP(OP_ZSPILL) MAGIC_OP(OP_COPY_INTERIOR) MAGIC_OP(OP_FINISH)
+    MAGIC_OP(OP_BC) MAGIC_OP(OP_BCUVW) MAGIC_OP(OP_BCZ) MAGIC_OP(OP_BACKUP) MAGIC_OP(OP_RESTORE) MAGIC_OP(OP_CONVERT)
+    MAGIC_OP(OP_DIFF_CROSS) MAGIC_OP(OP_DIFF) MAGIC_OP(OP_CONDUCT) MAGIC_OP(OP_COPY_T) MAGIC_OP(OP_FINISH)
     MAGIC_OP(OP_ADD_PARTS)
 #undef MAGIC_OP
     default: return nullptr;
@@ -223,31 +227,20 @@ const void *batch_op_fn<double>(int op)
 }
 
 // FP64 instantiations of the shared kernels
-template __global__ void k_bc_x<double, NoGate>(Dims, double *, int, int, int, NoGate);
-template __global__ void k_bc_y<double, NoGate>(Dims, double *, int, int, int, NoGate);
+template __global__ void k_bc<double, ZScale64, NoGate>(Dims, double *, int, Faces, int, ZScale64, NoGate);
+template __global__ void k_diff<double, true, NoGate>(Dims, DiffArgs<double>, int, NoGate);
+template __global__ void k_diff<double, false, NoGate>(Dims, DiffArgs<double>, int, NoGate);
 template __global__ void k_clamp<double, NoGate>(double *, long long, int, NoGate);
-template __global__ void k_zghost_uvw<double, NoGate>(Dims, double *, NoGate);
 template __global__ void k_bc_z<NoGate>(Dims, double *, int, int, int, const double *, const double *, const double *,
                                         const double *, const double *, NoGate);
 template __global__ void k_src_convert<false, NoGate>(Dims, const double *, double *, const Aux, NoGate, StepParts<double>);
 template __global__ void k_src_convert<true, NoGate>(Dims, const double *, double *, const Aux, NoGate, StepParts<double>);
 template __global__ void k_add_parts<double, NoGate>(Dims, double *, StepParts<double>, NoGate);
-template __global__ void k_src_finish<false, NoGate>(Dims, double *, int, const Aux, Forcing, NoGate);
-template __global__ void k_src_finish<true, NoGate>(Dims, double *, int, const Aux, Forcing, NoGate);
-template __global__ void k_diff_xyz<double, true, NoGate>(Dims, double *, const double *, const double *, double, double,
-                                                         double, int, NoGate);
+template __global__ void k_src_finish<false, NoGate>(Dims, double *, const double *, int, const Aux, Forcing, NoGate);
+template __global__ void k_src_finish<true, NoGate>(Dims, double *, const double *, int, const Aux, Forcing, NoGate);
 template __global__ void k_diff_cross<double, true, NoGate>(Dims, double *, const double *, const double *, double, double,
                                                            double, int, NoGate);
-template __global__ void k_pass<double, true, NoGate>(Dims, double *, const double *, const double *, const double *, double,
-                                                     int, NoGate);
-template __global__ void k_diff_xyz<double, false, NoGate>(Dims, double *, const double *, const double *, double, double,
-                                                          double, int, NoGate);
 template __global__ void k_diff_cross<double, false, NoGate>(Dims, double *, const double *, const double *, double, double, double,
                                                         int, NoGate);
 template __global__ void k_copy_interior<double, NoGate>(Dims, double *, const double *, int, NoGate);
-template __global__ void k_pass<double, false, NoGate>(Dims, double *, const double *, const double *, const double *, double, int,
-                                                  NoGate);
-template __global__ void k_conduct_zghost<double, NoGate>(Dims, double *, NoGate);
-template __global__ void k_conduct_zspill<double, NoGate>(Dims, double *, int, NoGate);
-
 }  // namespace magic

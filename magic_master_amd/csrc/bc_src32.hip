@@ -17,20 +17,12 @@
 namespace magic {
 
 // FP32 instantiations of the shared kernels (coefficients as columns)
-template __global__ void k_bc_x<float, NoGate>(Dims, float *, int, int, int, NoGate);
-template __global__ void k_bc_y<float, NoGate>(Dims, float *, int, int, int, NoGate);
+template __global__ void k_bc<float, ZScale32, NoGate>(Dims, float *, int, Faces, int, ZScale32, NoGate);
+template __global__ void k_diff<float, true, NoGate>(Dims, DiffArgs<float>, int, NoGate);
 template __global__ void k_clamp<float, NoGate>(float *, long long, int, NoGate);
-template __global__ void k_zghost_uvw<float, NoGate>(Dims, float *, NoGate);
-template __global__ void k_diff_xyz<float, true, NoGate>(Dims, float *, const float *, const float *, float, float, float,
-                                                        int, NoGate);
 template __global__ void k_diff_cross<float, true, NoGate>(Dims, float *, const float *, const float *, float, float, float,
                                                         int, NoGate);
 template __global__ void k_copy_interior<float, NoGate>(Dims, float *, const float *, int, NoGate);
-template __global__ void k_pass<float, true, NoGate>(Dims, float *, const float *, const float *, const float *, float, int,
-                                                  NoGate);
-template __global__ void k_conduct_zghost<float, NoGate>(Dims, float *, NoGate);
-template __global__ void k_conduct_zspill<float, NoGate>(Dims, float *, int, NoGate);
-
 // z faces (bc3_mpi.f:544-809).  The FP64 form writes
 //   q_ghost = aux_ghost + (q_boundary - aux_boundary) * sc
 // for rho, the horizontal momenta and E, and q_ghost = q_boundary * sc for
@@ -136,7 +128,7 @@ __global__ void k32_src_convert(Dims d, const float *qin, float *q, Col32 col, G
 // the heating adding dt*heat to T' first.  Positions and the forcing are
 // evaluated in FP64.
 template <class G>
-__device__ __forceinline__ void b32_src_finish(const uint3 BI, Dims d, float *q, int nc, Col32 col, Forcing f, const G &gate)
+__device__ __forceinline__ void b32_src_finish(const uint3 BI, Dims d, float *q, const float *t5, int nc, Col32 col, Forcing f, const G &gate)
 {
     if (!gate.on()) return;
     gate.forcing(f.t, f.dt, f.tgauss);
@@ -147,7 +139,7 @@ __device__ __forceinline__ void b32_src_finish(const uint3 BI, Dims d, float *q,
     const double rp = q[c], rho = rb + rp;
     const double m2 = q[P + c] * rho, m3 = q[2 * P + c] * rho;
     double m4 = q[3 * P + c] * rho;
-    double tp = q[4 * P + c];
+    double tp = t5[c];
     const double xcell = f.xlower + (i - 0.5) * f.dx - f.t * f.vsrcx;
     const double ycell = f.ylower + (j - 0.5) * f.dy;
     const double zcell = f.zlower + (k - 0.5) * f.dz;
@@ -173,18 +165,26 @@ __device__ __forceinline__ void b32_src_finish(const uint3 BI, Dims d, float *q,
     for (int m = 5; m < nc; m++) q[m * P + c] = fmaxD(0.0f, fminD(q[m * P + c], 1.0f));
 }
 template <class G>
-__global__ void k32_src_finish(Dims d, float *q, int nc, Col32 col, Forcing f, G gate)
+__global__ void k32_src_finish(Dims d, float *q, const float *t5, int nc, Col32 col, Forcing f, G gate)
 {
-    b32_src_finish(uint3{blockIdx.x, blockIdx.y, blockIdx.z}, d, q, nc, col, f, gate);
+    b32_src_finish(uint3{blockIdx.x, blockIdx.y, blockIdx.z}, d, q, t5, nc, col, f, gate);
 }
 
 
 // The FP32 form's own bodies for the batched work-list kernels (batch_ops.h)
 struct Form32 {
     // po: the operand block in memory (the factors are indexed by layer)
+    struct ZScaleC {
+        cptr<BatchOps<float>> po;
+        __device__ __forceinline__ float operator()(int m, int side, int kbc, float v, long long, long long, long long) const
+        {
+            return m >= 5 ? v : (float)((double)v * po->zr.s[side][kbc - 1]);
+        }
+    };
+    __device__ static ZScaleC zscale(const BatchOps<float> &, cptr<BatchOps<float>> po) { return {po}; }
     __device__ static void bc_z(uint3 bi, const BatchOps<float> &o, cptr<BatchOps<float>> po, const StepGate &g)
     {
-        b32_bc_z(bi, o.d, o.q, o.nc, lohi(o.bc[4]), lohi(o.bc[5]),
+        b32_bc_z(bi, o.d, o.q, o.nc, o.bcz ? o.bc.m[4] : 0, o.bcz ? o.bc.m[5] : 0,
                  [=](int side, int k) { return po->zr.s[side][k]; }, g);
     }
     __device__ static void convert(uint3 bi, const BatchOps<float> &o, const StepGate &g)
@@ -195,7 +195,7 @@ struct Form32 {
     }
     __device__ static void finish(uint3 bi, const BatchOps<float> &o, const StepGate &g)
     {
-        b32_src_finish(bi, o.d, o.q, o.nc, o.col, o.f, g);
+        b32_src_finish(bi, o.d, o.q, conducted(o, g), o.nc, o.col, o.f, g);
     }
     __device__ static const float *nu(const BatchOps<float> &o) { return o.nu32; }
     __device__ static const float *kap(const BatchOps<float> &o) { return o.kap32; }
@@ -206,9 +206,8 @@ const void *batch_op_fn<float>(int op)
 {
     switch (op) {
 #define MAGIC_OP(X) case X: return reinterpret_cast<const void *>(&k_batch_op<float, X, Form32>);
-    MAGIC_OP(OP_BCX) MAGIC_OP(OP_BCY) MAGIC_OP(OP_BCZ) MAGIC_OP(OP_CLAMP) MAGIC_OP(OP_BACKUP) MAGIC_OP(OP_RESTORE)
-    MAGIC_OP(OP_CONVERT) MAGIC_OP(OP_ZGHOST_UVW) MAGIC_OP(OP_DIFF_CROSS) MAGIC_OP(OP_DIFF_XYZ) MAGIC_OP(OP_COPY_Q5)
-    MAGIC_OP(OP_PASS) MAGIC_OP(OP_CONDUCT_ZGHOST) MAGIC_OP(OP_ZSPILL) MAGIC_OP(OP_COPY_INTERIOR) MAGIC_OP(OP_FINISH)
+    MAGIC_OP(OP_BC) MAGIC_OP(OP_BCUVW) MAGIC_OP(OP_BCZ) MAGIC_OP(OP_BACKUP) MAGIC_OP(OP_RESTORE) MAGIC_OP(OP_CONVERT)
+    MAGIC_OP(OP_DIFF_CROSS) MAGIC_OP(OP_DIFF) MAGIC_OP(OP_CONDUCT) MAGIC_OP(OP_COPY_T) MAGIC_OP(OP_FINISH)
     MAGIC_OP(OP_ADD_PARTS)
 #undef MAGIC_OP
     default: return nullptr;
@@ -220,7 +219,7 @@ const void *batch_op_fn<float>(int op)
 template __global__ void k32_bc_z<NoGate>(Dims, float *, int, int, int, Zr32, NoGate);
 template __global__ void k32_src_convert<NoGate>(Dims, const float *, float *, Col32, NoGate, StepParts<float>);
 template __global__ void k_add_parts<float, NoGate>(Dims, float *, StepParts<float>, NoGate);
-template __global__ void k32_src_finish<NoGate>(Dims, float *, int, Col32, Forcing, NoGate);
+template __global__ void k32_src_finish<NoGate>(Dims, float *, const float *, int, Col32, Forcing, NoGate);
 
 // reference AoS q(meqn, i, j, k) (FP64, full state) <-> perturbation planes:
 // the background is subtracted / added in FP64, then rounded.

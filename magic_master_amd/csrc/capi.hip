@@ -498,49 +498,51 @@ extern "C" int magic_host_free(void *p)
 }
 
 // ------------------------------------------------------------- bc3 -------
-static int bc3_launch(magic_ctx *c, const int *mthbc)
+static ZScale64 zscale(const magic_ctx *c, double)
+{
+    const double *A = c->aux;
+    return {A + AX_RHO * c->P, A + AX_MX * c->P, A + AX_MY * c->P, A + AX_E * c->P, c->zratio, c->mbc,
+            (long long)c->d.NX * c->d.NY};
+}
+static ZScale32 zscale(const magic_ctx *c, float) { return {c->zr32}; }
+static int bc_z_apart(magic_ctx *c, double *q, int lo, int hi)
+{
+    const ZScale64 z = zscale(c, 0.0);
+    k_bc_z<<<dim3(blocks(c->d.NX, 64), c->d.NY), 64, 0, c->stream>>>(c->d, q, c->meqn, lo, hi, z.aux1, z.aux2, z.aux3, z.aux5,
+                                                                     z.zratio, NoGate{});
+    return launch_check();
+}
+static int bc_z_apart(magic_ctx *c, float *q, int lo, int hi)
+{
+    k32_bc_z<<<dim3(blocks(c->d.NX, 64), c->d.NY), 64, 0, c->stream>>>(c->d, q, c->meqn, lo, hi, c->zr32, NoGate{});
+    return launch_check();
+}
+
+// bc3 on q, with b4step3's clamp (CLAMP_BC) or diffuse's z ghosts (UVW_BC) in
+// the same pass
+template <typename T>
+static int bc_launch(magic_ctx *c, T *q, const int *mthbc, int mode)
 {
     for (int f = 0; f < 6; f++)
         if (mthbc[f] == 0 || mthbc[f] >= 4) return MAGIC_EBC;
-    Span sp(c, TC_BC, 3);
+    Span sp(c, TC_BC, 1);
     const Dims &d = c->d;
-    const double *A = c->aux;
-    auto lohi = [](int m) { return m < 0 ? 0 : m; };
-    if (c->form == MAGIC_FORM_FP32P) {
-        if (mthbc[0] >= 0 || mthbc[1] >= 0) {
-            k_bc_x<<<dim3(blocks(d.NY, 64), d.NZ), 64, 0, c->stream>>>(d, c->q32, c->meqn, lohi(mthbc[0]),
-                                                                     lohi(mthbc[1]), NoGate{});
-            TRY(launch_check());
-        }
-        if (mthbc[2] >= 0 || mthbc[3] >= 0) {
-            k_bc_y<<<dim3(blocks(d.NX, 64), d.NZ), 64, 0, c->stream>>>(d, c->q32, c->meqn, lohi(mthbc[2]),
-                                                                     lohi(mthbc[3]), NoGate{});
-            TRY(launch_check());
-        }
-        if (mthbc[4] >= 0 || mthbc[5] >= 0) {
-            k32_bc_z<<<dim3(blocks(d.NX, 64), d.NY), 64, 0, c->stream>>>(d, c->q32, c->meqn, lohi(mthbc[4]),
-                                                                       lohi(mthbc[5]), c->zr32, NoGate{});
-            TRY(launch_check());
-        }
-        return MAGIC_OK;
-    }
-    if (mthbc[0] >= 0 || mthbc[1] >= 0) {
-        k_bc_x<<<dim3(blocks(d.NY, 64), d.NZ), 64, 0, c->stream>>>(d, c->q, c->meqn, lohi(mthbc[0]),
-                                                                 lohi(mthbc[1]), NoGate{});
-        TRY(launch_check());
-    }
-    if (mthbc[2] >= 0 || mthbc[3] >= 0) {
-        k_bc_y<<<dim3(blocks(d.NX, 64), d.NZ), 64, 0, c->stream>>>(d, c->q, c->meqn, lohi(mthbc[2]),
-                                                                 lohi(mthbc[3]), NoGate{});
-        TRY(launch_check());
-    }
-    if (mthbc[4] >= 0 || mthbc[5] >= 0) {
-        k_bc_z<<<dim3(blocks(d.NX, 64), d.NY), 64, 0, c->stream>>>(
-            d, c->q, c->meqn, lohi(mthbc[4]), lohi(mthbc[5]), A + AX_RHO * c->P, A + AX_MX * c->P,
-            A + AX_MY * c->P, A + AX_E * c->P, c->zratio, NoGate{});
-        TRY(launch_check());
-    }
-    return MAGIC_OK;
+    Faces fc;
+    for (int f = 0; f < 6; f++) fc.m[f] = mthbc[f] < 0 ? 0 : mthbc[f];
+    // fewer layers than ghost layers: a mirrored or periodic z ghost can come
+    // from the other side's ghosts, so the z faces follow in their own pass
+    const bool apart = c->mz < c->mbc && (fc.m[4] != 0 || fc.m[5] != 0);
+    const int lo = fc.m[4], hi = fc.m[5];
+    if (apart) fc.m[4] = fc.m[5] = 0;
+    const bool clamp = (mode & CLAMP_BC) != 0 && c->meqn > 5;
+    const long long n = (long long)bc_lanes(d, 0) + bc_lanes(d, 1) + bc_lanes(d, 2) + (clamp ? bc_lanes(d, 3) : 0);
+    k_bc<<<blocks(n, 256), 256, 0, c->stream>>>(d, q, c->meqn, fc, mode, zscale(c, T()), NoGate{});
+    TRY(launch_check());
+    return apart ? bc_z_apart(c, q, lo, hi) : MAGIC_OK;
+}
+static int bc3_launch(magic_ctx *c, const int *mthbc, int mode = 0)
+{
+    return c->form == MAGIC_FORM_FP32P ? bc_launch(c, c->q32, mthbc, mode) : bc_launch(c, c->q, mthbc, mode);
 }
 
 extern "C" int magic_bc3(magic_ctx *c, const int mthbc[6])
@@ -1023,17 +1025,66 @@ extern "C" int magic_tune(magic_ctx *c, double dt, int reps, int shapes_out[3], 
 }
 
 // ------------------------------------------------------------- src3 ------
+// The substeps of the source pass after its conversion (src3.f90:341-376 with
+// diffuse.f:37-210 and conduct.f:245-332): per substep the boundary pass with
+// diffuse's z ghosts, the cross terms, and the directional passes of the
+// velocities next to conduct's first substep; conduct's later substeps
+// follow one by one.  q's planes keep the values before the cross terms,
+// whose ghost layers the passes read (the reference's stale copy).  t5
+// returns T' after the last substep: conduct leaves it in ut or qt, from
+// where it goes back to q only between substeps.
+template <typename T, bool COLC>
+static int src3_substeps(magic_ctx *c, DiffArgs<T> a, const int *mthbc, int ndtr, double dtr, int ndtrc, double dtrc,
+                         const T **t5)
+{
+    const Dims &d = c->d;
+    const double fourthirds = 4.0 / 3.0;
+    double dtdx2 = (dtr) / (c->dx * c->dx), dtdy2 = (dtr) / (c->dy * c->dy), dtdz2 = (dtr) / (c->dz * c->dz);
+    for (int cc = 0; cc < 3; cc++) {   // diffuse.f:135-151
+        if (cc == 0) {
+            dtdx2 = fourthirds * dtdx2;
+        } else if (cc == 1) {
+            dtdy2 = fourthirds * dtdy2;
+            dtdx2 = dtdx2 / fourthirds;
+        } else {
+            dtdz2 = fourthirds * dtdz2;
+            dtdy2 = dtdy2 / fourthirds;
+        }
+        a.f[3 * cc] = (T)dtdx2; a.f[3 * cc + 1] = (T)dtdy2; a.f[3 * cc + 2] = (T)dtdz2;
+    }
+    a.f[9] = (T)((dtrc) / (c->dx * c->dx));
+    a.f[10] = (T)((dtrc) / (c->dy * c->dy));
+    a.f[11] = (T)((dtrc) / (c->dz * c->dz));
+    a.S = c->mz > c->mx ? c->mz - c->mx : 0;
+    a.kb = passes_kb(d);
+    const double dtr32 = dtr / 6.0;
+    const dim3 g4 = passes_grid(d, ndtrc > 0 ? 4 : 3), g1 = passes_grid(d, 1);
+    const T *res = ndtrc <= 0 ? a.q + 4 * d.P : (ndtrc & 1) ? a.ut : a.qt;
+    for (int nn = 1; nn <= ndtr; nn++) {
+        TRY(bc_launch(c, a.q, mthbc, UVW_BC));
+        Span sp(c, TC_SRC, 2 + (ndtrc > 1 ? ndtrc - 1 : 0) + (nn < ndtr ? 1 : 0));
+        k_diff_cross<T, COLC, NoGate><<<diff_grid(d), cell_block(), 0, c->stream>>>(
+            d, const_cast<T *>(a.u), a.q, a.nu, (T)(dtr32 / (c->dx * c->dy)), (T)(dtr32 / (c->dx * c->dz)),
+            (T)(dtr32 / (c->dy * c->dz)), diff_kb(d), NoGate{});
+        TRY(launch_check());
+        k_diff<T, COLC, NoGate><<<g4, cell_block(), 0, c->stream>>>(d, a, 1, NoGate{});
+        TRY(launch_check());
+        for (int kk = 2; kk <= ndtrc; kk++) k_diff<T, COLC, NoGate><<<g1, cell_block(), 0, c->stream>>>(d, a, kk, NoGate{});
+        if (nn < ndtr && ndtrc > 0)
+            k_copy_interior<<<interior_grid(d), cell_block(), 0, c->stream>>>(d, a.q + 4 * d.P, res, 1, NoGate{});
+        TRY(launch_check());
+    }
+    *t5 = ndtr > 0 ? res : a.q + 4 * d.P;
+    return MAGIC_OK;
+}
+
 // The source pass of the FP32 form: the FP64 form's passes (below) on the
 // perturbation planes, with nu and kappa as background columns.
 static int src3_passes32(magic_ctx *c, const int *mthbc, int ndtr, double dtr, int ndtrc, double dtrc,
                          const Forcing &f)
 {
     const Dims &d = c->d;
-    const long long P = c->P;
     const int NZ = d.NZ;
-    const dim3 gint = interior_grid(d);
-    const dim3 gface(blocks(d.NX, 64), d.NY);
-    const float *nu = c->col32 + C32_NU * NZ, *kap = c->col32 + C32_KAP * NZ;
     const Col32 col = col32_of(c);
     {
         Span sp(c, TC_SRC, 1);
@@ -1046,61 +1097,12 @@ static int src3_passes32(magic_ctx *c, const int *mthbc, int ndtr, double dtr, i
         if (c->pending_parts) std::swap(c->q32, c->qold32);
         c->pending_parts = false;
     }
-    for (int nn = 1; nn <= ndtr; nn++) {
-        TRY(bc3_launch(c, mthbc));
-        Span sp(c, TC_SRC, 6 + 6 * (ndtrc > 0 ? ndtrc : 0));
-        const double fourthirds = 4.0 / 3.0;
-        double dtdx2 = (dtr) / (c->dx * c->dx), dtdy2 = (dtr) / (c->dy * c->dy), dtdz2 = (dtr) / (c->dz * c->dz);
-        k_zghost_uvw<<<gface, 64, 0, c->stream>>>(d, c->q32, NoGate{});
-        TRY(launch_check());
-        const double dtr32 = dtr / 6.0;
-        k_diff_cross<float, true, NoGate><<<diff_grid(d), cell_block(), 0, c->stream>>>(d, c->u32, c->q32, nu,
-                                                             (float)(dtr32 / (c->dx * c->dy)),
-                                                             (float)(dtr32 / (c->dx * c->dz)),
-                                                             (float)(dtr32 / (c->dy * c->dz)), diff_kb(d), NoGate{});
-        TRY(launch_check());
-        for (int cc = 1; cc <= 3; cc++) {
-            if (cc == 1) {
-                dtdx2 = fourthirds * dtdx2;
-            } else if (cc == 2) {
-                dtdy2 = fourthirds * dtdy2;
-                dtdx2 = dtdx2 / fourthirds;
-            } else {
-                dtdz2 = fourthirds * dtdz2;
-                dtdy2 = dtdy2 / fourthirds;
-            }
-            k_diff_xyz<float, true, NoGate><<<diff_grid(d), cell_block(), 0, c->stream>>>(
-                d, c->q32 + cc * P, c->u32 + (cc - 1) * P, nu, (float)dtdx2, (float)dtdy2, (float)dtdz2, diff_kb(d),
-                NoGate{});
-            TRY(launch_check());
-        }
-        const float cx = (float)((dtrc) / (c->dx * c->dx)), cy = (float)((dtrc) / (c->dy * c->dy)),
-                    cz = (float)((dtrc) / (c->dz * c->dz));
-        float *q5 = c->q32 + 4 * P;
-        HIPCHECK(hipMemcpyAsync(c->ut32, q5, P * sizeof(float), hipMemcpyDeviceToDevice, c->stream));
-        for (int k = 1; k <= ndtrc; k++) {
-            k_pass<float, true, NoGate><<<gint, cell_block(), 0, c->stream>>>(d, c->qt32, c->ut32, c->ut32, kap, cx, 0, NoGate{});
-            k_pass<float, true, NoGate><<<gint, cell_block(), 0, c->stream>>>(d, c->ut32, c->qt32, c->ut32, kap, cy, 1, NoGate{});
-            k_conduct_zghost<<<gface, 64, 0, c->stream>>>(d, c->ut32, NoGate{});
-            if (c->mz > c->mx) {
-                const int S = c->mz - c->mx;
-                k_conduct_zspill<<<(S + 63) / 64, 64, 0, c->stream>>>(d, c->ut32, S, NoGate{});
-            }
-            if (k < ndtrc) {
-                k_pass<float, true, NoGate><<<gint, cell_block(), 0, c->stream>>>(d, c->qt32, c->ut32, c->ut32, kap, cz, 2, NoGate{});
-                k_copy_interior<<<gint, cell_block(), 0, c->stream>>>(d, c->ut32, c->qt32, 1, NoGate{});
-            } else {
-                k_pass<float, true, NoGate><<<gint, cell_block(), 0, c->stream>>>(d, q5, c->ut32, c->ut32, kap, cz, 2, NoGate{});
-            }
-            TRY(launch_check());
-        }
-    }
-    {
-        Span sp(c, TC_SRC, 1);
-        k32_src_finish<<<gint, cell_block(), 0, c->stream>>>(d, c->q32, c->meqn, col, f, NoGate{});
-        TRY(launch_check());
-    }
-    return MAGIC_OK;
+    const float *t5;
+    const DiffArgs<float> a = {c->q32, c->u32, c->ut32, c->qt32, c->col32 + C32_NU * NZ, c->col32 + C32_KAP * NZ, {}, 0, 0};
+    TRY((src3_substeps<float, true>(c, a, mthbc, ndtr, dtr, ndtrc, dtrc, &t5)));
+    Span sp(c, TC_SRC, 1);
+    k32_src_finish<<<interior_grid(d), cell_block(), 0, c->stream>>>(d, c->q32, t5, c->meqn, col, f, NoGate{});
+    return launch_check();
 }
 
 // The source pass of the FP64 form (src3.f90:203-634 with diffuse.f and
@@ -1111,15 +1113,10 @@ static int src3_passes64(magic_ctx *c, const int *mthbc, int ndtr, double dtr, i
                          const Forcing &f)
 {
     const Dims &d = c->d;
-    const long long P = c->P;
-    const int NZ = d.NZ;
     const double *A = COL ? c->col64 : c->aux;
-    const long long S = COL ? NZ : P;   // stride between slots
+    const long long S = COL ? d.NZ : c->P;   // stride between slots
     const Aux ax = {A + AX_RHO * S, A + AX_MX * S, A + AX_MY * S, A + AX_MZ * S, A + AX_E * S, A + AX_R * S,
                     A + AX_GAM * S};
-    const double *nu = A + AX_NU * S, *kap = A + AX_KAP * S;
-    const dim3 gint = interior_grid(d);
-    const dim3 gface(blocks(d.NX, 64), d.NY);
     {
         Span sp(c, TC_SRC, 1);
         if (!c->pending_parts) c->parts64.d[0].base = nullptr;
@@ -1131,67 +1128,12 @@ static int src3_passes64(magic_ctx *c, const int *mthbc, int ndtr, double dtr, i
         if (c->pending_parts) std::swap(c->q, c->qold);
         c->pending_parts = false;
     }
-    for (int nn = 1; nn <= ndtr; nn++) {
-        TRY(bc3_launch(c, mthbc));
-        Span sp(c, TC_SRC, 6 + 6 * (ndtrc > 0 ? ndtrc : 0));
-        // diffuse: diffuse.f:37-210.  After the z-ghost fill the cross terms
-        // of q(2:4) go to u's interior; each component then takes its three
-        // directional passes in one kernel, whose ghost input is q's own
-        // ghost layers (the reference's copy, stale as there), and whose
-        // result replaces q's interior.
-        const double fourthirds = 4.0 / 3.0;
-        double dtdx2 = (dtr) / (c->dx * c->dx), dtdy2 = (dtr) / (c->dy * c->dy), dtdz2 = (dtr) / (c->dz * c->dz);
-        k_zghost_uvw<<<gface, 64, 0, c->stream>>>(d, c->q, NoGate{});
-        TRY(launch_check());
-        const double dtr32 = dtr / 6.0;
-        k_diff_cross<double, COL, NoGate><<<diff_grid(d), cell_block(), 0, c->stream>>>(d, c->u, c->q, nu,
-                                                 dtr32 / (c->dx * c->dy), dtr32 / (c->dx * c->dz),
-                                                 dtr32 / (c->dy * c->dz), diff_kb(d), NoGate{});
-        TRY(launch_check());
-        for (int cc = 1; cc <= 3; cc++) {
-            if (cc == 1) {
-                dtdx2 = fourthirds * dtdx2;
-            } else if (cc == 2) {
-                dtdy2 = fourthirds * dtdy2;
-                dtdx2 = dtdx2 / fourthirds;
-            } else {
-                dtdz2 = fourthirds * dtdz2;
-                dtdy2 = dtdy2 / fourthirds;
-            }
-            k_diff_xyz<double, COL, NoGate><<<diff_grid(d), cell_block(), 0, c->stream>>>(
-                d, c->q + cc * P, c->u + (cc - 1) * P, nu, dtdx2, dtdy2, dtdz2, diff_kb(d), NoGate{});
-            TRY(launch_check());
-        }
-        // conduct: conduct.f:245-332.  ut = q(5) on every cell once; the
-        // interior ping-pongs between ut and qt, the ghost layers stay in ut
-        // (x/y ghosts never refreshed, z ghosts refreshed for i <= mz+mbc
-        // before each z pass); the last z pass writes q(5) directly.
-        const double cx = (dtrc) / (c->dx * c->dx), cy = (dtrc) / (c->dy * c->dy), cz = (dtrc) / (c->dz * c->dz);
-        double *q5 = c->q + 4 * P;
-        HIPCHECK(hipMemcpyAsync(c->ut, q5, P * sizeof(double), hipMemcpyDeviceToDevice, c->stream));
-        for (int k = 1; k <= ndtrc; k++) {
-            k_pass<double, COL, NoGate><<<gint, cell_block(), 0, c->stream>>>(d, c->qt, c->ut, c->ut, kap, cx, 0, NoGate{});
-            k_pass<double, COL, NoGate><<<gint, cell_block(), 0, c->stream>>>(d, c->ut, c->qt, c->ut, kap, cy, 1, NoGate{});
-            k_conduct_zghost<<<gface, 64, 0, c->stream>>>(d, c->ut, NoGate{});
-            if (c->mz > c->mx) {
-                const int S = c->mz - c->mx;
-                k_conduct_zspill<<<(S + 63) / 64, 64, 0, c->stream>>>(d, c->ut, S, NoGate{});
-            }
-            if (k < ndtrc) {
-                k_pass<double, COL, NoGate><<<gint, cell_block(), 0, c->stream>>>(d, c->qt, c->ut, c->ut, kap, cz, 2, NoGate{});
-                k_copy_interior<<<gint, cell_block(), 0, c->stream>>>(d, c->ut, c->qt, 1, NoGate{});
-            } else {
-                k_pass<double, COL, NoGate><<<gint, cell_block(), 0, c->stream>>>(d, q5, c->ut, c->ut, kap, cz, 2, NoGate{});
-            }
-            TRY(launch_check());
-        }
-    }
-    {
-        Span sp(c, TC_SRC, 1);
-        k_src_finish<COL><<<gint, cell_block(), 0, c->stream>>>(d, c->q, c->meqn, ax, f, NoGate{});
-        TRY(launch_check());
-    }
-    return MAGIC_OK;
+    const double *t5;
+    const DiffArgs<double> a = {c->q, c->u, c->ut, c->qt, A + AX_NU * S, A + AX_KAP * S, {}, 0, 0};
+    TRY((src3_substeps<double, COL>(c, a, mthbc, ndtr, dtr, ndtrc, dtrc, &t5)));
+    Span sp(c, TC_SRC, 1);
+    k_src_finish<COL><<<interior_grid(d), cell_block(), 0, c->stream>>>(d, c->q, t5, c->meqn, ax, f, NoGate{});
+    return launch_check();
 }
 
 static int src3_launch(magic_ctx *c, double t, double dt, const int *mthbc_in, int *ndtr_out,
@@ -1267,8 +1209,7 @@ extern "C" int magic_claw3(magic_ctx *c, double tstart, double *tend, double dtv
         const double told = t;
         if (told + dt > *tend && tstart < *tend) dt = *tend - told;   // claw3_mpi.f:741
         for (;;) {
-            if ((st = bc3_launch(c, mthbc))) goto out;
-            if ((st = b4step3_launch(c))) goto out;
+            if ((st = bc3_launch(c, mthbc, CLAMP_BC))) goto out;   // with b4step3
             if (!defer && (st = copy_state(c, true))) goto out;
             if ((st = step3_launch(c, dt, defer, defer))) goto out;
             if ((st = step3_finish(c, &cfl))) goto out;

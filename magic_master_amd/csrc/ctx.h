@@ -190,18 +190,29 @@ static inline int ntracer(const magic_ctx *c) { return c->meqn - 5; }
 static inline dim3 cell_block() { return dim3(64, 4, 1); }
 static inline dim3 interior_grid(const Dims &d) { return dim3(blocks(d.mx, 64), blocks(d.my, 4), d.mz); }
 static inline dim3 padded_cells(const Dims &d) { return dim3(blocks(d.NX, 64), blocks(d.NY, 4), d.NZ); }
-// k_diff_xyz: layers per workgroup so that a launch has about 8192
-// workgroups (at least 4 layers each; each workgroup recomputes the x and y
-// passes of two extra layers, and its layers run one after the other, so
-// many short workgroups hide the latency better), and its grid
-static inline int diff_kb(const Dims &d)
+// Layers per workgroup of the diffusion kernels.  Each workgroup's layers run
+// one after the other, so many short workgroups hide the latency better, but
+// each loads (cross terms) or recomputes (directional passes) two layers
+// beside its own: about 8192 workgroups, at least 4 layers each where that
+// still makes 512 of them (12 x 10 x 8: the passes 10.5 -> 6.5 us and the cross
+// terms 9.0 -> 5.0 us with one layer each).  The passes run four components
+// side by side in one launch.
+static inline int layers_kb(const Dims &d, int comps)
 {
-    const long long cols = (long long)blocks(d.mx, 64) * blocks(d.my, 4);
-    const long long chunks = (8192 + cols - 1) / cols;
-    const int kb = (int)((d.mz + chunks - 1) / chunks);
-    return kb < 4 ? 4 : kb;
+    const long long cols = (long long)blocks(d.mx, 64) * blocks(d.my, 4) * comps;
+    auto kb_for = [&](long long groups) {
+        const long long chunks = (groups + cols - 1) / cols;
+        return (int)((d.mz + chunks - 1) / chunks);
+    };
+    return std::max(kb_for(8192), std::min(4, kb_for(512)));
 }
+static inline int diff_kb(const Dims &d) { return layers_kb(d, 1); }
+static inline int passes_kb(const Dims &d) { return layers_kb(d, 4); }
 static inline dim3 diff_grid(const Dims &d) { return dim3(blocks(d.mx, 64), blocks(d.my, 4), blocks(d.mz, diff_kb(d))); }
+static inline dim3 passes_grid(const Dims &d, int comps)
+{
+    return dim3(blocks(d.mx, 64), blocks(d.my, 4), comps * blocks(d.mz, passes_kb(d)));
+}
 
 // every tracer count of meqn 5 .. 10 (rpt3euX.f:134-138 splits tracers 6 .. meqn)
 static inline bool sweep_supported(int ntr) { return ntr >= 0 && ntr <= 5; }

@@ -22,58 +22,129 @@ __device__ __forceinline__ long long cid(const Dims &d, int i, int j, int k)
     return ((long long)(k + d.mbc - 1) * d.NY + (j + d.mbc - 1)) * d.NX + (i + d.mbc - 1);
 }
 
-// x faces: bc3_mpi.f:97-312.  One thread per (j, k) of the padded face.
-template <typename T, class G>
-__device__ __forceinline__ void b_bc_x(const uint3 BI, Dims d, T *q, int nc, int lo, int hi, const G &gate)
+// The cell whose value bc3's x and y passes (bc3_mpi.f:97-312, 320-536) leave
+// at (i, j, k): its column, whether the x or y momentum changes sign on the
+// way, and whether any face writes the cell at all (else it is the cell
+// itself).  The y pass comes after the x pass, so a row beyond y takes its
+// source row's value with that row's x ghosts; periodic faces copy interior
+// layers only, in x interior rows only.
+struct GhostSrc {
+    int i, j;
+    bool fx, fy, def;
+};
+__device__ __forceinline__ GhostSrc xy_source(const Dims &d, const Faces &f, int i, int j, int k)
 {
-    if (!gate.on()) return;
-    const int j = (int)(BI.x * blockDim.x + threadIdx.x) + 1 - d.mbc;
-    const int k = (int)BI.y + 1 - d.mbc;
-    if (j > d.my + d.mbc || k > d.mz + d.mbc) return;
-    const bool inner = j >= 1 && j <= d.my && k >= 1 && k <= d.mz;
-    for (int m = 0; m < nc; m++) {
-        T *p = q + (long long)m * d.P;
-        for (int ibc = 1; ibc <= d.mbc; ibc++) {
-            if (lo == 1) p[cid(d, 1 - ibc, j, k)] = p[cid(d, 1, j, k)];
-            else if (lo == 3) p[cid(d, 1 - ibc, j, k)] = (m == 1 ? T(-1.0) : T(1.0)) * p[cid(d, ibc, j, k)];
-            else if (lo == 2 && inner) p[cid(d, 1 - ibc, j, k)] = p[cid(d, d.mx - d.mbc + (d.mbc + 1 - ibc), j, k)];
-            if (hi == 1) p[cid(d, d.mx + ibc, j, k)] = p[cid(d, d.mx, j, k)];
-            else if (hi == 3) p[cid(d, d.mx + ibc, j, k)] = (m == 1 ? T(-1.0) : T(1.0)) * p[cid(d, d.mx + 1 - ibc, j, k)];
-            else if (hi == 2 && inner) p[cid(d, d.mx + ibc, j, k)] = p[cid(d, ibc, j, k)];
-        }
+    GhostSrc s = {i, j, false, false, false};
+    const bool kin = k >= 1 && k <= d.mz;
+    while (s.j < 1 || s.j > d.my) {   // once, or more often where my < mbc
+        const bool lo = s.j < 1;
+        const int m = lo ? f.m[2] : f.m[3];
+        if (m == 1) s.j = lo ? 1 : d.my;
+        else if (m == 3) { s.j = (lo ? 1 : 2 * d.my + 1) - s.j; s.fy = !s.fy; }
+        else if (m == 2 && kin) s.j += lo ? d.my : -d.my;
+        else break;
+        s.def = true;
     }
-}
-template <typename T, class G>
-__global__ void k_bc_x(Dims d, T *q, int nc, int lo, int hi, G gate)
-{
-    b_bc_x(uint3{blockIdx.x, blockIdx.y, blockIdx.z}, d, q, nc, lo, hi, gate);
+    while (s.i < 1 || s.i > d.mx) {
+        const bool lo = s.i < 1;
+        const int m = lo ? f.m[0] : f.m[1];
+        if (m == 1) s.i = lo ? 1 : d.mx;
+        else if (m == 3) { s.i = (lo ? 1 : 2 * d.mx + 1) - s.i; s.fx = !s.fx; }
+        else if (m == 2 && kin && s.j >= 1 && s.j <= d.my) s.i += lo ? d.mx : -d.mx;
+        else break;
+        s.def = true;
+    }
+    return s;
 }
 
-// y faces: bc3_mpi.f:320-536.  One thread per (i, k).
-template <typename T, class G>
-__device__ __forceinline__ void b_bc_y(const uint3 BI, Dims d, T *q, int nc, int lo, int hi, const G &gate)
+// bc3 (bc3_mpi.f:5-812) in one pass: a lane per ghost cell writes what the
+// reference's x, y and z passes leave there, taken straight from the interior
+// cell that it comes from, all components; no lane reads a cell that another
+// writes.  The three passes as kernels of their own took 30 us on small
+// grids, most of it three launches of a few waves with a chain of loads each.
+// f.m: the faces (0: skipped).  zf(m, side, kbc, v, cg, cb, col): the z
+// pass's scaling of component m (stencil for faces 1 and 3; z faces need mz >=
+// mbc, the host runs them apart otherwise).  CLAMP_BC: b4step3 (b4step3.f:35-45,
+// tracers clamped to [0, 1] on every cell) with it.  UVW_BC: diffuse's own z
+// ghosts of q(2:4) (diffuse.f:48-54) after the x and y faces.
+template <typename T, class ZF, class G>
+__device__ __forceinline__ void b_bc(const uint3 BI, Dims d, T *q, int nc, const Faces &f, int mode, const ZF &zf,
+                                     const G &gate)
 {
     if (!gate.on()) return;
-    const int i = (int)(BI.x * blockDim.x + threadIdx.x) + 1 - d.mbc;
-    const int k = (int)BI.y + 1 - d.mbc;
-    if (i > d.mx + d.mbc || k > d.mz + d.mbc) return;
-    const bool inner = k >= 1 && k <= d.mz;
-    for (int m = 0; m < nc; m++) {
-        T *p = q + (long long)m * d.P;
-        for (int jbc = 1; jbc <= d.mbc; jbc++) {
-            if (lo == 1) p[cid(d, i, 1 - jbc, k)] = p[cid(d, i, 1, k)];
-            else if (lo == 3) p[cid(d, i, 1 - jbc, k)] = (m == 2 ? T(-1.0) : T(1.0)) * p[cid(d, i, jbc, k)];
-            else if (lo == 2 && inner) p[cid(d, i, 1 - jbc, k)] = p[cid(d, i, d.my - d.mbc + (d.mbc + 1 - jbc), k)];
-            if (hi == 1) p[cid(d, i, d.my + jbc, k)] = p[cid(d, i, d.my, k)];
-            else if (hi == 3) p[cid(d, i, d.my + jbc, k)] = (m == 2 ? T(-1.0) : T(1.0)) * p[cid(d, i, d.my + 1 - jbc, k)];
-            else if (hi == 2 && inner) p[cid(d, i, d.my + jbc, k)] = p[cid(d, i, jbc, k)];
-        }
+    unsigned e = BI.x * 256u + (unsigned)(threadIdx.y * blockDim.x + threadIdx.x);
+    const bool clamp = (mode & CLAMP_BC) != 0 && nc > 5;
+    int part = 0;
+    while (part < 4 && e >= bc_lanes(d, part)) e -= bc_lanes(d, part++);
+    if (part == 4 || (part == 3 && !clamp)) return;
+    const unsigned g = 2u * d.mbc;
+    auto ghost = [&](unsigned x, int n) { return (int)x < d.mbc ? (int)x + 1 - d.mbc : n + 1 + (int)x - d.mbc; };
+    int i, j, k;
+    if (part == 0) {
+        const unsigned r = e / d.NX;
+        i = (int)(e - r * d.NX) + 1 - d.mbc;
+        const unsigned l = r / d.NY;
+        j = (int)(r - l * d.NY) + 1 - d.mbc;
+        k = ghost(l, d.mz);
+    } else if (part == 1) {
+        const unsigned r = e / d.NX;
+        i = (int)(e - r * d.NX) + 1 - d.mbc;
+        const unsigned l = r / g;
+        j = ghost(r - l * g, d.my);
+        k = (int)l + 1;
+    } else if (part == 2) {
+        const unsigned r = e / g;
+        i = ghost(e - r * g, d.mx);
+        const unsigned l = r / d.my;
+        j = (int)(r - l * d.my) + 1;
+        k = (int)l + 1;
+    } else {
+        const unsigned r = e / d.mx;
+        i = (int)(e - r * d.mx) + 1;
+        const unsigned l = r / d.my;
+        j = (int)(r - l * d.my) + 1;
+        k = (int)l + 1;
+    }
+    const long long cg = cid(d, i, j, k);
+    const int side = k < 1 ? 0 : 1, kbc = k < 1 ? 1 - k : k - d.mz;
+    const int mz = part == 0 ? f.m[4 + side] : 0;
+    const int kb = part == 0 && (mz == 1 || mz == 3) ? (side == 0 ? 1 : d.mz) : mz == 2 ? (side == 0 ? k + d.mz : k - d.mz) : k;
+    const GhostSrc s = xy_source(d, f, i, j, kb);
+    const long long cb = cid(d, s.i, s.j, kb);
+    const bool def = s.def || mz != 0;
+    const long long col = (long long)(j + d.mbc - 1) * d.NX + (i + d.mbc - 1);
+    // the boundary cell of the cell's own column: the z pass's background
+    const long long cc = cid(d, i, j, kb);
+    // diffuse's z ghosts: the column's first or last interior layer
+    const bool uvw = (mode & UVW_BC) != 0 && part == 0;
+    GhostSrc s2 = s;
+    long long cu = cb;
+    if (uvw || mz == 3) {   // the mirrored layer of a wall, or the edge layer
+        const int kl = uvw ? (side == 0 ? 1 : d.mz) : (side == 0 ? kbc : d.mz + 1 - kbc);
+        s2 = xy_source(d, f, i, j, kl);
+        cu = cid(d, s2.i, s2.j, kl);
+    }
+#pragma unroll
+    for (int m = 0; m < 10; m++) {
+        if (m >= 5 && m >= nc) break;
+        const T *p = q + (long long)m * d.P;
+        const bool edge = (uvw && m >= 1 && m <= 3) || (mz == 3 && m == 3);
+        T v = p[edge ? cu : cb];
+        if (m == 1 && (edge ? s2.fx : s.fx)) v = -v;
+        if (m == 2 && (edge ? s2.fy : s.fy)) v = -v;
+        if (mz == 3 && m == 3) v = -v;
+        else if (mz == 1 || mz == 3) v = zf(m, side, kbc, v, cg, cc, col);
+        const bool cl = clamp && m >= 5;
+        const T raw = v;
+        if (cl) v = fmaxD(T(0.0), fminD(v, T(1.0)));
+        // an interior tracer already within its range is only read
+        if (part == 3 ? cl && !(v == raw) : (def || edge || cl)) q[(long long)m * d.P + cg] = v;
     }
 }
-template <typename T, class G>
-__global__ void k_bc_y(Dims d, T *q, int nc, int lo, int hi, G gate)
+template <typename T, class ZF, class G>
+__global__ __launch_bounds__(256) void k_bc(Dims d, T *q, int nc, Faces f, int mode, ZF zf, G gate)
 {
-    b_bc_y(uint3{blockIdx.x, blockIdx.y, blockIdx.z}, d, q, nc, lo, hi, gate);
+    b_bc(uint3{blockIdx.x, blockIdx.y, blockIdx.z}, d, q, nc, f, mode, zf, gate);
 }
 
 // b4step3.f:35-45: clamp tracers to [0, 1] on every cell.
@@ -92,29 +163,6 @@ template <typename T, class G>
 __global__ void k_clamp(T *q, long long P, int nc, G gate)
 {
     b_clamp(uint3{blockIdx.x, blockIdx.y, blockIdx.z}, q, P, nc, gate);
-}
-
-// diffuse.f:48-54: z ghosts of q(2:4) from the first/last interior layer.
-template <typename T, class G>
-__device__ __forceinline__ void b_zghost_uvw(const uint3 BI, Dims d, T *q, const G &gate)
-{
-    if (!gate.on()) return;
-    const int i = (int)(BI.x * blockDim.x + threadIdx.x) + 1 - d.mbc;
-    const int j = (int)BI.y + 1 - d.mbc;
-    if (i > d.mx + d.mbc || j > d.my + d.mbc) return;
-    for (int m = 1; m <= 3; m++) {
-        T *p = q + (long long)m * d.P;
-        const T lo = p[cid(d, i, j, 1)], hi = p[cid(d, i, j, d.mz)];
-        for (int kbc = 1; kbc <= d.mbc; kbc++) {
-            p[cid(d, i, j, 1 - kbc)] = lo;
-            p[cid(d, i, j, d.mz + kbc)] = hi;
-        }
-    }
-}
-template <typename T, class G>
-__global__ void k_zghost_uvw(Dims d, T *q, G gate)
-{
-    b_zghost_uvw(uint3{blockIdx.x, blockIdx.y, blockIdx.z}, d, q, gate);
 }
 
 // Interior thread mapping: x fastest.
@@ -210,28 +258,32 @@ __global__ __launch_bounds__(256) void k_diff_cross(Dims d, T *u, const T *q, co
     b_diff_cross<T, COLC>(uint3{blockIdx.x, blockIdx.y, blockIdx.z}, d, u, q, coef, dxy, dxz, dyz, kb, gate);
 }
 
-// diffuse.f:153-208 for one velocity component: the x, y and z passes of
-// one cycle of the component loop, fused.  u holds the cross-term result on
-// the interior; the plane q holds the values before the cross terms, whose
-// ghost layers are the reference's stale ghosts of every pass; the result
-// replaces q's interior.  Each pass is the reference's (k_pass below, same
-// operand order and roundings):
+// One component's x, y and z passes (diffuse.f:153-208 after the cross terms;
+// conduct.f:262-323), fused, each with the reference's operand order and
+// roundings:
 //   x: X = U + fx*co*((U[i+1]-U)-U+U[i-1])   on the interior rows
-//   y: Y = X + fy*co*((X[j+1]-X)-X+X[j-1])   (q's ghosts at j = 0, my+1)
-//   z: q = Y + fz*co*((Y[k-1]-Y)-Y+Y[k+1])   (q's ghosts at k = 0, mz+1)
-// A workgroup covers 64 x-cells by 4 y-rows and kb layers: per layer it
-// forms X on 6 rows (its rows and one on either side) in LDS, Y on its 4
-// rows, and keeps Y of three consecutive layers in registers for the z pass
-// (the layer below its first is recomputed).  Launch: block (64, 4), grid
-// (ceil(mx/64), ceil(my/4), ceil(mz/kb)).
-template <typename T, bool COLC, class G>
-__device__ __forceinline__ void b_diff_xyz(const uint3 BI, Dims d, T *q, const T *u, const T *coef, T fx, T fy, T fz, int kb, const G &gate)
+//   y: Y = X + fy*co*((X[j+1]-X)-X+X[j-1])
+//   z: q = Y + fz*co*((Y[k-1]-Y)-Y+Y[k+1])
+// u holds the interior before the passes, gh the ghost layers, which the
+// reference copies once and never refreshes between passes; except in
+// conduct (COND), where conduct.f:86-91 fills the z ghosts before the z pass:
+// for i in [1-mbc, mz+mbc], bounded by mz, not mx.  When mx > mz the columns
+// i > mz+mbc keep their stale z ghosts.  When mz > mx an out-of-row i
+// addresses the array linearly: within a layer the writes land on later rows
+// with those rows' own values, and S = mz-mx of them cross into the next
+// layer: at in-layer offsets r < S, layers 0 and 1 end up with layer 2's
+// values, whose columns then see no z difference in layer 1 and layer 2's
+// own value below layer 2; the ghost columns among them keep layer 2's
+// ghosts in layer 1 for later substeps (late).  (Writes past the last
+// layers change ghosts that nothing reads.)
+// A workgroup covers 64 x-cells by 4 y-rows and kb layers: per layer it forms
+// X on 6 rows (its rows and one on either side) in LDS, Y on its 4 rows, and
+// keeps Y of three consecutive layers in registers for the z pass (the layer
+// below its first is recomputed).
+template <typename T, bool COLC, bool COND>
+__device__ __forceinline__ void diff_passes(const uint3 BI, const Dims &d, T *out, const T *u, const T *gh, const T *coef, T fx,
+                                            T fy, T fz, int kb, int S, bool late, T (&sx)[6][64])
 {
-    if (!gate.on()) return;
-    fx = gate.f(fx, 0);
-    fy = gate.f(fy, 1);
-    fz = gate.f(fz, 2);
-    __shared__ T sx[6][64];
     const int tx = (int)threadIdx.x, ty = (int)threadIdx.y;
     const int i = (int)BI.x * 64 + tx + 1;
     const int j0 = (int)BI.y * 4 + 1;
@@ -241,6 +293,11 @@ __device__ __forceinline__ void b_diff_xyz(const uint3 BI, Dims d, T *q, const T
     const bool own = i <= d.mx && j <= d.my;
     const long long sy = d.NX, sz = (long long)d.NX * d.NY;
     auto co_at = [&](long long c, int k) { return coef[COLC ? (long long)(k + d.mbc - 1) : c]; };
+    auto spilt = [&](int ii, int jj) { return COND && (jj + d.mbc - 1) * d.NX + (ii + d.mbc - 1) < S; };
+    // ghost column (ii, jj) of layer kk at cell c
+    auto ghost = [&](long long c, int ii, int jj, int kk) {
+        return gh[COND && late && kk == 1 && spilt(ii, jj) ? c + sz : c];
+    };
     // Y at (i, j, kk) for an interior layer kk; every lane of the block calls it
     auto yres = [&](int kk) {
         __syncthreads();   // the previous layer's readers of sx are done
@@ -249,8 +306,8 @@ __device__ __forceinline__ void b_diff_xyz(const uint3 BI, Dims d, T *q, const T
             if (i <= d.mx && jr >= 1 && jr <= d.my) {
                 const long long c = cid(d, i, jr, kk);
                 const T aq = u[c];
-                const T am = i > 1 ? u[c - 1] : q[c - 1];
-                const T ap = i < d.mx ? u[c + 1] : q[c + 1];
+                const T am = i > 1 ? u[c - 1] : ghost(c - 1, 0, jr, kk);
+                const T ap = i < d.mx ? u[c + 1] : ghost(c + 1, d.mx + 1, jr, kk);
                 const T qt = ap - aq - aq + am;
                 sx[r][tx] = aq + fx * co_at(c, kk) * qt;
             }
@@ -260,32 +317,63 @@ __device__ __forceinline__ void b_diff_xyz(const uint3 BI, Dims d, T *q, const T
         if (own) {
             const long long c = cid(d, i, j, kk);
             const T aq = sx[ty + 1][tx];
-            const T am = j > 1 ? sx[ty][tx] : q[c - sy];
-            const T ap = j < d.my ? sx[ty + 2][tx] : q[c + sy];
+            const T am = j > 1 ? sx[ty][tx] : ghost(c - sy, i, 0, kk);
+            const T ap = j < d.my ? sx[ty + 2][tx] : ghost(c + sy, i, d.my + 1, kk);
             const T qt = ap - aq - aq + am;
             y = aq + fy * co_at(c, kk) * qt;
         }
         return y;
     };
     const long long cb = own ? cid(d, i, j, k0) : 0;
-    T ym = k0 > 1 ? yres(k0 - 1) : (own ? q[cb - sz] : T(0.0));
+    const bool fill = COND && i <= d.mz + d.mbc;   // conduct refreshes this column's z ghosts
+    const bool spill = spilt(i, j);
+    T ym = k0 > 1 ? yres(k0 - 1) : (own ? gh[cb - sz] : T(0.0));
     T y0 = yres(k0);
+    if (k0 == 1 && fill) ym = y0;
     for (int k = k0; k <= k1; k++) {
         const long long c = own ? cid(d, i, j, k) : 0;
-        const T yp = k < d.mz ? yres(k + 1) : (own ? q[c + sz] : T(0.0));
+        const T yp = k < d.mz ? yres(k + 1) : (fill ? y0 : own ? gh[c + sz] : T(0.0));
+        if (COND && spill && k <= 2) {
+            if (k == 1) y0 = yp;
+            ym = y0;
+        }
         if (own) {
             const T qt = ym - y0 - y0 + yp;
-            q[c] = y0 + fz * co_at(c, k) * qt;
+            out[c] = y0 + fz * co_at(c, k) * qt;
         }
         ym = y0;
         y0 = yp;
     }
 }
-template <typename T, bool COLC, class G>
-__global__ __launch_bounds__(256) void k_diff_xyz(Dims d, T *q, const T *u, const T *coef, T fx, T fy, T fz, int kb,
-                                                  G gate)
+
+// The diffusion passes of the three velocities and conduct's first substep
+// in one launch (components 0-3 side by side in the grid's z), or with only4
+// conduct's substep kk >= 2.  fac(3*cc + n): the factor of component cc along
+// axis n, from wherever the caller keeps them (an indexed copy of them would
+// live in scratch).  Launch: block (64, 4), grid (ceil(mx/64), ceil(my/4),
+// ncomp * ceil(mz/kb)).
+template <typename T, bool COLC, class G, class FAC>
+__device__ __forceinline__ void b_diff(const uint3 BI, Dims d, const DiffArgs<T> &a, const FAC &fac, int kk, const G &gate)
 {
-    b_diff_xyz<T, COLC>(uint3{blockIdx.x, blockIdx.y, blockIdx.z}, d, q, u, coef, fx, fy, fz, kb, gate);
+    if (!gate.on()) return;
+    __shared__ T sx[6][64];
+    const int nz = (d.mz + a.kb - 1) / a.kb;
+    const int cc = kk > 1 ? 3 : __builtin_amdgcn_readfirstlane((int)BI.z / nz);
+    const uint3 bi = {BI.x, BI.y, kk > 1 ? BI.z : BI.z - cc * nz};
+    const T fx = fac(3 * cc), fy = fac(3 * cc + 1), fz = fac(3 * cc + 2);
+    if (cc < 3) {
+        T *p = a.q + (cc + 1) * d.P;
+        diff_passes<T, COLC, false>(bi, d, p, a.u + cc * d.P, p, a.nu, fx, fy, fz, a.kb, 0, false, sx);
+    } else if (gate.conducts(kk)) {
+        const T *q5 = a.q + 4 * d.P;
+        const T *src = kk == 1 ? q5 : (kk & 1) ? a.qt : a.ut;
+        diff_passes<T, COLC, true>(bi, d, (kk & 1) ? a.ut : a.qt, src, q5, a.kap, fx, fy, fz, a.kb, a.S, kk > 1, sx);
+    }
+}
+template <typename T, bool COLC, class G>
+__global__ __launch_bounds__(256) void k_diff(Dims d, DiffArgs<T> a, int kk, G gate)
+{
+    b_diff<T, COLC>(uint3{blockIdx.x, blockIdx.y, blockIdx.z}, d, a, [&](int n) { return a.f[n]; }, kk, gate);
 }
 
 // interior copy of planes src -> dst (n planes with stride P)
@@ -300,93 +388,6 @@ template <typename T, class G>
 __global__ void k_copy_interior(Dims d, T *dst, const T *src, int nplanes, G gate)
 {
     b_copy_interior(uint3{blockIdx.x, blockIdx.y, blockIdx.z}, d, dst, src, nplanes, gate);
-}
-
-// One explicit directional diffusion pass (diffuse.f:153-208, conduct.f:262-323):
-//   out = u + f*coef*(second difference of u along axis),
-// computed on the interior.  The interior values of u come from src and the
-// values on the ghost layers (which the reference copies once per call and
-// never refreshes between passes) from ghost; src may equal ghost.  The
-// second difference keeps the reference's operand order: (up-mid-mid+down)
-// along x and y, (down-mid-mid+up) along z.
-template <typename T, bool COLC, class G>
-__device__ __forceinline__ void b_pass(const uint3 BI, Dims d, T *out, const T *src, const T *ghost, const T *coef, T f, int axis, const G &gate)
-{
-    if (!gate.on()) return;
-    f = gate.f(f, 0);
-    INTERIOR_IJK
-    long long s;
-    bool lo_in, hi_in;
-    if (axis == 0) { s = 1; lo_in = i > 1; hi_in = i < d.mx; }
-    else if (axis == 1) { s = d.NX; lo_in = j > 1; hi_in = j < d.my; }
-    else { s = (long long)d.NX * d.NY; lo_in = k > 1; hi_in = k < d.mz; }
-    const T aq = src[c];
-    const T am = lo_in ? src[c - s] : ghost[c - s];
-    const T ap = hi_in ? src[c + s] : ghost[c + s];
-    const T qt = axis == 2 ? (am - aq - aq + ap) : (ap - aq - aq + am);
-    out[c] = aq + f * coef[COLC ? (long long)(k + d.mbc - 1) : c] * qt;
-}
-template <typename T, bool COLC, class G>
-__global__ void k_pass(Dims d, T *out, const T *src, const T *ghost, const T *coef, T f, int axis, G gate)
-{
-    b_pass<T, COLC>(uint3{blockIdx.x, blockIdx.y, blockIdx.z}, d, out, src, ghost, coef, f, axis, gate);
-}
-
-// conduct.f:86-91: z ghosts of u, for j in [1-mbc, my+mbc] and i in
-// [1-mbc, mz+mbc] -- the reference bounds i by mz, not mx.  When mx > mz the
-// columns i > mz+mbc keep their stale z ghosts (which then enter the z
-// stencil of the interior cells of those columns).  When mz > mx the
-// out-of-row i addresses the array linearly: within a layer the writes land
-// on later rows of the same layer with those rows' own values (what the
-// in-row fill writes anyway), so this kernel fills whole rows and
-// k_conduct_zspill adds the writes that cross into the next layer.
-template <typename T, class G>
-__device__ __forceinline__ void b_conduct_zghost(const uint3 BI, Dims d, T *u, const G &gate)
-{
-    if (!gate.on()) return;
-    const int i = (int)(BI.x * blockDim.x + threadIdx.x) + 1 - d.mbc;
-    const int j = (int)BI.y + 1 - d.mbc;
-    const int ilast = (d.mz < d.mx ? d.mz : d.mx) + d.mbc;
-    if (i > ilast || j > d.my + d.mbc) return;
-    const T lo = u[cid(d, i, j, 1)], hi = u[cid(d, i, j, d.mz)];
-    for (int kbc = 1; kbc <= d.mbc; kbc++) {
-        u[cid(d, i, j, 1 - kbc)] = lo;
-        u[cid(d, i, j, d.mz + kbc)] = hi;
-    }
-}
-template <typename T, class G>
-__global__ void k_conduct_zghost(Dims d, T *u, G gate)
-{
-    b_conduct_zghost(uint3{blockIdx.x, blockIdx.y, blockIdx.z}, d, u, gate);
-}
-
-// The layer-crossing writes of conduct.f:86-91 when mz > mx.  The rows at
-// the end of a layer address i up to mz+mbc, S = mz-mx elements past the
-// layer's last cell, so at in-layer offsets r < S the loop writes
-//   layer 2-kbc <- layer 2          (u(i,j,1-kbc) = u(i,j,1), kbc = 1..mbc)
-//   layer mz+1+kbc <- layer mz+1    (u(i,j,mz+kbc) = u(i,j,mz))
-// after the in-row fills of the rows those offsets fall in (the host checks
-// that the rows written lie before the rows that write them).  Writes past
-// the last layer leave the reference's array; they are dropped here.
-// Layers are Fortran k indices; r counts from cell (1-mbc, 1-mbc).
-template <typename T, class G>
-__device__ __forceinline__ void b_conduct_zspill(const uint3 BI, Dims d, T *u, int S, const G &gate)
-{
-    if (!gate.on()) return;
-    const int r = (int)(BI.x * blockDim.x + threadIdx.x);
-    if (r >= S) return;
-    const long long NXY = (long long)d.NX * d.NY;
-    auto L = [&](int k) { return (long long)(k + d.mbc - 1) * NXY + r; };
-    const T lo = u[L(2)], hi = u[L(d.mz + 1)];
-    for (int kbc = 1; kbc <= d.mbc; kbc++) {
-        u[L(2 - kbc)] = lo;
-        if (d.mz + 1 + kbc <= d.mz + d.mbc) u[L(d.mz + 1 + kbc)] = hi;
-    }
-}
-template <typename T, class G>
-__global__ void k_conduct_zspill(Dims d, T *u, int S, G gate)
-{
-    b_conduct_zspill(uint3{blockIdx.x, blockIdx.y, blockIdx.z}, d, u, S, gate);
 }
 
 // plain copy of n elements (copyq3 and the working copies of the source pass)
