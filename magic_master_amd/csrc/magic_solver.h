@@ -261,7 +261,7 @@ struct LimT {
 
 // suppow (rpn3euX.f:709-731) with the interface's own Courant number as the
 // upwind one (its weight is then 1), so that each branch of the exponent
-// needs one reciprocal; zero for a ratio that is not positive.
+// needs one reciprocal; zero for a ratio that is not positive, NaN among them.
 template <typename T>
 __device__ __forceinline__ T suppow1(T r, T cfl)
 {
@@ -273,7 +273,7 @@ __device__ __forceinline__ T suppow1(T r, T cfl)
     const T pp = T(4.0) * (lo ? s3 : s2) * rcpL(lo ? e : T(1.0) - e);
     const T rfrac = fabs((T(1.0) - r) * rcpL(T(1.0) + r));
     const T y = (s3 + s2 * r) * one_minus_pow(rfrac, pp);
-    return r <= T(0.0) ? T(0.0) : y;
+    return r > T(0.0) ? y : T(0.0);
 }
 
 // Transverse split of a flux difference by the Roe eigensystem of the
@@ -334,6 +334,17 @@ struct WaveT {
     __device__ __forceinline__ WaveT(T x1, T x4, T xa, T xb, T x5, T snd)
         : s(x4), p(x1 + x5), n(snd * (x5 - x1)), a(xa), b(xb) {}
     __device__ __forceinline__ void add(const WaveT &o) { s += o.s; p += o.p; n += o.n; a += o.a; b += o.b; }
+    // k (x + c y)
+    __device__ __forceinline__ static WaveT comb(T k, const WaveT &x, T c, const WaveT &y)
+    {
+        WaveT o;
+        o.s = k * (x.s + c * y.s);
+        o.p = k * (x.p + c * y.p);
+        o.n = k * (x.n + c * y.n);
+        o.a = k * (x.a + c * y.a);
+        o.b = k * (x.b + c * y.b);
+        return o;
+    }
     // k e - (lo + hi): the middle one of three splits that sum to k e
     __device__ __forceinline__ static WaveT middle(const WaveT &lo, const WaveT &hi, T k, const WaveT &e)
     {

@@ -64,6 +64,16 @@ using gptr = __attribute__((address_space(1))) T *;
 template <typename T>
 __device__ __forceinline__ gptr<T> to_global(T *p) { return (gptr<T>)p; }
 
+// A value that nothing depends on: what an idle lane holds where the others
+// have computed one (a zero there would cost a move per value and plane).
+template <typename X>
+__device__ __forceinline__ X idle_value()
+{
+    X x;
+    asm volatile("" : "=v"(x));
+    return x;
+}
+
 template <typename AT>
 __device__ __forceinline__ void report_t(const AT &A, int code, int i, int pg, int ph)
 {
@@ -75,6 +85,15 @@ __device__ __forceinline__ void report_t(const AT &A, int code, int i, int pg, i
         A.status[1] = A.sweep; A.status[2] = fi; A.status[3] = fj; A.status[4] = fk;
     }
 }
+
+// x += v in LDS.  FP64: the hardware's add, which reads nothing back (13
+// cycles per wave; the sweeps of 250 x 200 x 300 5.3 -> 4.6 ms).  FP32 adds in
+// registers: ds_add_f32 takes 190 cycles per wave.
+__device__ __forceinline__ void lds_add(double &x, double v)
+{
+    __hip_atomic_fetch_add(&x, v, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WORKGROUP);
+}
+__device__ __forceinline__ void lds_add(float &x, float v) { x += v; }
 
 // One block (tile bt along the tile axis, chunk bk along the pencils, segment
 // bs along b) of direction A; called by every lane of a 256-lane workgroup.
@@ -100,15 +119,16 @@ __device__ __forceinline__ void tile_sweep_body(const SweepArgsT<T> &A, int bt, 
     __shared__ int s_need;
     __shared__ T LT[3 * NC * NPOS];
 
-    const int t = threadIdx.x;
-    const int pa = PM ? (t / CH) : (t % TA);    // pencil within the tile
-    const int c = PM ? (t % CH) : (t / TA);     // interface offset within the chunk
+    const int t0 = threadIdx.x;
+    int t = t0;
+    int pa = PM ? (t / CH) : (t % TA);    // pencil within the tile
+    int c = PM ? (t % CH) : (t / TA);     // interface offset within the chunk
     const int nb = PM ? 1 : TA;                 // lane distance between neighbouring interfaces
     const int n = A.n, a_is_g = A.a_is_g;
     const int A0 = bt * TA, B0 = bs << A.lgL;
     const int nplane = min(1 << A.lgL, A.nB + 2 - B0);   // planes B0 .. B0 + nplane - 1
-    const int a = A0 + pa;                      // tile-axis coordinate of this lane's pencil
-    const bool pen = a <= A.nA + 1;
+    int a = A0 + pa;                            // tile-axis coordinate of this lane's pencil
+    bool pen = a <= A.nA + 1;
     const T dtdn = T(A.dtdn);
     const T d = dtdn;
     const T ca = T(a_is_g ? A.fg : A.fh), cb2 = T(a_is_g ? A.fh : A.fg);   // dt/da, dt/db
@@ -128,7 +148,7 @@ __device__ __forceinline__ void tile_sweep_body(const SweepArgsT<T> &A, int bt, 
     double cflmax = 0.0;            // Courant number, reduced in FP64
 
     // cell I-1 of interface I on plane b; the states of a lane's interface
-    const long long cell0 = (long long)(a + A.mbc - 1) * A.sA + (long long)(c - 1 + A.mbc - 1) * A.sN;
+    long long cell0 = (long long)(a + A.mbc - 1) * A.sA + (long long)(c - 1 + A.mbc - 1) * A.sN;
     T pqa[NC], pqb[NC], pga = T(0.0), pgb = T(0.0), pvg = T(0.0);
     auto fetch = [&](int Iq, int b) {
         if (pen && Iq <= n + 2) {
@@ -136,8 +156,10 @@ __device__ __forceinline__ void tile_sweep_body(const SweepArgsT<T> &A, int bt, 
             const long long y = x + A.sN;
 #pragma unroll
             for (int m = 0; m < NC; m++) {
-                pqa[m] = qold[(long long)A.comp[m] * A.P + x];
-                pqb[m] = qold[(long long)A.comp[m] * A.P + y];
+                // transverse momenta in the order a, b
+                const int cm = A.comp[m == 2 ? (a_is_g ? 2 : 3) : m == 3 ? (a_is_g ? 3 : 2) : m];
+                pqa[m] = qold[(long long)cm * A.P + x];
+                pqb[m] = qold[(long long)cm * A.P + y];
             }
             if constexpr (!PERT) {
                 pga = gam[x];
@@ -146,31 +168,52 @@ __device__ __forceinline__ void tile_sweep_body(const SweepArgsT<T> &A, int bt, 
             }
         }
     };
-    // The next plane's states are loaded while the current plane's transverse
-    // terms are computed, so that part 3 hides their latency: in the FP32
-    // form, whose registers hold them next to two waves per SIMD.  In FP64
-    // they would not fit (two waves per SIMD hide the latency instead).
-    constexpr bool PREFETCH = sizeof(T) == 4;
-    const int I0 = bk * (CH - 2) + c;
+    // The next plane's states are loaded ahead: in the FP32 form while the
+    // current plane's transverse terms are computed, which hides the latency
+    // whole; in FP64, where they would not fit beside part 3, while the plane
+    // that is complete is flushed.
+    constexpr bool EARLY = sizeof(T) == 4;
+    int I0 = bk * (CH - 2) + c;
+    // In FP64 the registers are full: what a lane can form again from its
+    // index is formed again for every plane and every flush (the asm hides that
+    // it is the same each time), or the compiler keeps it all through the loop
+    // and spills, and each reload from scratch then waits for the flush's
+    // stores as well (28.4k -> 21.7k cycles per wave and plane with the
+    // hardware's LDS adds below).
+    constexpr bool RELOAD = sizeof(T) == 8;
 
     // one plane of the ring to the block's part, as it lies in LDS: whole
     // contiguous lines, nothing read back
     gptr<T> part = to_global(A.parts) + (long long)(bs * A.sS + bk * A.sK + bt * A.sT) * (((1 << A.lgL) + 2) * NC * NPOS);
     auto flush = [&](int p, int slot) {
+        int tf = t;
+        if constexpr (RELOAD) asm volatile("" : "+v"(tf));
         T *src = LT + slot * (NC * NPOS);
         const gptr<T> dst = part + p * (NC * NPOS);
 #pragma unroll
         for (int k = 0; k < (NC * NPOS + NT - 1) / NT; k++) {
-            const int e = t + k * NT;
+            const int e = tf + k * NT;
             if (e < NC * NPOS) {
+                T zero = T(0.0);
+                if constexpr (RELOAD) asm volatile("" : "+v"(zero));
                 dst[e] = src[e];
-                src[e] = T(0.0);
+                src[e] = zero;
             }
         }
     };
-    if constexpr (PREFETCH) fetch(I0, B0);
+    fetch(I0, B0);
 
     for (int plane = 0; plane < nplane; plane++) {
+        if constexpr (RELOAD) {
+            t = t0;
+            asm volatile("" : "+v"(t));
+            pa = PM ? (t / CH) : (t % TA);
+            c = PM ? (t % CH) : (t / TA);
+            a = A0 + pa;
+            pen = a <= A.nA + 1;
+            cell0 = (long long)(a + A.mbc - 1) * A.sA + (long long)(c - 1 + A.mbc - 1) * A.sN;
+            I0 = bk * (CH - 2) + c;
+        }
         const int b = B0 + plane;               // other transverse coordinate
         const int pg = a_is_g ? a : b, ph = a_is_g ? b : a;   // (g, h) coordinates
         // No barrier here: the previous plane's last readers of the s_*
@@ -181,7 +224,7 @@ __device__ __forceinline__ void tile_sweep_body(const SweepArgsT<T> &A, int bt, 
         asm volatile("" : "+s"(looked));        // one copy of the solve in the loop below
         RoeT<double> R;
         double b1, b2, b3, b4, b5, al1, al5, s1, s2, s3;
-        bool lf, f1, f2, f5, act1, act2;
+        bool lf, act1, act2;
         T trw[NTR > 0 ? NTR : 1];   // unlimited tracer waves
         T c1, c2, c3;
         int I;
@@ -189,7 +232,7 @@ __device__ __forceinline__ void tile_sweep_body(const SweepArgsT<T> &A, int bt, 
         I = kk * (CH - 2) + c;                  // Fortran interface index
         act1 = pen && I <= n + 2;
         act2 = act1 && c >= 1 && c <= CH - 2 && I >= 1 && I <= n + 1;
-        if (!PREFETCH || looked) fetch(I, b);
+        if (looked) fetch(I, b);
 
         // ---------------- part 1: Roe solve of interface I (rpn3euX.f:138-421)
         // The waves stay in their strengths (b1, b5 acoustic, b4 entropy, b2
@@ -197,10 +240,13 @@ __device__ __forceinline__ void tile_sweep_body(const SweepArgsT<T> &A, int bt, 
         // vectors of rpn3euX.f:217-271 are never formed.  al1, al5 and lf:
         // the left-going parts of waves 1, 3 and 2 (rpn3euX.f:311-399).
         // The solve runs in FP64 in both forms (see rcp1 in magic_solver.h).
-        R = {0, 0, 0, 0, 1, 0, 0, 0, 0};
-        b1 = b2 = b3 = b4 = b5 = al1 = al5 = s1 = s2 = s3 = 0;
-        lf = f1 = f2 = f5 = false;
-        c1 = c2 = c3 = 0;
+        for (double *v : {&R.u, &R.v, &R.w, &R.enth, &R.a, &R.u2v2w2, &R.g1a2, &R.euv, &R.i2a, &b1, &b2, &b3, &b4, &b5,
+                          &al1, &al5, &s1, &s2, &s3})
+            *v = idle_value<double>();
+        c1 = idle_value<T>(); c2 = idle_value<T>(); c3 = idle_value<T>();
+        lf = false;
+#pragma unroll
+        for (int k = 0; k < NTR; k++) trw[k] = idle_value<T>();
         if (act1) {
             constexpr bool RF = sizeof(T) == 4;
             double qa[NC], qb[NC], vgc = 0.0;
@@ -315,6 +361,7 @@ __device__ __forceinline__ void tile_sweep_body(const SweepArgsT<T> &A, int bt, 
                 }
                 if (super) al1 = 0.0;
                 lf = s2 < 0.0 && !super;
+                al5 = 0.0;
                 if (lf) {
                     const double ccb = gb * pr * qb[0];
                     // state ahead of wave 3, times s3
@@ -331,26 +378,25 @@ __device__ __forceinline__ void tile_sweep_body(const SweepArgsT<T> &A, int bt, 
                 }
             }
             c1 = fabs((T)s1 * dtdn); c2 = fabs((T)s2 * dtdn); c3 = fabs((T)s3 * dtdn);
-            f1 = b1 != 0.0; f2 = b2 != 0.0; f5 = b5 != 0.0;
             s_del[0][t] = d1; s_del[1][t] = d2; s_del[2][t] = d3; s_del[3][t] = d4; s_del[4][t] = d5;
             s_s2[t] = (T)s2;
 #pragma unroll
             for (int k = 0; k < NTR; k++) s_trw[k][t] = trw[k];
-            s_flag[t] = (c <= CH - 2 && I >= 1 && I <= n + 1 && (f1 || f2 || f5)) ? 1 : 0;
-            s_cfo[t] = f5 ? c3 : (f2 ? c2 : c1);
-            // the limiters may need the Courant number an earlier chunk left
-            if (bk > 0 && act2 && !f1 && !f2 && (b3 != 0.0 || b4 != 0.0)) s_need = 1;
-        } else {
-            s_flag[t] = 0;
+            // the limiters need the Courant number an earlier interface left
+            if (act2 && b1 == 0.0 && b2 == 0.0 && (b3 != 0.0 || b4 != 0.0)) s_need = 1;
         }
         __syncthreads();
         // CFLup (rpn3euX.f:563-619) is the Courant number last assigned along
-        // the pencil.  It is needed from an interface before this chunk only
-        // where waves 1 and 2 vanish exactly and wave 3 or 4 does not (pure
-        // shear or contact): then the earlier chunks are solved again, from
-        // the nearest back, until every pencil of the tile has met an
-        // assignment, and this chunk once more.
-        if (bk == 0 || s_need == 0 || (looked && kk == bk)) break;
+        // the pencil.  It is needed from an earlier interface only where waves
+        // 1 and 2 vanish exactly and wave 3 or 4 does not (pure shear or
+        // contact): then every interface says what it assigned; and the
+        // earlier chunks are solved again, from the nearest back, until every
+        // pencil of the tile has met an assignment, and this chunk once more.
+        if (s_need == 0) break;
+        s_flag[t] = (act1 && c <= CH - 2 && I >= 1 && I <= n + 1 && (b1 != 0.0 || b2 != 0.0 || b5 != 0.0)) ? 1 : 0;
+        s_cfo[t] = b5 != 0.0 ? c3 : (b2 != 0.0 ? c2 : c1);
+        __syncthreads();
+        if (bk == 0 || (looked && kk == bk)) break;
         if (!looked) {
             looked = 1;
             if (t < TA) { s_cprev[t] = T(0.0); s_found[t] = 0; }
@@ -367,16 +413,25 @@ __device__ __forceinline__ void tile_sweep_body(const SweepArgsT<T> &A, int bt, 
         // ---------------- part 2: limiters (rpn3euX.f:434-676) and the strengths
         // of the second-order correction (flux3fw.f:270-284).  From here on the
         // transverse directions are the tile axis a and the marching axis b.
-        T un = 0, ua = 0, ub = 0, snd = 1, isnd = 1, kin = 0, hk = 0;   // Roe state: kin = |u|^2/2, hk = H - kin
-        T x1 = 0, x4 = 0, xa = 0, xb = 0, x5 = 0, l1 = 0, l5 = 0;       // strengths, left-going acoustic parts
-        T q1 = 0, q4 = 0, qsa = 0, qsb = 0, q5 = 0;                     // strengths of cqxx
+        const T un = (T)R.u, ua = (T)R.v, ub = (T)R.w, snd = (T)R.a, isnd = (T)(2.0 * R.i2a);
+        const T kin = (T)(0.5 * R.u2v2w2), hk = (T)(R.enth - 0.5 * R.u2v2w2);   // |u|^2/2 and H - |u|^2/2
+        const T x1 = (T)b1, x4 = (T)b4, xa = (T)b2, xb = (T)b3, x5 = (T)b5;     // strengths
+        T l1 = (T)al1, l5 = (T)al5;                                            // left-going acoustic parts
+        T q1 = idle_value<T>(), q4 = idle_value<T>(), qsa = idle_value<T>(), qsb = idle_value<T>(),
+          q5 = idle_value<T>();   // strengths of cqxx
         T trq[NTR > 0 ? NTR : 1];
         T nrm[2][5];   // FP32 form: the cell's own normal update
+#pragma unroll
+        for (int k = 0; k < NTR; k++) trq[k] = idle_value<T>();
+        if constexpr (PERT) {
+#pragma unroll
+            for (int m = 0; m < 10; m++) nrm[m / 5][m % 5] = idle_value<T>();
+        }
         if (act2) {
             const T ts1 = (T)s1, ts2 = (T)s2, ts3 = (T)s3;
-            const T k1 = T(0.5) * copysign(T(1.0), ts1) * (T(1.0) - fabs(ts1) * dtdn);
-            const T k2 = T(0.5) * copysign(T(1.0), ts2) * (T(1.0) - fabs(ts2) * dtdn);
-            const T k3 = T(0.5) * copysign(T(1.0), ts3) * (T(1.0) - fabs(ts3) * dtdn);
+            // sign(s) / 2 * (1 - |s| dt/dn)
+            const T k1 = copysign(T(0.5), ts1) * (T(1.0) - c1), k2 = copysign(T(0.5), ts2) * (T(1.0) - c2),
+                    k3 = copysign(T(0.5), ts3) * (T(1.0) - c3);
             const int up1 = signbit(s1) ? t + nb : t - nb, up2 = signbit(s2) ? t + nb : t - nb,
                       up3 = signbit(s3) ? t + nb : t - nb;
             const LimT<T> lim2(c2);
@@ -393,48 +448,33 @@ __device__ __forceinline__ void tile_sweep_body(const SweepArgsT<T> &A, int bt, 
             }
             // the upwind interfaces' strengths in this interface's waves: those
             // of wave 2 come from one of the two acoustic waves' sides
-            double g1 = 0, g2 = 0, g3 = 0, g4 = 0, g5 = 0;
-            T wl1 = T(1.0), wl2 = T(1.0), wl3 = T(1.0), wl4 = T(1.0), wl5 = T(1.0);
-            if (b1 != 0.0 || b2 != 0.0 || b3 != 0.0 || b4 != 0.0 || b5 != 0.0) {
-                auto b4of = [&](int e) {
-                    return R.g1a2 * (R.euv * s_del[0][e] + R.u * s_del[1][e] + R.v * s_del[2][e] + R.w * s_del[3][e] -
-                                     s_del[4][e]);
-                };
-                auto b5of = [&](int e, double b4e) {
-                    return (s_del[1][e] + (R.a - R.u) * s_del[0][e] - R.a * b4e) * R.i2a;
-                };
-                const double b4l = b4of(up1), b4r = b4of(up3);
-                g1 = s_del[0][up1] - b4l - b5of(up1, b4l);
-                g5 = b5of(up3, b4r);
-                g4 = up2 == up1 ? b4l : b4r;
-                g2 = s_del[2][up2] - R.v * s_del[0][up2];
-                g3 = s_del[3][up2] - R.w * s_del[0][up2];
-                if (f1 || f5) {
-                    const T r1 = (T)(g1 / b1), r5 = (T)(g5 / b5);
-                    const T p1 = suppow1(r1, c1), p5 = suppow1(r5, c3);
-                    wl1 = f1 ? p1 : T(1.0);
-                    wl5 = f5 ? p5 : T(1.0);
+            auto b4of = [&](int e) {
+                return R.g1a2 * (R.euv * s_del[0][e] + R.u * s_del[1][e] + R.v * s_del[2][e] + R.w * s_del[3][e] -
+                                 s_del[4][e]);
+            };
+            auto b5of = [&](int e, double b4e) {
+                return (s_del[1][e] + (R.a - R.u) * s_del[0][e] - R.a * b4e) * R.i2a;
+            };
+            const double b4l = b4of(up1), b4r = b4of(up3);
+            const double g1 = s_del[0][up1] - b4l - b5of(up1, b4l), g5 = b5of(up3, b4r), g4 = up2 == up1 ? b4l : b4r;
+            const double g2 = s_del[2][up2] - R.v * s_del[0][up2], g3 = s_del[3][up2] - R.w * s_del[0][up2];
+            T wt = T(1.0);   // the upwind Courant number's weight: 1 where it is c2 itself
+            if (b2 == 0.0 && (b3 != 0.0 || b4 != 0.0)) {
+                T cflup;
+                if (b1 != 0.0) cflup = c1;
+                else {
+                    cflup = s_cprev[pa];
+                    for (int j = c - 1; j >= 0; j--)
+                        if (s_flag[t - (c - j) * nb]) { cflup = s_cfo[t - (c - j) * nb]; break; }
                 }
-                if (f2 || b3 != 0.0 || b4 != 0.0) {
-                    T wt = T(1.0);   // the upwind Courant number's weight: 1 where it is c2 itself
-                    if (!f2 && (b3 != 0.0 || b4 != 0.0)) {
-                        T cflup;
-                        if (f1) cflup = c1;
-                        else {
-                            cflup = s_cprev[pa];
-                            for (int j = c - 1; j >= 0; j--)
-                                if (s_flag[t - (c - j) * nb]) { cflup = s_cfo[t - (c - j) * nb]; break; }
-                        }
-                        wt = lim2.weight(cflup);
-                    }
-                    const T r2 = (T)(g2 / b2), r3 = (T)(g3 / b3), r4 = (T)(g4 / b4);
-                    const T p2 = lim2.bee(T(1.0), beta, r2, T(1.0)), p3 = lim2.bee(T(1.0), beta, r3, wt),
-                            p4 = lim2.bee(T(1.0), beta, r4, wt);
-                    wl2 = f2 ? p2 : T(1.0);
-                    wl3 = b3 != 0.0 ? p3 : T(1.0);
-                    wl4 = b4 != 0.0 ? p4 : T(1.0);
-                }
+                wt = lim2.weight(cflup);
             }
+            // A vanishing wave needs no case of its own: the limiters are
+            // finite for any ratio, NaN among them, and multiply a strength
+            // of zero.
+            const T wl1 = suppow1((T)(g1 / b1), c1), wl5 = suppow1((T)(g5 / b5), c3);
+            const T wl2 = lim2.bee(T(1.0), beta, (T)(g2 / b2), T(1.0)), wl3 = lim2.bee(T(1.0), beta, (T)(g3 / b3), wt),
+                    wl4 = lim2.bee(T(1.0), beta, (T)(g4 / b4), wt);
             // strengths of cqxx, in FP64 up to here
             const double w1 = (double)(k1 * wl1) * b1, w2 = (double)(k2 * wl2) * b2, w3 = (double)(k2 * wl3) * b3,
                          w4 = (double)(k2 * wl4) * b4, w5 = (double)(k3 * wl5) * b5;
@@ -457,30 +497,19 @@ __device__ __forceinline__ void tile_sweep_body(const SweepArgsT<T> &A, int bt, 
                     const double mv = R.v * rho + nv, mw = R.w * rho + nw;
                     nrm[ph2][0] = (T)rho;
                     nrm[ph2][1] = (T)(R.u * rho + nn);
-                    nrm[ph2][2] = (T)(a_is_g ? mv : mw);
-                    nrm[ph2][3] = (T)(a_is_g ? mw : mv);
+                    nrm[ph2][2] = (T)mv;
+                    nrm[ph2][3] = (T)mw;
                     nrm[ph2][4] = (T)((R.enth - kk) * pp + kk * rho + R.u * nn + R.v * nv + R.w * nw);
                 }
-                cflmax = fmaxF(cflmax, fmaxF(fmaxF(fabs((double)ts1), fabs((double)ts2)), fabs((double)ts3)) * A.dtdn);
+                cflmax = fmaxF(cflmax, fmaxF(fabs((double)ts1), fabs((double)ts3)) * A.dtdn);   // |u| is between them
             } else {
-                cflmax = fmaxF(cflmax, fmaxF(fmaxF(c1, c2), c3));
+                cflmax = fmaxF(cflmax, fmaxF(c1, c3));
             }
-            un = (T)R.u;
-            ua = (T)(a_is_g ? R.v : R.w);
-            ub = (T)(a_is_g ? R.w : R.v);
-            snd = (T)R.a;
-            isnd = (T)(2.0 * R.i2a);
-            kin = (T)(0.5 * R.u2v2w2);
-            hk = (T)(R.enth - 0.5 * R.u2v2w2);
-            x1 = (T)b1; x4 = (T)b4; x5 = (T)b5;
-            xa = (T)(a_is_g ? b2 : b3);
-            xb = (T)(a_is_g ? b3 : b2);
-            l1 = (T)al1; l5 = (T)al5;
             q1 = (T)w1; q4 = (T)w4; q5 = (T)w5;
-            qsa = (T)(a_is_g ? w2 : w3);
-            qsb = (T)(a_is_g ? w3 : w2);
+            qsa = (T)w2;
+            qsb = (T)w3;
         }
-        if (PREFETCH && plane + 1 < nplane) fetch(I0, b + 1);
+        if (EARLY && plane + 1 < nplane) fetch(I0, b + 1);
 
         // ---------------- part 3: transverse terms (flux3fw.f:297-625), two phases
         // The transverse splits by the interface's Roe eigensystem
@@ -505,6 +534,7 @@ __device__ __forceinline__ void tile_sweep_body(const SweepArgsT<T> &A, int bt, 
         const int r0 = plane % 3, r1 = r0 == 2 ? 0 : r0 + 1, r2 = r1 == 2 ? 0 : r1 + 1;
         const T kf = -(T(1.0) / T(6.0)) * d * ca * cb2, kea = -T(0.5) * d * ca, keb = -T(0.5) * d * cb2;
         const SpeedT<T> va(ua, snd), vb(ub, snd);
+        T hm = lf ? T(1.0) : T(0.0);   // 1 where the contact waves belong to the phase
 #pragma unroll 1
         for (int phase = 0; phase < 2; phase++) {
             // phase 0 (L): interface I -> cell I-1; phase 1 (R): -> cell I
@@ -512,19 +542,13 @@ __device__ __forceinline__ void tile_sweep_body(const SweepArgsT<T> &A, int bt, 
             const int ci = phase == 0 ? c - 1 : c;  // cell index within the chunk's tile
             if (phase == 1 && t == 0) s_need = 0;   // every lane has read it (phase 0's barrier)
             const T sg = phase == 0 ? T(1.0) : -T(1.0);
-            const bool has = (phase == 0) == lf;    // the contact waves belong to this phase
             WaveT<T> y[3], z[3], N;
             T yt[3][NTR > 0 ? NTR : 1], zt[3][NTR > 0 ? NTR : 1], Nt[NTR > 0 ? NTR : 1];
             if (on) {
-                const T a1 = phase == 0 ? l1 : x1 - l1, a5 = phase == 0 ? l5 : x5 - l5;
-                const T a4 = has ? x4 : T(0.0), aa = has ? xa : T(0.0), ab = has ? xb : T(0.0);
                 const T s3q = T(3.0) * sg, s2q = T(2.0) * sg;
-                const WaveT<T> F(kf * (a1 + s3q * q1), kf * (a4 + s3q * q4), kf * (aa + s3q * qsa), kf * (ab + s3q * qsb),
-                                 kf * (a5 + s3q * q5), snd);
-                const WaveT<T> E(a1 + s2q * q1, a4 + s2q * q4, aa + s2q * qsa, ab + s2q * qsb, a5 + s2q * q5, snd);
-                if constexpr (!PERT)
-                    N = WaveT<T>(-d * (a1 + sg * q1), -d * (a4 + sg * q4), -d * (aa + sg * qsa), -d * (ab + sg * qsb),
-                                 -d * (a5 + sg * q5), snd);
+                const WaveT<T> X(l1, hm * x4, hm * xa, hm * xb, l5, snd), Q(q1, q4, qsa, qsb, q5, snd);
+                const WaveT<T> F = WaveT<T>::comb(kf, X, s3q, Q), E = WaveT<T>::comb(T(1.0), X, s2q, Q);
+                if constexpr (!PERT) N = WaveT<T>::comb(-d, X, sg, Q);
                 y[0] = vb.template split_b<0>(F, snd, isnd);
                 y[2] = vb.template split_b<2>(F, snd, isnd);
                 z[0] = va.template split_a<0>(F, snd, isnd);
@@ -542,7 +566,7 @@ __device__ __forceinline__ void tile_sweep_body(const SweepArgsT<T> &A, int bt, 
                 z[1] = WaveT<T>::middle(z[0], z[2], keb, E);
 #pragma unroll
                 for (int k = 0; k < NTR; k++) {
-                    const T at = has ? trw[k] : T(0.0);
+                    const T at = hm * trw[k];
                     const T ft = kf * (at + s3q * trq[k]), et = at + s2q * trq[k];
                     Nt[k] = -d * (at + sg * trq[k]);
 #pragma unroll
@@ -572,12 +596,12 @@ __device__ __forceinline__ void tile_sweep_body(const SweepArgsT<T> &A, int bt, 
                             for (int m = 0; m < 5; m++) o[m] += phase == 0 ? nrm[0][m] : nrm[1][m];
                         }
 #pragma unroll
-                        for (int m = 0; m < 5; m++) row[m * NPOS] += o[m];
+                        for (int m = 0; m < 5; m++) lds_add(row[m * NPOS], o[m]);
 #pragma unroll
                         for (int k = 0; k < NTR; k++) {
                             T v = va.w2(r) * yt[j][k] + vb.w2(j) * zt[r][k];
                             if (r == 1 && j == 1) v += Nt[k];
-                            row[(5 + k) * NPOS] += v;
+                            lds_add(row[(5 + k) * NPOS], v);
                         }
                     };
                     target(IConst<0>{});
@@ -598,9 +622,13 @@ __device__ __forceinline__ void tile_sweep_body(const SweepArgsT<T> &A, int bt, 
             substep(IConst<0>{});
             substep(IConst<1>{});
             substep(IConst<2>{});
+            l1 = x1 - l1;   // phase 1: the right-going parts
+            l5 = x5 - l5;
+            hm = T(1.0) - hm;
         }
 
         // ---------------- flush: plane b-1 has all its increments
+        if (!EARLY && plane + 1 < nplane) fetch(I0, b + 1);
         flush(plane, r0);
     }
     flush(nplane, nplane % 3);
