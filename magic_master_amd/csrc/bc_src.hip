@@ -169,6 +169,7 @@ __device__ __forceinline__ void b_src_finish(const uint3 BI, Dims d, double *q, 
 template <bool COL, class G>
 __global__ void k_src_finish(Dims d, double *q, const double *t5, int nc, const Aux a, Forcing f, G gate)
 {
+    gate.report();
     b_src_finish<COL>(uint3{blockIdx.x, blockIdx.y, blockIdx.z}, d, q, t5, nc, a, f, gate);
 }
 
@@ -227,20 +228,20 @@ const void *batch_op_fn<double>(int op)
 }
 
 // FP64 instantiations of the shared kernels
-template __global__ void k_bc<double, ZScale64, NoGate>(Dims, double *, int, Faces, int, ZScale64, NoGate);
-template __global__ void k_diff<double, true, NoGate>(Dims, DiffArgs<double>, int, NoGate);
-template __global__ void k_diff<double, false, NoGate>(Dims, DiffArgs<double>, int, NoGate);
-template __global__ void k_clamp<double, NoGate>(double *, long long, int, NoGate);
-template __global__ void k_bc_z<NoGate>(Dims, double *, int, int, int, const double *, const double *, const double *,
-                                        const double *, const double *, NoGate);
-template __global__ void k_src_convert<false, NoGate>(Dims, const double *, double *, const Aux, NoGate, StepParts<double>);
-template __global__ void k_src_convert<true, NoGate>(Dims, const double *, double *, const Aux, NoGate, StepParts<double>);
-template __global__ void k_add_parts<double, NoGate>(Dims, double *, StepParts<double>, NoGate);
-template __global__ void k_src_finish<false, NoGate>(Dims, double *, const double *, int, const Aux, Forcing, NoGate);
-template __global__ void k_src_finish<true, NoGate>(Dims, double *, const double *, int, const Aux, Forcing, NoGate);
-template __global__ void k_diff_cross<double, true, NoGate>(Dims, double *, const double *, const double *, double, double,
-                                                           double, int, NoGate);
-template __global__ void k_diff_cross<double, false, NoGate>(Dims, double *, const double *, const double *, double, double, double,
-                                                        int, NoGate);
-template __global__ void k_copy_interior<double, NoGate>(Dims, double *, const double *, int, NoGate);
+template __global__ void k_bc<double, ZScale64, GridGate>(Dims, double *, int, Faces, int, ZScale64, GridGate);
+template __global__ void k_diff<double, true, GridGate>(Dims, DiffArgs<double>, int, GridGate);
+template __global__ void k_diff<double, false, GridGate>(Dims, DiffArgs<double>, int, GridGate);
+template __global__ void k_clamp<double, GridGate>(double *, long long, int, GridGate);
+template __global__ void k_bc_z<GridGate>(Dims, double *, int, int, int, const double *, const double *, const double *,
+                                        const double *, const double *, GridGate);
+template __global__ void k_src_convert<false, GridGate>(Dims, const double *, double *, const Aux, GridGate, StepParts<double>);
+template __global__ void k_src_convert<true, GridGate>(Dims, const double *, double *, const Aux, GridGate, StepParts<double>);
+template __global__ void k_add_parts<double, GridGate>(Dims, double *, StepParts<double>, GridGate);
+template __global__ void k_src_finish<false, GridGate>(Dims, double *, const double *, int, const Aux, Forcing, GridGate);
+template __global__ void k_src_finish<true, GridGate>(Dims, double *, const double *, int, const Aux, Forcing, GridGate);
+template __global__ void k_diff_cross<double, true, GridGate>(Dims, double *, const double *, const double *, double, double,
+                                                           double, int, GridGate);
+template __global__ void k_diff_cross<double, false, GridGate>(Dims, double *, const double *, const double *, double, double, double,
+                                                        int, GridGate);
+template __global__ void k_copy_interior<double, GridGate>(Dims, double *, const double *, int, GridGate);
 }  // namespace magic

@@ -17,12 +17,12 @@
 namespace magic {
 
 // FP32 instantiations of the shared kernels (coefficients as columns)
-template __global__ void k_bc<float, ZScale32, NoGate>(Dims, float *, int, Faces, int, ZScale32, NoGate);
-template __global__ void k_diff<float, true, NoGate>(Dims, DiffArgs<float>, int, NoGate);
-template __global__ void k_clamp<float, NoGate>(float *, long long, int, NoGate);
-template __global__ void k_diff_cross<float, true, NoGate>(Dims, float *, const float *, const float *, float, float, float,
-                                                        int, NoGate);
-template __global__ void k_copy_interior<float, NoGate>(Dims, float *, const float *, int, NoGate);
+template __global__ void k_bc<float, ZScale32, GridGate>(Dims, float *, int, Faces, int, ZScale32, GridGate);
+template __global__ void k_diff<float, true, GridGate>(Dims, DiffArgs<float>, int, GridGate);
+template __global__ void k_clamp<float, GridGate>(float *, long long, int, GridGate);
+template __global__ void k_diff_cross<float, true, GridGate>(Dims, float *, const float *, const float *, float, float, float,
+                                                        int, GridGate);
+template __global__ void k_copy_interior<float, GridGate>(Dims, float *, const float *, int, GridGate);
 // z faces (bc3_mpi.f:544-809).  The FP64 form writes
 //   q_ghost = aux_ghost + (q_boundary - aux_boundary) * sc
 // for rho, the horizontal momenta and E, and q_ghost = q_boundary * sc for
@@ -167,6 +167,7 @@ __device__ __forceinline__ void b32_src_finish(const uint3 BI, Dims d, float *q,
 template <class G>
 __global__ void k32_src_finish(Dims d, float *q, const float *t5, int nc, Col32 col, Forcing f, G gate)
 {
+    gate.report();
     b32_src_finish(uint3{blockIdx.x, blockIdx.y, blockIdx.z}, d, q, t5, nc, col, f, gate);
 }
 
@@ -216,10 +217,10 @@ const void *batch_op_fn<float>(int op)
 
 // instantiations of the single-grid kernels (the batched driver's are
 // k_batch_op, above)
-template __global__ void k32_bc_z<NoGate>(Dims, float *, int, int, int, Zr32, NoGate);
-template __global__ void k32_src_convert<NoGate>(Dims, const float *, float *, Col32, NoGate, StepParts<float>);
-template __global__ void k_add_parts<float, NoGate>(Dims, float *, StepParts<float>, NoGate);
-template __global__ void k32_src_finish<NoGate>(Dims, float *, const float *, int, Col32, Forcing, NoGate);
+template __global__ void k32_bc_z<GridGate>(Dims, float *, int, int, int, Zr32, GridGate);
+template __global__ void k32_src_convert<GridGate>(Dims, const float *, float *, Col32, GridGate, StepParts<float>);
+template __global__ void k_add_parts<float, GridGate>(Dims, float *, StepParts<float>, GridGate);
+template __global__ void k32_src_finish<GridGate>(Dims, float *, const float *, int, Col32, Forcing, GridGate);
 
 // reference AoS q(meqn, i, j, k) (FP64, full state) <-> perturbation planes:
 // the background is subtracted / added in FP64, then rounded.

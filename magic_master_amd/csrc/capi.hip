@@ -509,12 +509,12 @@ static int bc_z_apart(magic_ctx *c, double *q, int lo, int hi)
 {
     const ZScale64 z = zscale(c, 0.0);
     k_bc_z<<<dim3(blocks(c->d.NX, 64), c->d.NY), 64, 0, c->stream>>>(c->d, q, c->meqn, lo, hi, z.aux1, z.aux2, z.aux3, z.aux5,
-                                                                     z.zratio, NoGate{});
+                                                                     z.zratio, GridGate{});
     return launch_check();
 }
 static int bc_z_apart(magic_ctx *c, float *q, int lo, int hi)
 {
-    k32_bc_z<<<dim3(blocks(c->d.NX, 64), c->d.NY), 64, 0, c->stream>>>(c->d, q, c->meqn, lo, hi, c->zr32, NoGate{});
+    k32_bc_z<<<dim3(blocks(c->d.NX, 64), c->d.NY), 64, 0, c->stream>>>(c->d, q, c->meqn, lo, hi, c->zr32, GridGate{});
     return launch_check();
 }
 
@@ -536,7 +536,7 @@ static int bc_launch(magic_ctx *c, T *q, const int *mthbc, int mode)
     if (apart) fc.m[4] = fc.m[5] = 0;
     const bool clamp = (mode & CLAMP_BC) != 0 && c->meqn > 5;
     const long long n = (long long)bc_lanes(d, 0) + bc_lanes(d, 1) + bc_lanes(d, 2) + (clamp ? bc_lanes(d, 3) : 0);
-    k_bc<<<blocks(n, 256), 256, 0, c->stream>>>(d, q, c->meqn, fc, mode, zscale(c, T()), NoGate{});
+    k_bc<<<blocks(n, 256), 256, 0, c->stream>>>(d, q, c->meqn, fc, mode, zscale(c, T()), c->gate);
     TRY(launch_check());
     return apart ? bc_z_apart(c, q, lo, hi) : MAGIC_OK;
 }
@@ -558,8 +558,8 @@ static int b4step3_launch(magic_ctx *c)
 {
     if (c->meqn > 5) {
         Span sp(c, TC_OTHER, 1);
-        if (c->form == MAGIC_FORM_FP32P) k_clamp<<<blocks(c->P, 256), 256, 0, c->stream>>>(c->q32, c->P, c->meqn, NoGate{});
-        else k_clamp<<<blocks(c->P, 256), 256, 0, c->stream>>>(c->q, c->P, c->meqn, NoGate{});
+        if (c->form == MAGIC_FORM_FP32P) k_clamp<<<blocks(c->P, 256), 256, 0, c->stream>>>(c->q32, c->P, c->meqn, GridGate{});
+        else k_clamp<<<blocks(c->P, 256), 256, 0, c->stream>>>(c->q, c->P, c->meqn, GridGate{});
         TRY(launch_check());
     }
     return MAGIC_OK;
@@ -802,7 +802,7 @@ template <typename T>
 static int add_parts_launch(magic_ctx *c, T *q, const StepParts<T> &sp)
 {
     Span s(c, TC_OTHER, 1);
-    k_add_parts<T, NoGate><<<padded_cells(c->d), cell_block(), 0, c->stream>>>(c->d, q, sp, NoGate{});
+    k_add_parts<T, GridGate><<<padded_cells(c->d), cell_block(), 0, c->stream>>>(c->d, q, sp, GridGate{});
     return launch_check();
 }
 
@@ -905,7 +905,13 @@ static int setup_sweeps(magic_ctx *c)
 }
 static bool sweeps_defer(const magic_ctx *c) { return form_tile(c) && !c->parts_one; }
 
-// The sweeps of one step and the read-back of its reductions.  from_q: they
+static int scal_copy(magic_ctx *c)
+{
+    HIPCHECK(hipMemcpyAsync(c->hscal, c->dscal, 8 * sizeof(unsigned long long), hipMemcpyDeviceToHost, c->stream));
+    return MAGIC_OK;
+}
+
+// The sweeps of one step and (without defer) the read-back of its reductions.  from_q: they
 // read q itself (with deferred increments q does not change meanwhile);
 // else the backup.  The increments end up in q, or with defer stay pending
 // in the part buffer (c->pending_parts).
@@ -926,10 +932,9 @@ static int step3_launch(magic_ctx *c, double dt, bool from_q = false, bool defer
         TRY((step3_sweeps<double, false>(c, a, c->q, dt, c->parts64)));
         c->pending_parts = c->parts64.d[0].base != nullptr;
     }
-    HIPCHECK(hipMemcpyAsync(c->hscal, c->dscal, 8 * sizeof(unsigned long long), hipMemcpyDeviceToHost,
-                            c->stream));
-    if (!defer) TRY(parts_flush(c));
-    return MAGIC_OK;
+    if (defer) return MAGIC_OK;   // the source pass reports and adds the increments
+    TRY(scal_copy(c));
+    return parts_flush(c);
 }
 
 static int step3_finish(magic_ctx *c, double *cfl)
@@ -1063,15 +1068,15 @@ static int src3_substeps(magic_ctx *c, DiffArgs<T> a, const int *mthbc, int ndtr
     for (int nn = 1; nn <= ndtr; nn++) {
         TRY(bc_launch(c, a.q, mthbc, UVW_BC));
         Span sp(c, TC_SRC, 2 + (ndtrc > 1 ? ndtrc - 1 : 0) + (nn < ndtr ? 1 : 0));
-        k_diff_cross<T, COLC, NoGate><<<diff_grid(d), cell_block(), 0, c->stream>>>(
+        k_diff_cross<T, COLC, GridGate><<<diff_grid(d), cell_block(), 0, c->stream>>>(
             d, const_cast<T *>(a.u), a.q, a.nu, (T)(dtr32 / (c->dx * c->dy)), (T)(dtr32 / (c->dx * c->dz)),
-            (T)(dtr32 / (c->dy * c->dz)), diff_kb(d), NoGate{});
+            (T)(dtr32 / (c->dy * c->dz)), diff_kb(d), c->gate);
         TRY(launch_check());
-        k_diff<T, COLC, NoGate><<<g4, cell_block(), 0, c->stream>>>(d, a, 1, NoGate{});
+        k_diff<T, COLC, GridGate><<<g4, cell_block(), 0, c->stream>>>(d, a, 1, c->gate);
         TRY(launch_check());
-        for (int kk = 2; kk <= ndtrc; kk++) k_diff<T, COLC, NoGate><<<g1, cell_block(), 0, c->stream>>>(d, a, kk, NoGate{});
+        for (int kk = 2; kk <= ndtrc; kk++) k_diff<T, COLC, GridGate><<<g1, cell_block(), 0, c->stream>>>(d, a, kk, c->gate);
         if (nn < ndtr && ndtrc > 0)
-            k_copy_interior<<<interior_grid(d), cell_block(), 0, c->stream>>>(d, a.q + 4 * d.P, res, 1, NoGate{});
+            k_copy_interior<<<interior_grid(d), cell_block(), 0, c->stream>>>(d, a.q + 4 * d.P, res, 1, c->gate);
         TRY(launch_check());
     }
     *t5 = ndtr > 0 ? res : a.q + 4 * d.P;
@@ -1092,7 +1097,7 @@ static int src3_passes32(magic_ctx *c, const int *mthbc, int ndtr, double dtr, i
         // with pending increments the new state goes to the other buffer and
         // the old one stays behind as the backup
         float *to = c->pending_parts ? c->qold32 : c->q32;
-        k32_src_convert<<<padded_cells(c->d), cell_block(), 0, c->stream>>>(d, c->q32, to, col, NoGate{}, c->parts32);
+        k32_src_convert<<<padded_cells(c->d), cell_block(), 0, c->stream>>>(d, c->q32, to, col, c->gate, c->parts32);
         TRY(launch_check());
         if (c->pending_parts) std::swap(c->q32, c->qold32);
         c->pending_parts = false;
@@ -1101,7 +1106,7 @@ static int src3_passes32(magic_ctx *c, const int *mthbc, int ndtr, double dtr, i
     const DiffArgs<float> a = {c->q32, c->u32, c->ut32, c->qt32, c->col32 + C32_NU * NZ, c->col32 + C32_KAP * NZ, {}, 0, 0};
     TRY((src3_substeps<float, true>(c, a, mthbc, ndtr, dtr, ndtrc, dtrc, &t5)));
     Span sp(c, TC_SRC, 1);
-    k32_src_finish<<<interior_grid(d), cell_block(), 0, c->stream>>>(d, c->q32, t5, c->meqn, col, f, NoGate{});
+    k32_src_finish<<<interior_grid(d), cell_block(), 0, c->stream>>>(d, c->q32, t5, c->meqn, col, f, c->gate);
     return launch_check();
 }
 
@@ -1123,7 +1128,7 @@ static int src3_passes64(magic_ctx *c, const int *mthbc, int ndtr, double dtr, i
         // with pending increments the new state goes to the other buffer and
         // the old one stays behind as the backup
         double *to = c->pending_parts ? c->qold : c->q;
-        k_src_convert<COL><<<padded_cells(d), cell_block(), 0, c->stream>>>(d, c->q, to, ax, NoGate{}, c->parts64);
+        k_src_convert<COL><<<padded_cells(d), cell_block(), 0, c->stream>>>(d, c->q, to, ax, c->gate, c->parts64);
         TRY(launch_check());
         if (c->pending_parts) std::swap(c->q, c->qold);
         c->pending_parts = false;
@@ -1132,7 +1137,7 @@ static int src3_passes64(magic_ctx *c, const int *mthbc, int ndtr, double dtr, i
     const DiffArgs<double> a = {c->q, c->u, c->ut, c->qt, A + AX_NU * S, A + AX_KAP * S, {}, 0, 0};
     TRY((src3_substeps<double, COL>(c, a, mthbc, ndtr, dtr, ndtrc, dtrc, &t5)));
     Span sp(c, TC_SRC, 1);
-    k_src_finish<COL><<<interior_grid(d), cell_block(), 0, c->stream>>>(d, c->q, t5, c->meqn, ax, f, NoGate{});
+    k_src_finish<COL><<<interior_grid(d), cell_block(), 0, c->stream>>>(d, c->q, t5, c->meqn, ax, f, c->gate);
     return launch_check();
 }
 
@@ -1202,7 +1207,8 @@ extern "C" int magic_claw3(magic_ctx *c, double tstart, double *tend, double dtv
     // an accepted step's source pass (into the other state buffer): the state
     // before the step needs no copy and a rejected step no restoring.  A
     // batch's grid keeps its buffers' places (its captured kernels hold them)
-    // and takes the copying way.
+    // and takes the copying way.  The source pass is launched behind the sweeps
+    // under their result's gate, and the host waits once per attempt.
     if (maxn > 0 && (st = setup_sweeps(c))) return st;
     const bool defer = sweeps_defer(c) && c->own_stream;
     for (int n = 1; n <= maxn; n++) {
@@ -1212,7 +1218,20 @@ extern "C" int magic_claw3(magic_ctx *c, double tstart, double *tend, double dtv
             if ((st = bc3_launch(c, mthbc, CLAMP_BC))) goto out;   // with b4step3
             if (!defer && (st = copy_state(c, true))) goto out;
             if ((st = step3_launch(c, dt, defer, defer))) goto out;
-            if ((st = step3_finish(c, &cfl))) goto out;
+            int ss = MAGIC_OK, a, b;
+            if (defer) {
+                c->gate = GridGate{c->dscal, c->hscal, cflv[0]};
+                ss = src3_launch(c, told, dt, mthbc, &a, &b);   // claw3_mpi.f:900-905
+                c->gate = GridGate{};
+                if (ss && (st = scal_copy(c))) goto out;        // nothing was launched: a setting src3 refuses
+            }
+            st = step3_finish(c, &cfl);
+            if (defer && !ss && (st || !(cfl <= cflv[0]))) {    // no source pass ran: its target is the backup again
+                if (c->form == MAGIC_FORM_FP32P) std::swap(c->q32, c->qold32);
+                else std::swap(c->q, c->qold);
+                c->pending_parts = true;
+            }
+            if (st) goto out;
             t = told + dt;
             if (log_dt && nl < maxlog) {
                 log_dt[nl] = dt;
@@ -1222,16 +1241,14 @@ extern "C" int magic_claw3(magic_ctx *c, double tstart, double *tend, double dtv
             nl++;
             if (cfl <= cflv[0]) {                                  // claw3_mpi.f:861-886
                 cflmax = cflmax > cfl ? cflmax : cfl;
+                st = defer ? ss : src3_launch(c, told, dt, mthbc, &a, &b);
+                if (st) goto out;
                 break;
             }
             t = told;
             c->pending_parts = false;   // the rejected step's increments are dropped with it
             if (!defer && (st = copy_state(c, false))) goto out;
             dt = dtv[1] < dt * cflv[1] / cfl ? dtv[1] : dt * cflv[1] / cfl;
-        }
-        {
-            int a, b;
-            if ((st = src3_launch(c, told, dt, mthbc, &a, &b))) goto out;   // claw3_mpi.f:900-905
         }
         if (cfl == 0.0) dt = dtv[1];                               // claw3_mpi.f:910-919
         else dt = dtv[1] < dt * cflv[1] / cfl ? dtv[1] : dt * cflv[1] / cfl;

@@ -100,6 +100,7 @@ struct magic_ctx {
     int4 *items = nullptr;
     int item_off[4] = {0, 0, 0, 0};
     int item_shape[3] = {-1, -1, -1};      // the shapes the items were laid out for
+    GridGate gate;                         // of the kernels launched now (claw3's source pass)
     unsigned long long *hscal = nullptr;   // pinned host words: [0, 8) mirror dscal, [HSCAL_SUMS, +10) global sums
     void *sums_d = nullptr;                // global sums: partials and results (first magic_global_sums)
     magic_params prm;

@@ -91,3 +91,31 @@ def test_batch_substeps(form):
         assert (max(counts) >= (2, 2)) == (k < 3), counts
         assert states[k]["t"] == t and states[k]["dt"] == dt_next
         np.testing.assert_array_equal(qb[k], qs)
+
+
+@pytest.mark.parametrize("form", ["fp32", "fp64"])
+@pytest.mark.parametrize("dt", [0.5, 50.0])   # accepted, and rejected once before
+def test_claw3_refused_source(form, dt):
+    """A source pass that src3 refuses (a wind that changes with time) ends
+    claw3 with its error after the accepted sweeps: q holds their increments."""
+    from magic_master_amd.hip import FORM_FP32P, FORM_FP64, MagicError, MagicHIP
+    c, p, g, aux, q = perturbed(17, 12, 20, [2, 2, 1, 1, 3, 1], seed=5, vel=0.05)
+    p.omega1 = 1.0
+    d = MagicHIP(g, p, aux, q, form=FORM_FP32P if form == "fp32" else FORM_FP64)
+    try:
+        with pytest.raises(MagicError):
+            d.claw3(0.0, -1.0, [dt, c.dtv[1], 0, 0, 0], c.cflv, [1, 0], c.method, c.mthbc)
+        got = d.get_q()
+        d.set_q(q)
+        d.bc3(c.mthbc)
+        d.b4step3()
+        d.backup()
+        while (cfl := d.step3(dt)) > c.cflv[0]:
+            dt = min(c.dtv[1], dt * c.cflv[1] / cfl)
+            d.restore()
+            d.bc3(c.mthbc)
+            d.b4step3()
+            d.backup()
+        np.testing.assert_array_equal(got, d.get_q())
+    finally:
+        d.close()
