@@ -235,7 +235,7 @@ static dim3 list_block(int lg)
 // The block list each kernel class walks
 static int op_list(int op)
 {
-    static const int lg[NOP] = {LG_BC, LG_BCUVW, LG_BCZ, LG_CPY, LG_CPY, LG_PAD, LG_DIF, LG_DF4, LG_DIF, LG_INT, LG_INT, LG_PAD};
+    static const int lg[NOP] = {LG_BC, LG_BCUVW, LG_BCZ, LG_CPY, LG_CPY, LG_PAD, LG_DIF, LG_DF4, LG_DF1, LG_INT, LG_INT, LG_PAD};
     return lg[op];
 }
 
@@ -479,23 +479,29 @@ static void form_ops(const magic_ctx *c, BatchOps<double> &o)
     o.zratio = c->zratio;
 }
 
-// Layers per workgroup of a scenario's diffusion passes.  A workgroup
-// recomputes the x and y passes of the two layers around its own; one grid
-// takes few layers (diff_kb) to have enough workgroups, a batch has enough
-// from its scenarios and takes at least 16.  The result does not depend on
-// the layer count.
-static int batch_kb(const Dims &d) { return std::max(diff_kb(d), std::min(16, d.mz)); }
+// Layers per workgroup of the diffusion kernels of a batch.  A workgroup forms
+// the two layers around its own as well; one grid takes few layers (diff_kb)
+// to have enough workgroups, a batch has them from its scenarios: about 4096, of
+// 8 to 16 layers (24 FP32 grids of 40 x 36 x 60: the passes 68 us with 16
+// layers, 49 with 4, 45 with 8).  The result does not depend on the layer count.
+static int batch_kb(const magic_batch *b)
+{
+    long long work = 0;
+    for (const magic_ctx *c : b->sc)
+        if (c) work += 4ll * passes_cols(c->d).x * passes_cols(c->d).y * c->mz;
+    return (int)std::min<long long>(16, std::max<long long>(8, work / 4096));
+}
 
 // whether a scenario's z faces run after the others in their own pass (capi.hip's bc_launch)
 static bool z_apart(const magic_ctx *c, const int *bc) { return c->mz < c->mbc && (bc[4] > 0 || bc[5] > 0); }
 
 // Grid of list lg for one scenario (x, y, z blocks; x = 0: no blocks)
-static int4 list_grid(const magic_batch *b, const magic_ctx *c, const int *bc, int lg)
+static int4 list_grid(const magic_batch *b, const magic_ctx *c, const int *bc, int lg, int kb)
 {
     const Dims &d = c->d;
     const long long P = c->P;
     auto g1 = [](long long x) { return make_int4((int)x, 1, 1, 0); };
-    const int kb = batch_kb(d), nzb = (int)blocks(d.mz, kb);
+    const int nzb = (int)blocks(d.mz, kb);
     switch (lg) {
     case LG_BC: case LG_BCUVW: {
         long long n = (long long)bc_lanes(d, 0) + bc_lanes(d, 1) + bc_lanes(d, 2);
@@ -505,8 +511,8 @@ static int4 list_grid(const magic_batch *b, const magic_ctx *c, const int *bc, i
     case LG_BCZ: return z_apart(c, bc) ? make_int4(blocks(d.NX, 64), d.NY, 1, 0) : g1(0);
     case LG_CPY: return g1(std::min<long long>(8192, blocks(P * b->meqn, 256)));
     case LG_PAD: { const dim3 g = padded_cells(d); return make_int4(g.x, g.y, g.z, 0); }
-    case LG_DIF: return make_int4(blocks(d.mx, 64), blocks(d.my, 4), nzb, 0);
-    case LG_DF4: return make_int4(blocks(d.mx, 64), blocks(d.my, 4), 4 * nzb, 0);
+    case LG_DIF: return make_int4(diff_cols(d).x, diff_cols(d).y, nzb, 0);
+    case LG_DF1: case LG_DF4: return make_int4(passes_cols(d).x, passes_cols(d).y, (lg == LG_DF4 ? 4 : 1) * nzb, 0);
     case LG_INT: { const dim3 g = interior_grid(d); return make_int4(g.x, g.y, g.z, 0); }
     default: return g1(0);
     }
@@ -517,6 +523,7 @@ static int4 list_grid(const magic_batch *b, const magic_ctx *c, const int *bc, i
 template <typename T>
 static int build_ops(magic_batch *b)
 {
+    const int kb = batch_kb(b);
     std::vector<BatchOps<T>> ops(b->n);
     std::vector<int> off((size_t)NLG * (b->cap + 1), 0);
     std::vector<int4> gdim((size_t)NLG * b->cap, make_int4(0, 1, 1, 0));
@@ -528,7 +535,7 @@ static int build_ops(magic_batch *b)
             off[(size_t)lg * (b->cap + 1) + s] = (int)total;
             magic_ctx *c = b->sc[s];
             if (!c) continue;
-            const int4 g = list_grid(b, c, &b->mthbc[6 * s], lg);
+            const int4 g = list_grid(b, c, &b->mthbc[6 * s], lg, kb);
             gdim[(size_t)lg * b->cap + s] = g;
             total += (long long)g.x * g.y * g.z;
             if (total > 0x7fffffff) return MAGIC_EUNSUPPORTED;
@@ -546,7 +553,7 @@ static int build_ops(magic_batch *b)
         o.sp = slot_parts(b, s, T());
         o.one = b->parts_one;
         o.nc = c->meqn;
-        o.kb = batch_kb(c->d);
+        o.kb = kb;
         o.spill = c->mz > c->mx ? c->mz - c->mx : 0;
         for (int f = 0; f < 6; f++) o.bc.m[f] = std::max(0, b->mthbc[6 * s + f]);
         o.bcz = z_apart(c, &b->mthbc[6 * s]);

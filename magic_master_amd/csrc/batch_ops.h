@@ -54,10 +54,12 @@ enum {
 //   BCUVW boundary lanes (1-D, 256 lanes)
 //   BCZ bc3 z faces of grids with mz < mbc   (NX/64, NY)
 //   CPY grid-stride copy of meqn planes       PAD padded cells     (NX/64, NY/4, NZ)
-//   DIF cross terms, and conduct's substeps kk >= 2  (mx/64, my/4, mz/kb)
-//   DF4 directional passes of four components, conduct's first substep among them (mx/64, my/4, 4 * mz/kb)
+//   DIF cross terms      (mx/64, my/4, mz/kb)
+//   DF1 conduct's substeps kk >= 2  (mx/64, my/(4 DIFF_ROWS), mz/kb)
+//   DF4 directional passes of four components, conduct's first substep among them
+//       (mx/64, my/(4 DIFF_ROWS), 4 * mz/kb)
 //   INT interior cells   (mx/64, my/4, mz)
-enum { LG_BC = 0, LG_BCUVW, LG_BCZ, LG_CPY, LG_PAD, LG_DIF, LG_DF4, LG_INT, NLG };
+enum { LG_BC = 0, LG_BCUVW, LG_BCZ, LG_CPY, LG_PAD, LG_DIF, LG_DF1, LG_DF4, LG_INT, NLG };
 
 struct GateSpec {
     int mode, nn, kk, fslot;
@@ -187,7 +189,6 @@ __global__ __launch_bounds__(256) void k_batch_op(const BatchOps<T> *__restrict_
             // arg (OP_CONDUCT): the substep kk >= 2
             const DiffArgs<T> a = {o.q, o.u, o.ut, o.qt, FORM::nu(o), FORM::kap(o), {}, o.spill, o.kb};
             b_diff<T, true>(bi, o.d, a, [&](int i) { return g.f(T(0.0), i); }, OP == OP_DIFF ? 1 : arg, g);
-            __syncthreads();
         } else if constexpr (OP == OP_COPY_T) {
             b_copy_interior(bi, o.d, o.q + 4 * P, conducted(o, g), 1, g);
         } else if constexpr (OP == OP_FINISH) {

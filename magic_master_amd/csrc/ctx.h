@@ -191,28 +191,32 @@ static inline int ntracer(const magic_ctx *c) { return c->meqn - 5; }
 static inline dim3 cell_block() { return dim3(64, 4, 1); }
 static inline dim3 interior_grid(const Dims &d) { return dim3(blocks(d.mx, 64), blocks(d.my, 4), d.mz); }
 static inline dim3 padded_cells(const Dims &d) { return dim3(blocks(d.NX, 64), blocks(d.NY, 4), d.NZ); }
-// Layers per workgroup of the diffusion kernels.  Each workgroup's layers run
-// one after the other, so many short workgroups hide the latency better, but
-// each loads (cross terms) or recomputes (directional passes) two layers
-// beside its own: about 8192 workgroups, at least 4 layers each where that
-// still makes 512 of them (12 x 10 x 8: the passes 10.5 -> 6.5 us and the cross
-// terms 9.0 -> 5.0 us with one layer each).  The passes run four components
-// side by side in one launch.
-static inline int layers_kb(const Dims &d, int comps)
+// Layers per workgroup of the diffusion kernels, cols workgroups side by side.
+// Each workgroup's layers run one after the other, so many short workgroups
+// hide the latency better, but each loads (cross terms) or forms (directional
+// passes) two layers beside its own: about most workgroups, at least 4 layers
+// each where that still makes 512 of them (12 x 10 x 8: the cross terms 9.0 ->
+// 5.0 us with one layer each).
+static inline int layers_kb(const Dims &d, long long cols, long long most)
 {
-    const long long cols = (long long)blocks(d.mx, 64) * blocks(d.my, 4) * comps;
     auto kb_for = [&](long long groups) {
         const long long chunks = (groups + cols - 1) / cols;
         return (int)((d.mz + chunks - 1) / chunks);
     };
-    return std::max(kb_for(8192), std::min(4, kb_for(512)));
+    return std::max(kb_for(most), std::min(4, kb_for(512)));
 }
-static inline int diff_kb(const Dims &d) { return layers_kb(d, 1); }
-static inline int passes_kb(const Dims &d) { return layers_kb(d, 4); }
-static inline dim3 diff_grid(const Dims &d) { return dim3(blocks(d.mx, 64), blocks(d.my, 4), blocks(d.mz, diff_kb(d))); }
+static inline dim3 diff_cols(const Dims &d) { return dim3(blocks(d.mx, 64), blocks(d.my, 4)); }
+static inline dim3 passes_cols(const Dims &d) { return dim3(blocks(d.mx, 64), blocks(d.my, 4 * DIFF_ROWS)); }
+static inline int diff_kb(const Dims &d) { return layers_kb(d, (long long)diff_cols(d).x * diff_cols(d).y, 8192); }
+// (the directional passes of four components run side by side in one launch)
+static inline int passes_kb(const Dims &d)
+{
+    return layers_kb(d, 4ll * passes_cols(d).x * passes_cols(d).y, 4096);
+}
+static inline dim3 diff_grid(const Dims &d) { return dim3(diff_cols(d).x, diff_cols(d).y, blocks(d.mz, diff_kb(d))); }
 static inline dim3 passes_grid(const Dims &d, int comps)
 {
-    return dim3(blocks(d.mx, 64), blocks(d.my, 4), comps * blocks(d.mz, passes_kb(d)));
+    return dim3(passes_cols(d).x, passes_cols(d).y, comps * blocks(d.mz, passes_kb(d)));
 }
 
 // every tracer count of meqn 5 .. 10 (rpt3euX.f:134-138 splits tracers 6 .. meqn)

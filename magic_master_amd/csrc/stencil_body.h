@@ -102,7 +102,20 @@ __device__ __forceinline__ void b_bc(const uint3 BI, Dims d, T *q, int nc, const
         i = (int)(e - r * d.mx) + 1;
         const unsigned l = r / d.my;
         j = (int)(r - l * d.my) + 1;
-        k = (int)l + 1;
+        k = (int)l * CLAMP_LAYERS + 1;
+        const long long sz = (long long)d.NX * d.NY;
+        for (int m = 5; m < nc; m++) {
+            T *p = q + (long long)m * d.P + cid(d, i, j, k), v[CLAMP_LAYERS];
+#pragma unroll
+            for (int n = 0; n < CLAMP_LAYERS; n++)
+                if (k + n <= d.mz) v[n] = p[n * sz];
+#pragma unroll
+            for (int n = 0; n < CLAMP_LAYERS; n++) {
+                const T cl = fmaxD(T(0.0), fminD(v[n], T(1.0)));
+                if (k + n <= d.mz && !(cl == v[n])) p[n * sz] = cl;   // only read where in its range already
+            }
+        }
+        return;
     }
     const long long cg = cid(d, i, j, k);
     const int side = k < 1 ? 0 : 1, kbc = k < 1 ? 1 - k : k - d.mz;
@@ -134,10 +147,8 @@ __device__ __forceinline__ void b_bc(const uint3 BI, Dims d, T *q, int nc, const
         if (mz == 3 && m == 3) v = -v;
         else if (mz == 1 || mz == 3) v = zf(m, side, kbc, v, cg, cc, col);
         const bool cl = clamp && m >= 5;
-        const T raw = v;
         if (cl) v = fmaxD(T(0.0), fminD(v, T(1.0)));
-        // an interior tracer already within its range is only read
-        if (part == 3 ? cl && !(v == raw) : (def || edge || cl)) q[(long long)m * d.P + cg] = v;
+        if (def || edge || cl) q[(long long)m * d.P + cg] = v;
     }
 }
 template <typename T, class ZF, class G>
@@ -275,73 +286,117 @@ __global__ __launch_bounds__(256) void k_diff_cross(Dims d, T *u, const T *q, co
 // own value below layer 2; the ghost columns among them keep layer 2's
 // ghosts in layer 1 for later substeps (late).  (Writes past the last
 // layers change ghosts that nothing reads.)
-// A workgroup covers 64 x-cells by 4 y-rows and kb layers: per layer it forms
-// X on 6 rows (its rows and one on either side) in LDS, Y on its 4 rows, and
-// keeps Y of three consecutive layers in registers for the z pass (the layer
-// below its first is recomputed).
+// A wave covers 64 x-cells by DIFF_ROWS y-rows and marches over kb layers,
+// every lane holding its column of rows in registers: per layer it forms X on
+// its rows and one on either side, Y on its rows, and keeps Y of three
+// consecutive layers for the z pass (the layers around its first and last are
+// formed twice).  The next layer's values are loaded before the current one's
+// are used; nothing is shared between lanes, so no wave waits for another.
+// Bound by memory.  Against rows in LDS with two barriers per layer: 250 x 200
+// x 300 FP64 558 -> 412 us, FP32 batch of 8 grids of 200 x 200 x 300 1.60 ->
+// 0.78 ms (4 reads, 4 writes of 384 MB: 3.9 TB/s).
 template <typename T, bool COLC, bool COND>
 __device__ __forceinline__ void diff_passes(const uint3 BI, const Dims &d, T *out, const T *u, const T *gh, const T *coef, T fx,
-                                            T fy, T fz, int kb, int S, bool late, T (&sx)[6][64])
+                                            T fy, T fz, int kb, int S, bool late)
 {
-    const int tx = (int)threadIdx.x, ty = (int)threadIdx.y;
-    const int i = (int)BI.x * 64 + tx + 1;
-    const int j0 = (int)BI.y * 4 + 1;
-    const int j = j0 + ty;
+    constexpr int R = DIFF_ROWS;
+    const int tx = (int)threadIdx.x, ty = __builtin_amdgcn_readfirstlane((int)threadIdx.y);
+    const int il = (int)BI.x * 64 + tx + 1, i = il < d.mx ? il : d.mx;   // lanes past the end repeat the last column
+    const int j0 = ((int)BI.y * 4 + ty) * R + 1;
     const int k0 = (int)BI.z * kb + 1;
     const int k1 = k0 + kb - 1 < d.mz ? k0 + kb - 1 : d.mz;
-    const bool own = i <= d.mx && j <= d.my;
-    const long long sy = d.NX, sz = (long long)d.NX * d.NY;
+    if (j0 > d.my || k0 > d.mz) return;
+    const long long sz = (long long)d.NX * d.NY;
     auto co_at = [&](long long c, int k) { return coef[COLC ? (long long)(k + d.mbc - 1) : c]; };
     auto spilt = [&](int ii, int jj) { return COND && (jj + d.mbc - 1) * d.NX + (ii + d.mbc - 1) < S; };
     // ghost column (ii, jj) of layer kk at cell c
     auto ghost = [&](long long c, int ii, int jj, int kk) {
         return gh[COND && late && kk == 1 && spilt(ii, jj) ? c + sz : c];
     };
-    // Y at (i, j, kk) for an interior layer kk; every lane of the block calls it
-    auto yres = [&](int kk) {
-        __syncthreads();   // the previous layer's readers of sx are done
-        for (int r = ty; r < 6; r += 4) {
-            const int jr = j0 - 1 + r;
-            if (i <= d.mx && jr >= 1 && jr <= d.my) {
-                const long long c = cid(d, i, jr, kk);
-                const T aq = u[c];
-                const T am = i > 1 ? u[c - 1] : ghost(c - 1, 0, jr, kk);
-                const T ap = i < d.mx ? u[c + 1] : ghost(c + 1, d.mx + 1, jr, kk);
-                const T qt = ap - aq - aq + am;
-                sx[r][tx] = aq + fx * co_at(c, kk) * qt;
+    const bool first = i == 1, last = i == d.mx;
+    // rows j0-1 .. j0+R of the layer loaded last: the cell and its x neighbours
+    constexpr int NCO = COLC ? 1 : R + 2;
+    T wa[R + 2], wm[R + 2], wp[R + 2], wc[NCO];
+#pragma unroll
+    for (int r = 0; r < R + 2; r++) wa[r] = wm[r] = wp[r] = T(0.0);
+#pragma unroll
+    for (int r = 0; r < NCO; r++) wc[r] = T(0.0);
+    auto load = [&](int kk) __attribute__((always_inline)) {
+        if (COLC) wc[0] = co_at(0, kk);
+#pragma unroll
+        for (int r = 0; r < R + 2; r++) {
+            const int j = j0 - 1 + r;
+            const long long c = cid(d, i, j, kk);
+            T a = T(0.0), m = T(0.0), p = T(0.0), cc = T(0.0);
+            if (j >= 1 && j <= d.my) {
+                a = u[c];
+                m = first ? ghost(c - 1, 0, j, kk) : u[c - 1];
+                p = last ? ghost(c + 1, d.mx + 1, j, kk) : u[c + 1];
+                if (!COLC) cc = co_at(c, kk);
+            } else if (j <= d.my + 1) {
+                a = ghost(c, i, j, kk);
+            }
+            wa[r] = a;
+            wm[r] = m;
+            wp[r] = p;
+            if (!COLC) wc[COLC ? 0 : r] = cc;
+        }
+    };
+    // X, then Y of the loaded layer, whose coefficients go to co; layer kn is
+    // loaded (0: none) once X is formed
+    auto yres = [&](T (&y)[R], T (&co)[COLC ? 1 : R], int kn) __attribute__((always_inline)) {
+        T x[R + 2];
+#pragma unroll
+        for (int r = 0; r < R + 2; r++) {
+            const int j = j0 - 1 + r;
+            x[r] = wa[r];
+            if (j >= 1 && j <= d.my) {
+                const T qt = wp[r] - wa[r] - wa[r] + wm[r];
+                x[r] = wa[r] + fx * wc[COLC ? 0 : r] * qt;
             }
         }
-        __syncthreads();
-        T y = T(0.0);
-        if (own) {
-            const long long c = cid(d, i, j, kk);
-            const T aq = sx[ty + 1][tx];
-            const T am = j > 1 ? sx[ty][tx] : ghost(c - sy, i, 0, kk);
-            const T ap = j < d.my ? sx[ty + 2][tx] : ghost(c + sy, i, d.my + 1, kk);
-            const T qt = ap - aq - aq + am;
-            y = aq + fy * co_at(c, kk) * qt;
+#pragma unroll
+        for (int r = 0; r < (COLC ? 1 : R); r++) co[r] = wc[COLC ? 0 : r + 1];
+        if (kn > 0) load(kn);
+#pragma unroll
+        for (int r = 0; r < R; r++) {
+            const T qt = x[r + 2] - x[r + 1] - x[r + 1] + x[r];
+            y[r] = x[r + 1] + fy * co[COLC ? 0 : r] * qt;
         }
-        return y;
     };
-    const long long cb = own ? cid(d, i, j, k0) : 0;
     const bool fill = COND && i <= d.mz + d.mbc;   // conduct refreshes this column's z ghosts
-    const bool spill = spilt(i, j);
-    T ym = k0 > 1 ? yres(k0 - 1) : (own ? gh[cb - sz] : T(0.0));
-    T y0 = yres(k0);
-    if (k0 == 1 && fill) ym = y0;
+    T ym[R], y0[R], yp[R], co0[COLC ? 1 : R], con[COLC ? 1 : R];
+    const int kl = k1 < d.mz ? k1 + 1 : d.mz;   // last layer formed
+    if (k0 > 1) {
+        load(k0 - 1);
+        yres(ym, co0, k0);
+    } else {
+        load(k0);
+    }
+    yres(y0, co0, k0 < kl ? k0 + 1 : 0);
+    if (k0 == 1) {
+#pragma unroll
+        for (int r = 0; r < R; r++) ym[r] = fill || j0 + r > d.my ? y0[r] : gh[cid(d, i, j0 + r, 0)];
+    }
     for (int k = k0; k <= k1; k++) {
-        const long long c = own ? cid(d, i, j, k) : 0;
-        const T yp = k < d.mz ? yres(k + 1) : (fill ? y0 : own ? gh[c + sz] : T(0.0));
-        if (COND && spill && k <= 2) {
-            if (k == 1) y0 = yp;
-            ym = y0;
+        if (k < d.mz) yres(yp, con, k + 2 <= kl ? k + 2 : 0);
+        else
+#pragma unroll
+            for (int r = 0; r < R; r++) yp[r] = fill || j0 + r > d.my ? y0[r] : gh[cid(d, i, j0 + r, d.mz + 1)];
+#pragma unroll
+        for (int r = 0; r < R; r++) {
+            const int j = j0 + r;
+            if (COND && k <= 2 && spilt(i, j)) {
+                if (k == 1) y0[r] = yp[r];
+                ym[r] = y0[r];
+            }
+            const T qt = ym[r] - y0[r] - y0[r] + yp[r];
+            if (il <= d.mx && j <= d.my) out[cid(d, i, j, k)] = y0[r] + fz * co0[COLC ? 0 : r] * qt;
+            ym[r] = y0[r];
+            y0[r] = yp[r];
         }
-        if (own) {
-            const T qt = ym - y0 - y0 + yp;
-            out[c] = y0 + fz * co_at(c, k) * qt;
-        }
-        ym = y0;
-        y0 = yp;
+#pragma unroll
+        for (int r = 0; r < (COLC ? 1 : R); r++) co0[r] = con[r];
     }
 }
 
@@ -349,24 +404,23 @@ __device__ __forceinline__ void diff_passes(const uint3 BI, const Dims &d, T *ou
 // in one launch (components 0-3 side by side in the grid's z), or with only4
 // conduct's substep kk >= 2.  fac(3*cc + n): the factor of component cc along
 // axis n, from wherever the caller keeps them (an indexed copy of them would
-// live in scratch).  Launch: block (64, 4), grid (ceil(mx/64), ceil(my/4),
-// ncomp * ceil(mz/kb)).
+// live in scratch).  Launch: block (64, 4), grid (ceil(mx/64), ceil(my /
+// (4 DIFF_ROWS)), ncomp * ceil(mz/kb)).
 template <typename T, bool COLC, class G, class FAC>
 __device__ __forceinline__ void b_diff(const uint3 BI, Dims d, const DiffArgs<T> &a, const FAC &fac, int kk, const G &gate)
 {
     if (!gate.on()) return;
-    __shared__ T sx[6][64];
     const int nz = (d.mz + a.kb - 1) / a.kb;
     const int cc = kk > 1 ? 3 : __builtin_amdgcn_readfirstlane((int)BI.z / nz);
     const uint3 bi = {BI.x, BI.y, kk > 1 ? BI.z : BI.z - cc * nz};
     const T fx = fac(3 * cc), fy = fac(3 * cc + 1), fz = fac(3 * cc + 2);
     if (cc < 3) {
         T *p = a.q + (cc + 1) * d.P;
-        diff_passes<T, COLC, false>(bi, d, p, a.u + cc * d.P, p, a.nu, fx, fy, fz, a.kb, 0, false, sx);
+        diff_passes<T, COLC, false>(bi, d, p, a.u + cc * d.P, p, a.nu, fx, fy, fz, a.kb, 0, false);
     } else if (gate.conducts(kk)) {
         const T *q5 = a.q + 4 * d.P;
         const T *src = kk == 1 ? q5 : (kk & 1) ? a.qt : a.ut;
-        diff_passes<T, COLC, true>(bi, d, (kk & 1) ? a.ut : a.qt, src, q5, a.kap, fx, fy, fz, a.kb, a.S, kk > 1, sx);
+        diff_passes<T, COLC, true>(bi, d, (kk & 1) ? a.ut : a.qt, src, q5, a.kap, fx, fy, fz, a.kb, a.S, kk > 1);
     }
 }
 template <typename T, bool COLC, class G>
