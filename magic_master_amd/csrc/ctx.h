@@ -253,22 +253,29 @@ static inline const void *tile_fn(int ntr, int sh)
 
 // log2 of the planes per segment of a grid's sweeps.  Longer segments write
 // and read fewer edge planes (L + 2 for L) and start less often; shorter ones
-// give more workgroups.  The estimate, in planes of work: a segment costs L
-// and one more for its start and its two extra planes, 512 workgroups run at
-// once, and the last ones leave half a segment of the chip idle.  It depends
-// on the grid alone (not on the device or on a batch's other grids), since
-// the sums' grouping, and so the last bits, depend on it.  Full domain
-// (250 x 200 x 300): 16; 64 x 64 x 48: 8; a dozen cells: 1.
-static inline int segment_lg(const Dims &d)
+// give more workgroups.  The estimate, in planes of work: a segment costs its
+// planes and 1.5 for its start and its two extra planes, at_once workgroups run
+// at a time, and the last ones leave the chip idle for 0.65 of a segment (less
+// where hardly any are left after the first).  It depends on the grid alone
+// (not on the device or on a batch's other grids), since the sums' grouping,
+// and so the last bits, depend on it.  Measured, ms per step with 4, 8, 16, 32 planes:
+// 250 x 200 x 300 FP64 6.13, 5.82, 5.62, 5.54 (takes 32); 128 x 100 x 150 with
+// five tracers 1.87, 1.77, 1.74, 1.72 (16); 181 x 160 x 243 FP32 2.22, 2.08, 2.06,
+// 2.09 (16); 64 x 64 x 96 FP32 0.232, 0.222, 0.216, 0.340 (16); 64 x 64 x 48
+// FP64 0.185, 0.175, 0.259, 0.295 (8); 110 x 90 x 140 FP64 0.701, 0.684, 0.672,
+// 0.738 (8); 72 x 66 x 104 FP32 0.289, 0.282, 0.296, 0.348 (8).
+static inline int segment_lg(const Dims &d, double at_once)
 {
     auto cols = [](int n, int a) { return (long long)((a + 2 + 15) / 16) * ((n + 1 + 13) / 14); };
-    const long long cx = cols(d.mx, d.my), cy = cols(d.my, d.mx), cz = cols(d.mz, d.mx);
+    const long long cxy = cols(d.mx, d.my) + cols(d.my, d.mx), cz = cols(d.mz, d.mx);
     int best = 0;
     double fbest = 0.0;
     for (int lg = 0; lg <= 5; lg++) {
-        auto segs = [&](int nB) { return (long long)((nB + 2 + (1 << lg) - 1) >> lg); };
-        const double rounds = (double)(cx * segs(d.mz) + cy * segs(d.mz) + cz * segs(d.my)) / 512.0;
-        const double w = (1 << lg) + 1.0, f = rounds <= 1.0 ? w : (rounds + 0.5) * w;
+        const int L = 1 << lg;
+        auto segs = [&](int nB) { return (nB + 2 + L - 1) >> lg; };
+        const double rounds = (double)(cxy * segs(d.mz) + cz * segs(d.my)) / at_once;
+        const double work = (cxy * (d.mz + 2 + 1.5 * segs(d.mz)) + cz * (d.my + 2 + 1.5 * segs(d.my))) / at_once;
+        const double f = std::max(work, L + 1.5) + 0.65 * L * std::min(1.0, std::max(0.0, 10.0 * (rounds - 1.0)));
         if (lg == 0 || f < fbest) {
             best = lg;
             fbest = f;
@@ -304,7 +311,8 @@ static inline void sweep_geometry(const magic_ctx *c, int dir, int sh, SweepArgs
     memset(&p, 0, sizeof(p));
     p.n = a.n; p.nA = a.nA; p.nB = a.nB;
     p.lgTA = tile_lgta(sh);
-    p.lgL = segment_lg(d);
+    // two workgroups per compute unit, or the one whose LDS fits (FP64, 4 tracers or more)
+    p.lgL = segment_lg(d, sizeof(T) == 8 && c->meqn >= 9 ? 256.0 : 512.0);
     p.CI = tile_ci(sh);
     p.iCI = (unsigned)(((1ull << 32) + p.CI - 1) / p.CI);
     p.nt = (a.nA + 2 + tile_ta(sh) - 1) / tile_ta(sh);
