@@ -330,7 +330,7 @@ __device__ __forceinline__ void tsplit(const RoeT<T> &R, const T (&in)[NC], T (&
 template <typename T>
 struct WaveT {
     T s, p, n, a, b;
-    __device__ __forceinline__ WaveT() {}
+    __device__ __forceinline__ WaveT() : s(0), p(0), n(0), a(0), b(0) {}
     __device__ __forceinline__ WaveT(T x1, T x4, T xa, T xb, T x5, T snd)
         : s(x4), p(x1 + x5), n(snd * (x5 - x1)), a(xa), b(xb) {}
     __device__ __forceinline__ void add(const WaveT &o) { s += o.s; p += o.p; n += o.n; a += o.a; b += o.b; }

@@ -109,15 +109,22 @@ __device__ __forceinline__ void tile_sweep_body(const SweepArgsT<T> &A, int bt, 
     constexpr T beta = T(0.666666666666666);
     static_assert(TA * CH == NT && TA == tile_ta(SH) && NPOS == part_npos(SH), "tile is 256 lanes");
 
-    __shared__ double s_del[5][NT];   // FP64 in both forms: the limiters' upwind wave strengths
+    // What the limiters read of the neighbouring interfaces: the jumps (FP64 in
+    // both forms) and the tracer waves.  With four tracers or more in FP64 they
+    // lie in the ring's third plane, which takes increments only afterwards
+    // (and is cleared in between), so that two workgroups fit a compute unit.
+    constexpr bool OVERLAY = sizeof(T) == 8 && NTR >= 4;
+    constexpr int NSV = OVERLAY ? 1 : NT;
+    __shared__ double s_delv[5 * NSV];
+    __shared__ T s_trwv[(NTR > 0 ? NTR : 1) * NSV];
     __shared__ T s_s2[NT];
-    __shared__ T s_trw[NTR > 0 ? NTR : 1][NT];
     __shared__ T s_cfo[NT];
     __shared__ int s_flag[NT];
     __shared__ T s_cprev[TA];
     __shared__ int s_found[TA];
     __shared__ int s_need;
     __shared__ T LT[3 * NC * NPOS];
+    static_assert(!OVERLAY || (5 + NTR) * NT <= NC * NPOS, "the jumps and tracer waves fit a plane");
 
     const int t0 = threadIdx.x;
     int t = t0;
@@ -197,7 +204,7 @@ __device__ __forceinline__ void tile_sweep_body(const SweepArgsT<T> &A, int bt, 
                 T zero = T(0.0);
                 if constexpr (RELOAD) asm volatile("" : "+v"(zero));
                 dst[e] = src[e];
-                src[e] = zero;
+                if constexpr (!OVERLAY) src[e] = zero;
             }
         }
     };
@@ -216,9 +223,15 @@ __device__ __forceinline__ void tile_sweep_body(const SweepArgsT<T> &A, int bt, 
         }
         const int b = B0 + plane;               // other transverse coordinate
         const int pg = a_is_g ? a : b, ph = a_is_g ? b : a;   // (g, h) coordinates
-        // No barrier here: the previous plane's last readers of the s_*
-        // arrays (part 2) are behind its sub-step barriers, and its flush's
-        // accesses of the ring are behind this plane's barrier after part 1.
+        // the ring's planes of b-1, b and b+1
+        const int r0 = plane % 3, r1 = r0 == 2 ? 0 : r0 + 1, r2 = r1 == 2 ? 0 : r1 + 1;
+        double *const s_del = OVERLAY ? (double *)(LT + r2 * (NC * NPOS)) : s_delv;   // [5][NT]
+        T *const s_trw = OVERLAY ? LT + r2 * (NC * NPOS) + 5 * NT : s_trwv;           // [NTR][NT]
+        // No barrier here without the overlay: the previous plane's last
+        // readers of the s_* arrays (part 2) are behind its phase barriers, and
+        // its flush's accesses of the ring are behind this plane's barrier
+        // after part 1.  With it, the flush has to have read the plane.
+        if (OVERLAY && plane > 0) __syncthreads();
         int kk = bk;                            // chunk being solved (an earlier one while looking for CFLup)
         int looked = 0;
         asm volatile("" : "+s"(looked));        // one copy of the solve in the loop below
@@ -378,10 +391,10 @@ __device__ __forceinline__ void tile_sweep_body(const SweepArgsT<T> &A, int bt, 
                 }
             }
             c1 = fabs((T)s1 * dtdn); c2 = fabs((T)s2 * dtdn); c3 = fabs((T)s3 * dtdn);
-            s_del[0][t] = d1; s_del[1][t] = d2; s_del[2][t] = d3; s_del[3][t] = d4; s_del[4][t] = d5;
+            s_del[t] = d1; s_del[NT + t] = d2; s_del[2 * NT + t] = d3; s_del[3 * NT + t] = d4; s_del[4 * NT + t] = d5;
             s_s2[t] = (T)s2;
 #pragma unroll
-            for (int k = 0; k < NTR; k++) s_trw[k][t] = trw[k];
+            for (int k = 0; k < NTR; k++) s_trw[k * NT + t] = trw[k];
             // the limiters need the Courant number an earlier interface left
             if (act2 && b1 == 0.0 && b2 == 0.0 && (b3 != 0.0 || b4 != 0.0)) s_need = 1;
         }
@@ -440,7 +453,7 @@ __device__ __forceinline__ void tile_sweep_body(const SweepArgsT<T> &A, int bt, 
                 const T fc = trw[k];
                 T wl = T(0.0);
                 if (fc != T(0.0)) {
-                    const T r = s_trw[k][s2 > 0.0 ? t - nb : t + nb] / fc;
+                    const T r = s_trw[k * NT + (s2 > 0.0 ? t - nb : t + nb)] / fc;
                     if (k + 1 <= A.nspecadv) wl = lim2.bee(T(0.5), beta, r, lim2.weight(fabs(s_s2[up2] * dtdn)));
                     else wl = fmaxF(T(0.0), fminF(T(1.0), r));
                 }
@@ -449,15 +462,15 @@ __device__ __forceinline__ void tile_sweep_body(const SweepArgsT<T> &A, int bt, 
             // the upwind interfaces' strengths in this interface's waves: those
             // of wave 2 come from one of the two acoustic waves' sides
             auto b4of = [&](int e) {
-                return R.g1a2 * (R.euv * s_del[0][e] + R.u * s_del[1][e] + R.v * s_del[2][e] + R.w * s_del[3][e] -
-                                 s_del[4][e]);
+                return R.g1a2 * (R.euv * s_del[e] + R.u * s_del[NT + e] + R.v * s_del[2 * NT + e] + R.w * s_del[3 * NT + e] -
+                                 s_del[4 * NT + e]);
             };
             auto b5of = [&](int e, double b4e) {
-                return (s_del[1][e] + (R.a - R.u) * s_del[0][e] - R.a * b4e) * R.i2a;
+                return (s_del[NT + e] + (R.a - R.u) * s_del[e] - R.a * b4e) * R.i2a;
             };
             const double b4l = b4of(up1), b4r = b4of(up3);
-            const double g1 = s_del[0][up1] - b4l - b5of(up1, b4l), g5 = b5of(up3, b4r), g4 = up2 == up1 ? b4l : b4r;
-            const double g2 = s_del[2][up2] - R.v * s_del[0][up2], g3 = s_del[3][up2] - R.w * s_del[0][up2];
+            const double g1 = s_del[up1] - b4l - b5of(up1, b4l), g5 = b5of(up3, b4r), g4 = up2 == up1 ? b4l : b4r;
+            const double g2 = s_del[2 * NT + up2] - R.v * s_del[up2], g3 = s_del[3 * NT + up2] - R.w * s_del[up2];
             T wt = T(1.0);   // the upwind Courant number's weight: 1 where it is c2 itself
             if (b2 == 0.0 && (b3 != 0.0 || b4 != 0.0)) {
                 T cflup;
@@ -509,6 +522,22 @@ __device__ __forceinline__ void tile_sweep_body(const SweepArgsT<T> &A, int bt, 
             qsa = (T)w2;
             qsb = (T)w3;
         }
+        if constexpr (OVERLAY) {
+            // clear the third plane: a lane its own pencil's entries (and the
+            // tile's edge entries) of the cell that phase 0 adds to, so that
+            // with tile-axis-major lanes the wave's order is enough
+            __syncthreads();
+            T *cl = LT + r2 * (NC * NPOS);
+            if (c >= 1) {
+#pragma unroll
+                for (int m = 0; m < NC; m++) cl[m * NPOS + pix(pa, c - 1)] = T(0.0);
+                if (pa < 2)
+#pragma unroll
+                    for (int m = 0; m < NC; m++) cl[m * NPOS + pix(pa + TA, c - 1)] = T(0.0);
+            }
+            if constexpr (PM) __syncthreads();
+            else __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
+        }
         if (EARLY && plane + 1 < nplane) fetch(I0, b + 1);
 
         // ---------------- part 3: transverse terms (flux3fw.f:297-625), two phases
@@ -530,8 +559,6 @@ __device__ __forceinline__ void tile_sweep_body(const SweepArgsT<T> &A, int bt, 
         // once): deterministic.  Against splitting conserved vectors and
         // summing a 3 x 3 x NC register accumulator this halves the sweep's
         // arithmetic, and nothing wider than the y and z vectors stays live.
-        // the ring's planes of b-1, b and b+1
-        const int r0 = plane % 3, r1 = r0 == 2 ? 0 : r0 + 1, r2 = r1 == 2 ? 0 : r1 + 1;
         const T kf = -(T(1.0) / T(6.0)) * d * ca * cb2, kea = -T(0.5) * d * ca, keb = -T(0.5) * d * cb2;
         const SpeedT<T> va(ua, snd), vb(ub, snd);
         T hm = lf ? T(1.0) : T(0.0);   // 1 where the contact waves belong to the phase
@@ -542,9 +569,15 @@ __device__ __forceinline__ void tile_sweep_body(const SweepArgsT<T> &A, int bt, 
             const int ci = phase == 0 ? c - 1 : c;  // cell index within the chunk's tile
             if (phase == 1 && t == 0) s_need = 0;   // every lane has read it (phase 0's barrier)
             const T sg = phase == 0 ? T(1.0) : -T(1.0);
-            WaveT<T> y[3], z[3], N;
-            T yt[3][NTR > 0 ? NTR : 1], zt[3][NTR > 0 ? NTR : 1], Nt[NTR > 0 ? NTR : 1];
-            if (on) {
+            // One branch around the whole phase (pencil-major lanes all come
+            // along for its barriers): split into several, each branch's results
+            // live on as merged values and spill.  With it every tracer
+            // count runs two waves per SIMD in FP64 and three in FP32: 128 x 100
+            // x 150 with five tracers 1.74 -> 1.27 ms per step, with three
+            // 1.59 -> 1.09; FP32 181 x 160 x 243 2.06 -> 1.74.
+            if (PM || on) {
+            WaveT<T> y[3] = {}, z[3] = {}, N = {};
+            if (!PM || on) {
                 const T s3q = T(3.0) * sg, s2q = T(2.0) * sg;
                 const WaveT<T> X(l1, hm * x4, hm * xa, hm * xb, l5, snd), Q(q1, q4, qsa, qsb, q5, snd);
                 const WaveT<T> F = WaveT<T>::comb(kf, X, s3q, Q), E = WaveT<T>::comb(T(1.0), X, s2q, Q);
@@ -564,24 +597,43 @@ __device__ __forceinline__ void tile_sweep_body(const SweepArgsT<T> &A, int bt, 
                 }
                 y[1] = WaveT<T>::middle(y[0], y[2], kea, E);
                 z[1] = WaveT<T>::middle(z[0], z[2], keb, E);
+            }
+            // One tracer goes with the five components' targets, more come after
+            // them, one after the other: all at once they would hold 7 values
+            // each.
+            constexpr bool APART = NTR >= 2;
+            struct Tracer {
+                T y[3], z[3], n;
+            };
+            auto tracer = [&](int k) __attribute__((always_inline)) {
+                Tracer w;
+                const T at = hm * trw[k];
+                const T ft = kf * (at + T(3.0) * sg * trq[k]), et = at + T(2.0) * sg * trq[k];
+                w.n = -d * (at + sg * trq[k]);
 #pragma unroll
-                for (int k = 0; k < NTR; k++) {
-                    const T at = hm * trw[k];
-                    const T ft = kf * (at + s3q * trq[k]), et = at + s2q * trq[k];
-                    Nt[k] = -d * (at + sg * trq[k]);
-#pragma unroll
-                    for (int r = 0; r < 3; r += 2) {
-                        yt[r][k] = vb.w2(r) * ft;
-                        zt[r][k] = va.w2(r) * ft;
-                    }
-                    yt[1][k] = kea * et - (yt[0][k] + yt[2][k]);
-                    zt[1][k] = keb * et - (zt[0][k] + zt[2][k]);
+                for (int r = 0; r < 3; r += 2) {
+                    w.y[r] = vb.w2(r) * ft;
+                    w.z[r] = va.w2(r) * ft;
                 }
+                w.y[1] = kea * et - (w.y[0] + w.y[2]);
+                w.z[1] = keb * et - (w.z[0] + w.z[2]);
+                return w;
+            };
+            auto tracer_add = [&](T *row, int k, const Tracer &w, int r, int j) __attribute__((always_inline)) {
+                T v = va.w2(r) * w.y[j] + vb.w2(j) * w.z[r];
+                if (r == 1 && j == 1) v += w.n;
+                lds_add(row[(5 + k) * NPOS], v);
+            };
+            Tracer trs[!APART && NTR > 0 ? NTR : 1];
+            if constexpr (!APART) {
+#pragma unroll
+                for (int k = 0; k < NTR; k++)
+                    if (!PM || on) trs[k] = tracer(k);
             }
             // one sub-step per offset along a: lanes then add to distinct T entries
             auto substep = [&](auto rc) {
                 constexpr int r = decltype(rc)::value;
-                if (on) {
+                if (!PM || on) {
                     auto target = [&](auto jc) {
                         constexpr int j = decltype(jc)::value;
                         T *row = LT + (j == 0 ? r0 : j == 1 ? r1 : r2) * (NC * NPOS) + pix(pa + r, ci);
@@ -597,11 +649,9 @@ __device__ __forceinline__ void tile_sweep_body(const SweepArgsT<T> &A, int bt, 
                         }
 #pragma unroll
                         for (int m = 0; m < 5; m++) lds_add(row[m * NPOS], o[m]);
+                        if constexpr (!APART) {
 #pragma unroll
-                        for (int k = 0; k < NTR; k++) {
-                            T v = va.w2(r) * yt[j][k] + vb.w2(j) * zt[r][k];
-                            if (r == 1 && j == 1) v += Nt[k];
-                            lds_add(row[(5 + k) * NPOS], v);
+                            for (int k = 0; k < NTR; k++) tracer_add(row, k, trs[k], r, j);
                         }
                     };
                     target(IConst<0>{});
@@ -616,12 +666,31 @@ __device__ __forceinline__ void tile_sweep_body(const SweepArgsT<T> &A, int bt, 
                 // reads above the previous one's writes; it emits nothing),
                 // and the workgroup waits once per phase.  Pencil-major
                 // waves share entries: a barrier after every sub-step.
-                if (PM || r == 2) __syncthreads();
+                if constexpr (PM) __syncthreads();
                 else __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
             };
             substep(IConst<0>{});
             substep(IConst<1>{});
             substep(IConst<2>{});
+            if constexpr (APART) {
+#pragma unroll
+                for (int k = 0; k < NTR; k++) {
+                    Tracer w = {};
+                    if (!PM || on) w = tracer(k);
+#pragma unroll
+                    for (int r = 0; r < 3; r++) {
+                        if (!PM || on) {
+#pragma unroll
+                            for (int j = 0; j < 3; j++)
+                                tracer_add(LT + (j == 0 ? r0 : j == 1 ? r1 : r2) * (NC * NPOS) + pix(pa + r, ci), k, w, r, j);
+                        }
+                        if constexpr (PM) __syncthreads();
+                        else __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
+                    }
+                }
+            }
+            }
+            if constexpr (!PM) __syncthreads();
             l1 = x1 - l1;   // phase 1: the right-going parts
             l5 = x5 - l5;
             hm = T(1.0) - hm;
@@ -638,14 +707,11 @@ __device__ __forceinline__ void tile_sweep_body(const SweepArgsT<T> &A, int bt, 
 }
 
 
-// Waves per SIMD the register allocation aims at: two, except where the LDS
-// of two workgroups does not fit a compute unit (FP64 with four tracers or
-// more) or the registers would spill (pencil-major lanes).
+// Waves per SIMD the register allocation aims at
 template <typename T, int NTR, int SH>
 constexpr int tile_waves()
 {
-    if (TileShape<SH>::PM) return 1;
-    return sizeof(T) == 8 ? (NTR <= 3 ? 2 : 1) : (NTR <= 1 ? 2 : 1);
+    return sizeof(T) == 8 ? 2 : 3;
 }
 
 // The sweep kernel, for one grid and for a batch of grids alike (one
