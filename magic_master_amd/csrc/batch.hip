@@ -62,6 +62,7 @@ struct magic_batch {
     int4 *lgdim_d = nullptr;             //                  cap grid shapes each
     std::vector<int> loff;               // loff_d's host copy
     int ndtr_cap = 0, ndtrc_cap = 0;     // substep loops of the captured attempt
+    int ncu = 0;                         // compute units
     int opgrid[NOP] = {0};               // persistent grid of each kernel class
     bool overlap = false;                // accepted for the ABI; the order of the sums does not depend on it
     hipGraph_t graph = nullptr;
@@ -256,7 +257,16 @@ static int launch_op(magic_batch *b, int op, GateSpec gs, int arg = 0, int lo = 
     const int4 *gd = b->lgdim_d + (size_t)lg * b->cap + lo;
     int n = hi - lo;
     void *kargs[] = {&ops, &off, &gd, &n, &gs, &arg};
-    HIPCHECK(hipLaunchKernel(fn, dim3(std::min(total, b->opgrid[op])), list_block(lg), kargs, 0, b->stream));
+    int grid = b->opgrid[op];
+    // The conversion gathers from 18 or more places per cell.  Where the
+    // increments (256 cells to a block, three directions) come from memory
+    // and not from the 256 MB cache before it, fewer workgroups at once keep
+    // to fewer pages: 8 FP32 grids of 200 x 200 x 300 take 2.56 ms with three
+    // per compute unit, 2.75 with four, 2.87 with six; 24 of 40 x 36 x 60 (0.2 GB) 120,
+    // 106 and 95 us.
+    if (op == OP_CONVERT && (long long)total * 256 * 3 * b->meqn * (long long)sizeof(T) > 256ll << 20)
+        grid = std::min(grid, 3 * b->ncu);
+    HIPCHECK(hipLaunchKernel(fn, dim3(std::min(total, grid)), list_block(lg), kargs, 0, b->stream));
     return launch_check();
 }
 
@@ -583,16 +593,16 @@ static int build_ops(magic_batch *b)
 template <typename T>
 static int list_grids(magic_batch *b)
 {
-    int dev = 0, ncu = 0;
+    int dev = 0;
     HIPCHECK(hipGetDevice(&dev));
-    HIPCHECK(hipDeviceGetAttribute(&ncu, hipDeviceAttributeMultiprocessorCount, dev));
+    HIPCHECK(hipDeviceGetAttribute(&b->ncu, hipDeviceAttributeMultiprocessorCount, dev));
     for (int op = 0; op < NOP; op++) {
         const void *fn = batch_op_fn<T>(op);
         if (!fn) return MAGIC_EUNSUPPORTED;
         const dim3 blk = list_block(op_list(op));
         int occ = 0;
         HIPCHECK(hipOccupancyMaxActiveBlocksPerMultiprocessor(&occ, fn, (int)(blk.x * blk.y * blk.z), 0));
-        b->opgrid[op] = ncu * (occ > 0 ? occ : 1);
+        b->opgrid[op] = b->ncu * (occ > 0 ? occ : 1);
     }
     return MAGIC_OK;
 }
