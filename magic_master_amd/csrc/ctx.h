@@ -306,6 +306,8 @@ static inline void sweep_geometry(const magic_ctx *c, int dir, int sh, SweepArgs
     a.sA = dir == 0 ? d.NX : 1;
     a.sB = dir == 2 ? d.NX : NXY;
     a.a_is_g = dir != 1;
+    for (int m = 0; m < 10; m++)
+        a.cofs[m] = d.P * (m == 2 ? a.comp[a.a_is_g ? 2 : 3] : m == 3 ? a.comp[a.a_is_g ? 3 : 2] : m < c->meqn ? a.comp[m] : 0);
     a.gravity = dir == 2;
     a.sweep = dir + 1;
     memset(&p, 0, sizeof(p));

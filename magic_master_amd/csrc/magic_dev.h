@@ -41,6 +41,7 @@ struct SweepArgsT {
     // tiled sweep: sA/sB/nA/nB then describe the tile axis a and the marching
     // axis b; a_is_g: the tile axis is the sweep's g direction
     int a_is_g;
+    long long cofs[10];                // cells to the planes of rho, the momenta along n, a and b, E, tracers
     T *parts;                          // the direction's increment blocks (SweepParts)
     int lgL, sT, sK, sS;               // log2 planes per segment; blocks between tiles, chunks, segments
 };

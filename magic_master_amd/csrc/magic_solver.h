@@ -62,15 +62,25 @@ __device__ __forceinline__ float sqrtT<float>(float x) { return __builtin_amdgcn
 // steps, in FP64 to 3e-5-6e-5.  Its reciprocals and square roots need not
 // be correctly rounded there: the hardware's FP64 approximations refined by
 // one Newton step (relative error near 1e-15, far inside that form's error
-// bar).  RF selects them (true: the FP32 form) over the correctly rounded
-// operations of the FP64 form.
+// bar).  RF selects them (true: the FP32 form) over the operations of the
+// FP64 form: one third-order step from the hardware's 2**-24 (largest error
+// over 5e8 arguments 1.0 x 2**-53, as two Newton steps have, in three
+// operations for their four).
 template <bool RF>
 __device__ __forceinline__ double rcp1(double x)
 {
-    double r = __builtin_amdgcn_rcp(x);
-    r = fma(r, fma(-x, r, 1.0), r);
-    if constexpr (!RF) r = fma(r, fma(-x, r, 1.0), r);
-    return r;
+    const double r = __builtin_amdgcn_rcp(x), e = fma(-x, r, 1.0);
+    return fma(r, RF ? e : fma(e, e, e), r);
+}
+// g / b of the limiters: the FP32 form's rounds to FP32 afterwards, the FP64
+// form's is corrected by its remainder, as the correctly rounded quotient is,
+// without that one's scaling: NaN where b is zero or its reciprocal
+// overflows, which the limiters take (they then multiply b).
+template <bool RF>
+__device__ __forceinline__ double ratio(double g, double b)
+{
+    const double r = rcp1<RF>(b), q = g * r;
+    return RF ? q : fma(fma(-b, q, g), r, q);
 }
 // 1/x of the limiters' clamped Courant numbers and 1 + r (normal range)
 __device__ __forceinline__ double rcpL(double x) { return rcp1<false>(x); }
@@ -92,22 +102,20 @@ __device__ __forceinline__ double sqrt1(double x)
 }
 
 // Square root s and its reciprocal i of x > 0 together, from one hardware
-// reciprocal square root and Newton-Goldschmidt steps (one for the FP32
-// form; in FP64 two, and a last residual step for the root).
+// reciprocal square root and a Goldschmidt step (of first order for the FP32
+// form; in FP64 of second, and a last residual step for the root: largest
+// errors 1.0 x 2**-53 of the root and 2.0 x 2**-53 of the reciprocal, 1.0 and
+// 2.6 with two first-order steps).
 template <bool RF>
 __device__ __forceinline__ void root_rcp(double x, double &s, double &i)
 {
     const double y = __builtin_amdgcn_rsq(x);
     double g = x * y, h = 0.5 * y;
     double r = fma(-g, h, 0.5);
+    if constexpr (!RF) r = fma(1.5 * r, r, r);
     g = fma(g, r, g);
     h = fma(h, r, h);
-    if constexpr (!RF) {
-        r = fma(-g, h, 0.5);
-        g = fma(g, r, g);
-        h = fma(h, r, h);
-        g = fma(fma(-g, g, x), h, g);
-    }
+    if constexpr (!RF) g = fma(fma(-g, g, x), h, g);
     s = g;
     i = h + h;
 }
@@ -144,15 +152,12 @@ __device__ __forceinline__ float powT(float x, float y)
 // library function's special cases.
 __device__ __forceinline__ double one_minus_pow(double x, double p)
 {
-    int k;
-    double m = __builtin_frexp(fmaxT(x, 1e-300), &k);   // [1/2, 1); x = 0: the power is 0 either way
-    const bool low = m < 0.70710678118654752;
-    m = low ? m + m : m;
-    const double kd = (double)(low ? k - 1 : k);
-    const double f = m - 1.0, g = m + 1.0;
-    double i = __builtin_amdgcn_rcp(g);
-    i = fma(i, fma(-g, i, 1.0), i);
-    i = fma(i, fma(-g, i, 1.0), i);
+    const double xc = fmaxT(x, 1e-300);   // x = 0: the power is 0 either way
+    // k from the high words of x and sqrt(1/2) (0x3fe6a09e): m in [0.70711, 1.41422)
+    const int k = (__double2hiint(xc) - 0x3fe6a09e) >> 20;
+    const double m = __hiloint2double(__double2hiint(xc) - (k << 20), __double2loint(xc));
+    const double kd = (double)k;
+    const double f = m - 1.0, g = m + 1.0, i = rcp1<false>(g);
     // (m-1)/(m+1) = s + sl (m - (g - 1): what rounding m + 1 left out)
     const double s = f * i, sl = fma(-s, m - (g - 1.0), fma(-s, g, f)) * i;
     const double z = s * s;

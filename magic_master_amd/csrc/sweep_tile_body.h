@@ -163,10 +163,8 @@ __device__ __forceinline__ void tile_sweep_body(const SweepArgsT<T> &A, int bt, 
             const long long y = x + A.sN;
 #pragma unroll
             for (int m = 0; m < NC; m++) {
-                // transverse momenta in the order a, b
-                const int cm = A.comp[m == 2 ? (a_is_g ? 2 : 3) : m == 3 ? (a_is_g ? 3 : 2) : m];
-                pqa[m] = qold[(long long)cm * A.P + x];
-                pqb[m] = qold[(long long)cm * A.P + y];
+                pqa[m] = (qold + A.cofs[m])[x];
+                pqb[m] = (qold + A.cofs[m])[y];
             }
             if constexpr (!PERT) {
                 pga = gam[x];
@@ -182,11 +180,11 @@ __device__ __forceinline__ void tile_sweep_body(const SweepArgsT<T> &A, int bt, 
     constexpr bool EARLY = sizeof(T) == 4;
     int I0 = bk * (CH - 2) + c;
     // In FP64 the registers are full: what a lane can form again from its
-    // index is formed again for every plane and every flush (the asm hides that
-    // it is the same each time), or the compiler keeps it all through the loop
-    // and spills, and each reload from scratch then waits for the flush's
-    // stores as well (28.4k -> 21.7k cycles per wave and plane with the
-    // hardware's LDS adds below).
+    // index is formed again for every flush and, with two tracers or more, for
+    // every plane (the asm hides that it is the same each time), or the compiler
+    // keeps it all through the loop and spills, and each reload from scratch
+    // then waits for the flush's stores as well (28.4k -> 21.7k cycles per wave
+    // and plane with the hardware's LDS adds).
     constexpr bool RELOAD = sizeof(T) == 8;
 
     // one plane of the ring to the block's part, as it lies in LDS: whole
@@ -197,21 +195,27 @@ __device__ __forceinline__ void tile_sweep_body(const SweepArgsT<T> &A, int bt, 
         if constexpr (RELOAD) asm volatile("" : "+v"(tf));
         T *src = LT + slot * (NC * NPOS);
         const gptr<T> dst = part + p * (NC * NPOS);
+        // all read before the first is written: one wait
+        constexpr int NF = NC * NPOS / NT, REM = NC * NPOS % NT;
+        T v[NF + 1], zero = T(0.0);
+        if constexpr (RELOAD) asm volatile("" : "+v"(zero));
 #pragma unroll
-        for (int k = 0; k < (NC * NPOS + NT - 1) / NT; k++) {
-            const int e = tf + k * NT;
-            if (e < NC * NPOS) {
-                T zero = T(0.0);
-                if constexpr (RELOAD) asm volatile("" : "+v"(zero));
-                dst[e] = src[e];
-                if constexpr (!OVERLAY) src[e] = zero;
-            }
+        for (int k = 0; k < NF; k++) v[k] = src[tf + k * NT];
+        if (REM && tf < REM) v[NF] = src[tf + NF * NT];
+#pragma unroll
+        for (int k = 0; k < NF; k++) {
+            dst[tf + k * NT] = v[k];
+            if constexpr (!OVERLAY) src[tf + k * NT] = zero;
+        }
+        if (REM && tf < REM) {
+            dst[tf + NF * NT] = v[NF];
+            if constexpr (!OVERLAY) src[tf + NF * NT] = zero;
         }
     };
     fetch(I0, B0);
 
     for (int plane = 0; plane < nplane; plane++) {
-        if constexpr (RELOAD) {
+        if constexpr (RELOAD && NTR >= 2) {
             t = t0;
             asm volatile("" : "+v"(t));
             pa = PM ? (t / CH) : (t % TA);
@@ -485,9 +489,10 @@ __device__ __forceinline__ void tile_sweep_body(const SweepArgsT<T> &A, int bt, 
             // A vanishing wave needs no case of its own: the limiters are
             // finite for any ratio, NaN among them, and multiply a strength
             // of zero.
-            const T wl1 = suppow1((T)(g1 / b1), c1), wl5 = suppow1((T)(g5 / b5), c3);
-            const T wl2 = lim2.bee(T(1.0), beta, (T)(g2 / b2), T(1.0)), wl3 = lim2.bee(T(1.0), beta, (T)(g3 / b3), wt),
-                    wl4 = lim2.bee(T(1.0), beta, (T)(g4 / b4), wt);
+            constexpr bool RF = sizeof(T) == 4;
+            const T wl1 = suppow1((T)ratio<RF>(g1, b1), c1), wl5 = suppow1((T)ratio<RF>(g5, b5), c3);
+            const T wl2 = lim2.bee(T(1.0), beta, (T)ratio<RF>(g2, b2), T(1.0)), wl3 = lim2.bee(T(1.0), beta, (T)ratio<RF>(g3, b3), wt),
+                    wl4 = lim2.bee(T(1.0), beta, (T)ratio<RF>(g4, b4), wt);
             // strengths of cqxx, in FP64 up to here
             const double w1 = (double)(k1 * wl1) * b1, w2 = (double)(k2 * wl2) * b2, w3 = (double)(k2 * wl3) * b3,
                          w4 = (double)(k2 * wl4) * b4, w5 = (double)(k3 * wl5) * b5;
