@@ -75,7 +75,6 @@ static StepParts<double> &slot_parts(magic_batch *b, int s, double) { return b->
 static StepParts<float> &slot_parts(magic_batch *b, int s, float) { return b->sp32[s]; }
 static bool fp32(const magic_batch *b) { return b->form == MAGIC_FORM_FP32P; }
 static size_t elt(const magic_batch *b) { return fp32(b) ? sizeof(float) : sizeof(double); }
-static void *state_q(const magic_ctx *c) { return c->form == MAGIC_FORM_FP32P ? (void *)c->q32 : (void *)c->q; }
 static void *state_qold(const magic_ctx *c)
 {
     return c->form == MAGIC_FORM_FP32P ? (void *)c->qold32 : (void *)c->qold;
@@ -437,7 +436,7 @@ static int build_lists(magic_batch *b, bool tuning = false)
                 a.nspecadv = c->have_params ? c->prm.nspecadv : 0;
                 a.cfl_bits = &b->ctl_d[s].cfl_bits;
                 a.status = &b->ctl_d[s].err[0];
-                if (b->parts_one) a.qold = (const T *)state_qold(c);
+                if (b->parts_one || tuning) a.qold = (const T *)state_qold(c);
                 const double dt = b->ctl[s].dt > 0.0 ? b->ctl[s].dt : 1.0;
                 if (tuning) sweep_factors(c, dir, dt, a);
                 a.parts = next;
@@ -950,10 +949,7 @@ extern "C" int magic_batch_tune(magic_batch *b, int reps, int shapes_out[3], flo
     const int saved[3] = {b->shape[0], b->shape[1], b->shape[2]};
     TRY(drop_graph(b));   // the lists and argument blocks are rebuilt before the next attempt
     for (int s = 0; s < b->n; s++) {
-        magic_ctx *c = b->sc[s];
-        if (c)
-            HIPCHECK(hipMemcpyAsync(state_qold(c), state_q(c), (size_t)c->P * c->meqn * elt(b),
-                                    hipMemcpyDeviceToDevice, b->stream));
+        if (b->sc[s]) TRY(tune_state(b->sc[s]));
     }
     int st = fp32(b) ? tune_rounds<float, true>(b, reps, clk) : tune_rounds<double, false>(b, reps, clk);
     if (st == MAGIC_OK && hipStreamSynchronize(b->stream) != hipSuccess) st = MAGIC_EHIP;
