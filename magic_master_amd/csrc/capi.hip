@@ -9,6 +9,7 @@
 #include <condition_variable>
 #include <mutex>
 #include <thread>
+#include <unistd.h>
 
 #include "ctx.h"
 
@@ -54,6 +55,7 @@ size_t bounce_chunk(size_t bytes)
 // context (pool_open, pool_close).
 class CopyPool {
 public:
+    const pid_t pid = getpid();
     void copy(char *dst, const char *src, size_t n)
     {
         if (n < (size_t(1) << 20)) {
@@ -146,6 +148,7 @@ void pool_close()
 {
     std::lock_guard<std::mutex> lock(bounce_mu);
     if (--pool_users > 0) return;
+    if (pool->pid != getpid()) return;   // a forked child: the threads are its parent's
     pool->end();
     delete pool;
     pool = nullptr;
