@@ -62,10 +62,16 @@ def sums_row(ref: np.ndarray, other: np.ndarray) -> dict:
 PEAK_FLOOR = {"w": 1e-6, "T'": 1e-6, "rho'": 1e-9}
 
 
+def _set_order(d, first: bool):
+    """The order in which a step's increments are summed: the default tile
+    shapes' (first) or another one, that of shape 1 in every direction."""
+    d.set_tile_shapes([0, 0, 0] if first else [1, 1, 1])
+
+
 def compare_runs(c, p, g: Grid, aux: np.ndarray, q: np.ndarray, t_end: float, every: float, ref, other,
                  on_row=None) -> list:
     """Advance two configurations of the step, ref and other, each (form,
-    sweep overlap on/off), from the same state under claw3's step control, to
+    default order of additions or another one), from the same state under claw3's step control, to
     every multiple of `every` model seconds up to t_end (each claw3 call
     stops exactly at the output time, as the claw3ez frame loop does), and
     compare other against ref there.  Returns one row per output time:
@@ -75,10 +81,10 @@ def compare_runs(c, p, g: Grid, aux: np.ndarray, q: np.ndarray, t_end: float, ev
     devs = []
     rows = []
     try:
-        for form, overlap in cfgs:
+        for form, first in cfgs:
             d = MagicHIP(g, p, aux, q, form=form)
             devs.append(d)
-            d.set_sweep_overlap(overlap)
+            _set_order(d, first)
         t = [0.0, 0.0]
         dtv = [list(c.dtv), list(c.dtv)]
         steps = [0, 0]
@@ -107,10 +113,9 @@ def layer_error(scenario: int, nscen: int = 64, seed: int = 2024, t_end: float =
                 nmin=(64, 64, 96), nmax=(200, 200, 300)) -> dict:
     """Where in the column the FP32 form's error sits: scenario `scenario`
     of problem.ensemble(nscen, seed) stepped alone from rest to t_end in
-    three configurations, the FP64 form with the sweep overlap (the
-    reference), the FP64 form with the sweeps in turn (another order of
-    additions) and the FP32 form with the sweeps in turn (the batch's
-    order).  Returns {"grid", "amplitude", "peak": {field: FP64 peak},
+    three configurations, the FP64 form (the reference), the FP64 form with
+    another order of additions and the FP32 form (as the batch runs it).
+    Returns {"grid", "amplitude", "peak": {field: FP64 peak},
     "worst": {field: (k, j, i) of the FP32 form's largest error},
     "layers": one row per interior layer k: {"k", "rho_bar", field:
     {"fp32", "order", "value"}}, each the layer's largest |difference| (or
@@ -121,10 +126,10 @@ def layer_error(scenario: int, nscen: int = 64, seed: int = 2024, t_end: float =
     aux = np.ascontiguousarray(np.broadcast_to(col[:, None, None, :], g.shape_aux))
     q0 = P.qinit(g, aux)
     out = []
-    for form, overlap in ((FORM_FP64, True), (FORM_FP64, False), (FORM_FP32P, False)):
+    for form, first in ((FORM_FP64, True), (FORM_FP64, False), (FORM_FP32P, True)):
         d = MagicHIP(g, p, aux, q0, form=form)
         try:
-            d.set_sweep_overlap(overlap)
+            _set_order(d, first)
             t, dtv = 0.0, list(c.dtv)
             while t < t_end * (1 - 1e-12):
                 t, dtv, _, _, _ = d.claw3(t, t_end, dtv, c.cflv, [1 << 30, 0], c.method, c.mthbc)
@@ -150,7 +155,7 @@ def layer_error(scenario: int, nscen: int = 64, seed: int = 2024, t_end: float =
 def compare_forms(c, p, g: Grid, aux: np.ndarray, q: np.ndarray, t_end: float, every: float,
                   on_row=None) -> list:
     """The FP32 perturbation form against the FP64 form (compare_runs; both
-    with the default sweep overlap)."""
+    with the default order of additions)."""
     from .hip import FORM_FP32P, FORM_FP64
     return compare_runs(c, p, g, aux, q, t_end, every, (FORM_FP64, True), (FORM_FP32P, True), on_row)
 
@@ -228,8 +233,8 @@ def main(argv=None):
                     help="plume peak time (default: the workload's 2400 s)")
     ap.add_argument("--json", default=None, help="also write every row to this JSON file")
     ap.add_argument("--pair", default="fp32", choices=("fp32", "order"),
-                    help="fp32: the FP32 form against the FP64 form; order: the FP64 form with the sweeps "
-                         "in turn against the FP64 form with the sweep overlap (the same arithmetic in "
+                    help="fp32: the FP32 form against the FP64 form; order: the FP64 form with tile "
+                         "shapes 1, 1, 1 against the FP64 form with 0, 0, 0 (the same arithmetic in "
                          "another order of additions: how far rounding alone moves the solution)")
     ap.add_argument("--ensemble", type=int, default=0,
                     help="instead: the batched FP32 ensemble of this many seeded scenarios to --t-end, the "

@@ -103,3 +103,14 @@ def test_room_for_one_direction():
     np.testing.assert_allclose(dt0, dt1, rtol=1e-13)
     # one step's sums differ by a few roundings; three steps carry them on
     assert rel_err(q1, q0) <= 1e-11 and rel_err(b1, b0) <= 1e-11
+
+
+def test_report_orders_differ():
+    """The error report's two FP64 orders of additions: other last bits, the
+    same state to the report's bar (1e-12 of each field's peak)."""
+    from magic_master_amd import report
+    from magic_master_amd.hip import FORM_FP64
+    c, p, g, aux, q = perturbed(40, 20, 18, [1, 1, 1, 1, 3, 1], seed=5, vel=0.3)
+    rows = report.compare_runs(c, p, g, aux, q, 20.0, 20.0, (FORM_FP64, True), (FORM_FP64, False))
+    worst = [rows[0][k]["max_rel"] for k in ("w", "T'", "rho'")]
+    assert max(worst) > 0.0 and max(worst) <= 1e-12, worst
