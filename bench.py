@@ -34,20 +34,20 @@ METRIC = ("Mcell-updates/s FP64 vs FP32-batched on 1 MI355X at stated error; "
           "p50/p99 latency")
 HBM_PEAK_GBS = 8000.0
 # The step is bound by vector arithmetic, not by HBM.  Floating-point
-# operations per cell-update of the 18 sweep launches of a step, counted on
-# the full-domain workload with rocprofv3 (SQ_INSTS_VALU_{ADD,MUL,FMA,TRANS}
-# of each precision, times 64 lanes, an FMA counted twice; lanes masked off
-# at grid edges and the chunks' 2-interface overlap included): FP64 form
-# 12.71 k FP64; FP32 form 9.99 k FP32 + 1.73 k FP64.  MI355X vector peak
-# (non-matrix) is 78.6 TFLOP/s for FP64, and for FP32 too without packed
-# (two-wide) FP32 instructions, which this library does not use; the 157.3
-# TFLOP/s FP32 peak counts them.
-FLOP_PER_CELL_UPDATE = {"fp64": 12.71e3, "fp32": 9.99e3 + 1.73e3}
+# operations per cell-update of a step's sweeps, counted on the full-domain
+# workload with rocprofv3 (SQ_INSTS_VALU_{ADD,MUL,FMA,TRANS} of each
+# precision, times 64 lanes, an FMA counted twice; lanes masked off at grid
+# edges and the chunks' 2-interface overlap included): FP64 form 6.31 k FP64;
+# FP32 form 4.65 k FP32 + 1.25 k FP64.  MI355X vector peak (non-matrix) is 78.6
+# TFLOP/s for FP64, and for FP32 too without packed (two-wide) FP32
+# instructions, which this library does not use; the 157.3 TFLOP/s FP32 peak
+# counts them.
+FLOP_PER_CELL_UPDATE = {"fp64": 6.31e3, "fp32": 4.65e3 + 1.25e3}
 VECTOR_PEAK_TFLOPS = {"fp64": 78.6, "fp32": 78.6}
 # Algorithmic bytes per cell-update at meqn = 6.  Hyperbolic pass: read q,
 # write q (2 x 48 B) + aux(17), aux(19) (16 B), shared evenly by the three
-# sweep directions; a direction's launches (tile colours) each cover an equal
-# share of its cells.  Source pass: read q, write q, read aux 1-5, 11, 12, 18,
+# sweep directions (one launch sweeps all of a shape; its time is shared by
+# their blocks).  Source pass: read q, write q, read aux 1-5, 11, 12, 18,
 # 19 (96 + 72 B).
 HYP_BYTES_PER_CELL = 112.0
 SRC_BYTES_PER_CELL = 168.0
