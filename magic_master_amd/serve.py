@@ -67,8 +67,8 @@ class Outcome:
 
 
 def footprint_bytes(g: P.Grid) -> int:
-    """Device memory of one scenario of the FP32 form in a batch (sweeps in
-    turn, the batch's default): q' and its backup (2 x 4 B x meqn), the
+    """Device memory of one scenario of the FP32 form in a batch, beside the
+    batch's own buffer of increments (8 GB at most): q' and its backup (2 x 4 B x meqn), the
     source pass's scratch (5 x 4 B), the FP64 staging of q for upload and
     download (8 B x meqn), per padded cell, plus the columns."""
     cells = (g.mx + 2 * g.mbc) * (g.my + 2 * g.mbc) * (g.mz + 2 * g.mbc)
