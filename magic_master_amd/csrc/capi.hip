@@ -1335,14 +1335,18 @@ extern "C" int magic_claw3(magic_ctx *c, double tstart, double *tend, double dtv
             if (!defer && (st = copy_state(c, true))) goto out;
             if ((st = step3_launch(c, dt, defer, defer))) goto out;
             int ss = MAGIC_OK, a, b;
+            bool moved = false;   // the conversion's target is q already
             if (defer) {
+                const bool pending = c->pending_parts;
                 c->gate = GridGate{c->dscal, c->hscal, cflv[0]};
                 ss = src3_launch(c, told, dt, mthbc, &a, &b);   // claw3_mpi.f:900-905
                 c->gate = GridGate{};
-                if (ss && (st = scal_copy(c))) goto out;        // nothing was launched: a setting src3 refuses
+                moved = pending && !c->pending_parts;
+                // a setting src3 refuses, before it launches anything: the step itself goes on
+                if (ss && ss != MAGIC_EHIP && (st = scal_copy(c))) goto out;
             }
-            st = step3_finish(c, &cfl);
-            if (defer && !ss && (st || !(cfl <= cflv[0]))) {    // no source pass ran: its target is the backup again
+            st = ss == MAGIC_EHIP ? ss : step3_finish(c, &cfl);
+            if (moved && (st || !(cfl <= cflv[0]))) {           // no (whole) source pass ran: its target is the backup again
                 if (c->form == MAGIC_FORM_FP32P) std::swap(c->q32, c->qold32);
                 else std::swap(c->q, c->qold);
                 c->pending_parts = true;

@@ -1,0 +1,68 @@
+"""The library's host code where a run on the GPU cannot reach it: launches
+that fail half way, steps rejected by any factor, device memory that runs out.
+The library runs with a HIP runtime without a device (tests/hip_stub.cpp,
+preloaded into a process of its own): kernels do nothing, so no result of a
+step is checked here, only what the host decides."""
+import os
+import subprocess
+import sys
+import textwrap
+
+import pytest
+
+ROOT = os.path.dirname(os.path.dirname(os.path.abspath(__file__)))
+
+
+@pytest.fixture(scope="module")
+def host(tmp_path_factory):
+    """Runs a script with the stub; `stub` and the test inputs are in scope."""
+    so = str(tmp_path_factory.mktemp("stub") / "libhipstub.so")
+    subprocess.run(["g++", "-O1", "-std=c++17", "-shared", "-fPIC", "-o", so,
+                    os.path.join(ROOT, "tests", "hip_stub.cpp")], check=True)
+    head = f"""
+import ctypes as C
+import numpy as np
+from magic_master_amd import problem as P
+from magic_master_amd.hip import *
+from tests.helpers import perturbed
+stub = C.CDLL({so!r})
+stub.stub_launches.restype = C.c_char_p
+stub.stub_used.restype = C.c_size_t
+stub.stub_room.argtypes = [C.c_size_t]
+def courant(*c):
+    stub.stub_courant((C.c_double * len(c))(*c), len(c))
+def launches():
+    out = [l.split()[0] for l in stub.stub_launches().decode().splitlines()]
+    stub.stub_clear()
+    return out
+"""
+
+    def run(script):
+        env = dict(os.environ, LD_PRELOAD=so, PYTHONPATH=ROOT)
+        r = subprocess.run([sys.executable, "-c", head + textwrap.dedent(script)], env=env, cwd=ROOT,
+                           stdout=subprocess.PIPE, stderr=subprocess.STDOUT, text=True, timeout=100)
+        assert r.returncode == 0, r.stdout
+    return run
+
+
+@pytest.mark.parametrize("cfl", [0.5, 1.9])   # the attempt would be accepted, or rejected
+def test_claw3_launch_failure_in_the_source_pass(host, cfl):
+    """A launch that fails behind the source pass's conversion ends claw3 with
+    an error, on the state before the step (not on the older backup)."""
+    host(f"""
+    c, p, g, aux, q = perturbed(8, 7, 6, [1, 1, 1, 1, 3, 1])
+    d = MagicHIP(g, p, aux, q)
+    courant(0.5, {cfl}, 0.5)
+    one = lambda: d.claw3(0.0, -1.0, c.dtv, c.cflv, [10, 0], c.method, c.mthbc)
+    one()
+    assert np.all(d.get_q()[..., :5] == 1.0)      # the first step's source pass wrote its mark
+    stub.stub_fail(b"6k_diffI", 0)
+    try:
+        one()
+        raise SystemExit("no error")
+    except MagicError as e:
+        assert e.code == 6, e
+    assert np.all(d.get_q()[..., :5] == 1.0), d.get_q()[0, 0, 0]
+    d.restore()
+    assert np.all(d.get_q()[..., :5] == 1.0)
+    """)
