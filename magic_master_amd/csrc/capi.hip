@@ -1257,6 +1257,22 @@ static int src3_passes64(magic_ctx *c, const int *mthbc, int ndtr, double dtr, i
     return launch_check();
 }
 
+// Most launches of a source pass that claw3 queues behind the sweeps before
+// it knows their Courant number.  They end at once in a rejected attempt, but
+// each still takes 2-4 us, and the substeps of a dt far beyond the Courant
+// limit may be any number; a pass of more launches than this hardly gains by
+// the wait it saves (4-9 us).
+constexpr double MAX_AHEAD = 32.0;
+// About how many launches the source pass of a step dt takes, from its
+// substep counts (src3.f90:314-322)
+static double src_launches(const magic_ctx *c, double dt)
+{
+    const double dmin = std::min(std::min(c->dx, c->dy), c->dz), d2 = dmin * dmin;
+    const double n = std::ceil((dt * (4.0 / 3.0) * c->aux11_top / d2) / 0.45);
+    const double nc = n > 0.0 ? std::ceil((dt / n * c->aux12_top / d2) / 0.45) : 0.0;
+    return 2.0 + n * (4.0 + nc);
+}
+
 static int src3_launch(magic_ctx *c, double t, double dt, const int *mthbc_in, int *ndtr_out,
                        int *ndtrc_out)
 {
@@ -1323,8 +1339,8 @@ extern "C" int magic_claw3(magic_ctx *c, double tstart, double *tend, double dtv
     // an accepted step's source pass (into the other state buffer): the state
     // before the step needs no copy and a rejected step no restoring.  A
     // batch's grid keeps its buffers' places (its captured kernels hold them)
-    // and takes the copying way.  The source pass is launched behind the sweeps
-    // under their result's gate, and the host waits once per attempt.
+    // and takes the copying way.  A source pass of few launches is queued behind
+    // the sweeps under their result's gate, and the host waits once per attempt.
     if (maxn > 0 && (st = setup_sweeps(c))) return st;
     const bool defer = sweeps_defer(c) && c->own_stream;
     for (int n = 1; n <= maxn; n++) {
@@ -1336,7 +1352,9 @@ extern "C" int magic_claw3(magic_ctx *c, double tstart, double *tend, double dtv
             if ((st = step3_launch(c, dt, defer, defer))) goto out;
             int ss = MAGIC_OK, a, b;
             bool moved = false;   // the conversion's target is q already
-            if (defer) {
+            const bool ahead = defer && src_launches(c, dt) <= MAX_AHEAD;
+            if (defer && !ahead && (st = scal_copy(c))) goto out;
+            if (ahead) {
                 const bool pending = c->pending_parts;
                 c->gate = GridGate{c->dscal, c->hscal, cflv[0]};
                 ss = src3_launch(c, told, dt, mthbc, &a, &b);   // claw3_mpi.f:900-905
@@ -1361,7 +1379,7 @@ extern "C" int magic_claw3(magic_ctx *c, double tstart, double *tend, double dtv
             nl++;
             if (cfl <= cflv[0]) {                                  // claw3_mpi.f:861-886
                 cflmax = cflmax > cfl ? cflmax : cfl;
-                st = defer ? ss : src3_launch(c, told, dt, mthbc, &a, &b);
+                st = ahead ? ss : src3_launch(c, told, dt, mthbc, &a, &b);
                 if (st) goto out;
                 break;
             }

@@ -66,3 +66,24 @@ def test_claw3_launch_failure_in_the_source_pass(host, cfl):
     d.restore()
     assert np.all(d.get_q()[..., :5] == 1.0)
     """)
+
+
+@pytest.mark.parametrize("dt,rejected", [(1e5, True), (1e30, True), (1e5, False), (2.0, False)])
+def test_rejected_attempt_launches_no_substeps(host, dt, rejected):
+    """The diffusion substeps an attempt would need grow with its dt (here 999
+    at 1e5 s): an attempt that is rejected launches none of them, one that is
+    accepted all."""
+    host(f"""
+    dt, rejected = float("{dt}"), {rejected}
+    c, p, g, aux, q = perturbed(8, 7, 6, [1, 1, 1, 1, 3, 1], visc=1.0)
+    d2 = min(g.dx, g.dy, g.dz) ** 2
+    aux[..., 10] = aux[..., 11] = 1e3 * 0.45 * d2 / 1e5 * 0.75 * 0.999
+    d = MagicHIP(g, p, aux, q)
+    courant(*[1e4, 0.5] if rejected else [0.5])
+    d.claw3(0.0, -1.0, [dt, 1.0, 0, 0, 0], c.cflv, [10, 0], c.method, c.mthbc)
+    n = sum("k_diff_cross" in l for l in launches())
+    if rejected:
+        assert n == 1, n                  # those of the second attempt (dt 1)
+    else:
+        assert n == (999 if dt > 10 else 1), n
+    """)
