@@ -1128,12 +1128,14 @@ extern "C" int magic_tune(magic_ctx *c, double dt, int reps, int shapes_out[3], 
     TuneClock clk;
     if (!clk.ok) return MAGIC_EHIP;
     const int keep[3] = {c->shape[0], c->shape[1], c->shape[2]};
-    TRY(tune_state(c));
-    const int st = c->form == MAGIC_FORM_FP32P ? tune_rounds<float, true>(c, args32(c), dt, reps, clk)
-                                               : tune_rounds<double, false>(c, args64(c), dt, reps, clk);
+    int st = tune_state(c);
+    if (st == MAGIC_OK)
+        st = c->form == MAGIC_FORM_FP32P ? tune_rounds<float, true>(c, args32(c), dt, reps, clk)
+                                         : tune_rounds<double, false>(c, args64(c), dt, reps, clk);
     for (int k = 0; k < 3; k++) c->shape[k] = keep[k];
+    const int sc = copy_state(c, true);   // the ghosts too as in q, also after a failed round
     TRY(st);
-    TRY(copy_state(c, true));   // the ghosts too as in q
+    TRY(sc);
     int best[3];
     clk.result(reps, best, ms_out);
     k_zero_scalars<<<1, 64, 0, c->stream>>>(c->dscal);   // the candidates' Courant numbers and reports

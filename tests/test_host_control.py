@@ -87,3 +87,23 @@ def test_rejected_attempt_launches_no_substeps(host, dt, rejected):
     else:
         assert n == (999 if dt > 10 else 1), n
     """)
+
+
+@pytest.mark.parametrize("fails", [0, 7])   # the first candidate, a later one
+def test_tune_failure_restores_the_backup(host, fails):
+    """A tuner that ends with an error leaves the backup a copy of q, its ghost
+    cells among them."""
+    host(f"""
+    c, p, g, aux, q = perturbed(8, 7, 6, [1, 1, 1, 1, 3, 1])
+    d = MagicHIP(g, p, aux, q)
+    launches()
+    stub.stub_fail(b"tile_sweep", {fails})
+    try:
+        d.tune(1.0)
+        raise SystemExit("no error")
+    except MagicError:
+        pass
+    l = launches()
+    assert any("4k_bc" in n for n in l) and "copy" in l[[i for i, n in enumerate(l) if "4k_bc" in n][-1]:], l
+    assert d.tile_shapes() == [0, 0, 0]
+    """)
