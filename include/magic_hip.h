@@ -249,9 +249,10 @@ int magic_batch_state(magic_batch *b, int s, double real_out[5], int int_out[6])
 /* Tile shapes of the batch's x-, y- and z-sweeps (one per direction for all
  * scenarios; default 0, 0, 0); setting them captures the graph again.
  * magic_batch_tune is the autotuner of the batch: every shape of every
- * direction is timed as launches over the blocks of all scenarios (their current states and next dt; one untimed
- * and reps timed sweeps), and the fastest per direction is kept.  The
- * scenarios' states are unchanged bit for bit. */
+ * direction is timed as launches over the blocks of all scenarios (their
+ * current states and next dt; one untimed and reps timed sweeps), and the
+ * fastest per direction is kept.  The scenarios' states are unchanged bit
+ * for bit; their backup copies then hold them. */
 int magic_batch_set_tile_shapes(magic_batch *b, const int shapes[3]);
 int magic_batch_get_tile_shapes(magic_batch *b, int shapes[3]);
 int magic_batch_tune(magic_batch *b, int reps, int shapes_out[3], float *ms_out);

@@ -948,10 +948,14 @@ extern "C" int magic_batch_tune(magic_batch *b, int reps, int shapes_out[3], flo
     if (!clk.ok) return MAGIC_EHIP;
     const int saved[3] = {b->shape[0], b->shape[1], b->shape[2]};
     TRY(drop_graph(b));   // the lists and argument blocks are rebuilt before the next attempt
+    int st = MAGIC_OK;
+    for (int s = 0; s < b->n && st == MAGIC_OK; s++)
+        if (b->sc[s]) st = tune_state(b->sc[s]);
+    if (st == MAGIC_OK) st = fp32(b) ? tune_rounds<float, true>(b, reps, clk) : tune_rounds<double, false>(b, reps, clk);
     for (int s = 0; s < b->n; s++) {
-        if (b->sc[s]) TRY(tune_state(b->sc[s]));
+        const int sd = b->sc[s] ? tune_done(b->sc[s]) : MAGIC_OK;
+        if (st == MAGIC_OK) st = sd;
     }
-    int st = fp32(b) ? tune_rounds<float, true>(b, reps, clk) : tune_rounds<double, false>(b, reps, clk);
     if (st == MAGIC_OK && hipStreamSynchronize(b->stream) != hipSuccess) st = MAGIC_EHIP;
     if (st != MAGIC_OK) {
         for (int k = 0; k < 3; k++) b->shape[k] = saved[k];

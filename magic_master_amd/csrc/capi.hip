@@ -1121,6 +1121,10 @@ int tune_state(magic_ctx *c)
     return c->form == MAGIC_FORM_FP32P ? bc_launch(c, c->qold32, faces, 0) : bc_launch(c, c->qold, faces, 0);
 }
 
+// The backup a copy of q again, its ghosts too: after the tuners, whether
+// they succeeded or not
+int tune_done(magic_ctx *c) { return copy_state(c, true); }
+
 extern "C" int magic_tune(magic_ctx *c, double dt, int reps, int shapes_out[3], float *ms_out)
 {
     if (!c || !c->have_aux || !(dt > 0.0) || reps < 1) return MAGIC_EARG;
@@ -1133,7 +1137,7 @@ extern "C" int magic_tune(magic_ctx *c, double dt, int reps, int shapes_out[3], 
         st = c->form == MAGIC_FORM_FP32P ? tune_rounds<float, true>(c, args32(c), dt, reps, clk)
                                          : tune_rounds<double, false>(c, args64(c), dt, reps, clk);
     for (int k = 0; k < 3; k++) c->shape[k] = keep[k];
-    const int sc = copy_state(c, true);   // the ghosts too as in q, also after a failed round
+    const int sc = tune_done(c);
     TRY(st);
     TRY(sc);
     int best[3];

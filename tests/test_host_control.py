@@ -107,3 +107,25 @@ def test_tune_failure_restores_the_backup(host, fails):
     assert any("4k_bc" in n for n in l) and "copy" in l[[i for i, n in enumerate(l) if "4k_bc" in n][-1]:], l
     assert d.tile_shapes() == [0, 0, 0]
     """)
+
+
+@pytest.mark.parametrize("fails", [-1, 0, 7])   # none, the first candidate, a later one
+def test_batch_tune_restores_the_backups(host, fails):
+    """The batch's tuner leaves every scenario's backup a copy of its q, ghost
+    cells among them, whether it succeeds or not."""
+    host(f"""
+    b = MagicBatch([], [], [], meqn=6, mbc=2, maux=32, form=FORM_FP64)
+    for n in range(3):
+        c, p, g, aux, q = perturbed(8 + n, 7, 6, [1, 1, 1, 1, 3, 1])
+        b.add(g, p, aux[:, 0, 0, :].copy(), q)
+    launches()
+    stub.stub_fail(b"tile_sweep", {fails})
+    try:
+        b.tune()
+        assert {fails} < 0
+    except MagicError:
+        assert {fails} >= 0
+    l = launches()
+    last = [i for i, n in enumerate(l) if "4k_bc" in n][-1]
+    assert l[last:].count("copy") == 3, l[last:]
+    """)
