@@ -12,7 +12,7 @@
 
 namespace magic {
 
-enum { GATE_RUN = 0, GATE_ACCEPTED, GATE_REJECTED, GATE_DIFF, GATE_COND, GATE_MORE, GATE_SWEPT };
+enum { GATE_RUN = 0, GATE_ACCEPTED, GATE_DROPPED, GATE_DIFF, GATE_COND, GATE_MORE, GATE_SWEPT };
 
 // factor slots of ScenCtl::fac (source pass, src3.f90:314-322 and the
 // passes of diffuse.f / conduct.f)
@@ -68,7 +68,7 @@ struct StepGate {
         switch (mode) {
         case GATE_RUN: return c->run != 0;
         case GATE_ACCEPTED: return c->accepted != 0;
-        case GATE_REJECTED: return c->rejected != 0;
+        case GATE_DROPPED: return c->swept != 0 && c->accepted == 0;   // rejected, or failed
         case GATE_DIFF: return c->accepted != 0 && nn <= c->ndtr;
         case GATE_COND: return c->accepted != 0 && nn <= c->ndtr && kk <= c->ndtrc;
         case GATE_MORE: return c->accepted != 0 && nn < c->ndtr;

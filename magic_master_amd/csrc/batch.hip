@@ -40,6 +40,7 @@ struct magic_batch {
     std::vector<magic_ctx *> sc;         // nullptr: empty slot
     std::vector<ScenCtl> ctl;            // host copy of the control blocks
     std::vector<int> mthbc;              // 6 per scenario
+    std::vector<char> settled;           // a failed scenario's last step is in its q
     ScenCtl *ctl_d = nullptr;
     ScenCtl *ctl_pin = nullptr;          // pinned read-back buffer
     void *args_d = nullptr;              // SweepArgsT of the form, 3 per slot: one per direction
@@ -309,7 +310,7 @@ static int launch_group(magic_batch *b, const magic_batch::Group &g)
     }
     k_batch_decide<<<blocks(g.hi - g.lo, 256), 256, 0, b->stream>>>(b->ctl_d + g.lo, g.hi - g.lo);
     TRY(launch_check());
-    if (b->parts_one) TRY(launch_op<T>(b, OP_RESTORE, gs(GATE_REJECTED), 0, g.lo, g.hi));
+    if (b->parts_one) TRY(launch_op<T>(b, OP_RESTORE, gs(GATE_DROPPED), 0, g.lo, g.hi));
     return launch_op<T>(b, OP_CONVERT, gs(GATE_ACCEPTED), 0, g.lo, g.hi);
 }
 
@@ -707,6 +708,7 @@ extern "C" int magic_batch_add(magic_batch *b, const int dims[3], const double g
         b->sc.push_back(nullptr);
         b->ctl.push_back(ScenCtl());
         b->mthbc.insert(b->mthbc.end(), 6, 1);
+        b->settled.push_back(0);
     }
     b->sc[s] = c;
     memset(&b->ctl[s], 0, sizeof(ScenCtl));   // inactive until started
@@ -817,6 +819,7 @@ extern "C" int magic_batch_start(magic_batch *b, int s, double t, double tend, d
     h.rejects = 0;
     h.maxsteps = maxsteps;
     h.status = 0;
+    b->settled[s] = 0;
     h.dx = c->dx; h.dy = c->dy; h.dz = c->dz;
     double dmin = c->dx < c->dy ? c->dx : c->dy;
     dmin = dmin < c->dz ? dmin : c->dz;
@@ -868,6 +871,11 @@ extern "C" int magic_batch_run(magic_batch *b, int max_attempts, int check_every
     // a scenario that failed (rho <= 0, a**2 <= 0, more substeps than
     // captured) has stopped with its status in its control block, which
     // magic_batch_state reports; the others went on
+    for (int s = 0; s < b->n; s++)
+        if (b->sc[s] && !b->settled[s] && (b->ctl[s].status == MAGIC_ERHO || b->ctl[s].status == MAGIC_EA2)) {
+            b->settled[s] = 1;
+            TRY(failed_step(b->sc[s], b->shape, b->ctl[s].dt));
+        }
     return MAGIC_OK;
 }
 

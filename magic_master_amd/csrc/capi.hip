@@ -1064,6 +1064,29 @@ extern "C" int magic_step3(magic_ctx *c, double dt, double *cfl)
     return s;
 }
 
+// The end of a batch's scenario whose sweeps failed: q, which the attempt left
+// as it was (its sweeps read it, nothing is added before the decision), becomes
+// the backup, and the step's increments are added to it, as claw3 leaves a grid
+// that fails.  Sweeping again costs a failed scenario one step; gates for it
+// in the conversion cost every step (SGPRs spilt, or a wave fewer per SIMD).
+int failed_step(magic_ctx *c, const int *shape, double dt)
+{
+    int keep[3];
+    memcpy(keep, c->shape, sizeof(keep));
+    memcpy(c->shape, shape, sizeof(keep));
+    double cfl;
+    int st = copy_state(c, true);
+    if (st == MAGIC_OK) st = step3_launch(c, dt);
+    if (st == MAGIC_OK) st = step3_finish(c, &cfl);
+    memcpy(c->shape, keep, sizeof(keep));
+    hipFree(c->parts);   // a scenario has no sweeps of its own otherwise
+    hipFree(c->items);
+    c->parts = nullptr;
+    c->parts_bytes = 0;
+    c->items = nullptr;
+    return st == MAGIC_ERHO || st == MAGIC_EA2 ? MAGIC_OK : st;
+}
+
 // ------------------------------------------------------- tile shapes -----
 extern "C" int magic_set_tile_shapes(magic_ctx *c, const int shapes[3])
 {

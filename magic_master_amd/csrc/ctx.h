@@ -350,7 +350,9 @@ static inline void push_items(std::vector<int4> &items, const SweepParts<T> &p, 
             for (int t = 0; t < p.nt; t++) items.push_back(make_int4(arg, t, k, s));
 }
 
-int tune_state(magic_ctx *c), tune_done(magic_ctx *c);   // capi.hip
+// capi.hip
+int tune_state(magic_ctx *c), tune_done(magic_ctx *c);
+int failed_step(magic_ctx *c, const int *shape, double dt);
 
 // Event pairs of the autotuners, one per (direction, shape).  The shapes
 // are timed round-robin (every round times each candidate once), so that a
