@@ -392,6 +392,8 @@ static int build_groups(magic_batch *b)
             else return MAGIC_ENOMEM;
         }
         b->parts_bytes = got;
+    } else {
+        b->parts_one = false;   // what made it so is gone
     }
     b->groups.clear();
     const std::vector<size_t> &need = b->parts_one ? most : all;

@@ -129,3 +129,32 @@ def test_batch_tune_restores_the_backups(host, fails):
     last = [i for i, n in enumerate(l) if "4k_bc" in n][-1]
     assert l[last:].count("copy") == 3, l[last:]
     """)
+
+
+def test_batch_room_found_again(host):
+    """A batch that once had room for a part of a grid's increments only goes
+    the usual way again once what it holds fits."""
+    host("""
+    def add(dims):
+        c, p, g, aux, q = perturbed(*dims, [1, 1, 1, 1, 3, 1])
+        s = b.add(g, p, aux[:, 0, 0, :].copy(), q)
+        b.start(s, 0.0, 1e9, 1.0, c.dtv, c.cflv, 5, c.mthbc)
+        return s
+    backup = lambda: any("k_batch_opIdLi3E" in n for n in launches())
+    for share in np.linspace(8.0, 0.5, 30):      # of the big grid's q
+        b = MagicBatch([], [], [], meqn=6, mbc=2, maux=32, form=FORM_FP64)
+        big = add((60, 50, 40))
+        small = add((10, 9, 8))
+        launches()
+        stub.stub_room(stub.stub_used() + int(share * 64 * 54 * 44 * 48))
+        b.run(1, 1)
+        if backup():
+            break
+        b.close()
+        stub.stub_room(1 << 60)
+    else:
+        raise SystemExit("never out of room")
+    b.remove(big)
+    b.run(1, 1)
+    assert not backup()
+    """)
