@@ -200,6 +200,17 @@ int magic_tune(magic_ctx *ctx, double dt, int reps, int shapes_out[3], float *ms
  * Kept so that programs that set it keep working. */
 int magic_set_sweep_overlap(magic_ctx *ctx, int on);
 
+/* ---- Memory of the sweeps (no counterpart in the reference) -------------
+ * The sweeps' increments go to a buffer that the first sweep allocates.  Where
+ * it cannot hold the whole grid's, the grid is swept in slabs, narrow enough
+ * along x for it, one after the other: slower, with the same result bit for
+ * bit.  A context takes the whole grid's size or, where the device has less,
+ * what there is, and fails with MAGIC_ENOMEM only where that is not enough for
+ * slabs 16 cells wide.  magic_set_increment_room bounds the buffer to bytes
+ * (or those narrowest slabs, if they take more; 0: no bound) and gives back
+ * the one held. */
+int magic_set_increment_room(magic_ctx *ctx, size_t bytes);
+
 /* ---- Batched driver: many grids of one form advanced together ----------
  * Each scenario is a grid with its own state (a magic_ctx reachable through
  * magic_batch_ctx for parameters, aux and q); its step control is claw3's
@@ -207,11 +218,11 @@ int magic_set_sweep_overlap(magic_ctx *ctx, int on);
  * every scenario is one replay of a HIP graph captured at the first
  * magic_batch_run.  Each kernel of the attempt is one launch over all
  * scenarios (the sweeps over a list of the grids' blocks, in groups of
- * scenarios whose increments fit 8 GB, the boundary, copy and source-pass
+ * scenarios whose increments fit the batch's buffer, the boundary, copy and source-pass
  * kernels over the scenarios' grids laid end to end), so the launches per
  * attempt do not grow with the number of scenarios but by one group's three
- * per 8 GB of increments.  No counterpart in the
- * reference. */
+ * per buffer of increments (8 GB, or the largest grid's).  No counterpart in
+ * the reference. */
 typedef struct magic_batch magic_batch;
 /* dims: (mx, my, mz) per scenario; geom: (xlower, ylower, zlower, dx, dy, dz)
  * per scenario (nscen may be 0); form: MAGIC_FORM_FP32P or MAGIC_FORM_FP64
@@ -256,6 +267,10 @@ int magic_batch_state(magic_batch *b, int s, double real_out[5], int int_out[6])
 int magic_batch_set_tile_shapes(magic_batch *b, const int shapes[3]);
 int magic_batch_get_tile_shapes(magic_batch *b, int shapes[3]);
 int magic_batch_tune(magic_batch *b, int reps, int shapes_out[3], float *ms_out);
+/* magic_set_increment_room for the batch's buffer (0: 8 GB, or the largest
+ * grid's if that is more); grids that do not fit are swept in slabs.  Captures
+ * the graph again. */
+int magic_batch_set_increment_room(magic_batch *b, size_t bytes);
 /* As magic_set_sweep_overlap: accepted, without effect on the result.  A
  * scenario equals the same grid stepped alone bit for bit when both use the
  * same tile shapes.  Setting it captures the graph again. */

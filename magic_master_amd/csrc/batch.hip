@@ -47,14 +47,19 @@ struct magic_batch {
     const int **run_d = nullptr;         // per argument block: &ctl_d[s].run
     int4 *items_d = nullptr;
     // Groups of slots [lo, hi) whose increments the part buffer holds at
-    // once; blocks of the group's direction d at items_d[off[d], off[d + 1])
-    struct Group { int lo, hi, off[4]; };
+    // once; blocks of the group's direction d at items_d[off[d], off[d + 1]).
+    // A grid too large for the buffer is a group for each of its slabs.
+    struct Group {
+        int lo, hi, off[4];
+        int slab = -1, nslab = 0;        // of slot lo: which of how many (slab < 0: whole grids)
+    };
     std::vector<Group> groups;
+    std::vector<std::vector<Slab>> slabs;   // per slot; empty: swept whole
     std::vector<StepParts<double>> sp64; // per slot, by form: the increments of its sweeps
     std::vector<StepParts<float>> sp32;
     void *parts = nullptr;
     size_t parts_bytes = 0;
-    bool parts_one = false;              // room for one direction at a time only
+    size_t parts_room = 0;               // bytes the caller allows it (0: PARTS_BYTES)
     int shape[3] = {0, 0, 0};            // tile shape of the x-, y- and z-sweeps
     int *one_d = nullptr;                // a device 1: the run flag of every tile while tuning
     // boundary, copy and source-pass kernels (batch_ops.h)
@@ -76,6 +81,8 @@ static StepParts<double> &slot_parts(magic_batch *b, int s, double) { return b->
 static StepParts<float> &slot_parts(magic_batch *b, int s, float) { return b->sp32[s]; }
 static bool fp32(const magic_batch *b) { return b->form == MAGIC_FORM_FP32P; }
 static size_t elt(const magic_batch *b) { return fp32(b) ? sizeof(float) : sizeof(double); }
+static double *state_q(const magic_ctx *c, double) { return c->q; }
+static float *state_q(const magic_ctx *c, float) { return c->q32; }
 static void *state_qold(const magic_ctx *c)
 {
     return c->form == MAGIC_FORM_FP32P ? (void *)c->qold32 : (void *)c->qold;
@@ -236,7 +243,7 @@ static dim3 list_block(int lg)
 // The block list each kernel class walks
 static int op_list(int op)
 {
-    static const int lg[NOP] = {LG_BC, LG_BCUVW, LG_BCZ, LG_CPY, LG_CPY, LG_PAD, LG_DIF, LG_DF4, LG_DF1, LG_INT, LG_INT, LG_PAD};
+    static const int lg[NOP] = {LG_BC, LG_BCUVW, LG_BCZ, LG_CPY, LG_CPY, LG_PAD, LG_DIF, LG_DF4, LG_DF1, LG_INT, LG_INT};
     return lg[op];
 }
 
@@ -290,27 +297,66 @@ static int launch_src(magic_batch *b)
     return launch_op<T>(b, OP_FINISH, gs(GATE_ACCEPTED));
 }
 
-// Sweeps, decision and conversion of one group.  With room for one
-// direction's increments only, each direction's are added to q before the
-// next runs, from the copied backup, as one grid does (capi.hip).
+// The argument blocks of a slot's sweeps moved on to the blocks of a slab
+template <typename T>
+struct SlabArgs {
+    T *parts[3];
+    int sT[3], sK[3], sS[3];
+};
+template <typename T>
+__global__ void k_slab_args(SweepArgsT<T> *args, SlabArgs<T> a)
+{
+    const int d = (int)threadIdx.x;
+    if (d >= 3) return;
+    args[d].parts = a.parts[d];
+    args[d].sT = a.sT[d];
+    args[d].sK = a.sK[d];
+    args[d].sS = a.sS[d];
+}
+// Launches it; sp: the slab's increments
+template <typename T>
+static int put_slab(magic_batch *b, const magic_batch::Group &g, StepParts<T> &sp)
+{
+    const magic_ctx *c = b->sc[g.lo];
+    const Slab &slab = b->slabs[g.lo][g.slab];
+    SlabArgs<T> sa;
+    T *next = (T *)b->parts;
+    sp.nc = c->meqn;
+    for (int dir = 0; dir < 3; dir++) {
+        SweepArgsT<T> a;
+        sweep_geometry(c, dir, b->shape[dir], a, sp.d[dir]);
+        next = parts_layout(a, sp.d[dir], dir, slab.lo[dir], slab.hi[dir], c->meqn, b->shape[dir], next);
+        sa.parts[dir] = a.parts;
+        sa.sT[dir] = a.sT; sa.sK[dir] = a.sK; sa.sS[dir] = a.sS;
+    }
+    k_slab_args<T><<<1, 64, 0, b->stream>>>((SweepArgsT<T> *)b->args_d + 3 * g.lo, sa);
+    return launch_check();
+}
+
+// Sweeps, decision and conversion of one group.  A grid in slabs is swept from
+// the copied backup and each slab's increments are added to q at once, as one
+// grid does (capi.hip).
 template <typename T, bool PERT>
 static int launch_group(magic_batch *b, const magic_batch::Group &g)
 {
-    if (b->parts_one) {
-        TRY(launch_op<T>(b, OP_BACKUP, gs(GATE_RUN), 0, g.lo, g.hi));
-        for (int d = 0; d < 3; d++) {
-            TRY((launch_dirs<T, PERT>(b, g, d, d + 1)));
-            TRY(launch_op<T>(b, OP_ADD_PARTS, gs(GATE_SWEPT), d, g.lo, g.hi));
-        }
-    } else {
-        for (int d0 = 0, d1; d0 < 3; d0 = d1) {
-            for (d1 = d0 + 1; d1 < 3 && b->shape[d1] == b->shape[d0];) d1++;
-            TRY((launch_dirs<T, PERT>(b, g, d0, d1)));
-        }
+    StepParts<T> sp;
+    if (g.slab == 0) TRY(launch_op<T>(b, OP_BACKUP, gs(GATE_RUN), 0, g.lo, g.hi));
+    if (g.slab >= 0) TRY(put_slab<T>(b, g, sp));
+    for (int d0 = 0, d1; d0 < 3; d0 = d1) {
+        for (d1 = d0 + 1; d1 < 3 && b->shape[d1] == b->shape[d0];) d1++;
+        TRY((launch_dirs<T, PERT>(b, g, d0, d1)));
+    }
+    if (g.slab >= 0) {
+        const magic_ctx *c = b->sc[g.lo];
+        const Slab &s = b->slabs[g.lo][g.slab];
+        k_add_parts<T><<<slab_cells(c->d, s), cell_block(), 0, b->stream>>>(c->d, state_q(c, T()), sp, s.i0 + c->mbc - 1,
+                                                                            s.i1 + c->mbc - 1, &b->ctl_d[g.lo].swept);
+        TRY(launch_check());
+        if (g.slab + 1 < g.nslab) return MAGIC_OK;
     }
     k_batch_decide<<<blocks(g.hi - g.lo, 256), 256, 0, b->stream>>>(b->ctl_d + g.lo, g.hi - g.lo);
     TRY(launch_check());
-    if (b->parts_one) TRY(launch_op<T>(b, OP_RESTORE, gs(GATE_DROPPED), 0, g.lo, g.hi));
+    if (g.slab >= 0) TRY(launch_op<T>(b, OP_RESTORE, gs(GATE_DROPPED), 0, g.lo, g.hi));
     return launch_op<T>(b, OP_CONVERT, gs(GATE_ACCEPTED), 0, g.lo, g.hi);
 }
 
@@ -359,48 +405,43 @@ constexpr size_t PARTS_BYTES = size_t(8) << 30;
 template <typename T>
 static int build_groups(magic_batch *b)
 {
-    std::vector<size_t> all(b->n, 0), most(b->n, 0);
-    size_t sum = 0, big = 0, big1 = 0;
+    std::vector<size_t> need(b->n, 0);
+    size_t sum = 0, big = 0, least = 0;
     for (int s = 0; s < b->n; s++) {
         if (!b->sc[s]) continue;
-        for (int dir = 0; dir < 3; dir++) {
-            SweepArgsT<T> a;
-            SweepParts<T> p;
-            sweep_geometry(b->sc[s], dir, b->shape[dir], a, p);
-            const size_t bytes = (size_t)parts_size(p, b->meqn, b->shape[dir]) * sizeof(T);
-            all[s] += bytes;
-            most[s] = std::max(most[s], bytes);
-        }
-        sum += all[s];
-        big = std::max(big, all[s]);
-        big1 = std::max(big1, most[s]);
+        need[s] = whole_bytes<T>(b->sc[s], b->shape);
+        sum += need[s];
+        big = std::max(big, need[s]);
+        least = std::max(least, least_bytes<T>(b->sc[s], b->shape));
     }
-    const size_t want = std::max(big, std::min(sum, PARTS_BYTES));
+    const size_t want = b->parts_room ? std::min(sum, std::max(least, b->parts_room)) : std::max(big, std::min(sum, PARTS_BYTES));
     if (b->parts_bytes < want) {
         hipFree(b->parts);
         b->parts = nullptr;
         b->parts_bytes = 0;
-        b->parts_one = false;
         size_t got = want;
-        // less room: smaller groups, down to the largest grid; then one
-        // direction of it
+        // less room: smaller groups, then the largest grids in slabs
         while (hipMalloc(&b->parts, got) != hipSuccess) {
             (void)hipGetLastError();
             b->parts = nullptr;
-            if (got > big) got = std::max(big, got / 2);
-            else if (!b->parts_one) { b->parts_one = true; got = big1; }
-            else return MAGIC_ENOMEM;
+            if (got == least) return MAGIC_ENOMEM;
+            got = std::max(got > big ? big : least, got / 2);
         }
         b->parts_bytes = got;
-    } else {
-        b->parts_one = false;   // what made it so is gone
     }
     b->groups.clear();
-    const std::vector<size_t> &need = b->parts_one ? most : all;
+    b->slabs.assign(b->n, {});
     size_t used = 0;
     for (int s = 0; s < b->n; s++) {
-        if (b->groups.empty() || used + need[s] > b->parts_bytes) {
-            b->groups.push_back({s, s, {0, 0, 0, 0}});
+        magic_batch::Group g = {s, s + 1, {0, 0, 0, 0}};
+        if (need[s] > b->parts_bytes) {
+            b->slabs[s] = slabs_for<T>(b->sc[s], b->shape, b->parts_bytes);
+            g.nslab = (int)b->slabs[s].size();
+            for (g.slab = 0; g.slab < g.nslab; g.slab++) b->groups.push_back(g);
+            continue;
+        }
+        if (b->groups.empty() || b->groups.back().slab >= 0 || used + need[s] > b->parts_bytes) {
+            b->groups.push_back(g);
             used = 0;
         }
         used += need[s];
@@ -425,28 +466,32 @@ static int build_lists(magic_batch *b, bool tuning = false)
     for (auto &g : b->groups) {
         T *next = (T *)b->parts;
         for (int dir = 0; dir < 3; dir++) {
-            if (b->parts_one) next = (T *)b->parts;
             g.off[dir] = (int)items.size();
             for (int s = g.lo; s < g.hi; s++) {
                 magic_ctx *c = b->sc[s];
                 if (!c) continue;
                 SweepArgsT<T> &a = args[3 * s + dir];
                 StepParts<T> &sp = slot_parts(b, s, T());
+                SweepParts<T> &p = sp.d[dir];
                 memset(&a, 0, sizeof(a));
                 sweep_form_args(c, a);
-                sweep_geometry(c, dir, b->shape[dir], a, sp.d[dir]);
+                sweep_geometry(c, dir, b->shape[dir], a, p);
                 sp.nc = c->meqn;
                 a.nspecadv = c->have_params ? c->prm.nspecadv : 0;
                 a.cfl_bits = &b->ctl_d[s].cfl_bits;
                 a.status = &b->ctl_d[s].err[0];
-                if (b->parts_one || tuning) a.qold = (const T *)state_qold(c);
+                if (g.slab >= 0 || tuning) a.qold = (const T *)state_qold(c);
                 const double dt = b->ctl[s].dt > 0.0 ? b->ctl[s].dt : 1.0;
                 if (tuning) sweep_factors(c, dir, dt, a);
-                a.parts = next;
-                sp.d[dir].base = next;
-                next += parts_size(sp.d[dir], c->meqn, b->shape[dir]);
+                int lo = 0, hi = dir == 0 ? p.nk : p.nt;
+                if (g.slab >= 0) {   // put_slab places its parts
+                    lo = b->slabs[s][g.slab].lo[dir];
+                    hi = b->slabs[s][g.slab].hi[dir];
+                } else {
+                    next = parts_layout(a, p, dir, lo, hi, c->meqn, b->shape[dir], next);
+                }
                 run[3 * s + dir] = tuning ? b->one_d : &b->ctl_d[s].run;
-                push_items(items, sp.d[dir], 3 * s + dir);
+                push_items(items, p, dir, lo, hi, 3 * s + dir);
                 if (items.size() > 0x7fffffff) return MAGIC_EUNSUPPORTED;
             }
         }
@@ -563,7 +608,7 @@ static int build_ops(magic_batch *b)
         o.d = c->d;
         form_ops(c, o);
         o.sp = slot_parts(b, s, T());
-        o.one = b->parts_one;
+        o.added = !b->slabs[s].empty();
         o.nc = c->meqn;
         o.kb = kb;
         o.spill = c->mz > c->mx ? c->mz - c->mx : 0;
@@ -911,6 +956,17 @@ extern "C" int magic_batch_set_tile_shapes(magic_batch *b, const int shapes[3])
     return MAGIC_OK;
 }
 
+extern "C" int magic_batch_set_increment_room(magic_batch *b, size_t bytes)
+{
+    if (!b) return MAGIC_EARG;
+    TRY(drop_graph(b));   // its kernels hold the buffer's address
+    b->parts_room = bytes;
+    hipFree(b->parts);
+    b->parts = nullptr;
+    b->parts_bytes = 0;
+    return MAGIC_OK;
+}
+
 extern "C" int magic_batch_set_sweep_overlap(magic_batch *b, int on)
 {
     if (!b) return MAGIC_EARG;
@@ -939,7 +995,11 @@ static int tune_rounds(magic_batch *b, int reps, TuneClock &clk)
             TRY(build_lists<T>(b, true));
             for (int dir = 0; dir < 3; dir++) {
                 TRY(clk.mark(dir, sh, 0, b->stream));
-                for (const auto &g : b->groups) TRY((launch_dirs<T, PERT>(b, g, dir, dir + 1)));
+                for (const auto &g : b->groups) {
+                    StepParts<T> sp;
+                    if (g.slab >= 0) TRY(put_slab<T>(b, g, sp));
+                    TRY((launch_dirs<T, PERT>(b, g, dir, dir + 1)));
+                }
                 TRY(clk.mark(dir, sh, 1, b->stream));
             }
         }

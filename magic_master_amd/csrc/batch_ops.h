@@ -26,8 +26,8 @@ template <typename T>
 struct BatchOps {
     Dims d;
     T *q, *qold, *u, *qt, *ut;
-    StepParts<T> sp;  // the sweeps' increments, added in the conversion, or with one set by OP_ADD_PARTS
-    int one;          // the increments have room for one direction at a time
+    StepParts<T> sp;  // the sweeps' increments, added in the conversion
+    int added;        // they are in q already: the grid is swept in slabs
     int nc;          // meqn
     int kb;          // layers per block of the diffusion kernels (diff_kb)
     int spill;       // conduct.f:86-91 out-of-row writes (mz - mx when mz > mx, else 0)
@@ -47,7 +47,7 @@ struct BatchOps {
 // Kernel classes of the batched attempt
 enum {
     OP_BC = 0, OP_BCUVW, OP_BCZ, OP_BACKUP, OP_RESTORE, OP_CONVERT, OP_DIFF_CROSS, OP_DIFF, OP_CONDUCT, OP_COPY_T, OP_FINISH,
-    OP_ADD_PARTS, NOP
+    NOP
 };
 // Block lists, one per launch geometry:
 //   BC  boundary lanes and, with tracers, the interior's (1-D, 256 lanes)
@@ -97,7 +97,7 @@ __device__ __forceinline__ const T *conducted(const BatchOps<T> &o, const StepGa
 // end in LDS (pre: active blocks before each slot), then takes active
 // blocks blockIdx.x, blockIdx.x + gridDim.x, ...; a launch whose gates are
 // all off ends after that scan.  arg: conduct's substep of
-// OP_CONDUCT, the direction of OP_ADD_PARTS.  The form's own bodies
+// OP_CONDUCT.  The form's own bodies
 // are reached through the FORM functor (FP32: bc_src32.hip, FP64:
 // bc_src.hip).  n <= BATCH_MAX_SLOTS (the host checks).
 template <typename T, int OP, class FORM>
@@ -193,12 +193,6 @@ __global__ __launch_bounds__(256) void k_batch_op(const BatchOps<T> *__restrict_
             b_copy_interior(bi, o.d, o.q + 4 * P, conducted(o, g), 1, g);
         } else if constexpr (OP == OP_FINISH) {
             FORM::finish(bi, o, g);
-        } else if constexpr (OP == OP_ADD_PARTS) {
-            StepParts<T> one = o.sp;   // direction arg alone
-#pragma unroll
-            for (int k = 0; k < 3; k++)
-                if (k != arg) one.d[k].base = nullptr;
-            b_add_parts(bi, o.d, o.q, one, g);
         }
     }
 }

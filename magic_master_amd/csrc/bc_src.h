@@ -123,8 +123,6 @@ template <typename T>
 struct StepParts;
 template <bool COL, class G>
 __global__ void k_src_convert(Dims d, const double *qin, double *q, const Aux a, G gate, StepParts<double> sp);
-template <typename T, class G>
-__global__ void k_add_parts(Dims d, T *q, StepParts<T> sp, G gate);
 template <typename T, bool COLC, class G>
 __global__ void k_diff_cross(Dims d, T *u, const T *q, const T *coef, T dxy, T dxz, T dyz, int kb, G gate);
 // y-rows per lane of the directional passes (diff_passes): two load too much

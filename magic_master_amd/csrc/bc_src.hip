@@ -203,7 +203,7 @@ struct Form64 {
     __device__ static void convert(uint3 bi, const BatchOps<double> &o, const StepGate &g)
     {
         StepParts<double> sp = o.sp;
-        if (o.one) sp.d[0].base = nullptr;   // already in q
+        if (o.added) sp.d[0].base = nullptr;
         b_src_convert<true>(bi, o.d, o.q, o.q, o.qold, o.ax, g, sp);
     }
     __device__ static void finish(uint3 bi, const BatchOps<double> &o, const StepGate &g)
@@ -221,7 +221,6 @@ const void *batch_op_fn<double>(int op)
 #define MAGIC_OP(X) case X: return reinterpret_cast<const void *>(&k_batch_op<double, X, Form64>);
     MAGIC_OP(OP_BC) MAGIC_OP(OP_BCUVW) MAGIC_OP(OP_BCZ) MAGIC_OP(OP_BACKUP) MAGIC_OP(OP_RESTORE) MAGIC_OP(OP_CONVERT)
     MAGIC_OP(OP_DIFF_CROSS) MAGIC_OP(OP_DIFF) MAGIC_OP(OP_CONDUCT) MAGIC_OP(OP_COPY_T) MAGIC_OP(OP_FINISH)
-    MAGIC_OP(OP_ADD_PARTS)
 #undef MAGIC_OP
     default: return nullptr;
     }
@@ -236,7 +235,6 @@ template __global__ void k_bc_z<GridGate>(Dims, double *, int, int, int, const d
                                         const double *, const double *, GridGate);
 template __global__ void k_src_convert<false, GridGate>(Dims, const double *, double *, const Aux, GridGate, StepParts<double>);
 template __global__ void k_src_convert<true, GridGate>(Dims, const double *, double *, const Aux, GridGate, StepParts<double>);
-template __global__ void k_add_parts<double, GridGate>(Dims, double *, StepParts<double>, GridGate);
 template __global__ void k_src_finish<false, GridGate>(Dims, double *, const double *, int, const Aux, Forcing, GridGate);
 template __global__ void k_src_finish<true, GridGate>(Dims, double *, const double *, int, const Aux, Forcing, GridGate);
 template __global__ void k_diff_cross<double, true, GridGate>(Dims, double *, const double *, const double *, double, double,

@@ -191,7 +191,7 @@ struct Form32 {
     __device__ static void convert(uint3 bi, const BatchOps<float> &o, const StepGate &g)
     {
         StepParts<float> sp = o.sp;
-        if (o.one) sp.d[0].base = nullptr;   // already in q
+        if (o.added) sp.d[0].base = nullptr;
         b32_src_convert(bi, o.d, o.q, o.q, o.qold, o.col, g, sp);
     }
     __device__ static void finish(uint3 bi, const BatchOps<float> &o, const StepGate &g)
@@ -209,7 +209,6 @@ const void *batch_op_fn<float>(int op)
 #define MAGIC_OP(X) case X: return reinterpret_cast<const void *>(&k_batch_op<float, X, Form32>);
     MAGIC_OP(OP_BC) MAGIC_OP(OP_BCUVW) MAGIC_OP(OP_BCZ) MAGIC_OP(OP_BACKUP) MAGIC_OP(OP_RESTORE) MAGIC_OP(OP_CONVERT)
     MAGIC_OP(OP_DIFF_CROSS) MAGIC_OP(OP_DIFF) MAGIC_OP(OP_CONDUCT) MAGIC_OP(OP_COPY_T) MAGIC_OP(OP_FINISH)
-    MAGIC_OP(OP_ADD_PARTS)
 #undef MAGIC_OP
     default: return nullptr;
     }
@@ -219,7 +218,6 @@ const void *batch_op_fn<float>(int op)
 // k_batch_op, above)
 template __global__ void k32_bc_z<GridGate>(Dims, float *, int, int, int, Zr32, GridGate);
 template __global__ void k32_src_convert<GridGate>(Dims, const float *, float *, Col32, GridGate, StepParts<float>);
-template __global__ void k_add_parts<float, GridGate>(Dims, float *, StepParts<float>, GridGate);
 template __global__ void k32_src_finish<GridGate>(Dims, float *, const float *, int, Col32, Forcing, GridGate);
 
 // reference AoS q(meqn, i, j, k) (FP64, full state) <-> perturbation planes:

@@ -782,10 +782,20 @@ static void dir_args(const magic_ctx *c, SweepArgsT<T> &a, int dir, double dt)
     }
 }
 
+// The increment buffer given back; the next sweep sets it up again
+static void drop_parts(magic_ctx *c)
+{
+    hipFree(c->parts);
+    hipFree(c->items);
+    c->parts = nullptr;
+    c->parts_bytes = 0;
+    c->items = nullptr;
+}
+
 // Buffers of the tiled sweeps for the context's shapes: argument blocks and
 // run flags, the workgroups' blocks, and the increment buffer.  Where the
-// device has no room for the three directions' increments, one direction's
-// are kept and added to q before the next direction runs.
+// device (or the caller) has no room for the whole grid's increments, the
+// buffer holds a slab's, and the slabs are swept one after the other.
 template <typename T>
 static int sweep_setup(magic_ctx *c)
 {
@@ -803,55 +813,47 @@ static int sweep_setup(magic_ctx *c)
         HIPCHECK(hipMemcpy(c->lrun, run, sizeof(run), hipMemcpyHostToDevice));
     }
     if (c->items && memcmp(c->item_shape, c->shape, sizeof(c->shape)) == 0) return MAGIC_OK;
-    std::vector<int4> items;
-    int off[4] = {0, 0, 0, 0};
-    size_t all = 0, most = 0;
-    for (int dir = 0; dir < 3; dir++) {
-        SweepArgsT<T> a;
-        SweepParts<T> p;
-        sweep_geometry(c, dir, c->shape[dir], a, p);
-        push_items(items, p, dir);
-        off[dir + 1] = (int)items.size();
-        const size_t bytes = (size_t)parts_size(p, c->meqn, c->shape[dir]) * sizeof(T);
-        all += bytes;
-        most = std::max(most, bytes);
-    }
     HIPCHECK(hipStreamSynchronize(c->stream));   // nothing reads the old lists or increments any more
     hipFree(c->items);
     c->items = nullptr;
-    if (c->parts_bytes < all) {
+    const size_t least = least_bytes<T>(c, c->shape);
+    const size_t want = std::min(whole_bytes<T>(c, c->shape), std::max(least, c->parts_room));
+    if (c->parts_bytes < want) {
         hipFree(c->parts);
         c->parts = nullptr;
         c->parts_bytes = 0;
-        c->parts_one = false;
-        size_t got = all;
-        if (hipMalloc(&c->parts, all) != hipSuccess) {
+        size_t got = want;   // less room: narrower slabs
+        while (hipMalloc(&c->parts, got) != hipSuccess) {
             (void)hipGetLastError();
-            got = most;
-            c->parts_one = true;
-            if (hipMalloc(&c->parts, most) != hipSuccess) {
-                (void)hipGetLastError();
-                c->parts = nullptr;
-                return MAGIC_ENOMEM;
-            }
+            c->parts = nullptr;
+            if (got == least) return MAGIC_ENOMEM;
+            got = std::max(least, got / 2);
         }
         c->parts_bytes = got;
-    } else {
-        c->parts_one = false;
     }
+    c->slabs = slabs_for<T>(c, c->shape, c->parts_bytes);
+    std::vector<int4> items;
+    c->item_off.assign(1, 0);
+    for (const Slab &slab : c->slabs)
+        for (int dir = 0; dir < 3; dir++) {
+            SweepArgsT<T> a;
+            SweepParts<T> p;
+            sweep_geometry(c, dir, c->shape[dir], a, p);
+            push_items(items, p, dir, slab.lo[dir], slab.hi[dir], dir);
+            c->item_off.push_back((int)items.size());
+        }
     if (hipMalloc(&c->items, items.size() * sizeof(int4)) != hipSuccess) {
         (void)hipGetLastError();
         c->items = nullptr;
         return MAGIC_ENOMEM;
     }
     HIPCHECK(hipMemcpy(c->items, items.data(), items.size() * sizeof(int4), hipMemcpyHostToDevice));
-    memcpy(c->item_off, off, sizeof(off));
     memcpy(c->item_shape, c->shape, sizeof(c->shape));
     return MAGIC_OK;
 }
 
-// The argument blocks of one step's sweeps, and the step's reductions back
-// to zero.  Launched before the sweeps on their stream.
+// The argument blocks of a slab's sweeps, and (scal) the step's reductions
+// back to zero.  Launched before the sweeps on their stream.
 template <typename T>
 struct StepArgs {
     SweepArgsT<T> d[3];
@@ -860,53 +862,52 @@ template <typename T>
 __global__ void k_put_step_args(SweepArgsT<T> *slots, StepArgs<T> a, unsigned long long *scal)
 {
     if (threadIdx.x < 3) slots[threadIdx.x] = a.d[threadIdx.x];
-    else if (threadIdx.x >= 8 && threadIdx.x < 16) scal[threadIdx.x - 8] = 0ull;
+    else if (scal && threadIdx.x >= 8 && threadIdx.x < 16) scal[threadIdx.x - 8] = 0ull;
 }
 
-// Argument blocks for step dt from base (state pointers and form-specific
-// fields set), and the descriptors of the parts they fill
+// Argument blocks for step dt of slab s from base (state pointers and
+// form-specific fields set), and the descriptors of the parts they fill
 template <typename T>
-static int put_step_args(magic_ctx *c, const SweepArgsT<T> &base, double dt, StepParts<T> &sp)
+static int put_step_args(magic_ctx *c, const SweepArgsT<T> &base, double dt, size_t s, StepParts<T> &sp)
 {
-    TRY(sweep_setup<T>(c));
-    StepArgs<T> s;
+    StepArgs<T> sa;
+    const Slab &slab = c->slabs[s];
     sp.nc = c->meqn;
     T *next = (T *)c->parts;
     for (int dir = 0; dir < 3; dir++) {
-        s.d[dir] = base;
-        sweep_geometry(c, dir, c->shape[dir], s.d[dir], sp.d[dir]);
-        sweep_factors(c, dir, dt, s.d[dir]);
-        s.d[dir].parts = next;
-        sp.d[dir].base = next;
-        if (!c->parts_one) next += parts_size(sp.d[dir], c->meqn, c->shape[dir]);
+        sa.d[dir] = base;
+        sweep_geometry(c, dir, c->shape[dir], sa.d[dir], sp.d[dir]);
+        sweep_factors(c, dir, dt, sa.d[dir]);
+        next = parts_layout(sa.d[dir], sp.d[dir], dir, slab.lo[dir], slab.hi[dir], c->meqn, c->shape[dir], next);
     }
-    k_put_step_args<T><<<1, 64, 0, c->stream>>>((SweepArgsT<T> *)c->largs, s, c->dscal);
+    k_put_step_args<T><<<1, 64, 0, c->stream>>>((SweepArgsT<T> *)c->largs, sa, s == 0 ? c->dscal : nullptr);
     return launch_check();
 }
 
-// One launch over the blocks of directions d0 .. d1-1 (of one shape)
+// One launch over the blocks of slab s and directions d0 .. d1-1 (of one shape)
 template <typename T, bool PERT>
-static int launch_tile(magic_ctx *c, int d0, int d1)
+static int launch_tile(magic_ctx *c, size_t s, int d0, int d1)
 {
     const void *fn = tile_fn<T, PERT>(ntracer(c), c->shape[d0]);
     if (!fn) return MAGIC_EARG;
     const SweepArgsT<T> *args = (const SweepArgsT<T> *)c->largs;
-    const int4 *items = c->items + c->item_off[d0];
+    const int *off = &c->item_off[3 * s];
+    const int4 *items = c->items + off[d0];
     const int *const *run = c->lrun;
     void *kargs[] = {&args, &items, &run};
     Span sp(c, NTC, 1);
-    const float blocks_ = (float)(c->item_off[d1] - c->item_off[d0]);
-    for (int d = d0; d < d1; d++) sp.share[d] = (c->item_off[d + 1] - c->item_off[d]) / blocks_;
-    HIPCHECK(hipLaunchKernel(fn, dim3((unsigned)(c->item_off[d1] - c->item_off[d0])), dim3(256), kargs, 0, c->stream));
+    const float blocks_ = (float)(off[d1] - off[d0]);
+    for (int d = d0; d < d1; d++) sp.share[d] = (off[d + 1] - off[d]) / blocks_;
+    HIPCHECK(hipLaunchKernel(fn, dim3((unsigned)(off[d1] - off[d0])), dim3(256), kargs, 0, c->stream));
     return MAGIC_OK;
 }
 
-// q += the increments of sp (directions with a base), every cell
+// q += the increments of sp, the cells of slab s
 template <typename T>
-static int add_parts_launch(magic_ctx *c, T *q, const StepParts<T> &sp)
+static int add_parts_launch(magic_ctx *c, T *q, const StepParts<T> &sp, const Slab &s)
 {
-    Span s(c, TC_OTHER, 1);
-    k_add_parts<T, GridGate><<<padded_cells(c->d), cell_block(), 0, c->stream>>>(c->d, q, sp, GridGate{});
+    Span t(c, TC_OTHER, 1);
+    k_add_parts<T><<<slab_cells(c->d, s), cell_block(), 0, c->stream>>>(c->d, q, sp, s.i0 + c->mbc - 1, s.i1 + c->mbc - 1, nullptr);
     return launch_check();
 }
 
@@ -915,27 +916,22 @@ static int add_parts_launch(magic_ctx *c, T *q, const StepParts<T> &sp)
 // read a.qold and write their blocks' increments, so they are one launch
 // (one per run of directions that share a tile shape); sp returns the
 // increments, which add_parts or the source pass's conversion adds to q.
-// With one direction's room (parts_one) each direction's increments are
-// added to q at once, and sp is left empty.
+// In slabs, each slab's increments are added to q at once, the same sum for
+// every cell, and sp is left empty.
 template <typename T, bool PERT>
 static int step3_sweeps(magic_ctx *c, const SweepArgsT<T> &a, T *q, double dt, StepParts<T> &sp)
 {
-    TRY(put_step_args<T>(c, a, dt, sp));
-    if (c->parts_one) {
-        for (int dir = 0; dir < 3; dir++) {
-            TRY((launch_tile<T, PERT>(c, dir, dir + 1)));
-            StepParts<T> one = sp;
-            for (int k = 0; k < 3; k++)
-                if (k != dir) one.d[k].base = nullptr;
-            TRY(add_parts_launch(c, q, one));
+    TRY(sweep_setup<T>(c));
+    for (size_t s = 0; s < c->slabs.size(); s++) {
+        TRY(put_step_args<T>(c, a, dt, s, sp));
+        for (int d0 = 0, d1; d0 < 3; d0 = d1) {
+            for (d1 = d0 + 1; d1 < 3 && c->shape[d1] == c->shape[d0];) d1++;
+            TRY((launch_tile<T, PERT>(c, s, d0, d1)));
         }
+        if (c->slabs.size() > 1) TRY(add_parts_launch(c, q, sp, c->slabs[s]));
+    }
+    if (c->slabs.size() > 1)
         for (auto &p : sp.d) p.base = nullptr;
-        return MAGIC_OK;
-    }
-    for (int d0 = 0, d1; d0 < 3; d0 = d1) {
-        for (d1 = d0 + 1; d1 < 3 && c->shape[d1] == c->shape[d0];) d1++;
-        TRY((launch_tile<T, PERT>(c, d0, d1)));
-    }
     return MAGIC_OK;
 }
 
@@ -996,7 +992,8 @@ static int parts_flush(magic_ctx *c)
 {
     if (!c->pending_parts) return MAGIC_OK;
     c->pending_parts = false;
-    return c->form == MAGIC_FORM_FP32P ? add_parts_launch(c, c->q32, c->parts32) : add_parts_launch(c, c->q, c->parts64);
+    return c->form == MAGIC_FORM_FP32P ? add_parts_launch(c, c->q32, c->parts32, c->slabs[0])
+                                       : add_parts_launch(c, c->q, c->parts64, c->slabs[0]);
 }
 
 // whether the sweeps leave their increments in the part buffer (known once
@@ -1007,7 +1004,7 @@ static int setup_sweeps(magic_ctx *c)
     if (!form_tile(c)) return MAGIC_OK;
     return c->form == MAGIC_FORM_FP32P ? sweep_setup<float>(c) : sweep_setup<double>(c);
 }
-static bool sweeps_defer(const magic_ctx *c) { return form_tile(c) && !c->parts_one; }
+static bool sweeps_defer(const magic_ctx *c) { return form_tile(c) && c->slabs.size() == 1; }
 
 static int scal_copy(magic_ctx *c)
 {
@@ -1079,11 +1076,7 @@ int failed_step(magic_ctx *c, const int *shape, double dt)
     if (st == MAGIC_OK) st = step3_launch(c, dt);
     if (st == MAGIC_OK) st = step3_finish(c, &cfl);
     memcpy(c->shape, keep, sizeof(keep));
-    hipFree(c->parts);   // a scenario has no sweeps of its own otherwise
-    hipFree(c->items);
-    c->parts = nullptr;
-    c->parts_bytes = 0;
-    c->items = nullptr;
+    drop_parts(c);   // a scenario has no sweeps of its own otherwise
     return st == MAGIC_ERHO || st == MAGIC_EA2 ? MAGIC_OK : st;
 }
 
@@ -1099,6 +1092,15 @@ extern "C" int magic_get_tile_shapes(magic_ctx *c, int shapes[3])
 {
     if (!c || !shapes) return MAGIC_EARG;
     for (int k = 0; k < 3; k++) shapes[k] = c->shape[k];
+    return MAGIC_OK;
+}
+
+extern "C" int magic_set_increment_room(magic_ctx *c, size_t bytes)
+{
+    if (!c) return MAGIC_EARG;
+    HIPCHECK(hipStreamSynchronize(c->stream));
+    c->parts_room = bytes ? bytes : ~size_t(0);
+    drop_parts(c);
     return MAGIC_OK;
 }
 
@@ -1120,11 +1122,16 @@ static int tune_rounds(magic_ctx *c, const SweepArgsT<T> &a, double dt, int reps
     for (int r = 0; r <= reps; r++) {   // repetition 0 warms up and is not timed
         for (int sh = 0; sh < TILE_NSHAPE; sh++) {
             for (int k = 0; k < 3; k++) c->shape[k] = sh;
+            TRY(sweep_setup<T>(c));
             StepParts<T> sp;
-            TRY(put_step_args<T>(c, a, dt, sp));
+            const size_t n = c->slabs.size();
+            if (n == 1) TRY(put_step_args<T>(c, a, dt, 0, sp));
             for (int dir = 0; dir < 3; dir++) {
                 TRY(clk.mark(dir, sh, 0, c->stream));
-                TRY((launch_tile<T, PERT>(c, dir, dir + 1)));
+                for (size_t s = 0; s < n; s++) {
+                    if (n > 1) TRY(put_step_args<T>(c, a, dt, s, sp));
+                    TRY((launch_tile<T, PERT>(c, s, dir, dir + 1)));
+                }
                 TRY(clk.mark(dir, sh, 1, c->stream));
             }
         }

@@ -46,6 +46,14 @@ struct TimedSpan {
     float share[3];        // of each direction (cls = NTC)
 };
 
+// A slab of a grid swept on its own: its cells (Fortran i) i0 .. i1-1 of all
+// rows and layers, and the blocks that hold increments of theirs: chunks of the
+// x-sweep, tiles of the others, lo .. hi-1 of each direction.
+struct Slab {
+    int i0, i1;
+    int lo[3], hi[3];
+};
+
 struct magic_ctx {
     int form = MAGIC_FORM_FP64;
     int mx, my, mz, meqn, mbc, maux;
@@ -67,12 +75,13 @@ struct magic_ctx {
     double *col64 = nullptr;
     bool aux_layered = false;
     bool own_stream = true;   // false when a batch lends its stream
-    // The sweeps' increment blocks (SweepParts) of one step, for all three
-    // directions at once or, where the device has no room for that, for one
-    // direction at a time (parts_one).  Allocated on first use.
+    // The sweeps' increment blocks (SweepParts) of one step, of the whole grid
+    // or, where the device has no room for that, of one of its slabs at a time.
+    // Allocated on first use.
     void *parts = nullptr;
     size_t parts_bytes = 0;
-    bool parts_one = false;
+    size_t parts_room = ~size_t(0);   // bytes the caller allows them
+    std::vector<Slab> slabs;          // one: the whole grid
     // Inside magic_claw3 the increments of a step are left to the source
     // pass's conversion (pending), which adds them on its way
     bool pending_parts = false;
@@ -92,13 +101,13 @@ struct magic_ctx {
     // The sweep kernel's operands (set up on the first tiled sweep): an
     // argument block per direction (written by a kernel at the start of each
     // step3 or of each tuner round), run flags all pointing at a device 1, and
-    // the workgroups' blocks, direction by direction (those of direction d at
-    // [item_off[d], item_off[d + 1]))
+    // the workgroups' blocks, slab by slab and direction by direction (those of
+    // slab s and direction d at [item_off[3 s + d], item_off[3 s + d + 1]))
     void *largs = nullptr;
     const int **lrun = nullptr;
     int *lone = nullptr;
     int4 *items = nullptr;
-    int item_off[4] = {0, 0, 0, 0};
+    std::vector<int> item_off;
     int item_shape[3] = {-1, -1, -1};      // the shapes the items were laid out for
     GridGate gate;                         // of the kernels launched now (claw3's source pass)
     unsigned long long *hscal = nullptr;   // pinned host words: [0, 8) mirror dscal, [HSCAL_SUMS, +10) global sums
@@ -190,6 +199,7 @@ static inline int ntracer(const magic_ctx *c) { return c->meqn - 5; }
 // along x by 4 rows along y per workgroup, one layer per grid z index.
 static inline dim3 cell_block() { return dim3(64, 4, 1); }
 static inline dim3 interior_grid(const Dims &d) { return dim3(blocks(d.mx, 64), blocks(d.my, 4), d.mz); }
+static inline dim3 slab_cells(const Dims &d, const Slab &s) { return dim3(blocks(s.i1 - s.i0, 64), blocks(d.NY, 4), d.NZ); }
 static inline dim3 padded_cells(const Dims &d) { return dim3(blocks(d.NX, 64), blocks(d.NY, 4), d.NZ); }
 // Layers per workgroup of the diffusion kernels, cols workgroups side by side.
 // Each workgroup's layers run one after the other, so many short workgroups
@@ -336,18 +346,108 @@ static inline void sweep_factors(const magic_ctx *c, int dir, double dt, SweepAr
     a.fg = dir == 0 ? y : dir == 1 ? z : x;
     a.fh = dir == 0 ? z : dir == 1 ? x : y;
 }
+// Elements of one block
 template <typename T>
-static inline long long parts_size(const SweepParts<T> &p, int nc, int sh)   // elements
+static inline long long block_size(const SweepParts<T> &p, int nc, int sh)
 {
-    return (long long)p.ns * p.nk * p.nt * ((1 << p.lgL) + 2) * nc * part_npos(sh);
+    return (long long)((1 << p.lgL) + 2) * nc * part_npos(sh);
 }
-// the blocks of one direction, as they lie in the part buffer
+// The blocks lo .. hi-1 along x of direction dir laid out from next on;
+// returns the element behind them.
 template <typename T>
-static inline void push_items(std::vector<int4> &items, const SweepParts<T> &p, int arg)
+static inline T *parts_layout(SweepArgsT<T> &a, SweepParts<T> &p, int dir, int lo, int hi, int nc, int sh, T *next)
 {
+    const int w = hi - lo;
+    p.sT = dir == 0 ? w : 1;
+    p.sK = dir == 0 ? 1 : w;
+    p.sS = w * (dir == 0 ? p.nt : p.nk);
+    const long long bs = block_size(p, nc, sh);
+    a.parts = next - lo * bs;
+    p.base = a.parts;
+    a.sT = p.sT; a.sK = p.sK; a.sS = p.sS;
+    return next + bs * p.sS * p.ns;
+}
+// the blocks lo .. hi-1 along x of one direction, as they lie in the part buffer
+template <typename T>
+static inline void push_items(std::vector<int4> &items, const SweepParts<T> &p, int dir, int lo, int hi, int arg)
+{
+    const int kl = dir == 0 ? lo : 0, kh = dir == 0 ? hi : p.nk, tl = dir == 0 ? 0 : lo, th = dir == 0 ? p.nt : hi;
     for (int s = 0; s < p.ns; s++)
-        for (int k = 0; k < p.nk; k++)
-            for (int t = 0; t < p.nt; t++) items.push_back(make_int4(arg, t, k, s));
+        for (int k = kl; k < kh; k++)
+            for (int t = tl; t < th; t++) items.push_back(make_int4(arg, t, k, s));
+}
+
+// The blocks along x that hold entries of the cells i0 .. i1-1, as add_parts
+// (parts.h) looks them up: a cell's own block and, next to an edge, the
+// neighbouring one; cells without entries look at the nearest column's.
+template <typename T>
+static inline void slab_blocks(const SweepParts<T> &p, int dir, int i0, int i1, int &lo, int &hi)
+{
+    auto clamp = [](int x, int a, int b) { return std::min(std::max(x, a), b); };
+    if (dir == 0) {
+        const int x = clamp(i1 - 2, 0, p.n - 1);
+        lo = clamp(i0 - 1, 0, p.n - 1) / p.CI;
+        hi = x / p.CI + (x % p.CI == p.CI - 1 ? 2 : 1);
+    } else {
+        const int TA = 1 << p.lgTA;
+        const int x = clamp(i0, -1, p.nA + 2), y = clamp(i1 - 1, -1, p.nA + 2);
+        lo = x < 0 ? 0 : x / TA - (x >= 1 && x % TA == 0 ? 1 : 0);
+        hi = y < 0 ? 1 : std::min(p.nt, y / TA + (y % TA == TA - 1 ? 2 : 1));
+    }
+}
+
+// Slabs w cells wide of a grid's sweeps in shapes sh; bytes returns what the
+// largest one's increments take, all three directions
+template <typename T>
+static inline std::vector<Slab> cut_slabs(const magic_ctx *c, const int *sh, int w, size_t &bytes)
+{
+    std::vector<Slab> out;
+    bytes = 0;
+    for (int x = 0; x < c->mx + 2; x += w) {
+        Slab s;
+        s.i0 = x == 0 ? 1 - c->mbc : x;
+        s.i1 = x + w < c->mx + 2 ? x + w : c->mx + c->mbc + 1;
+        long long n = 0;
+        for (int dir = 0; dir < 3; dir++) {
+            SweepArgsT<T> a;
+            SweepParts<T> p;
+            sweep_geometry(c, dir, sh[dir], a, p);
+            slab_blocks(p, dir, s.i0, s.i1, s.lo[dir], s.hi[dir]);
+            n += block_size(p, c->meqn, sh[dir]) * (s.hi[dir] - s.lo[dir]) * (dir == 0 ? p.nt : p.nk) * p.ns;
+        }
+        bytes = std::max(bytes, (size_t)n * sizeof(T));
+        out.push_back(s);
+    }
+    return out;
+}
+// What the increments of a whole grid take, and those of its narrowest slabs.
+// A slab sweeps every block that holds entries of its cells, so each cell's
+// sum is whole and in its one order; slabs share the blocks at their borders,
+// which are swept twice: 16 cells wide, about three times the work.
+constexpr int SLAB_MIN = 16;
+template <typename T>
+static inline size_t whole_bytes(const magic_ctx *c, const int *sh)
+{
+    size_t n;
+    cut_slabs<T>(c, sh, c->mx + 2, n);
+    return n;
+}
+template <typename T>
+static inline size_t least_bytes(const magic_ctx *c, const int *sh)
+{
+    size_t n;
+    cut_slabs<T>(c, sh, SLAB_MIN, n);
+    return n;
+}
+// The widest slabs whose increments take at most room bytes (at least
+// least_bytes)
+template <typename T>
+static inline std::vector<Slab> slabs_for(const magic_ctx *c, const int *sh, size_t room)
+{
+    size_t n;
+    std::vector<Slab> s = cut_slabs<T>(c, sh, c->mx + 2, n);
+    for (int w = (c->mx + 1) / SLAB_MIN * SLAB_MIN; n > room && w >= SLAB_MIN; w -= SLAB_MIN) s = cut_slabs<T>(c, sh, w, n);
+    return s;
 }
 
 // capi.hip

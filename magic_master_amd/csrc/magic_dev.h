@@ -78,7 +78,7 @@ __global__ void tile_sweep(const SweepArgsT<T> *args, const int4 *items, const i
 // that add them to q do.
 template <typename T>
 struct SweepParts {
-    const T *base;         // nullptr: no increments pending
+    const T *base;         // block 0 (not in the buffer where a slab starts further on); nullptr: no increments pending
     int n, nA, nB;         // interior cells along the pencils, a and b
     int lgTA, lgL;         // log2 pencils per tile, planes per segment
     int CI;                // cells a chunk completes

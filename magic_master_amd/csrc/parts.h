@@ -38,7 +38,8 @@ __device__ __forceinline__ Cand cand_ab(int q, int x, int lg, int nblk, int last
 }
 
 // acc[m] += direction DIR's increments of cell (i, j, k); j and k are the
-// wave's own (scalar), i the lane's.  Along x a lane takes its own block's
+// wave's own (scalar), i the lane's.  Lanes without an entry read the nearest
+// column's, which a slab that holds them has too.  Along x a lane takes its own block's
 // entry and, at an edge, one neighbour's, both loaded without a branch (a
 // lane that is at no edge loads its own entry again and drops it), so that
 // all loads of a direction are in flight together; the blocks along the other
@@ -66,7 +67,7 @@ __device__ __forceinline__ void add_parts(const SweepParts<T> &p, int nc, int i,
     bool own, edge;
     if (DIR == 0) {
         own = i >= 1 && i <= p.n;
-        const int x = own ? i - 1 : 0;
+        const int x = min(max(i - 1, 0), p.n - 1);
         lb = (int)__umulhi((unsigned)x, p.iCI);
         lo = x - lb * p.CI + 1;
         edge = own && lo == p.CI;
@@ -74,7 +75,7 @@ __device__ __forceinline__ void add_parts(const SweepParts<T> &p, int nc, int i,
         eo = 0;
     } else {
         const bool in = i >= -1 && i <= p.nA + 2;
-        const int x = in ? i : 0;
+        const int x = min(max(i, -1), p.nA + 2);
         lb = x >> p.lgTA;
         lo = (x & (TA - 1)) + 1;
         own = in && x >= 0 && lb < p.nt;
@@ -82,7 +83,7 @@ __device__ __forceinline__ void add_parts(const SweepParts<T> &p, int nc, int i,
         edge = in && (before || after);
         eb = before ? lb - 1 : lb + 1;
         eo = before ? TA + 1 : 0;
-        if (!own) { lb = edge ? eb : 0; lo = edge ? eo : 1; }
+        if (lb < 0 || lb >= p.nt) { lb = eb; lo = eo; }   // before the first tile or past the last
     }
     if (!edge) { eb = lb; eo = lo; }
     // blocks run fastest along x: the lanes' blocks are neighbours
@@ -140,27 +141,22 @@ __device__ __forceinline__ void step_parts(const StepParts<T> &sp, int ip, int j
     add_parts<2>(sp.d[2], sp.nc, i, j, k, acc);
 }
 
-// q += the step's increments, every cell (launch: padded_cells)
-template <typename T, class G>
-__device__ __forceinline__ void b_add_parts(const uint3 BI, Dims d, T *q, const StepParts<T> &sp, const G &gate)
+// q += the step's increments, columns ip0 .. ip1-1 of the padded grid (launch:
+// slab_cells); on: the control flag of a batch's scenario, or nullptr
+template <typename T>
+__global__ void k_add_parts(Dims d, T *q, StepParts<T> sp, int ip0, int ip1, const int *on)
 {
-    if (!gate.on()) return;
-    const int ip = (int)(BI.x * blockDim.x + threadIdx.x);
-    const int jp = (int)(BI.y * blockDim.y + threadIdx.y);
-    if (ip >= d.NX || jp >= d.NY) return;
-    const int kk = (int)BI.z;
+    if (on && *on == 0) return;
+    const int ip = ip0 + (int)(blockIdx.x * blockDim.x + threadIdx.x);
+    const int jp = (int)(blockIdx.y * blockDim.y + threadIdx.y);
+    if (ip >= ip1 || jp >= d.NY) return;
+    const int kk = (int)blockIdx.z;
     const long long c = ((long long)kk * d.NY + jp) * d.NX + ip;
     T acc[10];
     step_parts(sp, ip, jp, kk, d.mbc, acc);
 #pragma unroll
     for (int m = 0; m < 10; m++)
         if (m < sp.nc) q[m * d.P + c] = q[m * d.P + c] + acc[m];
-}
-
-template <typename T, class G>
-__global__ void k_add_parts(Dims d, T *q, StepParts<T> sp, G gate)
-{
-    b_add_parts(uint3{blockIdx.x, blockIdx.y, blockIdx.z}, d, q, sp, gate);
 }
 
 }  // namespace magic

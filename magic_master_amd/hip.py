@@ -45,7 +45,7 @@ EXPORTS = ["magic_create", "magic_create_form", "magic_destroy", "magic_strerror
            "magic_batch_set_tile_shapes", "magic_batch_get_tile_shapes", "magic_batch_tune",
            "magic_set_sweep_overlap", "magic_batch_set_sweep_overlap", "magic_global_sums",
            "magic_global_sums_noalloc", "magic_snapshot_begin", "magic_snapshot_wait", "magic_host_alloc",
-           "magic_host_free"]
+           "magic_host_free", "magic_set_increment_room", "magic_batch_set_increment_room"]
 
 TILE_NSHAPE = 4   # MAGIC_TILE_NSHAPE
 # (pencils per tile, lane order) of each tile shape
@@ -175,6 +175,8 @@ def load_library(path: str = LIB_PATH):
     L.magic_batch_tune.argtypes = [vp, C.c_int, _ip, _fp]
     L.magic_set_sweep_overlap.argtypes = [vp, C.c_int]
     L.magic_batch_set_sweep_overlap.argtypes = [vp, C.c_int]
+    L.magic_set_increment_room.argtypes = [vp, C.c_size_t]
+    L.magic_batch_set_increment_room.argtypes = [vp, C.c_size_t]
     L.magic_global_sums.argtypes = [vp, _dp]
     L.magic_global_sums_noalloc.argtypes = [vp, _dp]
     _LIB = L
@@ -360,6 +362,11 @@ class MagicHIP:
         and their sums have one order, whatever it says."""
         self._check(self.L.magic_set_sweep_overlap(self.h, 1 if on else 0), "magic_set_sweep_overlap")
 
+    def set_increment_room(self, nbytes: int):
+        """At most nbytes of device memory for the sweeps' increments (0: no
+        bound); a grid that needs more is swept in slabs, with the same result."""
+        self._check(self.L.magic_set_increment_room(self.h, int(nbytes)), "magic_set_increment_room")
+
     def tune(self, dt: float, reps: int = 3):
         """Autotuner: times every tile shape of every sweep direction on the
         current state and keeps the fastest; returns (shapes, ms[3][NSHAPE])."""
@@ -491,6 +498,10 @@ class MagicBatch:
     def set_sweep_overlap(self, on: bool):
         """Accepted, without effect, as MagicHIP.set_sweep_overlap."""
         self._check(self.L.magic_batch_set_sweep_overlap(self.h, 1 if on else 0), "magic_batch_set_sweep_overlap")
+
+    def set_increment_room(self, nbytes: int):
+        """MagicHIP.set_increment_room for the batch's buffer (0: 8 GB)."""
+        self._check(self.L.magic_batch_set_increment_room(self.h, int(nbytes)), "magic_batch_set_increment_room")
 
     def tile_shapes(self):
         sh = (C.c_int * 3)()
