@@ -59,6 +59,7 @@ struct magic_batch {
     std::vector<StepParts<float>> sp32;
     void *parts = nullptr;
     size_t parts_bytes = 0;
+    magic_ctx *parts_of = nullptr;       // the scenario whose staging buffer it is: there is no room beside it
     size_t parts_room = 0;               // bytes the caller allows it (0: PARTS_BYTES)
     int shape[3] = {0, 0, 0};            // tile shape of the x-, y- and z-sweeps
     int *one_d = nullptr;                // a device 1: the run flag of every tile while tuning
@@ -401,14 +402,25 @@ static void sweep_form_args(const magic_ctx *c, SweepArgsT<double> &a)
 // scenarios' own states take.
 constexpr size_t PARTS_BYTES = size_t(8) << 30;
 
+// The part buffer given back; the next list build sets it up again
+static void drop_parts(magic_batch *b)
+{
+    if (!b->parts_of) hipFree(b->parts);
+    b->parts = nullptr;
+    b->parts_bytes = 0;
+    b->parts_of = nullptr;
+}
+
 // The part buffer and the groups for the batch's shapes
 template <typename T>
 static int build_groups(magic_batch *b)
 {
     std::vector<size_t> need(b->n, 0);
     size_t sum = 0, big = 0, least = 0;
+    magic_ctx *roomy = nullptr;   // the scenario with the largest staging buffer
     for (int s = 0; s < b->n; s++) {
         if (!b->sc[s]) continue;
+        if (!roomy || stage_bytes(b->sc[s]) > stage_bytes(roomy)) roomy = b->sc[s];
         need[s] = whole_bytes<T>(b->sc[s], b->shape);
         sum += need[s];
         big = std::max(big, need[s]);
@@ -416,15 +428,20 @@ static int build_groups(magic_batch *b)
     }
     const size_t want = b->parts_room ? std::min(sum, std::max(least, b->parts_room)) : std::max(big, std::min(sum, PARTS_BYTES));
     if (b->parts_bytes < want) {
-        hipFree(b->parts);
-        b->parts = nullptr;
-        b->parts_bytes = 0;
+        drop_parts(b);
         size_t got = want;
-        // less room: smaller groups, then the largest grids in slabs
+        // less room: smaller groups, then the largest grids in slabs, at last
+        // in a staging buffer, idle in an attempt
         while (hipMalloc(&b->parts, got) != hipSuccess) {
             (void)hipGetLastError();
             b->parts = nullptr;
-            if (got == least) return MAGIC_ENOMEM;
+            if (got == least) {
+                if (stage_bytes(roomy) < least) return MAGIC_ENOMEM;
+                b->parts = roomy->stage;
+                b->parts_of = roomy;
+                got = stage_bytes(roomy);
+                break;
+            }
             got = std::max(got > big ? big : least, got / 2);
         }
         b->parts_bytes = got;
@@ -769,6 +786,7 @@ extern "C" int magic_batch_remove(magic_batch *b, int s)
 {
     if (!b || s < 0 || s >= b->n || !b->sc[s]) return MAGIC_EARG;
     TRY(drop_graph(b));
+    if (b->parts_of == b->sc[s]) drop_parts(b);
     magic_destroy(b->sc[s]);
     b->sc[s] = nullptr;
     memset(&b->ctl[s], 0, sizeof(ScenCtl));
@@ -814,9 +832,10 @@ extern "C" int magic_batch_destroy(magic_batch *b)
 {
     if (!b) return MAGIC_OK;
     drop_graph(b);
+    drop_parts(b);
     for (auto c : b->sc)
         if (c) magic_destroy(c);
-    hipFree(b->ctl_d); hipFree(b->args_d); hipFree(b->run_d); hipFree(b->items_d); hipFree(b->parts);
+    hipFree(b->ctl_d); hipFree(b->args_d); hipFree(b->run_d); hipFree(b->items_d);
     hipFree(b->one_d); hipFree(b->ops_d); hipFree(b->loff_d); hipFree(b->lgdim_d);
     if (b->ctl_pin) hipHostFree(b->ctl_pin);
     if (b->stream) hipStreamDestroy(b->stream);
@@ -902,6 +921,7 @@ extern "C" int magic_batch_run(magic_batch *b, int max_attempts, int check_every
         HIPCHECK(hipMemcpyAsync(b->ctl_d, b->ctl.data(), b->n * sizeof(ScenCtl), hipMemcpyHostToDevice, b->stream));
         b->dirty = false;
     }
+    if (b->parts_of) TRY(stage_ready(b->parts_of));   // a snapshot may still be copied out of it
     int done = 0;
     bool any = true;
     while (done < max_attempts && any) {
@@ -961,9 +981,7 @@ extern "C" int magic_batch_set_increment_room(magic_batch *b, size_t bytes)
     if (!b) return MAGIC_EARG;
     TRY(drop_graph(b));   // its kernels hold the buffer's address
     b->parts_room = bytes;
-    hipFree(b->parts);
-    b->parts = nullptr;
-    b->parts_bytes = 0;
+    drop_parts(b);
     return MAGIC_OK;
 }
 
@@ -993,6 +1011,7 @@ static int tune_rounds(magic_batch *b, int reps, TuneClock &clk)
         for (int sh = 0; sh < TILE_NSHAPE; sh++) {
             for (int k = 0; k < 3; k++) b->shape[k] = sh;
             TRY(build_lists<T>(b, true));
+            if (b->parts_of) TRY(stage_ready(b->parts_of));
             for (int dir = 0; dir < 3; dir++) {
                 TRY(clk.mark(dir, sh, 0, b->stream));
                 for (const auto &g : b->groups) {

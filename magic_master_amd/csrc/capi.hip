@@ -315,7 +315,8 @@ extern "C" int magic_destroy(magic_ctx *c)
     hipFree(c->u); hipFree(c->qt); hipFree(c->ut); hipFree(c->dscal);
     hipFree(c->q32); hipFree(c->qold32); hipFree(c->u32); hipFree(c->qt32); hipFree(c->ut32);
     hipFree(c->col32); hipFree(c->bg64); hipFree(c->col64); hipFree(c->sums_d);
-    hipFree(c->largs); hipFree(c->lrun); hipFree(c->lone); hipFree(c->items); hipFree(c->parts);
+    hipFree(c->largs); hipFree(c->lrun); hipFree(c->lone); hipFree(c->items);
+    if (!c->parts_stage) hipFree(c->parts);
     if (c->hscal) hipHostFree(c->hscal);
     if (c->snap_conv) hipEventDestroy(c->snap_conv);
     if (c->snap_done) hipEventDestroy(c->snap_done);
@@ -483,7 +484,7 @@ extern "C" int magic_set_aux_column(magic_ctx *c, const double *col)
 
 // stage may be read by a snapshot's copy still in flight: the stream waits
 // for it before anything writes stage
-static int stage_ready(magic_ctx *c)
+int stage_ready(magic_ctx *c)
 {
     if (c->snap_pending) HIPCHECK(hipStreamWaitEvent(c->stream, c->snap_done, 0));
     return MAGIC_OK;
@@ -785,10 +786,11 @@ static void dir_args(const magic_ctx *c, SweepArgsT<T> &a, int dir, double dt)
 // The increment buffer given back; the next sweep sets it up again
 static void drop_parts(magic_ctx *c)
 {
-    hipFree(c->parts);
+    if (!c->parts_stage) hipFree(c->parts);
     hipFree(c->items);
     c->parts = nullptr;
     c->parts_bytes = 0;
+    c->parts_stage = false;
     c->items = nullptr;
 }
 
@@ -819,14 +821,18 @@ static int sweep_setup(magic_ctx *c)
     const size_t least = least_bytes<T>(c, c->shape);
     const size_t want = std::min(whole_bytes<T>(c, c->shape), std::max(least, c->parts_room));
     if (c->parts_bytes < want) {
-        hipFree(c->parts);
-        c->parts = nullptr;
-        c->parts_bytes = 0;
-        size_t got = want;   // less room: narrower slabs
+        drop_parts(c);
+        size_t got = want;   // less room: narrower slabs, at last in the staging buffer, idle in a step
         while (hipMalloc(&c->parts, got) != hipSuccess) {
             (void)hipGetLastError();
             c->parts = nullptr;
-            if (got == least) return MAGIC_ENOMEM;
+            if (got == least) {
+                if (stage_bytes(c) < least) return MAGIC_ENOMEM;
+                c->parts = c->stage;
+                c->parts_stage = true;
+                got = stage_bytes(c);
+                break;
+            }
             got = std::max(least, got / 2);
         }
         c->parts_bytes = got;
@@ -870,6 +876,7 @@ __global__ void k_put_step_args(SweepArgsT<T> *slots, StepArgs<T> a, unsigned lo
 template <typename T>
 static int put_step_args(magic_ctx *c, const SweepArgsT<T> &base, double dt, size_t s, StepParts<T> &sp)
 {
+    if (c->parts_stage) TRY(stage_ready(c));
     StepArgs<T> sa;
     const Slab &slab = c->slabs[s];
     sp.nc = c->meqn;

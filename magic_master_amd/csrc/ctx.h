@@ -80,6 +80,7 @@ struct magic_ctx {
     // Allocated on first use.
     void *parts = nullptr;
     size_t parts_bytes = 0;
+    bool parts_stage = false;         // they lie in stage: there is no room beside it
     size_t parts_room = ~size_t(0);   // bytes the caller allows them
     std::vector<Slab> slabs;          // one: the whole grid
     // Inside magic_claw3 the increments of a step are left to the source
@@ -453,6 +454,8 @@ static inline std::vector<Slab> slabs_for(const magic_ctx *c, const int *sh, siz
 // capi.hip
 int tune_state(magic_ctx *c), tune_done(magic_ctx *c);
 int failed_step(magic_ctx *c, const int *shape, double dt);
+int stage_ready(magic_ctx *c);
+static inline size_t stage_bytes(const magic_ctx *c) { return (size_t)c->P * c->meqn * sizeof(double); }
 
 // Event pairs of the autotuners, one per (direction, shape).  The shapes
 // are timed round-robin (every round times each candidate once), so that a

@@ -93,3 +93,39 @@ def test_batch_with_little_room(form, share):
                 d.close()
     finally:
         b.close()
+
+
+def test_no_room_beside_the_grid():
+    """A grid whose increments have to go to its staging buffer, with a snapshot
+    still on its way out of that buffer."""
+    import ctypes as C
+    from magic_master_amd.hip import MagicHIP, PinnedBuffer, load_library, snapshot_wait
+    L = load_library()      # its HIP runtime's own calls, found through its dependencies
+    c, p, g, aux, q = perturbed(400, 150, 100, [1, 1, 1, 1, 3, 1], seed=6, vel=0.05, visc=1.0)
+    buf = PinnedBuffer(8 * q.size)
+    out = []
+    d = MagicHIP(g, p, aux, q)
+    fill = C.c_void_p()
+    try:
+        for full in (True, False):
+            if not full:    # leave 100 MB; slabs 16 cells wide take 190 MB beside the grid
+                d.set_increment_room(0)
+                free, total = C.c_size_t(), C.c_size_t()
+                assert L.hipMemGetInfo(C.byref(free), C.byref(total)) == 0
+                assert L.hipMalloc(C.byref(fill), C.c_size_t(free.value - 100_000_000)) == 0
+            print(f"[no room] full {full}", flush=True)
+            d.set_q(q)
+            d.timing(True)
+            d.timing_reset()
+            h = d.snapshot_begin(buf)
+            t, dtv, log = d.run_steps(c, 2, dt0=60.0)
+            snapshot_wait(h)
+            assert full == (d.timing_read()["sweep_x"][1] == len(log.dt))
+            out.append([t, log.dt, log.cfl, buf.array(g.shape_q).copy(), d.get_q()])
+    finally:
+        d.close()
+        L.hipFree(fill)
+        buf.close()
+    for a, b in zip(*out):
+        np.testing.assert_array_equal(a, b)
+    np.testing.assert_array_equal(out[0][3], q)

@@ -158,3 +158,41 @@ def test_batch_room_found_again(host):
     b.run(1, 1)
     assert not backup()
     """)
+
+
+def test_no_room_beside_the_grid(host):
+    """A grid that fills the device is stepped all the same (its increments go
+    to the staging buffer), and a snapshot that is still being copied out of
+    that buffer is waited for."""
+    host("""
+    c, p, g, aux, q = perturbed(400, 30, 30, [1, 1, 1, 1, 3, 1])
+    d = MagicHIP(g, p, aux, q)
+    stub.stub_room(stub.stub_used() + (1 << 20))        # 6.5 MB are the least beside it
+    d.step3(1.0)
+    launches()
+    buf = PinnedBuffer(8 * q.size)
+    h = d.snapshot_begin(buf)
+    d.run_steps(c, 2)
+    l = launches()
+    first = [i for i, n in enumerate(l) if "tile_sweep" in n][0]
+    assert "wait" in l[:first][l.index("wait") + 1:], l[:first]   # beside the copy stream's own
+    snapshot_wait(h)
+    d.close()
+    stub.stub_room(1 << 60)
+    b = MagicBatch([g], [p], [aux[:, 0, 0, :].copy()], [q], form=FORM_FP64)
+    stub.stub_room(stub.stub_used() + (1 << 20))
+    b.start(0, 0.0, 1e9, 1.0, c.dtv, c.cflv, 5, c.mthbc)
+    b.run(1, 1)
+    assert b.state(0)["status"] == 0
+    launches()
+    h = b.snapshot_begin(0, buf)
+    b.run(1, 1)
+    assert launches().count("wait") == 2
+    snapshot_wait(h)
+    b.remove(0)
+    stub.stub_room(1 << 60)
+    s = b.add(g, p, aux[:, 0, 0, :].copy(), q)
+    b.start(s, 0.0, 1e9, 1.0, c.dtv, c.cflv, 5, c.mthbc)
+    b.run(1, 1)
+    b.close()
+    """)
