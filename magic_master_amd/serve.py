@@ -68,11 +68,21 @@ class Outcome:
 
 def footprint_bytes(g: P.Grid) -> int:
     """Device memory of one scenario of the FP32 form in a batch, beside the
-    batch's own buffer of increments (8 GB at most): q' and its backup (2 x 4 B x meqn), the
-    source pass's scratch (5 x 4 B), the FP64 staging of q for upload and
-    download (8 B x meqn), per padded cell, plus the columns."""
+    batch's own buffer of increments (increment_room): q' and its backup (2 x
+    4 B x meqn), the source pass's scratch (5 x 4 B), the FP64 staging of q for
+    upload and download (8 B x meqn), per padded cell, plus the columns."""
     cells = (g.mx + 2 * g.mbc) * (g.my + 2 * g.mbc) * (g.mz + 2 * g.mbc)
     return cells * (8 * g.meqn + 20 + 8 * g.meqn) + 12 * (g.mz + 2 * g.mbc) * 8
+
+
+def increment_room(budget_bytes: float, grids) -> int:
+    """The part of an admission budget that the batch's buffer of the sweeps'
+    increments gets: 8 GB (scenarios beyond that are swept in groups, at no
+    cost), or enough for the largest grid at once (about five times its q'),
+    but an eighth of the budget at most; a grid that needs more is swept in
+    slabs."""
+    q = max(4 * g.meqn * (g.mx + 2 * g.mbc) * (g.my + 2 * g.mbc) * (g.mz + 2 * g.mbc) for g in grids)
+    return max(1, int(min(budget_bytes / 8, max(8 << 30, 5 * q))))
 
 
 class _PinnedPool:
@@ -161,7 +171,9 @@ class Server:
         keeps stepping, and a writer thread finishes them.  tile_shapes: the
         sweeps' tile shapes (x, y, z) for the whole run (None: the library's
         default), fixed so that a request's result does not depend on when
-        it ran.  progress: print a status line every that many wall-clock
+        it ran.  budget_bytes: device memory of the scenarios that run at once
+        and of the sweeps' increments (of very small grids these may take more
+        than their part of it).  progress: print a status line every that many wall-clock
         seconds."""
         if snapshots not in ("hdf5", "download", "none"):
             raise ValueError(snapshots)
@@ -195,6 +207,8 @@ class Server:
         waiting: List[Request] = []
         active = {}                  # slot -> (request, frame, footprint)
         used = 0.0
+        full_room = room = increment_room(self.budget, [r.grid for r in reqs])
+        batch.set_increment_room(room)
         cells_steps = 0
         max_active = 0
         max_used = 0.0
@@ -215,8 +229,13 @@ class Server:
                     fp = footprint_bytes(r.grid)
                     if fp > self.budget:
                         raise ValueError(f"request {r.rid} needs {fp:.3g} B, more than the budget")
-                    if used + fp > self.budget:
+                    # next to the others and the increments' buffer; a request
+                    # that leaves it less room runs alone
+                    if used + fp + full_room > self.budget and used > 0:
                         break
+                    if used + fp + room > self.budget or room < full_room:
+                        room = max(1, int(min(full_room, self.budget - used - fp)))
+                        batch.set_increment_room(room)
                     waiting.pop(0)
                     s = batch.add(r.grid, r.prob, r.column, r.q0)
                     c = r.claw
@@ -225,7 +244,7 @@ class Server:
                     used += fp
                     out[r.rid].admitted = time.perf_counter() - t0
                 max_active = max(max_active, len(active))
-                max_used = max(max_used, used)
+                max_used = max(max_used, used + room)
                 if not active:
                     if pending:
                         time.sleep(max(0.0, pending[0].arrival - (time.perf_counter() - t0)))
