@@ -72,15 +72,20 @@ __device__ __forceinline__ double rcp1(double x)
     const double r = __builtin_amdgcn_rcp(x), e = fma(-x, r, 1.0);
     return fma(r, RF ? e : fma(e, e, e), r);
 }
-// g / b of the limiters: the FP32 form's rounds to FP32 afterwards, the FP64
-// form's is corrected by its remainder, as the correctly rounded quotient is,
-// without that one's scaling: NaN where b is zero or its reciprocal
-// overflows, which the limiters take (they then multiply b).
+// num / den from an approximate reciprocal r of den: corrected by its
+// remainder, as the correctly rounded quotient is, without that one's scaling.
+// One rounding (a unit of 2**-53) whatever error r has up to 1e-14 or so.
+__host__ __device__ __forceinline__ double quot(double num, double den, double r)
+{
+    const double q = num * r;
+    return fma(fma(-den, q, num), r, q);
+}
+// g / b of the limiters: NaN where b is zero or its reciprocal overflows,
+// which the limiters take (they then multiply b).
 template <bool RF>
 __device__ __forceinline__ double ratio(double g, double b)
 {
-    const double r = rcp1<RF>(b), q = g * r;
-    return RF ? q : fma(fma(-b, q, g), r, q);
+    return quot(g, b, rcp1<RF>(b));
 }
 // 1/x of the limiters' clamped Courant numbers and 1 + r (normal range)
 __device__ __forceinline__ double rcpL(double x) { return rcp1<false>(x); }

@@ -309,8 +309,8 @@ __device__ __forceinline__ void tile_sweep_body(const SweepArgsT<T> &A, int bt, 
             const double gamma1 = gamma - 1.0;
             if constexpr (PERT) {
                 // p - p_bar = (gamma-1) (E' - kinetic energy), p_bar = (gamma-1) E_bar
-                ppa = (ga - 1.0) * (ppa - 0.5 * (qa[1] * qa[1] + qa[2] * qa[2] + qa[3] * qa[3]) * iqa);
-                ppb = (gb - 1.0) * (ppb - 0.5 * (qb[1] * qb[1] + qb[2] * qb[2] + qb[3] * qb[3]) * iqb);
+                ppa = (ga - 1.0) * (ppa - 0.5 * quot(qa[1] * qa[1] + qa[2] * qa[2] + qa[3] * qa[3], qa[0], iqa));
+                ppb = (gb - 1.0) * (ppb - 0.5 * quot(qb[1] * qb[1] + qb[2] * qb[2] + qb[3] * qb[3], qb[0], iqb));
             }
             const double pl = pressure_nc(ga, qa[4], qa[1], qa[2], qa[3], iqa);
             const double pr = pressure_nc(gb, qb[4], qb[1], qb[2], qb[3], iqb);
@@ -324,7 +324,7 @@ __device__ __forceinline__ void tile_sweep_body(const SweepArgsT<T> &A, int bt, 
             double ia;
             root_rcp<RF>(a2, R.a, ia);
             R.i2a = 0.5 * ia;
-            R.g1a2 = gamma1 * (ia * ia);
+            R.g1a2 = quot(gamma1, a2, ia * ia);
             R.euv = R.enth - R.u2v2w2;
             const double ur = qb[1] * iqb, ul = qa[1] * iqa;
             const double d1 = qb[1] - qa[1];
