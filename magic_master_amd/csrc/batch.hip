@@ -517,7 +517,11 @@ static int build_lists(magic_batch *b, bool tuning = false)
     const size_t total = items.size();
     hipFree(b->items_d);
     b->items_d = nullptr;
-    HIPCHECK(hipMalloc(&b->items_d, (total ? total : 1) * sizeof(int4)));
+    if (hipMalloc(&b->items_d, (total ? total : 1) * sizeof(int4)) != hipSuccess) {
+        (void)hipGetLastError();
+        b->items_d = nullptr;
+        return MAGIC_ENOMEM;
+    }
     HIPCHECK(hipMemcpyAsync(b->items_d, items.data(), total * sizeof(int4), hipMemcpyHostToDevice, b->stream));
     HIPCHECK(hipMemcpyAsync(b->args_d, args.data(), args.size() * sizeof(args[0]), hipMemcpyHostToDevice, b->stream));
     HIPCHECK(hipMemcpyAsync(b->run_d, run.data(), run.size() * sizeof(run[0]), hipMemcpyHostToDevice, b->stream));

@@ -196,3 +196,35 @@ def test_no_room_beside_the_grid(host):
     b.run(1, 1)
     b.close()
     """)
+
+
+@pytest.mark.parametrize("batch", [False, True])
+def test_lists_without_room(host, batch):
+    """Where the blocks' lists find no room the call ends with MAGIC_ENOMEM,
+    and the next one, with room again, goes on."""
+    host(f"""
+    c, p, g, aux, q = perturbed(60, 30, 30, [1, 1, 1, 1, 3, 1])
+    def grid():
+        if not {batch}:
+            d = MagicHIP(g, p, aux, q)
+            return d, lambda: d.step3(1.0)
+        b = MagicBatch([g], [p], [aux[:, 0, 0, :].copy()], [q], form=FORM_FP64)
+        b.start(0, 0.0, 1e9, 1.0, c.dtv, c.cflv, 5, c.mthbc)
+        return b, lambda: b.run(1, 1)
+    d, step = grid()
+    before = stub.stub_used()
+    step()
+    whole = stub.stub_used() - before
+    d.close()
+    for miss in (1 << 9, 1 << 12):           # the lists take 20 KB, the last allocation of all
+        d, step = grid()
+        stub.stub_room(stub.stub_used() + whole - miss)
+        try:
+            step()
+            raise SystemExit("no error")
+        except MagicError as e:
+            assert e.code == 7, e
+        stub.stub_room(1 << 60)
+        step()
+        d.close()
+    """)
