@@ -271,9 +271,9 @@ int magic_batch_tune(magic_batch *b, int reps, int shapes_out[3], float *ms_out)
  * grid's if that is more); grids that do not fit are swept in slabs.  Captures
  * the graph again. */
 int magic_batch_set_increment_room(magic_batch *b, size_t bytes);
-/* As magic_set_sweep_overlap: accepted, without effect on the result.  A
- * scenario equals the same grid stepped alone bit for bit when both use the
- * same tile shapes.  Setting it captures the graph again. */
+/* As magic_set_sweep_overlap: accepted, without effect.  A scenario equals
+ * the same grid stepped alone bit for bit when both use the same tile
+ * shapes. */
 int magic_batch_set_sweep_overlap(magic_batch *b, int on);
 
 #ifdef __cplusplus

@@ -71,7 +71,6 @@ struct magic_batch {
     int ndtr_cap = 0, ndtrc_cap = 0;     // substep loops of the captured attempt
     int ncu = 0;                         // compute units
     int opgrid[NOP] = {0};               // persistent grid of each kernel class
-    bool overlap = false;                // accepted for the ABI; the order of the sums does not depend on it
     hipGraph_t graph = nullptr;
     hipGraphExec_t exec = nullptr;
     bool dirty = true;                   // control blocks changed on the host
@@ -989,13 +988,7 @@ extern "C" int magic_batch_set_increment_room(magic_batch *b, size_t bytes)
     return MAGIC_OK;
 }
 
-extern "C" int magic_batch_set_sweep_overlap(magic_batch *b, int on)
-{
-    if (!b) return MAGIC_EARG;
-    b->overlap = on != 0;
-    b->graph_ok = false;
-    return MAGIC_OK;
-}
+extern "C" int magic_batch_set_sweep_overlap(magic_batch *b, int) { return b ? MAGIC_OK : MAGIC_EARG; }
 
 extern "C" int magic_batch_get_tile_shapes(magic_batch *b, int shapes[3])
 {

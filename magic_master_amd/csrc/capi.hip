@@ -1111,12 +1111,7 @@ extern "C" int magic_set_increment_room(magic_ctx *c, size_t bytes)
     return MAGIC_OK;
 }
 
-extern "C" int magic_set_sweep_overlap(magic_ctx *c, int on)
-{
-    if (!c) return MAGIC_EARG;
-    c->overlap = on != 0;
-    return MAGIC_OK;
-}
+extern "C" int magic_set_sweep_overlap(magic_ctx *c, int) { return c ? MAGIC_OK : MAGIC_EARG; }
 
 // Autotuner: every tile shape of every sweep direction is timed on this
 // grid's current state (one untimed sweep, then reps timed ones, HIP events

@@ -88,7 +88,6 @@ struct magic_ctx {
     bool pending_parts = false;
     StepParts<double> parts64;   // the last sweeps' increments, by form
     StepParts<float> parts32;
-    bool overlap = true;   // accepted for the ABI; the sweeps of a step are one launch
     // Asynchronous snapshots (magic_snapshot_begin): the conversion into
     // stage runs on the context's stream, the copy out of stage on cstream
     // (created on first use), so that later work on the stream need not

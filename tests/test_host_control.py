@@ -228,3 +228,18 @@ def test_lists_without_room(host, batch):
         step()
         d.close()
     """)
+
+
+def test_sweep_overlap_setting_keeps_the_graph(host):
+    """The setting that has no effect does not make a batch capture again."""
+    host("""
+    c, p, g, aux, q = perturbed(12, 10, 8, [1, 1, 1, 1, 3, 1])
+    b = MagicBatch([g], [p], [aux[:, 0, 0, :].copy()], [q], form=FORM_FP64)
+    b.start(0, 0.0, 1e9, 1.0, c.dtv, c.cflv, 5, c.mthbc)
+    b.run(1, 1)
+    assert launches()
+    for on in (True, False):
+        b.set_sweep_overlap(on)
+        b.run(1, 1)
+        assert not launches()
+    """)
