@@ -175,8 +175,6 @@ template <class G>
 __global__ void k32_src_convert(Dims d, const float *qin, float *q, Col32 col, G gate, StepParts<float> sp);
 template <class G>
 __global__ void k32_src_finish(Dims d, float *q, const float *t5, int nc, Col32 col, Forcing f, G gate);
-template <typename T, class G>
-__global__ void k_copy(T *dst, const T *src, long long n, G gate);
 __global__ void k32_aos_to_pert(Dims d, float *q, const double *aos, int nc, const double *bgrho,
                                 const double *bgE);
 __global__ void k32_pert_to_aos(Dims d, double *aos, const float *q, int nc, const double *bgrho,

@@ -33,7 +33,6 @@ struct SweepArgsT {
     double dtdn, fg, fh;               // dt/dn, dt/dg, dt/dh
     unsigned long long *cfl_bits;      // running max of the Courant number
     int *status;                       // [0] code, [1..4] sweep,i,j,k of first failure
-    int i0, j0, k0;                    // Fortran index of (cell 0 along n, a = 0, b = 0) mapping helpers
     // perturbation form only: background columns indexed by k + mbc - 1
     // (rho_bar, E_bar, gamma, aux17, and the background's own z jump
     // p_bar(k) - p_bar(k-1) - .5 (rho_bar(k) + rho_bar(k-1)) aux17(k))
@@ -60,7 +59,6 @@ __global__ void sweep_kernel(SweepArgs a);
 constexpr int TILE_NSHAPE = 4;
 __host__ __device__ constexpr int tile_ta(int sh) { return sh == 0 ? 16 : sh == 3 ? 4 : 8; }
 __host__ __device__ constexpr int tile_lgta(int sh) { return sh == 0 ? 4 : sh == 3 ? 2 : 3; }
-__host__ __device__ constexpr bool tile_pm(int sh) { return sh >= 2; }
 // cells along the pencil a chunk completes, and positions of a part's plane
 __host__ __device__ constexpr int tile_ci(int sh) { return 256 / tile_ta(sh) - 2; }
 __host__ __device__ constexpr int part_npos(int sh) { return (tile_ta(sh) + 2) * (tile_ci(sh) + 1); }

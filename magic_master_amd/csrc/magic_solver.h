@@ -1,8 +1,10 @@
-// Per-interface solver math shared by the sweep kernels: Roe state,
-// limiters, transverse splits and the 9-point increment accumulator, for a
+// Per-interface solver math of the sweep kernels: Roe state, limiters,
+// transverse splits and the 9-point increment accumulator, for a
 // floating-point type T (double: the FP64 form; float: the FP32 perturbation
-// form).  Constants are written as T(...) so that the double instantiation
-// performs exactly the reference's operations.
+// form).  What the pencil kernel uses (cflsupbee, suppow, tsplit, Acc) performs
+// exactly the reference's operations.  The tiled sweep's own (rcp1, quot,
+// root_rcp, one_minus_pow, LimT, suppow1, WaveT) round otherwise, within the
+// errors stated at each.
 #pragma once
 #include "magic_dev.h"
 
@@ -40,32 +42,18 @@ __device__ __forceinline__ T gravity_jump_nc(T d, T ra, T rb, T vg)
     return d - T(0.5) * (rb + ra) * vg;
 }
 
-// Reciprocal and square root of the Riemann solver's densities, sound
-// speeds and wave speeds: correctly rounded in FP64 (as the reference); in
-// the FP32 form, whose error bar is a fraction of the field peak, the
-// hardware's single-instruction approximations (about one unit in the last
-// place).  Never used for a ratio of two quantities that can both be tiny.
-template <typename T>
-__device__ __forceinline__ T rcpT(T x) { return T(1.0) / x; }
-template <>
-__device__ __forceinline__ float rcpT<float>(float x) { return __builtin_amdgcn_rcpf(x); }
-template <typename T>
-__device__ __forceinline__ T sqrtT(T x) { return sqrt(x); }
-template <>
-__device__ __forceinline__ float sqrtT<float>(float x) { return __builtin_amdgcn_sqrtf(x); }
-
 // The FP32 form solves the normal Riemann problem in FP64 (the sweep's
 // part 1): its jumps and wave strengths subtract background-sized products
 // (enthalpy times velocity, enthalpy times the density jump), whose FP32
 // rounding the flow carries up into the thin upper layers; in FP32 the
 // form's temperature error there grew to 3e-4 of the field peak in 300
-// steps, in FP64 to 3e-5-6e-5.  Its reciprocals and square roots need not
-// be correctly rounded there: the hardware's FP64 approximations refined by
-// one Newton step (relative error near 1e-15, far inside that form's error
-// bar).  RF selects them (true: the FP32 form) over the operations of the
-// FP64 form: one third-order step from the hardware's 2**-24 (largest error
-// over 5e8 arguments 1.0 x 2**-53, as two Newton steps have, in three
-// operations for their four).
+// steps, in FP64 to 3e-5-6e-5.  Its reciprocals and square roots are the
+// hardware's FP64 approximations refined by one Newton step (relative error
+// near 1e-14, far inside that form's error bar).  RF selects them (true: the
+// FP32 form) over those of the FP64 form: one third-order step from the
+// hardware's 2**-24 (largest error over 5e8 arguments 1.0 x 2**-53, the bound of
+// a correctly rounded quotient, as two Newton steps have, in three operations
+// for their four).  Quotients are corrected by their remainder (quot).
 template <bool RF>
 __device__ __forceinline__ double rcp1(double x)
 {
@@ -138,15 +126,6 @@ __device__ __forceinline__ double fmaxT(double a, double b) { return __builtin_f
 __device__ __forceinline__ float fminT(float a, float b) { return __builtin_fminf(a, b); }
 __device__ __forceinline__ float fmaxT(float a, float b) { return __builtin_fmaxf(a, b); }
 
-// x**y for 0 <= x < 1, y > 0 (suppow's rfrac**pp): the library pow in FP64;
-// in the FP32 form 2**(y log2 x) from the hardware's exp2 and log2
-// (log2 0 = -inf gives 0, as pow does).
-__device__ __forceinline__ double powT(double x, double y) { return pow(x, y); }
-__device__ __forceinline__ float powT(float x, float y)
-{
-    return __builtin_amdgcn_exp2f(y * __builtin_amdgcn_logf(x));
-}
-
 // 1 - x**p for 0 <= x <= 1, p > 0 (suppow's 1 - rfrac**pp).  FP64: ln x from
 // the odd series of ln((1+s)/(1-s)) with x = m 2**k, sqrt(1/2) <= m <
 // sqrt(2), s = (m-1)/(m+1), and -expm1(p ln x) from the Taylor series of the
@@ -202,47 +181,41 @@ __device__ __forceinline__ double one_minus_pow(double x, double p)
     const double sc = __builtin_ldexp(1.0, (int)n);
     return fma(-sc, em1, 1.0 - sc);
 }
-__device__ __forceinline__ float one_minus_pow(float x, float p) { return 1.0f - powT(x, p); }
+// FP32 form: 2**(p log2 x) from the hardware's exp2 and log2 (log2 0 = -inf
+// gives 0, as pow does)
+__device__ __forceinline__ float one_minus_pow(float x, float p)
+{
+    return 1.0f - __builtin_amdgcn_exp2f(p * __builtin_amdgcn_logf(x));
+}
 
 // rpn3euX.f:686-705
-template <typename T>
-__device__ __forceinline__ T cflsupbee(T theta, T beta, T r, T cfl, T cflup)
+__device__ __forceinline__ double cflsupbee(double theta, double beta, double r, double cfl, double cflup)
 {
-    T cfle = fmaxF(T(0.001), fminF(T(0.999), cfl));
-    T cflupe = fmaxF(T(0.001), fminF(T(0.999), cflup));
+    const double cfle = fmaxF(0.001, fminF(0.999, cfl)), cflupe = fmaxF(0.001, fminF(0.999, cflup));
     // cfle is clamped to [0.001, 0.999]: its reciprocals are taken once
-    const T i1mc = rcpT(T(1.0) - cfle), icfle = rcpT(cfle);
-    T weight = (T(1.0) - cflupe) * i1mc;
-    T s1 = theta * weight * T(2.0) * icfle;
-    T s2 = (T(1.0) + cfle) * (T(1.0) / T(3.0));
-    T phimax = theta * T(2.0) * i1mc;
-    T ultra = fmaxF(T(0.0), fminF(s1 * r, phimax));
-    T c1 = T(1.0) + (s2 - beta / T(2.0)) * (r - T(1.0));
-    T c2 = T(1.0) + (s2 + beta / T(2.0)) * (r - T(1.0));
-    return fmaxF(T(0.0), fminF(ultra, fmaxF(c1, c2)));
+    const double i1mc = 1.0 / (1.0 - cfle), icfle = 1.0 / cfle;
+    const double weight = (1.0 - cflupe) * i1mc;
+    const double s1 = theta * weight * 2.0 * icfle;
+    const double s2 = (1.0 + cfle) * (1.0 / 3.0);
+    const double phimax = theta * 2.0 * i1mc;
+    const double ultra = fmaxF(0.0, fminF(s1 * r, phimax));
+    const double c1 = 1.0 + (s2 - beta / 2.0) * (r - 1.0);
+    const double c2 = 1.0 + (s2 + beta / 2.0) * (r - 1.0);
+    return fmaxF(0.0, fminF(ultra, fmaxF(c1, c2)));
 }
 
 // rpn3euX.f:709-731
-template <typename T>
-__device__ __forceinline__ T suppow(T r, T cfl, T cflup)
+__device__ __forceinline__ double suppow(double r, double cfl, double cflup)
 {
-    if constexpr (sizeof(T) == 4) {
-        // FP32: a denormal wave strength can make the ratio r overflow to
-        // +-inf, and (1-|r|)/(1+|r|) is then NaN.  For |r| >= 1e30 the
-        // result is already 0 in both precisions (rfrac rounds to 1).
-        r = fminF(fmaxF(r, T(-1e30)), T(1e30));
-    }
-    T cfle = fmaxF(T(0.001), fminF(T(0.999), cfl));
-    T cflupe = fmaxF(T(0.001), fminF(T(0.999), cflup));
-    const T i1mc = rcpT(T(1.0) - cfle), icfle = rcpT(cfle);
-    T s2 = (T(1.0) + cfle) * (T(1.0) / T(3.0));
-    T s3 = T(1.0) - s2;
-    T weight = (T(1.0) - cflupe) * i1mc;
-    T pp = (r <= T(1.0)) ? weight * (T(2.0) * icfle) * T(2.0) * s3 : fabs(T(2.0) * i1mc) * T(2.0) * s2;
-    T rabs = fabs(r);
-    T rfrac = fabs((T(1.0) - rabs) * rcpT(T(1.0) + rabs));
-    T signum = fmaxF(T(0.0), copysign(T(1.0), r));
-    return signum * (s3 + s2 * r) * (T(1.0) - powT(rfrac, pp));
+    const double cfle = fmaxF(0.001, fminF(0.999, cfl)), cflupe = fmaxF(0.001, fminF(0.999, cflup));
+    const double i1mc = 1.0 / (1.0 - cfle), icfle = 1.0 / cfle;
+    const double s2 = (1.0 + cfle) * (1.0 / 3.0), s3 = 1.0 - s2;
+    const double weight = (1.0 - cflupe) * i1mc;
+    const double pp = (r <= 1.0) ? weight * (2.0 * icfle) * 2.0 * s3 : fabs(2.0 * i1mc) * 2.0 * s2;
+    const double rabs = fabs(r);
+    const double rfrac = fabs((1.0 - rabs) * (1.0 / (1.0 + rabs)));
+    const double signum = fmaxF(0.0, copysign(1.0, r));
+    return signum * (s3 + s2 * r) * (1.0 - pow(rfrac, pp));
 }
 
 // The limiters of one interface's waves that move at one speed: with the

@@ -452,10 +452,5 @@ __device__ __forceinline__ void b_copy(const uint3 BI, unsigned nblk, T *dst, co
          e += (long long)nblk * blockDim.x)
         dst[e] = src[e];
 }
-template <typename T, class G>
-__global__ void k_copy(T *dst, const T *src, long long n, G gate)
-{
-    b_copy(uint3{blockIdx.x, blockIdx.y, blockIdx.z}, gridDim.x, dst, src, n, gate);
-}
 
 }  // namespace magic
