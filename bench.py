@@ -37,12 +37,12 @@ HBM_PEAK_GBS = 8000.0
 # operations per cell-update of a step's sweeps, counted on the full-domain
 # workload with rocprofv3 (SQ_INSTS_VALU_{ADD,MUL,FMA,TRANS} of each
 # precision, times 64 lanes, an FMA counted twice; lanes masked off at grid
-# edges and the chunks' 2-interface overlap included): FP64 form 6.31 k FP64;
-# FP32 form 4.65 k FP32 + 1.25 k FP64.  MI355X vector peak (non-matrix) is 78.6
+# edges and the chunks' 2-interface overlap included): FP64 form 6.32 k FP64;
+# FP32 form 4.65 k FP32 + 1.38 k FP64.  MI355X vector peak (non-matrix) is 78.6
 # TFLOP/s for FP64, and for FP32 too without packed (two-wide) FP32
 # instructions, which this library does not use; the 157.3 TFLOP/s FP32 peak
 # counts them.
-FLOP_PER_CELL_UPDATE = {"fp64": 6.31e3, "fp32": 4.65e3 + 1.25e3}
+FLOP_PER_CELL_UPDATE = {"fp64": 6.32e3, "fp32": 4.65e3 + 1.38e3}
 VECTOR_PEAK_TFLOPS = {"fp64": 78.6, "fp32": 78.6}
 # Algorithmic bytes per cell-update at meqn = 6.  Hyperbolic pass: read q,
 # write q (2 x 48 B) + aux(17), aux(19) (16 B), shared evenly by the three

@@ -74,8 +74,8 @@ __global__ void k_bc_z(Dims d, double *q, int nc, int lo, int hi, const double *
 // read from qin and written to q: one grid hands over its two state buffers,
 // so that the state before the step stays behind as copyq3's backup without
 // a copy; a batch works in place (qin = q) and writes that state to keep.
-// Against adding a finished increment buffer this pass reads up to 1.36
-// times the increments, but they were written once and never added to.
+// Against adding a finished increment buffer this pass reads the blocks' edges
+// too (parts.h), but they were written once and never added to.
 template <bool COL, class G>
 __device__ __forceinline__ void b_src_convert(const uint3 BI, Dims d, const double *qin, double *q, double *keep, const Aux a,
                                               const G &gate, const StepParts<double> &sp)

@@ -2,12 +2,16 @@
 // its entry of every block that holds one, the directions in the order x, y,
 // z and the blocks of a direction in a fixed order, so the sum does not
 // depend on which workgroup wrote first.  Bound by memory: a block's planes
-// are read once (plus the neighbours' edge entries, up to 36 % at 16 planes
-// per segment), in runs along x, with one lane per cell and no branch between
-// a direction's loads.  The source pass's conversion with this in it takes
-// 1.01 ms on the full domain (250 x 200 x 300, FP64: 4.6 GB, 4.6 TB/s, what a
-// large copy reaches), 0.30 ms in FP32 on 181 x 160 x 243; with the parts in
-// the tiles' lane order and a branch per neighbour it took 1.59 and 0.48.
+// are read once, in runs along x, with one lane per cell and no branch between
+// a direction's loads.  With L planes per segment, TA pencils and CI cells a
+// direction holds (L + 2) / L x (TA + 2) / TA x (CI + 1) / CI times q, and more
+// where the grid does not fill its last blocks: the three directions 3.9 to
+// 4.5 times q on large grids, 6 on 64 x 64 x 48, 10 to 16 on grids of 10 to 20
+// cells.  The source pass's conversion with this in it takes 0.97 ms on the full
+// domain (250 x 200 x 300, FP64): it moves 6.2 GB, 6.4 TB/s, some of it still in
+// the last-level cache (a copy of 6 GB runs at 4.9 TB/s); 0.30 ms in FP32 on 181
+// x 160 x 243.  With the parts in the tiles' lane order and a branch per
+// neighbour it took 1.59 and 0.48.
 #pragma once
 #include "bc_src.h"
 #include "magic_dev.h"

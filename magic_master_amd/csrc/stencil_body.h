@@ -10,7 +10,8 @@
 #pragma once
 #include "bc_src.h"
 
-// Every kernel below takes a gate G: GridGate (factors as passed) for one grid; the batched driver passes a gate that reads its scenario's
+// Every kernel below takes a gate G: GridGate (factors as passed) for one
+// grid; the batched driver passes a gate that reads its scenario's
 // step-control block on the device (skip when the scenario is idle in this
 // stage, factors that depend on the scenario's dt).
 

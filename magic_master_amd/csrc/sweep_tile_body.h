@@ -409,6 +409,11 @@ __device__ __forceinline__ void tile_sweep_body(const SweepArgsT<T> &A, int bt, 
         // contact): then every interface says what it assigned; and the
         // earlier chunks are solved again, from the nearest back, until every
         // pencil of the tile has met an assignment, and this chunk once more.
+        // A block that marched along the pencil would carry the value for
+        // nothing; here a sheared sheet across 250 x 200 x 300 cells (FP64, 4
+        // interfaces) costs 10 % of the three sweeps (3.25 -> 3.57 ms), shear at
+        // every interface of the x-sweep without any assignment, the worst case,
+        // 7.5 ms.
         if (s_need == 0) break;
         s_flag[t] = (act1 && c <= CH - 2 && I >= 1 && I <= n + 1 && (b1 != 0.0 || b2 != 0.0 || b5 != 0.0)) ? 1 : 0;
         s_cfo[t] = b5 != 0.0 ? c3 : (b2 != 0.0 ? c2 : c1);
@@ -486,6 +491,9 @@ __device__ __forceinline__ void tile_sweep_body(const SweepArgsT<T> &A, int bt, 
                 }
                 wt = lim2.weight(cflup);
             }
+            // Whether a shear strength vanishes is asked of the strength itself;
+            // the reference asks what is left of it in the wave's momentum,
+            // (b2 + v b4) - v b4, which rounding can make zero or not.
             // A vanishing wave needs no case of its own: the limiters are
             // finite for any ratio, NaN among them, and multiply a strength
             // of zero.

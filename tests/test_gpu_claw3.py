@@ -49,3 +49,30 @@ def test_many_substeps(form, substeps, dt):
         assert np.isfinite(got[interior(g)]).all()
     finally:
         d.close()
+
+
+@pytest.mark.parametrize("form", ["fp32", "fp64"])
+def test_sweep_overlap_setting_changes_nothing(form):
+    """set_sweep_overlap on and off: the same state, dt and t, bit for bit, on
+    one grid and in a batch."""
+    from magic_master_amd.hip import FORM_FP32P, FORM_FP64, MagicBatch, MagicHIP
+    fm = FORM_FP32P if form == "fp32" else FORM_FP64
+    c, p, g, aux, q = perturbed(33, 20, 18, [2, 2, 1, 1, 3, 1], seed=3, vel=0.05, visc=1.0)
+    out = []
+    for on in (True, False):
+        d = MagicHIP(g, p, aux, q, form=fm)
+        b = MagicBatch([g], [p], [aux[:, 0, 0, :].copy()], [q], form=fm)
+        try:
+            d.set_sweep_overlap(on)
+            b.set_sweep_overlap(on)
+            t, dtv, log = d.run_steps(c, 3, dt0=50.0)
+            b.start(0, 0.0, 1e9, 50.0, c.dtv, c.cflv, 3, c.mthbc)
+            b.run()
+            st = b.state(0)
+            out += [(t, dtv[4], d.get_q()), (st["t"], st["dt"], b.get_q(0))]
+        finally:
+            d.close()
+            b.close()
+    for o in out[1:]:
+        assert o[:2] == out[0][:2]
+        np.testing.assert_array_equal(o[2], out[0][2])
