@@ -420,10 +420,11 @@ static int build_groups(magic_batch *b)
     for (int s = 0; s < b->n; s++) {
         if (!b->sc[s]) continue;
         if (!roomy || stage_bytes(b->sc[s]) > stage_bytes(roomy)) roomy = b->sc[s];
-        need[s] = whole_bytes<T>(b->sc[s], b->shape);
+        const Slabs<T> slabs(b->sc[s], b->shape);
+        need[s] = slabs.whole();
         sum += need[s];
         big = std::max(big, need[s]);
-        least = std::max(least, least_bytes<T>(b->sc[s], b->shape));
+        least = std::max(least, slabs.least());
     }
     const size_t want = b->parts_room ? std::min(sum, std::max(least, b->parts_room)) : std::max(big, std::min(sum, PARTS_BYTES));
     if (b->parts_bytes < want) {
@@ -451,7 +452,7 @@ static int build_groups(magic_batch *b)
     for (int s = 0; s < b->n; s++) {
         magic_batch::Group g = {s, s + 1, {0, 0, 0, 0}};
         if (need[s] > b->parts_bytes) {
-            b->slabs[s] = slabs_for<T>(b->sc[s], b->shape, b->parts_bytes);
+            b->slabs[s] = Slabs<T>(b->sc[s], b->shape).within(b->parts_bytes);
             g.nslab = (int)b->slabs[s].size();
             for (g.slab = 0; g.slab < g.nslab; g.slab++) b->groups.push_back(g);
             continue;

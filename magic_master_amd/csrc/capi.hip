@@ -818,8 +818,8 @@ static int sweep_setup(magic_ctx *c)
     HIPCHECK(hipStreamSynchronize(c->stream));   // nothing reads the old lists or increments any more
     hipFree(c->items);
     c->items = nullptr;
-    const size_t least = least_bytes<T>(c, c->shape);
-    const size_t want = std::min(whole_bytes<T>(c, c->shape), std::max(least, c->parts_room));
+    const Slabs<T> slabs(c, c->shape);
+    const size_t least = slabs.least(), want = std::min(slabs.whole(), std::max(least, c->parts_room));
     if (c->parts_bytes < want) {
         drop_parts(c);
         size_t got = want;   // less room: narrower slabs, at last in the staging buffer, idle in a step
@@ -837,15 +837,12 @@ static int sweep_setup(magic_ctx *c)
         }
         c->parts_bytes = got;
     }
-    c->slabs = slabs_for<T>(c, c->shape, c->parts_bytes);
+    c->slabs = slabs.within(c->parts_bytes);
     std::vector<int4> items;
     c->item_off.assign(1, 0);
     for (const Slab &slab : c->slabs)
         for (int dir = 0; dir < 3; dir++) {
-            SweepArgsT<T> a;
-            SweepParts<T> p;
-            sweep_geometry(c, dir, c->shape[dir], a, p);
-            push_items(items, p, dir, slab.lo[dir], slab.hi[dir], dir);
+            push_items(items, slabs.p[dir], dir, slab.lo[dir], slab.hi[dir], dir);
             c->item_off.push_back((int)items.size());
         }
     if (hipMalloc(&c->items, items.size() * sizeof(int4)) != hipSuccess) {

@@ -396,59 +396,73 @@ static inline void slab_blocks(const SweepParts<T> &p, int dir, int i0, int i1, 
     }
 }
 
-// Slabs w cells wide of a grid's sweeps in shapes sh; bytes returns what the
-// largest one's increments take, all three directions
-template <typename T>
-static inline std::vector<Slab> cut_slabs(const magic_ctx *c, const int *sh, int w, size_t &bytes)
-{
-    std::vector<Slab> out;
-    bytes = 0;
-    for (int x = 0; x < c->mx + 2; x += w) {
-        Slab s;
-        s.i0 = x == 0 ? 1 - c->mbc : x;
-        s.i1 = x + w < c->mx + 2 ? x + w : c->mx + c->mbc + 1;
-        long long n = 0;
-        for (int dir = 0; dir < 3; dir++) {
-            SweepArgsT<T> a;
-            SweepParts<T> p;
-            sweep_geometry(c, dir, sh[dir], a, p);
-            slab_blocks(p, dir, s.i0, s.i1, s.lo[dir], s.hi[dir]);
-            n += block_size(p, c->meqn, sh[dir]) * (s.hi[dir] - s.lo[dir]) * (dir == 0 ? p.nt : p.nk) * p.ns;
-        }
-        bytes = std::max(bytes, (size_t)n * sizeof(T));
-        out.push_back(s);
-    }
-    return out;
-}
-// What the increments of a whole grid take, and those of its narrowest slabs.
-// A slab sweeps every block that holds entries of its cells, so each cell's
-// sum is whole and in its one order; slabs share the blocks at their borders,
-// which are swept twice: 16 cells wide, about three times the work.
+// Slabs of a grid's sweeps in shapes sh.  A slab sweeps every block that holds
+// entries of its cells, so each cell's sum is whole and in its one order; slabs
+// share the blocks at their borders, which are swept twice: 16 cells wide, about
+// three times the work.
 constexpr int SLAB_MIN = 16;
 template <typename T>
-static inline size_t whole_bytes(const magic_ctx *c, const int *sh)
-{
-    size_t n;
-    cut_slabs<T>(c, sh, c->mx + 2, n);
-    return n;
-}
-template <typename T>
-static inline size_t least_bytes(const magic_ctx *c, const int *sh)
-{
-    size_t n;
-    cut_slabs<T>(c, sh, SLAB_MIN, n);
-    return n;
-}
-// The widest slabs whose increments take at most room bytes (at least
-// least_bytes)
-template <typename T>
-static inline std::vector<Slab> slabs_for(const magic_ctx *c, const int *sh, size_t room)
-{
-    size_t n;
-    std::vector<Slab> s = cut_slabs<T>(c, sh, c->mx + 2, n);
-    for (int w = (c->mx + 1) / SLAB_MIN * SLAB_MIN; n > room && w >= SLAB_MIN; w -= SLAB_MIN) s = cut_slabs<T>(c, sh, w, n);
-    return s;
-}
+struct Slabs {
+    int mx, mbc;
+    SweepParts<T> p[3];
+    long long row[3];   // bytes of the blocks at one place along x
+    Slabs(const magic_ctx *c, const int *sh) : mx(c->mx), mbc(c->mbc)
+    {
+        for (int dir = 0; dir < 3; dir++) {
+            SweepArgsT<T> a;
+            sweep_geometry(c, dir, sh[dir], a, p[dir]);
+            row[dir] = block_size(p[dir], c->meqn, sh[dir]) * (dir == 0 ? p[dir].nt : p[dir].nk) * p[dir].ns * (long long)sizeof(T);
+        }
+    }
+    // the slab of the cells x .. x+w-1 and what its increments take
+    Slab at(int x, int w, size_t &bytes) const
+    {
+        Slab s;
+        s.i0 = x == 0 ? 1 - mbc : x;
+        s.i1 = x + w < mx + 2 ? x + w : mx + mbc + 1;
+        bytes = 0;
+        for (int dir = 0; dir < 3; dir++) {
+            slab_blocks(p[dir], dir, s.i0, s.i1, s.lo[dir], s.hi[dir]);
+            bytes += (size_t)(row[dir] * (s.hi[dir] - s.lo[dir]));
+        }
+        return s;
+    }
+    // slabs w cells wide; bytes: of the largest
+    std::vector<Slab> cut(int w, size_t &bytes) const
+    {
+        std::vector<Slab> out;
+        bytes = 0;
+        for (int x = 0; x < mx + 2; x += w) {
+            size_t n;
+            out.push_back(at(x, w, n));
+            bytes = std::max(bytes, n);
+        }
+        return out;
+    }
+    size_t whole() const   // what the increments of the whole grid take
+    {
+        size_t n;
+        at(0, mx + 2, n);
+        return n;
+    }
+    size_t least() const   // and those of the narrowest slabs
+    {
+        size_t n, most = 0;
+        for (int x = 0; x < mx + 2; x += SLAB_MIN) {
+            at(x, SLAB_MIN, n);
+            most = std::max(most, n);
+        }
+        return most;
+    }
+    // the widest slabs whose increments take at most room bytes (least() at the least)
+    std::vector<Slab> within(size_t room) const
+    {
+        size_t n;
+        std::vector<Slab> s = cut(mx + 2, n);
+        for (int w = (mx + 1) / SLAB_MIN * SLAB_MIN; n > room && w >= SLAB_MIN; w -= SLAB_MIN) s = cut(w, n);
+        return s;
+    }
+};
 
 // capi.hip
 int tune_state(magic_ctx *c), tune_done(magic_ctx *c);

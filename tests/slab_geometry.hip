@@ -12,7 +12,7 @@ extern "C" int slab_table(const int *dims, int meqn, const int *sh, int w, long 
     c.d.NX = c.mx + 2 * c.mbc; c.d.NY = c.my + 2 * c.mbc; c.d.NZ = c.mz + 2 * c.mbc;
     c.P = c.d.P = (long long)c.d.NX * c.d.NY * c.d.NZ;
     size_t bytes;
-    const std::vector<Slab> slabs = cut_slabs<double>(&c, sh, w ? w : c.mx + 2, bytes);
+    const std::vector<Slab> slabs = Slabs<double>(&c, sh).cut(w ? w : c.mx + 2, bytes);
     long long *o = out;
     for (size_t s = 0; s < slabs.size() && (int)s < maxslab; s++) {
         double *const buf = (double *)(size_t(1) << 40), *next = buf;
