@@ -205,10 +205,11 @@ int magic_set_sweep_overlap(magic_ctx *ctx, int on);
  * it cannot hold the whole grid's, the grid is swept in slabs, narrow enough
  * along x for it, one after the other: slower, with the same result bit for
  * bit.  A context takes the whole grid's size or, where the device has less,
- * what there is, and fails with MAGIC_ENOMEM only where that is not enough for
- * slabs 16 cells wide.  magic_set_increment_room bounds the buffer to bytes
- * (or those narrowest slabs, if they take more; 0: no bound) and gives back
- * the one held. */
+ * what there is, at last the staging buffer of magic_set_q and magic_get_q; it
+ * fails with MAGIC_ENOMEM only where that cannot hold slabs 16 cells wide
+ * either (small grids; some MB).  magic_set_increment_room bounds the buffer to
+ * bytes (or those narrowest slabs, if they take more; 0: no bound) and gives
+ * back the one held. */
 int magic_set_increment_room(magic_ctx *ctx, size_t bytes);
 
 /* ---- Batched driver: many grids of one form advanced together ----------

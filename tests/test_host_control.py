@@ -38,7 +38,8 @@ def launches():
 """
 
     def run(script):
-        env = dict(os.environ, LD_PRELOAD=so, PYTHONPATH=ROOT)
+        preload = " ".join(filter(None, [so, os.environ.get("LD_PRELOAD")]))
+        env = dict(os.environ, LD_PRELOAD=preload, PYTHONPATH=ROOT)
         r = subprocess.run([sys.executable, "-c", head + textwrap.dedent(script)], env=env, cwd=ROOT,
                            stdout=subprocess.PIPE, stderr=subprocess.STDOUT, text=True, timeout=100)
         assert r.returncode == 0, r.stdout
