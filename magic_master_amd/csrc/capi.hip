@@ -1357,6 +1357,16 @@ extern "C" int magic_src3(magic_ctx *c, double t, double dt, const int mthbc[6],
 }
 
 // ------------------------------------------------------------ claw3 ------
+// No source pass, or not the whole of one, ran behind a conversion: the state
+// that it read is q again, the increments are still to be added, and its target
+// is the backup.
+static void take_back(magic_ctx *c)
+{
+    if (c->form == MAGIC_FORM_FP32P) std::swap(c->q32, c->qold32);
+    else std::swap(c->q, c->qold);
+    c->pending_parts = true;
+}
+
 extern "C" int magic_claw3(magic_ctx *c, double tstart, double *tend, double dtv[5], double cflv[4],
                            int nv[2], const int method[7], const int mthbc[6], double *log_dt,
                            double *log_cfl, int *log_acc, int maxlog, int *nlog)
@@ -1399,11 +1409,7 @@ extern "C" int magic_claw3(magic_ctx *c, double tstart, double *tend, double dtv
                 if (ss && ss != MAGIC_EHIP && (st = scal_copy(c))) goto out;
             }
             st = ss == MAGIC_EHIP ? ss : step3_finish(c, &cfl);
-            if (moved && (st || !(cfl <= cflv[0]))) {           // no (whole) source pass ran: its target is the backup again
-                if (c->form == MAGIC_FORM_FP32P) std::swap(c->q32, c->qold32);
-                else std::swap(c->q, c->qold);
-                c->pending_parts = true;
-            }
+            if (moved && (st || !(cfl <= cflv[0]))) take_back(c);
             if (st) goto out;
             t = told + dt;
             if (log_dt && nl < maxlog) {
@@ -1414,7 +1420,9 @@ extern "C" int magic_claw3(magic_ctx *c, double tstart, double *tend, double dtv
             nl++;
             if (cfl <= cflv[0]) {                                  // claw3_mpi.f:861-886
                 cflmax = cflmax > cfl ? cflmax : cfl;
+                const bool pending = c->pending_parts;
                 st = ahead ? ss : src3_launch(c, told, dt, mthbc, &a, &b);
+                if (st && pending && !c->pending_parts) take_back(c);
                 if (st) goto out;
                 break;
             }

@@ -46,12 +46,15 @@ def launches():
     return run
 
 
+@pytest.mark.parametrize("substeps", [1, 40])
 @pytest.mark.parametrize("cfl", [0.5, 1.9])   # the attempt would be accepted, or rejected
-def test_claw3_launch_failure_in_the_source_pass(host, cfl):
+def test_claw3_launch_failure_in_the_source_pass(host, cfl, substeps):
     """A launch that fails behind the source pass's conversion ends claw3 with
-    an error, on the state before the step (not on the older backup)."""
+    an error, on the state before the step (not on the older backup).  A long
+    source pass is launched only once its attempt is accepted."""
     host(f"""
     c, p, g, aux, q = perturbed(8, 7, 6, [1, 1, 1, 1, 3, 1])
+    aux[..., 10] = 0.75 * ({substeps} - 0.5) * 0.45 * min(g.dx, g.dy, g.dz) ** 2 / c.dtv[0]
     d = MagicHIP(g, p, aux, q)
     courant(0.5, {cfl}, 0.5)
     one = lambda: d.claw3(0.0, -1.0, c.dtv, c.cflv, [10, 0], c.method, c.mthbc)
