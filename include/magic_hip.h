@@ -253,7 +253,9 @@ int magic_batch_start(magic_batch *b, int s, double t, double tend, double dt, c
  * and HIP errors: a scenario that fails (MAGIC_ERHO, MAGIC_EA2, or
  * MAGIC_EUNSUPPORTED when its source pass needs more substeps than were
  * captured) stops with that status, which magic_batch_state reports, and
- * the other scenarios go on. */
+ * the other scenarios go on.  After MAGIC_ERHO or MAGIC_EA2 its q holds the
+ * failed step's increments and its backup the state before them, as
+ * magic_claw3 leaves a grid that fails. */
 int magic_batch_run(magic_batch *b, int max_attempts, int check_every, int *attempts_done);
 /* real_out: t, dt (next), cfl (last attempt), cflmax, tend;
  * int_out: accepted steps, attempts, rejected attempts, active, status, ndtr. */
